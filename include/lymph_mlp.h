@@ -64,7 +64,7 @@ int lymph_mlp_train(LymphMlp* net, int n_steps, int batch, const int32_t* order,
  * parameter gradients in the parameter layout. */
 int lymph_mlp_gradients(LymphMlp* net, int batch, const float* x, const float* y, float* grads,
                         float* loss);
-/* Forward pass of n inputs (any n; processed in batches of max_batch). */
+/* Forward pass of n inputs (any n). */
 int lymph_mlp_predict(LymphMlp* net, int n, const float* x, float* y);
 /* Device time of forward passes over the first n samples of the training
  * set (device-resident inputs), mean over reps, in ms. */

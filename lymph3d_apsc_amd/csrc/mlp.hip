@@ -12,7 +12,8 @@
 // the forward pass (X W^T), the input gradient (dZ W) and the weight
 // gradient (dZ^T X) without transposed copies.  Epilogues fuse bias + GELU
 // (forward, keeping the FP32 pre-activation) and the GELU derivative
-// (backward).
+// (backward).  Networks up to 512 wide take the fragment-order kernels further
+// down instead (k_slab, k_layer, k_update).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,6 +21,7 @@
 #include <cstdint>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/lymph_mlp.h"
@@ -29,6 +31,7 @@ namespace {
 typedef uint16_t bf16_t;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 thread_local std::string g_err;
 int fail(int code, std::string m) {
@@ -327,24 +330,491 @@ __global__ __launch_bounds__(256) void k_colsum(const bf16_t* __restrict__ D, in
   }
 }
 
+__global__ void k_to_bf16(const float* __restrict__ a, bf16_t* __restrict__ b, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) b[i] = f2bf(a[i]);
+}
+
+
+// ---------------------------------------------------------------------------
+// Networks whose layers are all at most kSlabW wide (the receiver network).
+//
+// Weights are kept in the order the matrix cores read them (pack_pos: W for
+// the forward pass, its columns for the input gradients), and so are the
+// activations and gradients between layers, so that one 16-byte load per lane
+// is a whole MFMA fragment and a wave's load is 1 KB in one piece: no LDS
+// staging, no transposes.  The products run over k in the same 32-wide steps,
+// in the same order, as k_gemm's: the same bits.
+constexpr int kSlabW = 512;       // widest layer: 8 waves x 4 tiles of 16 columns in one pass
+constexpr int kSlabL = 16;        // most layers
+constexpr int kSlabLd = kSlabW + 8;  // LDS row of activations: 16-byte reads of 8 rows in distinct banks
+
+// fragment order of a [R][C] matrix contracted over C: tile r / 16, step
+// c / 32, then lane (c % 32) / 8 * 16 + r % 16 holding c % 8; `steps` per tile
+__host__ __device__ inline size_t pack_pos(int r, int c, int steps) {
+  return ((size_t)(r >> 4) * steps + (c >> 5)) * 512 + ((((c >> 3) & 3) << 4) + (r & 15)) * 8 + (c & 7);
+}
+__host__ __device__ inline int steps_of(int c) { return (c + 31) >> 5; }
+__host__ __device__ inline int tiles_of(int r) { return (r + 15) >> 4; }
+// tiles per wave (8 waves), and the packed matrix' tiles: whole passes, so no
+// load needs a bound (the padding is zero)
+__host__ __device__ inline int tpw_of(int r) { return (tiles_of(r) + 7) >> 3; }
+__host__ __device__ inline size_t pack_size(int r, int c) { return (size_t)tpw_of(r) * 8 * steps_of(c) * 512; }
+
+struct SlabArgs {
+  int L, B;                 // layers, valid rows
+  int w[kSlabL + 1];        // widths
+  const bf16_t* Wf[kSlabL]; // W_l packed
+  const float* bias[kSlabL];
+  const float* X;           // inputs [B][w[0]]
+  float* Y;                 // outputs [B][w[L]]
+};
+
+// fragment f of the packed matrix: a uniform base and the lane's 16 bytes
+__device__ __forceinline__ u32x4 frag(const bf16_t* W, size_t f, int lane) {
+  return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(W + f * 512) + (uint32_t)lane * 16u);
+}
+
+// the first fragments of a wave's tiles (PF of them, step by step)
+template <int PF, int TPW>
+__device__ __forceinline__ void frag_first(u32x4 (&pf)[PF], const bf16_t* W, int steps, int wave, int lane) {
+  constexpr int CH = PF / TPW;  // steps in flight
+#pragma unroll
+  for (int s = 0; s < CH; ++s)
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)
+      pf[s * TPW + i] = frag(W, (size_t)(wave + 8 * i) * steps + min(s, steps - 1), lane);
+}
+template <int PF>
+__device__ __forceinline__ void frag_first_any(u32x4 (&pf)[PF], const bf16_t* W, int tpw, int steps, int wave,
+                                               int lane) {
+  if (tpw == 4) frag_first<PF, 4>(pf, W, steps, wave, lane);
+  else if (tpw == 3) frag_first<PF, 3>(pf, W, steps, wave, lane);
+  else if (tpw == 2) frag_first<PF, 2>(pf, W, steps, wave, lane);
+  else frag_first<PF, 1>(pf, W, steps, wave, lane);
+}
+
+// acc[i][m] += W tile (wave + 8 i) times the slab's rows 16 m..16 m + 15; pf
+// holds the first fragments (frag_first), each refilled as it is used
+template <int MR, int PF, int TPW>
+__device__ __forceinline__ void slab_product(f32x4 (&acc)[4][MR / 16], u32x4 (&pf)[PF], const bf16_t* W, int steps,
+                                             const bf16_t* sH, int wave, int lane) {
+  constexpr int CH = PF / TPW;  // steps in flight
+  const bf16_t* a = sH + (lane & 15) * kSlabLd + (lane >> 4) * 8;
+#pragma unroll
+  for (int i = 0; i < TPW; ++i)
+#pragma unroll
+    for (int m = 0; m < MR / 16; ++m) acc[i][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 h[MR / 16], hn[MR / 16];
+  auto rows = [&](bf16x8 (&v)[MR / 16], int step) {
+#pragma unroll
+    for (int m = 0; m < MR / 16; ++m) v[m] = *reinterpret_cast<const bf16x8*>(a + m * 16 * kSlabLd + step * 32);
+  };
+  auto use = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      const bf16x8 w = __builtin_bit_cast(bf16x8, pf[s * TPW + i]);
+#pragma unroll
+      for (int m = 0; m < MR / 16; ++m)
+        acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, h[m], acc[i][m], 0, 0, 0);
+    }
+  };
+  rows(h, 0);
+  // whole chunks refill without a branch (the last step again past the end):
+  // with one, every use would wait for all loads in flight; and in this order,
+  // or the compiler gathers the refills at the chunk's end
+  const int whole = steps / CH * CH;
+#pragma unroll 1
+  for (int s0 = 0; s0 < whole; s0 += CH)
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      rows(hn, min(s0 + s + 1, steps - 1));
+      use(s);
+#pragma unroll
+      for (int i = 0; i < TPW; ++i)
+        pf[s * TPW + i] = frag(W, (size_t)(wave + 8 * i) * steps + min(s0 + s + CH, steps - 1), lane);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < MR / 16; ++m) h[m] = hn[m];
+    }
+#pragma unroll
+  for (int s = 0; s < CH; ++s)
+    if (whole + s < steps) {
+      rows(h, whole + s);
+      use(s);
+    }
+}
+template <int MR, int PF>
+__device__ __forceinline__ void slab_product_any(f32x4 (&acc)[4][MR / 16], u32x4 (&pf)[PF], const bf16_t* W, int tpw,
+                                                 int steps, const bf16_t* sH, int wave, int lane) {
+  if (tpw == 4) slab_product<MR, PF, 4>(acc, pf, W, steps, sH, wave, lane);
+  else if (tpw == 3) slab_product<MR, PF, 3>(acc, pf, W, steps, sH, wave, lane);
+  else if (tpw == 2) slab_product<MR, PF, 2>(acc, pf, W, steps, sH, wave, lane);
+  else slab_product<MR, PF, 1>(acc, pf, W, steps, sH, wave, lane);
+}
+
+// Four neighbouring columns n0..n0+3 of slab row m into LDS; columns past the
+// layer's width are zeros (the next contraction runs in whole steps of 32)
+__device__ __forceinline__ void slab_put(bf16_t* sH, int m, int n0, const uint32_t (&h)[4]) {
+  *reinterpret_cast<uint2*>(sH + m * kSlabLd + n0) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+}
+
+// Forward pass of one slab of MR rows through the whole network: rows are
+// independent, so a workgroup needs no other's results and the activations
+// never leave LDS.  8 waves x TPW column tiles; D fragments: lane holds
+// columns 16 t + 4 (lane / 16) + r of row 16 m + lane % 16.  Bound by the
+// weights' way into the CUs (each slab reads all of them from L2) and the
+// error functions.  Receiver network (32-512x5-64), 16,384 rows: 64 batches
+// of 7 launches took 5.6 ms, one launch takes 0.106 ms (340 TFLOP/s).
+template <int MR, int PF>
+__global__ __launch_bounds__(512, 2) void k_slab(SlabArgs g) {
+  constexpr int MT = MR / 16;
+  __shared__ __attribute__((aligned(16))) bf16_t sH[MR * kSlabLd];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int b0 = blockIdx.x * MR;
+  const int q4 = (lane >> 4) * 4, mr = lane & 15;
+  u32x4 pf[PF];
+  frag_first_any<PF>(pf, g.Wf[0], tpw_of(g.w[1]), steps_of(g.w[0]), wave, lane);
+  {  // the slab's inputs in bf16, zeros past the rows and past the width
+    const int K = g.w[0], Kp = steps_of(K) * 32;
+    for (int e = tid; e < MR * (Kp / 4); e += 512) {
+      const int m = e / (Kp / 4), k = (e % (Kp / 4)) * 4;
+      uint32_t h[4] = {0u, 0u, 0u, 0u};
+      if (b0 + m < g.B && k < K) {
+        const float4 x = *reinterpret_cast<const float4*>(g.X + (size_t)(b0 + m) * K + k);
+        h[0] = f2bf(x.x); h[1] = f2bf(x.y); h[2] = f2bf(x.z); h[3] = f2bf(x.w);
+      }
+      slab_put(sH, m, k, h);
+    }
+  }
+  __syncthreads();
+  f32x4 acc[4][MT];
+  for (int l = 0; l < g.L; ++l) {
+    const int N = g.w[l + 1], tpw = tpw_of(N), nt = tiles_of(N);
+    const bool last = l + 1 == g.L;
+    slab_product_any<MR, PF>(acc, pf, g.Wf[l], tpw, steps_of(g.w[l]), sH, wave, lane);
+    if (!last) frag_first_any<PF>(pf, g.Wf[l + 1], tpw_of(g.w[l + 2]), steps_of(N), wave, lane);
+    __syncthreads();  // every wave has read this layer's input
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = wave + 8 * i;
+      if (i >= tpw || t >= nt) continue;
+      const int n0 = t * 16 + q4;
+      const bool in = n0 < N;  // widths are multiples of 8: all four columns or none
+      const float4 bv = in ? *reinterpret_cast<const float4*>(g.bias[l] + n0) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float b[4] = {bv.x, bv.y, bv.z, bv.w};
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const int row = b0 + m * 16 + mr;
+        if (last) {
+          if (in && row < g.B)
+            *reinterpret_cast<float4*>(g.Y + (size_t)row * N + n0) =
+                make_float4(acc[i][m][0] + b[0], acc[i][m][1] + b[1], acc[i][m][2] + b[2], acc[i][m][3] + b[3]);
+          continue;
+        }
+        uint32_t h[4] = {0u, 0u, 0u, 0u};
+        if (in)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) h[r] = f2bf(gelu(acc[i][m][r] + b[r]));
+        slab_put(sH, m * 16 + mr, n0, h);
+      }
+    }
+    if (nt & 1) {  // the last step's second tile
+      const uint32_t zero[4] = {0u, 0u, 0u, 0u};
+      for (int e = tid; e < MR * 4; e += 512) slab_put(sH, e >> 2, nt * 16 + (e & 3) * 4, zero);
+    }
+    __syncthreads();
+  }
+}
+
+// Training: one launch per layer and direction.  A slab kernel as above left
+// the chip idle here -- 16 slabs at batch 256, each pulling all 2.3 MB of
+// weights into one CU at about 60 GB/s, 84 us forward and back -- so every
+// 16 x 16 tile of a layer is a wave of its own (512 of them at 256 x 512),
+// all its fragments in flight at once: one trip to memory per launch, 3.7 to
+// 4.7 us each.  Receiver network, batch 256: a step of 30 launches took 178
+// us, these 12 take 61 us (k_update 17 us of them).
+enum { LAYER_FWD = 0, LAYER_LOSS = 1, LAYER_BWD = 2 };
+struct LayerArgs {
+  int N, K, B, ldb;    // output width, contraction, rows
+  const bf16_t* W;     // packed [N][K]
+  const bf16_t* in;    // packed [rows][K]; null: rows idx[b] of X
+  const float* X;
+  const int* idx;
+  bf16_t* XT;          // X's rows in bf16, transposed [K][ldb]
+  const float* bias;   // forward
+  bf16_t* out;         // packed [rows][N]: gelu(z), dY or dZ
+  bf16_t* outT;        // transposed [N][ldb]
+  f32x4* dg;           // gelu'(z) as the lanes hold it, one per tile and lane
+  const float* T;      // loss: targets, row idx[b]
+  float scale;         // loss: 2 / (B N)
+  float* part;         // loss: per tile, sum of (y - t)^2
+};
+
+// workgroups of 2 waves: column tile wg % tiles, row tiles 2 (wg / tiles) + wave
+__host__ __device__ inline int layer_wgs(int N, int B) { return tiles_of(N) * ((B + 31) >> 5); }
+
+template <int EPI, bool GATHER>
+__device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt = tiles_of(g.N), t = wg % nt, mt = wg / nt * 2 + wave;
+  if (mt * 16 >= g.B) return;
+  const int steps = steps_of(g.K);
+  const int mr = lane & 15, row = mt * 16 + mr, n0 = t * 16 + (lane >> 4) * 4;
+  const bool in = n0 < g.N, ok = in && row < g.B;  // widths are multiples of 8: all four columns or none
+  f32x4 dg = {0.f, 0.f, 0.f, 0.f};
+  if (EPI == LAYER_BWD) dg = g.dg[((size_t)mt * nt + t) * 64 + lane];
+  float4 bv = make_float4(0.f, 0.f, 0.f, 0.f), tv = bv;
+  if (EPI != LAYER_BWD && in) bv = *reinterpret_cast<const float4*>(g.bias + n0);
+  if (EPI == LAYER_LOSS && ok) tv = *reinterpret_cast<const float4*>(g.T + (size_t)g.idx[row] * g.N + n0);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  constexpr int CH = GATHER ? 4 : 16;  // steps in flight
+#pragma unroll 1
+  for (int s0 = 0; s0 < steps; s0 += CH) {
+    u32x4 w[CH], h[CH];
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      const int st = min(s0 + s, steps - 1);
+      w[s] = frag(g.W, (size_t)t * steps + st, lane);
+      if (!GATHER) {
+        h[s] = frag(g.in, (size_t)mt * steps + st, lane);
+      } else {
+        const int k = st * 32 + (lane >> 4) * 8;
+        uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+        if (row < g.B && k < g.K) {
+          const float* x = g.X + (size_t)g.idx[row] * g.K + k;
+          const float4 a = *reinterpret_cast<const float4*>(x), b = *reinterpret_cast<const float4*>(x + 4);
+          v[0] = f2bf(a.x); v[1] = f2bf(a.y); v[2] = f2bf(a.z); v[3] = f2bf(a.w);
+          v[4] = f2bf(b.x); v[5] = f2bf(b.y); v[6] = f2bf(b.z); v[7] = f2bf(b.w);
+          if (t == 0 && s0 + s < steps)
+#pragma unroll
+            for (int r = 0; r < 8; ++r) g.XT[(size_t)(k + r) * g.ldb + row] = (bf16_t)v[r];
+        }
+        h[s] = u32x4{v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < CH; ++s)
+      if (s0 + s < steps)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[s]),
+                                                      __builtin_bit_cast(bf16x8, h[s]), acc, 0, 0, 0);
+  }
+  const float b[4] = {bv.x, bv.y, bv.z, bv.w}, tt[4] = {tv.x, tv.y, tv.z, tv.w};
+  uint32_t h[4] = {0u, 0u, 0u, 0u};
+  float d2 = 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (EPI == LAYER_FWD) {
+      const float z = acc[r] + b[r];
+      const float e1 = 1.0f + erff(z * 0.70710678118654752f);
+      h[r] = f2bf(0.5f * z * e1);
+      dg[r] = 0.5f * e1 + z * 0.39894228040143268f * expf(-0.5f * z * z);
+    } else if (EPI == LAYER_BWD) {
+      h[r] = f2bf(acc[r] * dg[r]);
+    } else {
+      const float d = (acc[r] + b[r]) - tt[r];
+      if (ok) d2 += d * d;
+      h[r] = f2bf(g.scale * d);
+    }
+  }
+  if (EPI == LAYER_FWD) g.dg[((size_t)mt * nt + t) * 64 + lane] = dg;
+  if (ok) {
+    if (g.out)
+      *reinterpret_cast<uint2*>(g.out + pack_pos(row, n0, steps_of(g.N))) =
+          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) g.outT[(size_t)(n0 + r) * g.ldb + row] = (bf16_t)h[r];
+  }
+  if (EPI == LAYER_LOSS) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) d2 += __shfl_down(d2, o, 64);
+    if (lane == 0) g.part[(size_t)mt * nt + t] = d2;
+  }
+}
+
+struct AdamArgs {
+  float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ float adam_one(float& w, float& m, float& v, float g, const AdamArgs& a) {
+  const float mi = a.b1 * m + (1.f - a.b1) * g;
+  const float vi = a.b2 * v + (1.f - a.b2) * g * g;
+  m = mi;
+  v = vi;
+  w = w - a.lr * (mi * a.c1) / (sqrtf(vi * a.c2) + a.eps);
+  return w;
+}
+
 __global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ gr, bf16_t* __restrict__ wb, size_t n, float lr,
-                       float b1, float b2, float eps, float c1, float c2) {
+                       const float* __restrict__ gr, bf16_t* __restrict__ wb, size_t n, AdamArgs a) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const float g = gr[i];
-  const float mi = b1 * m[i] + (1.f - b1) * g;
-  const float vi = b2 * v[i] + (1.f - b2) * g * g;
+  float wi = w[i], mi = m[i], vi = v[i];
+  adam_one(wi, mi, vi, gr[i], a);
   m[i] = mi;
   v[i] = vi;
-  const float wi = w[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
   w[i] = wi;
   if (wb) wb[i] = f2bf(wi);
 }
 
-__global__ void k_to_bf16(const float* __restrict__ a, bf16_t* __restrict__ b, size_t n) {
+struct UpdateLayer {
+  int N, K, first;      // W is [N][K]; first workgroup of its weight tiles
+  const bf16_t *DT, *HT;  // dZ^T [N][ldb], H^T [K][ldb]
+  size_t woff, boff;
+  bf16_t *Wf, *Wd, *Wb;  // packed copies and the row-major copy, where kept
+};
+struct UpdateArgs {
+  int L, B, ldb, first_bias, n_part;
+  UpdateLayer y[kSlabL];
+  float *P, *M, *V;  // ADAM: updated in place
+  float* G;          // !ADAM: gradients
+  AdamArgs a;
+  const float* part;
+  float part_scale;
+  float* loss;
+};
+
+// Weight gradients dW_l = dZ_l^T H_l of every layer in one launch, with the
+// Adam update of the master weights, both moments and the bf16 copies in the
+// epilogue (ADAM), or the gradients stored (!ADAM).  64 x 16 (k x n) of W per
+// workgroup of 2 waves, 32 x 16 per wave, fragments straight from the
+// transposed operands (both contiguous along the batch, 16 bytes a lane); D
+// fragments hold four neighbouring k of one n, so masters and moments move in
+// 16-byte pieces.  Bound by their 24 bytes per weight and by the trip to
+// memory (a gradient buffer in between would add 8 bytes and a launch).
+// Joined to the launch of a lower layer's input gradient instead, each layer's
+// update made those launches 8.3 us long where they take 4.2: 75 us a step
+// against 63.  The workgroups from first_bias on sum the biases' columns (in
+// k_colsum's order), the last one the loss.
+template <bool ADAM>
+__global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wg = blockIdx.x;
+  if (wg == (int)gridDim.x - 1) {  // the loss
+    __shared__ double red[128];
+    double s = 0.0;
+    for (int i = tid; i < u.n_part; i += 128) s += u.part[i];
+    red[tid] = s;
+    __syncthreads();
+    for (int w = 64; w > 0; w >>= 1) {
+      if (tid < w) red[tid] += red[tid + w];
+      __syncthreads();
+    }
+    if (tid == 0) u.loss[0] = (float)(red[0] * u.part_scale);
+    return;
+  }
+  if (wg >= u.first_bias) {  // 4 bias entries per workgroup, 32 lanes each
+    int o = wg - u.first_bias, l = 0;
+    while (o >= u.y[l].N / 4) o -= u.y[l++].N / 4;
+    const UpdateLayer& y = u.y[l];
+    const int gp = lane & 31, half = lane >> 5;
+    const int n = o * 4 + wave * 2 + half;  // widths are multiples of 8
+    float s = 0.f;
+    for (int b = gp; b < u.B; b += 32) s += bf2f(y.DT[(size_t)n * u.ldb + b]);
+    float t = 0.f;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) t += __shfl(s, half * 32 + j, 64);
+    if (gp == 0) {
+      const size_t i = y.boff + n;
+      if (ADAM) {
+        float w = u.P[i], m = u.M[i], v = u.V[i];
+        adam_one(w, m, v, t, u.a);
+        u.P[i] = w; u.M[i] = m; u.V[i] = v;
+      } else {
+        u.G[i] = t;
+      }
+    }
+    return;
+  }
+  int l = u.L - 1;
+  while (wg < u.y[l].first) --l;
+  const UpdateLayer& y = u.y[l];
+  const int tk = (y.K + 63) / 64, o = wg - y.first;
+  const int k0 = (o % tk) * 64 + wave * 32, n0 = (o / tk) * 16;
+  if (k0 >= y.K || n0 >= y.N) return;
+  const int fr = lane & 15, fk = (lane >> 4) * 8;
+  f32x4 acc[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // masters and moments on their way while the products run
+  float4 pw[2], pm[2], pv[2];
+  if (ADAM) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = k0 + 16 * i + (lane >> 4) * 4, n = n0 + fr;
+      if (k < y.K && n < y.N) {
+        const size_t at = y.woff + (size_t)n * y.K + k;
+        pw[i] = *reinterpret_cast<const float4*>(u.P + at);
+        pm[i] = *reinterpret_cast<const float4*>(u.M + at);
+        pv[i] = *reinterpret_cast<const float4*>(u.V + at);
+      }
+    }
+  }
+  constexpr int CH = 4;
+#pragma unroll 1
+  for (int s0 = 0; s0 < u.B; s0 += 32 * CH) {
+    uint4 a[CH][2], b[CH];
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      const int bb = s0 + 32 * s + fk, n = n0 + fr;
+      b[s] = a[s][0] = a[s][1] = make_uint4(0u, 0u, 0u, 0u);
+      if (bb < u.B && n < y.N) b[s] = *reinterpret_cast<const uint4*>(y.DT + (size_t)n * u.ldb + bb);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int k = k0 + 16 * i + fr;
+        if (bb < u.B && k < y.K) a[s][i] = *reinterpret_cast<const uint4*>(y.HT + (size_t)k * u.ldb + bb);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < CH; ++s)
+      if (s0 + 32 * s < u.B)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s][i]),
+                                                           __builtin_bit_cast(bf16x8, b[s]), acc[i], 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int k = k0 + 16 * i + (lane >> 4) * 4, n = n0 + fr;
+    if (k >= y.K || n >= y.N) continue;
+    const size_t at = y.woff + (size_t)n * y.K + k;
+    if (!ADAM) {
+      *reinterpret_cast<float4*>(u.G + at) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+      continue;
+    }
+    float4 w = pw[i], m = pm[i], v = pv[i];
+    const uint32_t h0 = f2bf(adam_one(w.x, m.x, v.x, acc[i][0], u.a));
+    const uint32_t h1 = f2bf(adam_one(w.y, m.y, v.y, acc[i][1], u.a));
+    const uint32_t h2 = f2bf(adam_one(w.z, m.z, v.z, acc[i][2], u.a));
+    const uint32_t h3 = f2bf(adam_one(w.w, m.w, v.w, acc[i][3], u.a));
+    *reinterpret_cast<float4*>(u.P + at) = w;
+    *reinterpret_cast<float4*>(u.M + at) = m;
+    *reinterpret_cast<float4*>(u.V + at) = v;
+    const uint2 hw = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
+    if (y.Wb) *reinterpret_cast<uint2*>(y.Wb + (size_t)n * y.K + k) = hw;
+    if (y.Wf) *reinterpret_cast<uint2*>(y.Wf + pack_pos(n, k, steps_of(y.K))) = hw;
+    if (y.Wd) {
+      const int sn = steps_of(y.N);
+      y.Wd[pack_pos(k, n, sn)] = (bf16_t)h0;
+      y.Wd[pack_pos(k + 1, n, sn)] = (bf16_t)h1;
+      y.Wd[pack_pos(k + 2, n, sn)] = (bf16_t)h2;
+      y.Wd[pack_pos(k + 3, n, sn)] = (bf16_t)h3;
+    }
+  }
+}
+
+template <int EPI, bool GATHER>
+__global__ __launch_bounds__(128) void k_layer(LayerArgs g) {
+  layer_tile<EPI, GATHER>(g, blockIdx.x);
+}
+
+// bf16 copies of W [N][K] in both fragment orders
+__global__ void k_pack(const float* __restrict__ W, int N, int K, bf16_t* __restrict__ Wf, bf16_t* __restrict__ Wd) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = f2bf(a[i]);
+  if (i >= (size_t)N * K) return;
+  const int n = (int)(i / K), k = (int)(i % K);
+  const bf16_t h = f2bf(W[i]);
+  if (Wf) Wf[pack_pos(n, k, steps_of(K))] = h;
+  if (Wd) Wd[pack_pos(k, n, steps_of(N))] = h;
 }
 
 unsigned blocks(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
@@ -374,6 +844,18 @@ struct LymphMlp {
   size_t dorder_cap = 0;
   float* dloss = nullptr;
   size_t dloss_cap = 0;
+  // slab networks (all widths <= kSlabW): packed weights, transposed
+  // activations and gradients, gelu' per slab; grown with the batch
+  bool slab = false;
+  std::vector<bf16_t*> Wf, Wd, HT, DT, HP, DP;
+  std::vector<f32x4*> dg;
+  // inputs and outputs of host-side calls: one batch with the network, grown
+  // (own) to the largest call
+  struct Buf {
+    float* p = nullptr;
+    size_t cap = 0;
+    bool own = false;
+  } in, out;
   std::vector<void*> owned;
   // every kernel and copy of this network runs on its own stream, so that
   // networks trained from different host threads overlap on the GPU
@@ -485,6 +967,106 @@ int backward(LymphMlp* m, int B, const float* T, const int* idx, float* loss_out
   return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("backward: ") + hipGetErrorString(e));
 }
 
+int grow(LymphMlp* m, LymphMlp::Buf& b, size_t n) {
+  if (n <= b.cap) return 0;
+  HIP_TRY(hipStreamSynchronize(m->stream));
+  float* q = nullptr;
+  if (hipMalloc((void**)&q, n * sizeof(float)) != hipSuccess)
+    return fail(LYMPH_MLP_ERR_HIP, "hipMalloc(" + std::to_string(n * sizeof(float)) + " B) failed");
+  if (b.own) (void)hipFree(b.p);
+  b = {q, n, true};
+  return 0;
+}
+
+// Outputs of n rows (device).  16 rows a slab until every CU has one (4096
+// rows), then 32: the weights are read once per slab, and two slabs of 32 fit
+// a CU's registers.
+int slab_forward(LymphMlp* m, int n, const float* X, float* Y) {
+  if (n <= 0) return 0;
+  SlabArgs a{};
+  a.L = m->L;
+  a.B = n;
+  for (int l = 0; l <= m->L; ++l) a.w[l] = m->w[l];
+  for (int l = 0; l < m->L; ++l) {
+    a.Wf[l] = m->Wf[l];
+    a.bias[l] = m->P + m->boff[l];
+  }
+  a.X = X;
+  a.Y = Y;
+  if (n <= 4096)
+    k_slab<16, 16><<<blocks(n, 16), 512, 0, m->stream>>>(a);
+  else
+    k_slab<32, 16><<<blocks(n, 32), 512, 0, m->stream>>>(a);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("k_slab: ") + hipGetErrorString(e));
+}
+
+// One step on rows idx of X, T: gradients into G (adam == null) or applied.
+// L forward launches, L - 1 backward, one update.
+int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx, float* loss,
+              const AdamArgs* adam) {
+  const size_t ny = (size_t)B * m->w[m->L];
+  const int L = m->L;
+  hipStream_t st = m->stream;
+  for (int l = 0; l < L; ++l) {
+    LayerArgs a{};
+    a.N = m->w[l + 1]; a.K = m->w[l]; a.B = B; a.ldb = m->max_batch;
+    a.W = m->Wf[l];
+    a.in = m->HP[l];
+    a.X = X; a.idx = idx; a.XT = m->HT[0];
+    a.bias = m->P + m->boff[l];
+    const unsigned wgs = (unsigned)layer_wgs(a.N, B);
+    if (l + 1 < L) {
+      a.out = m->HP[l + 1]; a.outT = m->HT[l + 1]; a.dg = m->dg[l];
+      if (l == 0) k_layer<LAYER_FWD, true><<<wgs, 128, 0, st>>>(a);
+      else k_layer<LAYER_FWD, false><<<wgs, 128, 0, st>>>(a);
+    } else {
+      a.out = m->DP[l]; a.outT = m->DT[l];
+      a.T = T; a.scale = 2.0f / (float)ny; a.part = m->part;
+      if (l == 0) k_layer<LAYER_LOSS, true><<<wgs, 128, 0, st>>>(a);
+      else k_layer<LAYER_LOSS, false><<<wgs, 128, 0, st>>>(a);
+    }
+  }
+  for (int l = L - 1; l >= 1; --l) {  // dZ_{l-1} = (dZ_l W_l) gelu'(z_{l-1})
+    LayerArgs a{};
+    a.N = m->w[l]; a.K = m->w[l + 1]; a.B = B; a.ldb = m->max_batch;
+    a.W = m->Wd[l];
+    a.in = m->DP[l];
+    a.out = l > 1 ? m->DP[l - 1] : nullptr; a.outT = m->DT[l - 1]; a.dg = m->dg[l - 1];
+    k_layer<LAYER_BWD, false><<<(unsigned)layer_wgs(a.N, B), 128, 0, st>>>(a);
+  }
+  UpdateArgs u{};
+  u.L = L;
+  u.B = B;
+  u.ldb = m->max_batch;
+  u.P = m->P; u.M = m->Mo; u.V = m->Vo; u.G = m->G;
+  if (adam) u.a = *adam;
+  int wgs = 0, bias = 0;
+  for (int l = 0; l < L; ++l) {
+    UpdateLayer& y = u.y[l];
+    y.N = m->w[l + 1];
+    y.K = m->w[l];
+    y.first = wgs;
+    wgs += (int)(blocks(y.N, 16) * blocks(y.K, 64));
+    bias += y.N / 4;
+    y.DT = m->DT[l];
+    y.HT = m->HT[l];
+    y.woff = m->woff[l];
+    y.boff = m->boff[l];
+    y.Wf = m->Wf[l];
+    y.Wd = m->Wd[l];
+  }
+  u.first_bias = wgs;
+  u.part = m->part;
+  u.n_part = tiles_of(B) * tiles_of(m->w[L]);
+  u.part_scale = 1.0f / (float)ny;
+  u.loss = loss;
+  if (adam) k_update<true><<<wgs + bias + 1, 128, 0, st>>>(u);
+  else k_update<false><<<wgs + bias + 1, 128, 0, st>>>(u);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("training step: ") + hipGetErrorString(e));
+}
+
 int need(const LymphMlp* m) { return m ? 0 : fail(LYMPH_MLP_ERR_ARG, "null network"); }
 
 }  // namespace
@@ -500,6 +1082,8 @@ int lymph_mlp_destroy(LymphMlp* m) {
   if (m->ws) (void)hipFree(m->ws);
   if (m->dorder) (void)hipFree(m->dorder);
   if (m->dloss) (void)hipFree(m->dloss);
+  if (m->in.own) (void)hipFree(m->in.p);
+  if (m->out.own) (void)hipFree(m->out.p);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
   return 0;
@@ -533,35 +1117,67 @@ int lymph_mlp_create(int n_layers, const int32_t* widths, int max_batch, LymphMl
     if (l + 1 < n_layers) maxh = std::max(maxh, m->w[l + 1]);
   }
   m->n_params = off;
-  int rc = 0;
-  auto al = [&](auto** p, size_t n) {
-    if (!rc) rc = dalloc(m, p, n);
-  };
-  al(&m->P, off);
+  // one allocation: the buffers that start as zeros first, then the others
+  struct Want { void** p; size_t bytes; };
+  std::vector<Want> zeros, rest;
+  auto zero = [&](auto** p, size_t n) { zeros.push_back({(void**)p, n * sizeof(**p)}); };
+  auto al = [&](auto** p, size_t n) { rest.push_back({(void**)p, n * sizeof(**p)}); };
+  zero(&m->P, off);
+  zero(&m->Mo, off);
+  zero(&m->Vo, off);
   al(&m->G, off);
-  al(&m->Mo, off);
-  al(&m->Vo, off);
-  al(&m->Wb, off);
-  m->H.assign(n_layers, nullptr);
-  m->Z.assign(n_layers, nullptr);
-  for (int l = 0; l < n_layers; ++l) al(&m->H[l], (size_t)max_batch * m->w[l]);
-  for (int l = 0; l + 1 < n_layers; ++l) al(&m->Z[l], (size_t)max_batch * m->w[l + 1]);
   const int NL = m->w[n_layers];
-  al(&m->Y, (size_t)max_batch * NL);
-  al(&m->dY, (size_t)max_batch * NL);
-  al(&m->dZa, (size_t)max_batch * maxh);
-  al(&m->dZb, (size_t)max_batch * maxh);
-  al(&m->part, blocks((size_t)max_batch * NL, 256));
+  m->slab = n_layers <= kSlabL && *std::max_element(m->w.begin(), m->w.end()) <= kSlabW;
+  const size_t ldb = (size_t)max_batch;
+  if (m->slab) {
+    for (auto* v : {&m->Wf, &m->Wd, &m->HT, &m->DT, &m->HP, &m->DP}) v->assign(n_layers, nullptr);
+    m->dg.assign(n_layers, nullptr);
+    for (int l = 0; l < n_layers; ++l) {
+      const int N = m->w[l + 1], K = m->w[l];
+      zero(&m->Wf[l], pack_size(N, K));
+      al(&m->HT[l], ldb * K);
+      al(&m->DT[l], ldb * N);
+      if (l > 0) {  // operands of the next layer's launch, either way
+        zero(&m->Wd[l], pack_size(K, N));
+        zero(&m->HP[l], pack_size(max_batch, K));
+        zero(&m->DP[l], pack_size(max_batch, N));
+      }
+      if (l + 1 < n_layers) al(&m->dg[l], (size_t)tiles_of(max_batch) * tiles_of(N) * 64);
+    }
+  } else {
+    zero(&m->Wb, off);
+    m->H.assign(n_layers, nullptr);
+    m->Z.assign(n_layers, nullptr);
+    for (int l = 0; l < n_layers; ++l) al(&m->H[l], (size_t)max_batch * m->w[l]);
+    for (int l = 0; l + 1 < n_layers; ++l) al(&m->Z[l], (size_t)max_batch * m->w[l + 1]);
+    al(&m->Y, (size_t)max_batch * NL);
+    al(&m->dY, (size_t)max_batch * NL);
+    al(&m->dZa, (size_t)max_batch * maxh);
+    al(&m->dZb, (size_t)max_batch * maxh);
+  }
+  al(&m->part, std::max((size_t)blocks((size_t)max_batch * NL, 256), (size_t)tiles_of(max_batch) * tiles_of(NL)));
   al(&m->loss, 1);
   al(&m->idx, (size_t)max_batch);
-  if (rc) {
+  m->in.cap = (size_t)max_batch * m->w[0];
+  m->out.cap = (size_t)max_batch * NL;
+  al(&m->in.p, m->in.cap);
+  al(&m->out.p, m->out.cap);
+  size_t total = 0, cleared = 0;
+  for (auto* v : {&zeros, &rest}) {
+    for (auto& q : *v) total += (q.bytes + 255) / 256 * 256;
+    if (v == &zeros) cleared = total;
+  }
+  char* base = nullptr;
+  if (int rc = dalloc(m, &base, total)) {
     lymph_mlp_destroy(m);
     return rc;
   }
-  if (hipMemsetAsync(m->P, 0, off * 4, m->stream) != hipSuccess ||
-      hipMemsetAsync(m->Mo, 0, off * 4, m->stream) != hipSuccess ||
-      hipMemsetAsync(m->Vo, 0, off * 4, m->stream) != hipSuccess ||
-      hipMemsetAsync(m->Wb, 0, off * 2, m->stream) != hipSuccess ||
+  for (auto* v : {&zeros, &rest})
+    for (auto& q : *v) {
+      *q.p = base;
+      base += (q.bytes + 255) / 256 * 256;
+    }
+  if (hipMemsetAsync(m->P, 0, cleared, m->stream) != hipSuccess ||
       hipStreamSynchronize(m->stream) != hipSuccess) {
     lymph_mlp_destroy(m);
     return fail(LYMPH_MLP_ERR_HIP, "hipMemset failed");
@@ -580,7 +1196,13 @@ int lymph_mlp_set_params(LymphMlp* m, const float* p) {
   if (int rc = need(m)) return rc;
   if (!p) return fail(LYMPH_MLP_ERR_ARG, "null params");
   HIP_TRY(hipMemcpyAsync(m->P, p, m->n_params * 4, hipMemcpyHostToDevice, m->stream));
-  k_to_bf16<<<blocks(m->n_params, 256), 256, 0, m->stream>>>(m->P, m->Wb, m->n_params);
+  if (m->slab) {
+    for (int l = 0; l < m->L; ++l)
+      k_pack<<<blocks((size_t)m->w[l + 1] * m->w[l], 256), 256, 0, m->stream>>>(m->P + m->woff[l], m->w[l + 1],
+                                                                                m->w[l], m->Wf[l], m->Wd[l]);
+  } else {
+    k_to_bf16<<<blocks(m->n_params, 256), 256, 0, m->stream>>>(m->P, m->Wb, m->n_params);
+  }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemsetAsync(m->Mo, 0, m->n_params * 4, m->stream));
   HIP_TRY(hipMemsetAsync(m->Vo, 0, m->n_params * 4, m->stream));
@@ -648,15 +1270,21 @@ int lymph_mlp_train(LymphMlp* m, int n_steps, int batch, const int32_t* order, f
   int rc = 0;
   for (int s = 0; s < n_steps && !rc; ++s) {
     const int* idx = dorder + (size_t)s * batch;
+    m->adam_t++;
+    const AdamArgs ad{lr, beta1, beta2, eps, 1.0f / (1.0f - std::pow(beta1, (float)m->adam_t)),
+                      1.0f / (1.0f - std::pow(beta2, (float)m->adam_t))};
+    if (m->slab) {
+      rc = slab_step(m, batch, m->X, m->T, idx, dloss + s, &ad);
+      if (rc) m->adam_t--;
+      continue;
+    }
     k_gather<<<blocks((size_t)batch * m->w[0], 256), 256, 0, m->stream>>>(m->X, m->w[0], idx, batch, m->H[0]);
     rc = forward(m, batch);
     if (!rc) rc = backward(m, batch, m->T, idx, dloss + s);
-    if (!rc) {
-      m->adam_t++;
-      const float c1 = 1.0f / (1.0f - std::pow(beta1, (float)m->adam_t));
-      const float c2 = 1.0f / (1.0f - std::pow(beta2, (float)m->adam_t));
-      k_adam<<<blocks(m->n_params, 256), 256, 0, m->stream>>>(m->P, m->Mo, m->Vo, m->G, m->Wb, m->n_params, lr,
-                                                beta1, beta2, eps, c1, c2);
+    if (rc) {
+      m->adam_t--;
+    } else {
+      k_adam<<<blocks(m->n_params, 256), 256, 0, m->stream>>>(m->P, m->Mo, m->Vo, m->G, m->Wb, m->n_params, ad);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) rc = fail(LYMPH_MLP_ERR_HIP, std::string("k_adam: ") + hipGetErrorString(e));
     }
@@ -675,12 +1303,9 @@ int lymph_mlp_gradients(LymphMlp* m, int batch, const float* x, const float* y, 
     return fail(LYMPH_MLP_ERR_ARG, "batch must be a multiple of 8 and at most max_batch");
   if (!x || !y) return fail(LYMPH_MLP_ERR_ARG, "null batch");
   const size_t nx = (size_t)batch * m->w[0], ny = (size_t)batch * m->w[m->L];
-  float *dx = nullptr, *dy = nullptr;
-  HIP_TRY(hipMalloc(&dx, nx * 4));
-  if (hipMalloc(&dy, ny * 4) != hipSuccess) {
-    (void)hipFree(dx);
-    return fail(LYMPH_MLP_ERR_HIP, "hipMalloc failed");
-  }
+  if (int rc = grow(m, m->in, nx)) return rc;
+  if (int rc = grow(m, m->out, ny)) return rc;
+  float *dx = m->in.p, *dy = m->out.p;
   std::vector<int> id(batch);
   for (int i = 0; i < batch; ++i) id[i] = i;
   int rc = 0;
@@ -688,19 +1313,19 @@ int lymph_mlp_gradients(LymphMlp* m, int batch, const float* x, const float* y, 
       hipMemcpyAsync(dy, y, ny * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
       hipMemcpyAsync(m->idx, id.data(), 4 * batch, hipMemcpyHostToDevice, m->stream) != hipSuccess)
     rc = fail(LYMPH_MLP_ERR_HIP, "upload failed");
-  if (!rc) {
+  if (!rc && m->slab) {
+    rc = slab_step(m, batch, dx, dy, m->idx, m->loss, nullptr);
+  } else if (!rc) {
     k_gather<<<blocks(nx, 256), 256, 0, m->stream>>>(dx, m->w[0], m->idx, batch, m->H[0]);
     rc = forward(m, batch);
+    if (!rc) rc = backward(m, batch, dy, m->idx, m->loss);
   }
-  if (!rc) rc = backward(m, batch, dy, m->idx, m->loss);
   if (!rc && grads &&
       hipMemcpyAsync(grads, m->G, m->n_params * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
     rc = fail(LYMPH_MLP_ERR_HIP, "gradient copy failed");
   if (!rc && loss && hipMemcpyAsync(loss, m->loss, 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
     rc = fail(LYMPH_MLP_ERR_HIP, "loss copy failed");
-  (void)hipStreamSynchronize(m->stream);
-  (void)hipFree(dx);
-  (void)hipFree(dy);
+  if (hipStreamSynchronize(m->stream) != hipSuccess && !rc) rc = fail(LYMPH_MLP_ERR_HIP, "gradients failed");
   return rc;
 }
 
@@ -708,12 +1333,21 @@ int lymph_mlp_predict(LymphMlp* m, int n, const float* x, float* y) {
   if (int rc = need(m)) return rc;
   if (n < 0 || (n > 0 && (!x || !y))) return fail(LYMPH_MLP_ERR_ARG, "bad inputs");
   const int w0 = m->w[0], NL = m->w[m->L];
-  float* dx = nullptr;
-  HIP_TRY(hipMalloc(&dx, (size_t)std::max(1, n) * w0 * 4));
+  if (int rc = grow(m, m->in, (size_t)std::max(1, n) * w0)) return rc;
+  float* dx = m->in.p;
   int rc = 0;
   if (n > 0 &&
       hipMemcpyAsync(dx, x, (size_t)n * w0 * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
     rc = fail(LYMPH_MLP_ERR_HIP, "upload failed");
+  if (m->slab) {
+    if (!rc) rc = grow(m, m->out, (size_t)std::max(1, n) * NL);
+    if (!rc) rc = slab_forward(m, n, dx, m->out.p);
+    if (!rc && n > 0 &&
+        hipMemcpyAsync(y, m->out.p, (size_t)n * NL * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
+      rc = fail(LYMPH_MLP_ERR_HIP, "download failed");
+    if (hipStreamSynchronize(m->stream) != hipSuccess && !rc) rc = fail(LYMPH_MLP_ERR_HIP, "prediction failed");
+    return rc;
+  }
   std::vector<int> id(m->max_batch);
   for (int i = 0; i < m->max_batch; ++i) id[i] = i;
   if (!rc &&
@@ -727,8 +1361,7 @@ int lymph_mlp_predict(LymphMlp* m, int n, const float* x, float* y) {
                               m->stream) != hipSuccess)
       rc = fail(LYMPH_MLP_ERR_HIP, "download failed");
   }
-  (void)hipStreamSynchronize(m->stream);
-  (void)hipFree(dx);
+  if (hipStreamSynchronize(m->stream) != hipSuccess && !rc) rc = fail(LYMPH_MLP_ERR_HIP, "prediction failed");
   return rc;
 }
 
@@ -738,18 +1371,25 @@ int lymph_mlp_time_predict(LymphMlp* m, int n, int reps, double* ms) {
   std::vector<int> id(m->max_batch);
   for (int i = 0; i < m->max_batch; ++i) id[i] = i;
   HIP_TRY(hipMemcpyAsync(m->idx, id.data(), 4 * m->max_batch, hipMemcpyHostToDevice, m->stream));
+  if (m->slab)
+    if (int rc = grow(m, m->out, (size_t)n * m->w[m->L])) return rc;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   int rc = 0;
   HIP_TRY(hipEventRecord(e0, m->stream));
-  for (int r = 0; r < reps && !rc; ++r)
+  for (int r = 0; r < reps && !rc; ++r) {
+    if (m->slab) {
+      rc = slab_forward(m, n, m->X, m->out.p);
+      continue;
+    }
     for (int b0 = 0; b0 < n && !rc; b0 += m->max_batch) {
       const int B = std::min(m->max_batch, n - b0);
       k_gather<<<blocks((size_t)B * m->w[0], 256), 256, 0, m->stream>>>(m->X + (size_t)b0 * m->w[0], m->w[0],
                                                           m->idx, B, m->H[0]);
       rc = forward(m, B);
     }
+  }
   HIP_TRY(hipEventRecord(e1, m->stream));
   HIP_TRY(hipEventSynchronize(e1));
   float f = 0.f;

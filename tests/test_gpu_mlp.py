@@ -83,3 +83,48 @@ def test_adam_step_matches_oracle_and_training_reduces_loss():
         assert losses[-1] < 0.1 * losses[0]
         yp = net.predict(x)
         assert rel(yp, y) < 0.25
+
+
+# networks on the fragment-order kernels (all widths <= 512) at their edges:
+# one layer, widths of one tile and of odd tile counts, the widest, batches of
+# half a tile, of a tile and a half and of several slabs; 520 takes the GEMMs
+EDGES = [([8, 8], 8), ([16, 24], 24), ([8, 16, 8], 16), ([40, 264, 72, 24], 40), ([32, 512, 512, 512], 72),
+         ([512, 8, 504, 16], 8), ([24, 136, 392, 88, 40, 512], 264), ([8, 520, 64, 16], 24)]
+
+
+@pytest.mark.parametrize("widths,batch", EDGES)
+def test_narrow_networks_at_tile_edges_match_oracle(widths, batch):
+    """Outputs, loss, gradients and one Adam step against the oracle, to the
+    tolerances above (bfloat16 operands, 2^-9 per rounding); every row's
+    output is the same bits whatever rows come with it (1, 15, 17 and 4200
+    rows: the two slab sizes)."""
+    from lymph3d_apsc_amd.mlp import Mlp
+    say(f"[mlp edges] {widths} batch {batch}")
+    rng = np.random.default_rng(sum(widths) + batch)
+    x = rng.standard_normal((4200, widths[0])).astype(np.float32)
+    t = rng.standard_normal((batch, widths[-1])).astype(np.float32)
+    with Mlp(widths, max_batch=batch + 8, seed=4) as net:
+        p = net.params().astype(np.float64)
+        y = net.predict(x)
+        y_ref, _ = R.forward(p, widths, x[:64], emulate=True)
+        assert rel(y[:64], y_ref) < 5e-3
+        for n in (1, 15, 17):
+            assert np.array_equal(net.predict(x[:n]), y[:n])
+        loss, g = net.gradients(x[:batch], t)
+        loss_ref, g_ref = R.loss_and_grads(p, widths, x[:batch], t, emulate=True)
+        assert abs(loss - loss_ref) < 1e-3 * loss_ref
+        o = 0
+        for k, n in zip(widths[:-1], widths[1:]):
+            for size in (n * k, n):
+                assert rel(g[o:o + size], g_ref[o:o + size]) < 2e-2, (k, n, size)
+                o += size
+        net.set_data(x[:batch], t)
+        losses = net.train(np.arange(batch, dtype=np.int32), batch, lr=1e-3)
+        q, _, _ = R.adam(p, g.astype(np.float64), 0.0, 0.0, 1, 1e-3)
+        assert np.allclose(net.params(), q, rtol=1e-5, atol=1e-7)
+        assert abs(losses[0] - loss) <= 1e-6 * loss
+        # the packed copies follow the master weights: outputs of a network
+        # given the updated parameters are the same bits
+        with Mlp(widths, max_batch=batch, seed=0) as other:
+            other.set_params(net.params())
+            assert np.array_equal(other.predict(x[:33]), net.predict(x[:33]))
