@@ -891,14 +891,14 @@ int errors_dev(LymphCtx* c, const double* uh, const double* ue, double* l2sq, do
     if (l2sq) {
       k_l2_terms<P><<<grid1(3 * (size_t)c->n_poly, 128), 128, 0, c->stream>>>(c->Mm, uh, ue, c->part,
                                                                                c->n_poly);
-      k_seq_sum<<<1, 64, 0, c->stream>>>(c->part, 3 * c->n_poly, c->dsum);
+      k_sum_terms<<<1, 1024, 0, c->stream>>>(c->part, 3 * c->n_poly, c->dsum);
     }
     if (dgsq) {
       k_sub<<<grid1(n, 256), 256, 0, c->stream>>>(uh, ue, c->stage[2], n);
       launch_leapfrog<P, 2>(0, c->n_poly, c->stream, c->A, c->md.row_ptr, c->md.col, nullptr,
                             nullptr, nullptr, c->stage[2], nullptr, c->part, 0.0, 0.0, 0.0,
                             nullptr, nullptr, c->order, 0);
-      k_seq_sum<<<1, 64, 0, c->stream>>>(c->part, c->n_poly, c->dsum + 1);
+      k_sum_terms<<<1, 1024, 0, c->stream>>>(c->part, c->n_poly, c->dsum + 1);
     }
     return check_launch("error kernels");
   });
@@ -908,6 +908,26 @@ int errors_dev(LymphCtx* c, const double* uh, const double* ue, double* l2sq, do
   if (l2sq) *l2sq = res[0];
   if (dgsq) *dgsq = res[1];
   return 0;
+}
+
+// zeros into a vector by a kernel (a fill of hipMemsetAsync recorded into a
+// captured solve is not replayed reliably)
+int fill_zero(LymphCtx* c, double* v) {
+  k_fill<<<(unsigned)std::min<size_t>(grid1(vec_n(c), 256), 4096), 256, 0, c->stream>>>(v, 0.0, vec_n(c));
+  return check_launch("k_fill");
+}
+
+// COMPUTE_MODAL_COEFFICIENTS_FREE of a built-in field into a device vector.
+// The zero field's coefficients are zeros: no quadrature is run for it (the
+// two projections of a start from rest took 7.3 ms per p = 4 solve on 20^3
+// uneven polyhedra, a fill 5 us).
+int project_field(LymphCtx* c, int fn, double* v) {
+  if (fn == LYMPH_FN_ZERO) return fill_zero(c, v);
+  return dispatch_p(c->p, [&](auto pc) -> int {
+    constexpr int P = decltype(pc)::value;
+    k_project<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, fn, c->RMm, v, nullptr);
+    return check_launch("k_project");
+  });
 }
 
 int need_ctx(const LymphCtx* c) {
@@ -1231,24 +1251,21 @@ int lymph_build_operator(LymphCtx* c) {
     c->bytes += nk * sizeof(double);
   }
   c->built = false;
-  HIP_TRY(hipMemsetAsync(c->K, 0, nk * sizeof(double), c->stream));
-  if (c->A) HIP_TRY(hipMemsetAsync(c->A, 0, nk * sizeof(double), c->stream));
-  HIP_TRY(hipMemsetAsync(c->M, 0, (size_t)c->n_poly * c->Np * c->Np * sizeof(double), c->stream));
-  HIP_TRY(hipMemsetAsync(c->Mm, 0, (size_t)c->n_poly * c->Np * c->Np * sizeof(double), c->stream));
   HIP_TRY(hipMemsetAsync(c->status, 0, sizeof(int), c->stream));
   int rc = dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    const int chunk = 1 << 16;
-    for (int p0 = 0; p0 < c->n_poly; p0 += chunk) {
-      const int n = std::min(chunk, c->n_poly - p0);
-      if (c->build_mode == LYMPH_BUILD_FACTORED)
-        k_build_factored<P><<<n, factored_threads<P>(), 0, c->stream>>>(c->md, c->alpha, c->theta, c->K, c->A, c->M,
-                                                      c->Mm, p0);
-      else
-        k_build_operator<P><<<n, 256, 0, c->stream>>>(c->md, c->alpha, c->theta, c->K, c->A, c->M,
-                                                     c->Mm, p0);
-      if (int r = check_launch("k_build_operator")) return r;
-    }
+    // every entry of K, A_dg and the mass blocks is stored, none needs clearing
+    const unsigned wgs = grid1(c->n_poly, Build<P>::GP) * Build<P>::SPLIT;
+    auto go = [&](auto ref, auto adg) {
+      k_build<P, decltype(ref)::value, decltype(adg)::value><<<wgs, Build<P>::TPB, 0, c->stream>>>(
+          c->md, c->alpha, c->theta, c->K, c->A, c->M, c->Mm, c->n_poly);
+    };
+    const bool ref = c->build_mode != LYMPH_BUILD_FACTORED;
+    if (ref && c->A) go(std::true_type{}, std::true_type{});
+    else if (ref) go(std::true_type{}, std::false_type{});
+    else if (c->A) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
+    if (int r = check_launch("k_build")) return r;
     k_cholesky<P><<<(unsigned)c->n_poly, 64, 0, c->stream>>>(c->M, c->Mm, c->RM, c->RMm,
                                                               c->n_poly, c->status);
     if (int r = check_launch("k_cholesky")) return r;
@@ -1348,12 +1365,16 @@ int lymph_build_rhs(LymphCtx* c, int problem, int slot, double* rhs_out) {
   if (slot < 0 || slot >= LYMPH_NUM_SLOTS) return fail(LYMPH_ERR_ARG, "bad slot");
   if (problem < LYMPH_PROB_NULL || problem > LYMPH_PROB_RICKER)
     return fail(LYMPH_ERR_ARG, "unknown problem");
-  int rc = dispatch_p(c->p, [&](auto pc) -> int {
-    constexpr int P = decltype(pc)::value;
-    k_rhs<P><<<c->n_poly, 128, 0, c->stream>>>(c->md, problem, c->alpha, c->theta, c->slot[slot],
-                                                nullptr, nullptr);
-    return check_launch("k_rhs");
-  });
+  int rc = 0;
+  if (problem == LYMPH_PROB_NULL || problem == LYMPH_PROB_RICKER)  // no volume or boundary data
+    rc = fill_zero(c, c->slot[slot]);
+  else
+    rc = dispatch_p(c->p, [&](auto pc) -> int {
+      constexpr int P = decltype(pc)::value;
+      k_rhs<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, problem, c->alpha, c->theta, c->slot[slot],
+                                                              nullptr, nullptr);
+      return check_launch("k_rhs");
+    });
   if (rc) return rc;
   if (rhs_out) return d2h_vec(c, c->slot[slot], rhs_out);
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1394,7 +1415,7 @@ int lymph_project_fn(LymphCtx* c, lymph_field_fn fld, void* user, int slot, doub
   HIP_TRY_OR(hipMemcpy(dv, tv.data(), 3 * nv * sizeof(double), hipMemcpyHostToDevice), done);
   rc = dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    k_project<P><<<c->n_poly, 128, 0, c->stream>>>(c->md, LYMPH_FN_ZERO, c->RMm, c->slot[slot], dv);
+    k_project<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, LYMPH_FN_ZERO, c->RMm, c->slot[slot], dv);
     return check_launch("k_project");
   });
   if (rc) return done(rc);
@@ -1480,7 +1501,7 @@ int lymph_build_rhs_fn(LymphCtx* c, lymph_forcing_fn f, lymph_dirichlet_fn gd, l
   HIP_TRY_OR(hipMemcpy(df, tf.data(), 3 * nf * sizeof(double), hipMemcpyHostToDevice), done);
   rc = dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    k_rhs<P><<<c->n_poly, 128, 0, c->stream>>>(c->md, LYMPH_PROB_NULL, c->alpha, c->theta,
+    k_rhs<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, LYMPH_PROB_NULL, c->alpha, c->theta,
                                                 c->slot[slot], dv, df);
     return check_launch("k_rhs");
   });
@@ -1493,11 +1514,7 @@ int lymph_project(LymphCtx* c, int fn, int slot, double* out) {
   if (int rc = need_built(c)) return rc;
   if (slot < 0 || slot >= LYMPH_NUM_SLOTS) return fail(LYMPH_ERR_ARG, "bad slot");
   if (fn < LYMPH_FN_ZERO || fn > LYMPH_FN_CUBE_U) return fail(LYMPH_ERR_ARG, "unknown field");
-  int rc = dispatch_p(c->p, [&](auto pc) -> int {
-    constexpr int P = decltype(pc)::value;
-    k_project<P><<<c->n_poly, 128, 0, c->stream>>>(c->md, fn, c->RMm, c->slot[slot], nullptr);
-    return check_launch("k_project");
-  });
+  const int rc = project_field(c, fn, c->slot[slot]);
   if (rc) return rc;
   if (out) return d2h_vec(c, c->slot[slot], out);
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -2024,16 +2041,10 @@ int lymph_capture_solve(LymphCtx* c, int problem, double dt, int nsteps, int eve
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->n_rec = 0;
   HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  // zero initial state (projection kernels, no memset nodes), first step at
+  // zero initial state (fill kernels, no memset nodes), first step at
   // t = 0, then the loop; every launch goes to the capturing stream
-  int rc = dispatch_p(c->p, [&](auto pc) -> int {
-    constexpr int P = decltype(pc)::value;
-    k_project<P><<<c->n_poly, 128, 0, c->stream>>>(c->md, LYMPH_FN_ZERO, c->RMm,
-                                                   c->slot[LYMPH_SLOT_U_PREV], nullptr);
-    k_project<P><<<c->n_poly, 128, 0, c->stream>>>(c->md, LYMPH_FN_ZERO, c->RMm,
-                                                   c->slot[LYMPH_SLOT_V0], nullptr);
-    return check_launch("k_project");
-  });
+  int rc = project_field(c, LYMPH_FN_ZERO, c->slot[LYMPH_SLOT_U_PREV]);
+  if (!rc) rc = project_field(c, LYMPH_FN_ZERO, c->slot[LYMPH_SLOT_V0]);
   double t = 0.0;
   double g0 = 0.0;
   bool grouped = false;

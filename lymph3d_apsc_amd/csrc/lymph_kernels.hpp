@@ -139,206 +139,82 @@ struct MeshDev {
 };
 
 // ---------------------------------------------------------------------------
-// Operator build: MAKE_MATRICES_FREE (src/matrix_free.f90:27-464).
-// One 256-thread workgroup per polyhedron; its tets are processed in order
-// (volume term, then faces 1..4), each output entry owned by one thread for
-// the whole kernel so every entry accumulates in the reference's order.
+// Basis tables.  At a point the basis functions are products of 1-D values
+// v_d[k] = L_k(x_d) / sqrt(h_d) and their derivatives; each 1-D value costs a
+// square root and a division, so a workgroup forms them once per point,
+// dimension and degree (tab1d) and the products from LDS (basis_row), in
+// basis_at's operand order.  Tables run over the functions first ([q][f]):
+// lanes hold neighbouring functions, and their reads fall in distinct banks
+// ([f][q] put all of them in one).
 // ---------------------------------------------------------------------------
-template <int P>
-__global__ __launch_bounds__(256) void k_build_operator(MeshDev m, double alpha, double theta,
-                                                         double* __restrict__ K,
-                                                         double* __restrict__ A,
-                                                         double* __restrict__ M,
-                                                         double* __restrict__ Mm, int poly0) {
-  using D = Dims<P>;
-  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2;
-  constexpr int VOLSZ = 4 * NP * NQ3, FACESZ = 8 * NP * NQ2;
-  constexpr int SHSZ = VOLSZ > FACESZ ? VOLSZ : FACESZ;
-  __shared__ double sh[SHSZ];
-  __shared__ double spt[NQ3 * 3];
-  __shared__ int sbl[NP * 3];
-  const int tid = threadIdx.x;
-  const int Pp = poly0 + blockIdx.x;
-  for (int i = tid; i < NP * 3; i += blockDim.x) sbl[i] = m.blist[i];
-  double bbP[6];
-  for (int d = 0; d < 6; ++d) bbP[d] = m.bbox[Pp * 6 + d];
-  const double hkP = m.hk[Pp];
-  double* Ks = K + (size_t)m.row_ptr[Pp] * D::BS;
-  const bool keepA = A != nullptr;  // A_dg may be dropped for batched runs
-  double* As = keepA ? A + (size_t)m.row_ptr[Pp] * D::BS : nullptr;
-  double* MP = M + (size_t)Pp * NP * NP;
-  double* MmP = Mm + (size_t)Pp * NP * NP;
-  // volume-phase views
-  double* phi = sh;                // [NP][NQ3]
-  double* dphi = sh + NP * NQ3;    // [3][NP][NQ3]
-  // face-phase views
-  double* p1 = sh;                      // [NP][NQ2]
-  double* p2 = sh + NP * NQ2;           // [NP][NQ2]
-  double* g1 = sh + 2 * NP * NQ2;       // [3][NP][NQ2]
-  double* g2 = sh + 5 * NP * NQ2;       // [3][NP][NQ2]
-
-  for (int a = m.ptet_ptr[Pp]; a < m.ptet_ptr[Pp + 1]; ++a) {
-    const int t = m.ptet[a];
-    double v[12], Fk[12], Jdet;
-    for (int i = 0; i < 12; ++i) v[i] = m.tet_xyz[(size_t)t * 12 + i];
-    affine_map(v, Fk, Jdet);
-    const double aJ = fabs(Jdet);
-    const double rho = m.rho[t], lam = m.lam[t], mu = m.mu[t];
-    const double l2m = lam + 2 * mu;
-    __syncthreads();
-    for (int q = tid; q < NQ3; q += blockDim.x) map_point(Fk, &m.qtet[q * 4], &spt[q * 3]);
-    __syncthreads();
-    for (int e = tid; e < NP * NQ3; e += blockDim.x) {
-      const int f = e / NQ3, q = e % NQ3;
-      double ph, d0, d1, d2;
-      basis_at(&sbl[f * 3], bbP, &spt[q * 3], ph, d0, d1, d2);
-      phi[e] = ph;
-      dphi[(0 * NP + f) * NQ3 + q] = d0;
-      dphi[(1 * NP + f) * NQ3 + q] = d1;
-      dphi[(2 * NP + f) * NQ3 + q] = d2;
-    }
-    __syncthreads();
-    // mass (MAKE_MATRICES_FREE :224-233 with MAKE_MASS_VOLUME)
-    for (int e = tid; e < NP * NP; e += blockDim.x) {
-      const int mm = e / NP, nn = e % NP;
-      double s = 0.0;
-      for (int q = 0; q < NQ3; ++q)
-        s = s + 1.0 * m.wtet[q] * aJ * phi[mm * NQ3 + q] * phi[nn * NQ3 + q];
-      MmP[e] = MmP[e] + s;
-      MP[e] = MP[e] + s * rho;
-    }
-    // volume stiffness (MAKE_STIFFNESS_VOLUME, assemble_element :24-77)
-    for (int e = tid; e < 9 * NP * NP; e += blockDim.x) {
-      const int i = e / (3 * NP * NP), j = (e / (NP * NP)) % 3;
-      const int mm = (e / NP) % NP, nn = e % NP;
-      const int oi = i == 0 ? 1 : 0, oi2 = i == 2 ? 1 : 2;  // the other two directions
-      double s = 0.0;
-      const double* Dm = dphi + mm * NQ3;
-      const double* Dn = dphi + nn * NQ3;
-      constexpr int SD = NP * NQ3;
-      for (int q = 0; q < NQ3; ++q) {
-        const double wj = m.wtet[q] * aJ;
-        double tv;
-        if (i == j)
-          tv = l2m * Dm[i * SD + q] * Dn[i * SD + q] + mu * Dm[oi * SD + q] * Dn[oi * SD + q] +
-               mu * Dm[oi2 * SD + q] * Dn[oi2 * SD + q];
-        else
-          tv = lam * Dm[i * SD + q] * Dn[j * SD + q] + mu * Dm[j * SD + q] * Dn[i * SD + q];
-        s = s + wj * tv;
-      }
-      const size_t o = kpos(N3, i * NP + mm, j * NP + nn);
-      Ks[o] = Ks[o] + s;
-      if (keepA) As[o] = As[o] + s;
-    }
-    // faces (MAKE_STIFFNESS_FACE, assemble_element :404-661; insertion
-    // src/matrix_free.f90:371-441)
-    for (int f = 0; f < 4; ++f) {
-      const int e2 = m.neigh[t * 4 + f];
-      int Q = -1;
-      if (e2 >= 0) {
-        Q = m.tet_poly[e2];
-        if (Q == Pp) continue;  // intra-polyhedron face
-      }
-      if (e2 == -2) continue;  // Neumann: no stiffness contribution
-      __syncthreads();
-      for (int q = tid; q < NQ2; q += blockDim.x) face_point(Fk, f, &m.qtri[q * 4], &spt[q * 3]);
-      __syncthreads();
-      double bbQ[6];
-      if (Q >= 0)
-        for (int d = 0; d < 6; ++d) bbQ[d] = m.bbox[Q * 6 + d];
-      for (int e = tid; e < NP * NQ2; e += blockDim.x) {
-        const int fb = e / NQ2, q = e % NQ2;
-        double ph, d0, d1, d2;
-        basis_at(&sbl[fb * 3], bbP, &spt[q * 3], ph, d0, d1, d2);
-        p1[e] = ph;
-        g1[(0 * NP + fb) * NQ2 + q] = d0;
-        g1[(1 * NP + fb) * NQ2 + q] = d1;
-        g1[(2 * NP + fb) * NQ2 + q] = d2;
-        if (Q >= 0) {
-          basis_at(&sbl[fb * 3], bbQ, &spt[q * 3], ph, d0, d1, d2);
-          p2[e] = ph;
-          g2[(0 * NP + fb) * NQ2 + q] = d0;
-          g2[(1 * NP + fb) * NQ2 + q] = d1;
-          g2[(2 * NP + fb) * NQ2 + q] = d2;
-        }
-      }
-      __syncthreads();
-      const double* nrm = &m.normal[(t * 4 + f) * 3];
-      const double n1 = nrm[0], n2 = nrm[1], n3 = nrm[2];
-      const double ar = m.area[t * 4 + f];
-      const double Dbar = lam + 2 * mu;
-      const double hmin = (Q >= 0) ? (hkP < m.hk[Q] ? hkP : m.hk[Q]) : hkP;
-      const double sigma = alpha * (P * P) / hmin * Dbar;
-      const double d11 = fabs(n1) * fabs(n1) + 0.5 * (fabs(n2) * fabs(n2)) + 0.5 * (fabs(n3) * fabs(n3));
-      const double d22 = fabs(n2) * fabs(n2) + 0.5 * (fabs(n1) * fabs(n1)) + 0.5 * (fabs(n3) * fabs(n3));
-      const double d33 = fabs(n3) * fabs(n3) + 0.5 * (fabs(n1) * fabs(n1)) + 0.5 * (fabs(n2) * fabs(n2));
-      const double dd[3] = {d11, d22, d33};
-      const bool interior = Q >= 0;
-      double* Kb = interior ? K + (size_t)m.face_blk[t * 4 + f] * D::BS : nullptr;
-      double* Ab = interior && keepA ? A + (size_t)m.face_blk[t * 4 + f] * D::BS : nullptr;
-      constexpr int SG = NP * NQ2;
-      for (int e = tid; e < 9 * NP * NP; e += blockDim.x) {
-        const int i = e / (3 * NP * NP), j = (e / (NP * NP)) % 3;
-        const int mm = (e / NP) % NP, nn = e % NP;
-        const double ni = nrm[i < j ? i : j], nj = nrm[i < j ? j : i];  // reference order n(min)*n(max)
-        double s1 = 0.0, i1 = 0.0, i1t = 0.0, i2 = 0.0, it2 = 0.0, s2 = 0.0;
-        for (int q = 0; q < NQ2; ++q) {
-          const double w = m.wtri[q];
-          // S_E1 (:476-490)
-          double ts = (i == j) ? (p1[mm * NQ2 + q] * p1[nn * NQ2 + q]) * dd[i]
-                               : 0.5 * p1[mm * NQ2 + q] * p1[nn * NQ2 + q] * ni * nj;
-          s1 = s1 + sigma * w * ts * ar;
-          // I(i,j,m,n) = sigma(grad_m) : (phi_n (x) n) with the component pattern
-          // of :504-515; a = grad side, b = phi side.
-          auto itemp = [&](const double* G, int gm, double phv, int ii, int jj) -> double {
-            if (ii == jj) {
-              if (ii == 0)
-                return l2m * G[0 * SG + gm * NQ2 + q] * phv * n1 + mu * G[1 * SG + gm * NQ2 + q] * phv * n2 +
-                       mu * G[2 * SG + gm * NQ2 + q] * phv * n3;
-              if (ii == 1)
-                return l2m * G[1 * SG + gm * NQ2 + q] * phv * n2 + mu * G[0 * SG + gm * NQ2 + q] * phv * n1 +
-                       mu * G[2 * SG + gm * NQ2 + q] * phv * n3;
-              return l2m * G[2 * SG + gm * NQ2 + q] * phv * n3 + mu * G[1 * SG + gm * NQ2 + q] * phv * n2 +
-                     mu * G[0 * SG + gm * NQ2 + q] * phv * n1;
-            }
-            return lam * G[ii * SG + gm * NQ2 + q] * phv * nrm[jj] +
-                   mu * G[jj * SG + gm * NQ2 + q] * phv * nrm[ii];
-          };
-          const double tI = itemp(g1, mm, p1[nn * NQ2 + q], i, j);
-          const double tIt = itemp(g1, nn, p1[mm * NQ2 + q], j, i);
-          if (!interior) {
-            i1 = i1 + w * ar * tI;
-            i1t = i1t + w * ar * tIt;
-          } else {
-            i1 = i1 + 0.5 * w * ar * tI;
-            i1t = i1t + 0.5 * w * ar * tIt;
-            const double tI2 = itemp(g1, mm, p2[nn * NQ2 + q], i, j);
-            i2 = i2 - 0.5 * w * ar * tI2;
-            const double tIT2 = itemp(g2, nn, p1[mm * NQ2 + q], i, j);
-            it2 = it2 + 0.5 * w * ar * tIT2;
-            double t3 = (i == j) ? (p1[mm * NQ2 + q] * p2[nn * NQ2 + q]) * dd[i]
-                                 : 0.5 * p1[mm * NQ2 + q] * p2[nn * NQ2 + q] * ni * nj;
-            s2 = s2 - sigma * w * t3 * ar;
-          }
-        }
-        const size_t o = kpos(N3, i * NP + mm, j * NP + nn);
-        Ks[o] = Ks[o] + s1;
-        if (keepA) As[o] = As[o] + s1;
-        Ks[o] = Ks[o] + theta * i1 - i1t;
-        if (interior) {
-          Kb[o] = Kb[o] + theta * i2 + s2;
-          if (keepA) Ab[o] = Ab[o] + s2;
-          Kb[o] = Kb[o] - it2;
-        }
-      }
-    }
+// Row d of affine_map's matrix from the tet's vertices (same expressions).
+__device__ __forceinline__ void affine_row(const double* __restrict__ v, int d, double (&r)[4]) {
+  const double x1 = v[d], x2 = v[3 + d], x3 = v[6 + d], x4 = v[9 + d];
+  r[0] = ((0.0 + -1 * x1) + 1 * x2) + 0 * x3 + 0 * x4;
+  r[1] = ((0.0 + -1 * x1) + 0 * x2) + 1 * x3 + 0 * x4;
+  r[2] = ((0.0 + -1 * x1) + 0 * x2) + 0 * x3 + 1 * x4;
+  r[3] = ((0.0 + 1 * x1) + 0 * x2) + 0 * x3 + 0 * x4;
+}
+// Coordinate d of map_point / face_point from row d.
+__device__ __forceinline__ double map_coord(const double (&r)[4], const double* __restrict__ nod4) {
+  double s = 0.0;
+#pragma unroll
+  for (int l = 0; l < 4; ++l) s = s + r[l] * nod4[l];
+  return s;
+}
+__device__ __forceinline__ double face_coord(const double (&r)[4], int face, const double* __restrict__ tri4) {
+  double s = 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    double t = 0.0;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) t = t + r[l] * node_map(face, l, q);
+    s = s + t * tri4[q];
   }
+  return s;
 }
 
-// Operator build, factored form (same operator, fewer flops).  The face and
-// volume terms of MAKE_STIFFNESS_VOLUME / MAKE_STIFFNESS_FACE are bilinear in
-// the basis values, so each is a combination of a few quadrature sums per
-// basis pair (m, n):
+// 1-D values of one bounding box at NQ points: v[d][k][q], dv[d][k][q]
+template <int P, int NQ>
+struct Tab1 {
+  double v[3][P + 1][NQ], dv[3][P + 1][NQ];
+};
+template <int P, int NQ>
+__device__ __forceinline__ void tab1d(Tab1<P, NQ>& t, int d, int q, double x, double lo, double hi) {
+  const double hb = (hi - lo) / 2.0;
+  const double mb = (hi + lo) / 2.0;
+  const double sq = sqrt(hb);
+  const double xp = (x - mb) / hb;
+#pragma unroll
+  for (int k = 0; k <= P; ++k) {
+    t.v[d][k][q] = leg(k, xp) / sq;
+    t.dv[d][k][q] = dleg(k, xp) / (hb * sq);
+  }
+}
+// phi and gradient of the function with degrees (a, b, c) at point q
+template <int P, int NQ>
+__device__ __forceinline__ void basis_row(const Tab1<P, NQ>& t, int a, int b, int c, int q, double& phi, double& d0,
+                                          double& d1, double& d2) {
+  const double v0 = t.v[0][a][q], v1 = t.v[1][b][q], v2 = t.v[2][c][q];
+  phi = v0 * v1 * v2;
+  d0 = t.dv[0][a][q] * v1 * v2;
+  d1 = v0 * t.dv[1][b][q] * v2;
+  d2 = v0 * v1 * t.dv[2][c][q];
+}
+
+// ---------------------------------------------------------------------------
+// Operator build: MAKE_MATRICES_FREE (src/matrix_free.f90:27-464).  A group of
+// TG threads per polyhedron, a basis pair (m, n) with its nine component
+// entries per thread; the tets are
+// processed in order (volume term, then faces 1..4), and the self block's
+// entries stay in registers to the end, so every entry accumulates in the
+// reference's order and is written once; a neighbour's block is stored at its
+// first face and added to at the others.
+//
+// REF evaluates the reference's terms in its operand order.  !REF uses that
+// the face and volume terms of MAKE_STIFFNESS_VOLUME / MAKE_STIFFNESS_FACE are
+// bilinear in the basis values, so each is a combination of a few quadrature
+// sums per basis pair (m, n):
 //   volume:  D_ab = sum_q w|J| d_a phi_m d_b phi_n  (a, b = x, y, z)
 //     V_ii = (l+2m) D_ii + m sum_{a != i} D_aa,  V_ij = l D_ij + m D_ji;
 //   face:    PP = sum w phiP_m phiP_n,  PQ = sum w phiP_m phiQ_n,
@@ -349,226 +225,450 @@ __global__ __launch_bounds__(256) void k_build_operator(MeshDev m, double alpha,
 //     S+ = s ar PP c_ij, I+ = k ar T(i,j;BP), I+^T = k ar T(j,i;BPt),
 //     I- = -ar/2 T(i,j;CP), I-^T = ar/2 T(i,j;DQ), S- = -s ar PQ c_ij,
 //     c_ii = dd_i, c_ij = n_i n_j / 2, k = 1 (Dirichlet) or 1/2 (interior);
-// inserted like k_build_operator (per tet: volume, then faces 1..4).  Each
-// thread owns basis pairs (m, n) for the whole polyhedron and keeps its
-// self-block entries in registers, so every entry accumulates in one fixed
-// order; sums are regrouped relative to the reference, so entries agree with
-// it to rounding (1e-15 relative), not bit for bit.  The mass blocks are
-// summed exactly as k_build_operator does.
-// Threads per workgroup of k_build_factored: at p <= 2 the basis pairs
-// rounded up to whole waves (one pair per thread: 64 and 128 threads, the
-// build 3x and 1.6x faster than with 256); from p = 3 on 256 threads of two
-// or five pairs, two workgroups per CU at p = 3 (448 threads of one pair left
-// room for one and measured 126 ms against 113 ms at 64,000 polyhedra) and no
-// register spills at p = 4.
+// sums are regrouped relative to the reference, so entries agree with it to
+// rounding (1e-15 relative), not bit for bit.  The mass blocks are summed the
+// same way in both.
+//
+// Bound by FP64 instructions (no contraction: the reference's roundings).  A
+// face's transposed consistency term of entry (i, j; m, n) is its plain one of
+// (j, i; n, m), so REF exchanges it through LDS instead of summing it again.
+// What it replaced read its tables with every lane in one bank, evaluated each
+// function's 1-D values (three square roots, six divisions) per point anew and
+// added every tet and face into the blocks in memory.  Milliseconds, then ->
+// now, reference / factored order, both operators, agglomerated cubes: p = 1
+// (64,000 polyhedra) 17.6 -> 1.3 / 7.1 -> 1.1; p = 2 (32,768) 35.9 -> 6.5 / 11.7
+// -> 4.0; p = 3 (13,824) 123 -> 20 / 29.6 -> 10.5; p = 4 (4,096) 233 -> 32 / 31
+// -> 11.  At p = 3 the reference order keeps the FP64 units 62% busy; the
+// factored one waits on LDS and barriers.
+// ---------------------------------------------------------------------------
 template <int P>
-constexpr int factored_threads() {
-  constexpr int pairs = np_of(P) * np_of(P);
-  return pairs <= 128 ? (pairs + 63) / 64 * 64 : 256;
+struct Build {
+  static constexpr int PAIRS = np_of(P) * np_of(P);
+  // p = 1: 16 pairs, four polyhedra a wave; p = 2: 100 pairs in two waves; p =
+  // 3: 400 in seven; p = 4: 1225 in two workgroups of ten (two pairs a thread
+  // in one spilled 210 registers)
+  static constexpr int GP = P == 1 ? 4 : 1;
+  static constexpr int TG = P == 1 ? 16 : (P == 2 ? 128 : (P == 3 ? 448 : 640));
+  static constexpr int SPLIT = (PAIRS + TG - 1) / TG;
+  static constexpr int SHARE = (PAIRS + SPLIT - 1) / SPLIT;  // pairs per workgroup
+  static constexpr int TPB = GP * TG;
+  static constexpr int NQ2 = (P + 1) * (P + 1), NQ3 = NQ2 * (P + 1);
+  static constexpr int NB = P == 1 ? 2 : 8;  // tets fetched at a time
+  static constexpr int QC = P <= 2 ? NQ3 : 2 * NQ2 <= 32 ? 32 : NQ2;  // volume points per table
+  static_assert(NQ3 % QC == 0, "whole chunks of the volume rule");
+};
+
+// acc[3 i + j] += c I(i, j), the consistency term sigma(grad) : (phi (x) n) of
+// :504-515 with the component pattern: gradient (G0, G1, G2) on one side,
+// value ph on the other.
+__device__ __forceinline__ void face_terms(double (&acc)[9], double c, double G0, double G1, double G2, double ph,
+                                           double lam, double mu, double l2m, double n1, double n2, double n3) {
+  const double a0 = l2m * G0 * ph, a1 = l2m * G1 * ph, a2 = l2m * G2 * ph;
+  const double u0 = mu * G0 * ph, u1 = mu * G1 * ph, u2 = mu * G2 * ph;
+  const double l0 = lam * G0 * ph, l1 = lam * G1 * ph, l2 = lam * G2 * ph;
+  const double w0 = u0 * n1, w1 = u1 * n2, w2 = u2 * n3;
+  acc[0] = acc[0] + c * (a0 * n1 + w1 + w2);
+  acc[4] = acc[4] + c * (a1 * n2 + w0 + w2);
+  acc[8] = acc[8] + c * (a2 * n3 + w1 + w0);
+  acc[1] = acc[1] + c * (l0 * n2 + u1 * n1);
+  acc[2] = acc[2] + c * (l0 * n3 + u2 * n1);
+  acc[3] = acc[3] + c * (l1 * n1 + u0 * n2);
+  acc[5] = acc[5] + c * (l1 * n3 + u2 * n2);
+  acc[6] = acc[6] + c * (l2 * n1 + u0 * n3);
+  acc[7] = acc[7] + c * (l2 * n2 + u1 * n3);
 }
 
-template <int P>
-__global__ __launch_bounds__(factored_threads<P>()) void k_build_factored(MeshDev m, double alpha, double theta,
-                                                         double* __restrict__ K,
-                                                         double* __restrict__ A,
-                                                         double* __restrict__ M,
-                                                         double* __restrict__ Mm, int poly0) {
+// What a workgroup needs of a few tets ahead, fetched for all of them at once
+// (one walk tet -> neighbour -> polyhedron -> its box per polyhedron instead
+// of one per face).
+struct BuildFace {
+  double n[3], ar, sigma, bb[6];  // normal, area, penalty, the neighbour's box
+  int Q, blk;                     // neighbour polyhedron (-1: Dirichlet), its block; Q = -2: no term
+};
+struct BuildTet {
+  double v[12], aJ, rho, lam, mu;
+  BuildFace f[4];
+};
+
+template <int P, bool REF, bool ADG>
+__global__ __launch_bounds__(Build<P>::TPB, !REF && (P == 2 || P == 3) ? 4 : 2) void k_build(MeshDev m, double alpha, double theta,
+                                                         double* __restrict__ K, double* __restrict__ A,
+                                                         double* __restrict__ M, double* __restrict__ Mm,
+                                                         int n_poly) {
   using D = Dims<P>;
-  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2;
-  constexpr int VOLSZ = 4 * NP * NQ3, FACESZ = 8 * NP * NQ2;
-  constexpr int SHSZ = VOLSZ > FACESZ ? VOLSZ : FACESZ;
-  constexpr int PAIRS = NP * NP;
-  constexpr int TPB = factored_threads<P>();
-  constexpr int PPT = (PAIRS + TPB - 1) / TPB;  // pairs per thread
-  __shared__ double sh[SHSZ];
-  __shared__ double spt[NQ3 * 3];
-  __shared__ double swq[NQ3];
+  using B = Build<P>;
+  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2, QC = B::QC, GP = B::GP, TG = B::TG,
+                PAIRS = B::PAIRS;
+  constexpr bool XCHG = REF && B::SPLIT == 1;  // the transposed pair's term is in this workgroup
+  constexpr int VOLSZ = 4 * NP * QC, FACESZ = 8 * NP * NQ2, NB = B::NB;
+  union Tabs {
+    Tab1<P, QC> vol;
+    Tab1<P, NQ2> face[2];
+  };
+  __shared__ double shT[GP][VOLSZ > FACESZ ? VOLSZ : FACESZ];
+  __shared__ Tabs sh1[GP];
+  __shared__ double shw[GP][QC > NQ2 ? QC : NQ2][2];
+  __shared__ double shX[GP][XCHG ? 9 : 1][XCHG ? PAIRS : 1];
+  __shared__ BuildTet shS[GP][NB];
+  __shared__ double sq3[NQ3 * 4], sw3[NQ3], sq2[NQ2 * 4], sw2[NQ2], sbb[GP][6];
   __shared__ int sbl[NP * 3];
-  const int tid = threadIdx.x;
-  const int Pp = poly0 + blockIdx.x;
-  const bool keepA = A != nullptr;
-  for (int i = tid; i < NP * 3; i += blockDim.x) sbl[i] = m.blist[i];
-  double bbP[6];
-  for (int d = 0; d < 6; ++d) bbP[d] = m.bbox[Pp * 6 + d];
+  const int tid = threadIdx.x, grp = GP == 1 ? 0 : tid / TG, lt = GP == 1 ? tid : tid % TG;
+  const int Pr = (int)(blockIdx.x / B::SPLIT) * GP + grp, half = blockIdx.x % B::SPLIT;
+  const bool poly = GP == 1 || Pr < n_poly;
+  const int Pp = poly ? Pr : n_poly - 1;  // a group past the end computes along and stores nothing
+  double* const T = shT[grp];
+  Tabs& t1 = sh1[grp];
+  double(*const sw)[2] = shw[grp];
+  for (int i = tid; i < NP * 3; i += B::TPB) sbl[i] = m.blist[i];
+  for (int i = tid; i < NQ3 * 4; i += B::TPB) sq3[i] = m.qtet[i];
+  for (int i = tid; i < NQ2 * 4; i += B::TPB) sq2[i] = m.qtri[i];
+  for (int i = tid; i < NQ3; i += B::TPB) sw3[i] = m.wtet[i];
+  for (int i = tid; i < NQ2; i += B::TPB) sw2[i] = m.wtri[i];
+  double* const bbP = sbb[grp];
+  if (lt < 6) bbP[lt] = m.bbox[(size_t)Pp * 6 + lt];
   const double hkP = m.hk[Pp];
-  double* Ks = K + (size_t)m.row_ptr[Pp] * D::BS;
-  double* As = keepA ? A + (size_t)m.row_ptr[Pp] * D::BS : nullptr;
-  double* phi = sh;               // [NP][NQ3]
-  double* dphi = sh + NP * NQ3;   // [3][NP][NQ3]
-  double* p1 = sh;                // [NP][NQ2]
-  double* p2 = sh + NP * NQ2;
-  double* g1 = sh + 2 * NP * NQ2; // [3][NP][NQ2]
-  double* g2 = sh + 5 * NP * NQ2;
-  double* MP = M + (size_t)Pp * NP * NP;
-  double* MmP = Mm + (size_t)Pp * NP * NP;
-  for (int a = m.ptet_ptr[Pp]; a < m.ptet_ptr[Pp + 1]; ++a) {
-    const int t = m.ptet[a];
-    double v[12], Fk[12], Jdet;
-    for (int i = 0; i < 12; ++i) v[i] = m.tet_xyz[(size_t)t * 12 + i];
-    affine_map(v, Fk, Jdet);
-    const double aJ = fabs(Jdet);
-    const double rho = m.rho[t], lam = m.lam[t], mu = m.mu[t];
-    const double l2m = lam + 2 * mu;
-    __syncthreads();
-    for (int q = tid; q < NQ3; q += blockDim.x) {
-      map_point(Fk, &m.qtet[q * 4], &spt[q * 3]);
-      swq[q] = m.wtet[q] * aJ;
-    }
-    __syncthreads();
-    for (int e = tid; e < NP * NQ3; e += blockDim.x) {
-      const int f = e / NQ3, q = e % NQ3;
-      double ph, d0, d1, d2;
-      basis_at(&sbl[f * 3], bbP, &spt[q * 3], ph, d0, d1, d2);
-      phi[e] = ph;
-      dphi[(0 * NP + f) * NQ3 + q] = d0;
-      dphi[(1 * NP + f) * NQ3 + q] = d1;
-      dphi[(2 * NP + f) * NQ3 + q] = d2;
-    }
-    __syncthreads();
-    constexpr int SD = NP * NQ3;
-#pragma unroll 1
-    for (int k = 0; k < PPT; ++k) {
-      const int pr = tid + TPB * k;
-      if (pr >= PAIRS) continue;
-      const int mm = pr / NP, nn = pr % NP;
-      double sm = 0.0, Dv[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-#pragma unroll 2
-      for (int q = 0; q < NQ3; ++q) {
-        // mass exactly as k_build_operator sums it
-        sm = sm + 1.0 * m.wtet[q] * aJ * phi[mm * NQ3 + q] * phi[nn * NQ3 + q];
-        const double wq = swq[q];
-        const double gm0 = dphi[mm * NQ3 + q], gm1 = dphi[SD + mm * NQ3 + q],
-                     gm2 = dphi[2 * SD + mm * NQ3 + q];
-        const double gn0 = wq * dphi[nn * NQ3 + q], gn1 = wq * dphi[SD + nn * NQ3 + q],
-                     gn2 = wq * dphi[2 * SD + nn * NQ3 + q];
-        Dv[0][0] += gm0 * gn0; Dv[0][1] += gm0 * gn1; Dv[0][2] += gm0 * gn2;
-        Dv[1][0] += gm1 * gn0; Dv[1][1] += gm1 * gn1; Dv[1][2] += gm1 * gn2;
-        Dv[2][0] += gm2 * gn0; Dv[2][1] += gm2 * gn1; Dv[2][2] += gm2 * gn2;
+  const int r0 = m.row_ptr[Pp], r1 = m.row_ptr[Pp + 1];
+  const int pr = half * B::SHARE + lt;
+  const bool on = lt < B::SHARE && pr < PAIRS;
+  // lanes along the rows: their stores cover whole lines of the column-pair layout
+  const int mm = on ? pr % NP : 0, nn = on ? pr / NP : 0;
+  double sK[9], sA[9], sM = 0.0, sMr = 0.0;
+#pragma unroll
+  for (int e = 0; e < 9; ++e) sK[e] = sA[e] = 0.0;
+  // entry (i, j) of this thread's pair in a block
+  auto at = [&](int i, int j) { return (uint32_t)kpos(N3, i * NP + mm, j * NP + nn); };
+  // blocks of this row stored already (bit = block - r0; longer rows: cleared here)
+  unsigned long long seen = 0ull;
+  if (poly && on)
+    for (int b = r0 + 64; b < r1; ++b)
+      for (int e = 0; e < 9; ++e) {
+        K[(size_t)b * D::BS + at(e / 3, e % 3)] = 0.0;
+        if (ADG) A[(size_t)b * D::BS + at(e / 3, e % 3)] = 0.0;
       }
-      MmP[pr] = MmP[pr] + sm;
-      MP[pr] = MP[pr] + sm * rho;
+  const int a0 = m.ptet_ptr[Pp], cnt = m.ptet_ptr[Pp + 1] - a0;
+  int steps = cnt;  // the workgroup's polyhedra walk their tets together
+  if constexpr (GP > 1) {
+#pragma unroll
+    for (int o = TG; o < 64; o <<= 1) steps = max(steps, __shfl_xor(steps, o, 64));
+  }
+  for (int a = 0; a < steps; ++a) {
+    if (a % NB == 0) {
+      __syncthreads();
+      for (int i = lt; i < 4 * NB; i += TG) {
+        const int c = a + i / 4, f = i % 4;
+        if (c >= cnt) continue;
+        BuildTet& ts = shS[grp][i / 4];
+        const int t = m.ptet[a0 + c], e2 = m.neigh[t * 4 + f];
+        const double lam = m.lam[t], mu = m.mu[t];
+        double v[12];
+        for (int e = 0; e < 12; ++e) v[e] = m.tet_xyz[(size_t)t * 12 + e];
+        const int Q = e2 >= 0 ? m.tet_poly[e2] : -1;
+        BuildFace& fs = ts.f[f];
+        // neither a face inside the polyhedron nor a Neumann face has a term
+        fs.Q = (e2 >= 0 ? Q != Pp : e2 != -2) ? Q : -2;
+        fs.blk = m.face_blk[t * 4 + f];
+        for (int d = 0; d < 3; ++d) fs.n[d] = m.normal[(t * 4 + f) * 3 + d];
+        fs.ar = m.area[t * 4 + f];
+        const double hkQ = Q >= 0 ? m.hk[Q] : hkP;
+        const double Dbar = lam + 2 * mu;
+        const double hmin = hkP < hkQ ? hkP : hkQ;
+        fs.sigma = alpha * (P * P) / hmin * Dbar;
+        if (Q >= 0)
+          for (int e = 0; e < 6; ++e) fs.bb[e] = m.bbox[(size_t)Q * 6 + e];
+        if (f == 0) {
+          double Fk[12], Jdet;
+          affine_map(v, Fk, Jdet);
+          for (int e = 0; e < 12; ++e) ts.v[e] = v[e];
+          ts.aJ = fabs(Jdet);
+          ts.rho = m.rho[t];
+          ts.lam = lam;
+          ts.mu = mu;
+        }
+      }
+      __syncthreads();
+    }
+    const bool tet = a < cnt;
+    const BuildTet& ts = shS[grp][tet ? a % NB : 0];
+    const double lam = ts.lam, mu = ts.mu;
+    const double l2m = lam + 2 * mu;
+    // mass (MAKE_MATRICES_FREE :224-233 with MAKE_MASS_VOLUME) and volume
+    // stiffness (MAKE_STIFFNESS_VOLUME, assemble_element :24-77)
+    double s[9], ms = 0.0;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) s[e] = 0.0;
+#pragma unroll 1
+    for (int q0 = 0; q0 < NQ3; q0 += QC) {
+      for (int i = lt; i < 3 * QC; i += TG) {
+        const int d = i / QC, q = i % QC;
+        double r[4];
+        affine_row(ts.v, d, r);
+        tab1d<P, QC>(t1.vol, d, q, map_coord(r, &sq3[(q0 + q) * 4]), bbP[2 * d], bbP[2 * d + 1]);
+        if (d == 0) sw[q][0] = sw3[q0 + q] * ts.aJ;
+      }
+      __syncthreads();
+      double *phi = T, *dphi = T + NP * QC;  // [q][f], [d][q][f]
+      for (int e = lt; e < NP * QC; e += TG) {
+        const int q = e / NP, f = e % NP;
+        basis_row<P, QC>(t1.vol, sbl[f * 3], sbl[f * 3 + 1], sbl[f * 3 + 2], q, phi[e], dphi[e],
+                         dphi[NP * QC + e], dphi[2 * NP * QC + e]);
+      }
+      __syncthreads();
+#pragma unroll 2
+      for (int q = 0; q < QC; ++q) {
+        const double wj = sw[q][0];
+        ms = ms + wj * phi[q * NP + mm] * phi[q * NP + nn];
+        const double x0 = dphi[q * NP + mm], x1 = dphi[(QC + q) * NP + mm], x2 = dphi[(2 * QC + q) * NP + mm];
+        const double y0 = dphi[q * NP + nn], y1 = dphi[(QC + q) * NP + nn], y2 = dphi[(2 * QC + q) * NP + nn];
+        if constexpr (REF) {
+          const double u0 = mu * x0, u1 = mu * x1, u2 = mu * x2;
+          const double b0 = u0 * y0, b1 = u1 * y1, b2 = u2 * y2;
+          const double l0 = lam * x0, l1 = lam * x1, l2 = lam * x2;
+          s[0] = s[0] + wj * (l2m * x0 * y0 + b1 + b2);
+          s[4] = s[4] + wj * (l2m * x1 * y1 + b0 + b2);
+          s[8] = s[8] + wj * (l2m * x2 * y2 + b0 + b1);
+          s[1] = s[1] + wj * (l0 * y1 + u1 * y0);
+          s[2] = s[2] + wj * (l0 * y2 + u2 * y0);
+          s[3] = s[3] + wj * (l1 * y0 + u0 * y1);
+          s[5] = s[5] + wj * (l1 * y2 + u2 * y1);
+          s[6] = s[6] + wj * (l2 * y0 + u0 * y2);
+          s[7] = s[7] + wj * (l2 * y1 + u1 * y2);
+        } else {
+          const double z0 = wj * y0, z1 = wj * y1, z2 = wj * y2;
+          s[0] += x0 * z0; s[1] += x0 * z1; s[2] += x0 * z2;
+          s[3] += x1 * z0; s[4] += x1 * z1; s[5] += x1 * z2;
+          s[6] += x2 * z0; s[7] += x2 * z1; s[8] += x2 * z2;
+        }
+      }
+      __syncthreads();  // the tables' reads are done before they are filled again
+    }
+    if (tet) {
+      sM = sM + ms;
+      sMr = sMr + ms * ts.rho;
 #pragma unroll
       for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-          double val;
-          if (i == j)
-            val = l2m * Dv[i][i] + mu * Dv[(i + 1) % 3][(i + 1) % 3] + mu * Dv[(i + 2) % 3][(i + 2) % 3];
-          else
-            val = lam * Dv[i][j] + mu * Dv[j][i];
-          const size_t o = kpos(N3, i * NP + mm, j * NP + nn);
-          Ks[o] = Ks[o] + val;
-          if (keepA) As[o] = As[o] + val;
+          const int e = 3 * i + j;
+          double val = s[e];
+          if constexpr (!REF) {
+            if (i == j)
+              val = l2m * s[e] + mu * s[4 * ((i + 1) % 3)] + mu * s[4 * ((i + 2) % 3)];
+            else
+              val = lam * s[e] + mu * s[3 * j + i];
+          }
+          sK[e] = sK[e] + val;
+          if (ADG) sA[e] = sA[e] + val;
         }
     }
+    // faces (MAKE_STIFFNESS_FACE, assemble_element :404-661; insertion
+    // src/matrix_free.f90:371-441)
 #pragma unroll 1
     for (int f = 0; f < 4; ++f) {
-      const int e2 = m.neigh[t * 4 + f];
-      int Q = -1;
-      if (e2 >= 0) {
-        Q = m.tet_poly[e2];
-        if (Q == Pp) continue;  // intra-polyhedron face
-      }
-      if (e2 == -2) continue;  // Neumann: no stiffness contribution
-      __syncthreads();
-      for (int q = tid; q < NQ2; q += blockDim.x) face_point(Fk, f, &m.qtri[q * 4], &spt[q * 3]);
-      __syncthreads();
-      double bbQ[6];
-      if (Q >= 0)
-        for (int d = 0; d < 6; ++d) bbQ[d] = m.bbox[Q * 6 + d];
-      for (int e = tid; e < NP * NQ2; e += blockDim.x) {
-        const int fb = e / NQ2, q = e % NQ2;
-        double ph, d0, d1, d2;
-        basis_at(&sbl[fb * 3], bbP, &spt[q * 3], ph, d0, d1, d2);
-        p1[e] = ph;
-        g1[(0 * NP + fb) * NQ2 + q] = d0;
-        g1[(1 * NP + fb) * NQ2 + q] = d1;
-        g1[(2 * NP + fb) * NQ2 + q] = d2;
-        if (Q >= 0) {
-          basis_at(&sbl[fb * 3], bbQ, &spt[q * 3], ph, d0, d1, d2);
-          p2[e] = ph;
-          g2[(0 * NP + fb) * NQ2 + q] = d0;
-          g2[(1 * NP + fb) * NQ2 + q] = d1;
-          g2[(2 * NP + fb) * NQ2 + q] = d2;
-        }
-      }
-      __syncthreads();
-      const double* nrm = &m.normal[(t * 4 + f) * 3];
-      const double n1 = nrm[0], n2 = nrm[1], n3 = nrm[2];
-      const double nv[3] = {n1, n2, n3};
-      const double ar = m.area[t * 4 + f];
-      const double Dbar = lam + 2 * mu;
-      const double hmin = (Q >= 0) ? (hkP < m.hk[Q] ? hkP : m.hk[Q]) : hkP;
-      const double sigma = alpha * (P * P) / hmin * Dbar;
+      const BuildFace& fs = ts.f[f];
+      const int Q = tet ? fs.Q : -2;
+      const bool act = Q != -2, interior = Q >= 0;
+      if (GP == 1 ? !act : !__any(act)) continue;
+      const double n1 = fs.n[0], n2 = fs.n[1], n3 = fs.n[2];
+      const double ar = fs.ar;
       const double d11 = fabs(n1) * fabs(n1) + 0.5 * (fabs(n2) * fabs(n2)) + 0.5 * (fabs(n3) * fabs(n3));
       const double d22 = fabs(n2) * fabs(n2) + 0.5 * (fabs(n1) * fabs(n1)) + 0.5 * (fabs(n3) * fabs(n3));
       const double d33 = fabs(n3) * fabs(n3) + 0.5 * (fabs(n1) * fabs(n1)) + 0.5 * (fabs(n2) * fabs(n2));
       const double dd[3] = {d11, d22, d33};
-      const bool interior = Q >= 0;
-      const double kk = interior ? 0.5 : 1.0;
-      double* Kb = interior ? K + (size_t)m.face_blk[t * 4 + f] * D::BS : nullptr;
-      double* Ab = interior && keepA ? A + (size_t)m.face_blk[t * 4 + f] * D::BS : nullptr;
+      for (int i = lt; i < 3 * NQ2 * (interior ? 2 : 1); i += TG) {
+        const int side = i / (3 * NQ2), d = i / NQ2 % 3, q = i % NQ2;
+        double r[4];
+        affine_row(ts.v, d, r);
+        const double x = face_coord(r, f, &sq2[q * 4]);
+        const double* bb = side ? fs.bb : bbP;
+        tab1d<P, NQ2>(t1.face[side], d, q, x, bb[2 * d], bb[2 * d + 1]);
+        if (side == 0 && d == 0) {
+          const double w = sw2[q];
+          sw[q][0] = REF ? (interior ? 0.5 * w * ar : w * ar) : w;
+          sw[q][1] = fs.sigma * w;
+        }
+      }
+      __syncthreads();
+      double *p1 = T, *p2 = T + NP * NQ2, *g1 = T + 2 * NP * NQ2, *g2 = T + 5 * NP * NQ2;  // [q][f], [d][q][f]
       constexpr int SG = NP * NQ2;
-      // T(i,j;X): the traction pattern of itemp
-      auto Tij = [&](int i, int j, const double* X) -> double {
-        if (i == j) return l2m * nv[i] * X[i] + mu * nv[(i + 1) % 3] * X[(i + 1) % 3] +
-                           mu * nv[(i + 2) % 3] * X[(i + 2) % 3];
-        return lam * nv[j] * X[i] + mu * nv[i] * X[j];
-      };
-#pragma unroll 1
-      for (int k = 0; k < PPT; ++k) {
-        const int pr = tid + TPB * k;
-        if (pr >= PAIRS) continue;
-        const int mm = pr / NP, nn = pr % NP;
-        double PPs = 0.0, PQs = 0.0, BP[3] = {0, 0, 0}, BPt[3] = {0, 0, 0}, CP[3] = {0, 0, 0},
-               DQ[3] = {0, 0, 0};
-#pragma unroll 2
-        for (int q = 0; q < NQ2; ++q) {
-          const double w = m.wtri[q];
-          const double pm = p1[mm * NQ2 + q], pn = p1[nn * NQ2 + q];
-          const double wpm = w * pm, wpn = w * pn;
-          PPs += wpm * pn;
+      for (int e = lt; e < SG * (interior ? 2 : 1); e += TG) {
+        const int side = e / SG, o = e % SG, q = o / NP, fb = o % NP;
+        double* g = side ? g2 : g1;
+        basis_row<P, NQ2>(t1.face[side], sbl[fb * 3], sbl[fb * 3 + 1], sbl[fb * 3 + 2], q,
+                          (side ? p2 : p1)[o], g[o], g[SG + o], g[2 * SG + o]);
+      }
+      __syncthreads();
+      // the neighbour's block: first face to touch it stores, the others add
+      const int blk = interior ? fs.blk : r0;
+      const int bit = blk - r0;
+      const bool fresh = bit < 64 && !(seen >> (bit & 63) & 1ull);
+      if (interior && bit < 64) seen |= 1ull << bit;
+      double* Kb = K + (size_t)blk * D::BS;
+      double* Ab = ADG ? A + (size_t)blk * D::BS : nullptr;
+      if constexpr (REF) {
+        double i1[9], i1t[9];  // the term and its transpose: entry (j, i) of the pair (n, m)
+        // S_E1 (:476-490): the same for (i, j) and (j, i); entries 00 11 22 01 02 12
+        double s1[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            BP[d] += g1[d * SG + mm * NQ2 + q] * wpn;
-            BPt[d] += g1[d * SG + nn * NQ2 + q] * wpm;
+        for (int e = 0; e < 9; ++e) i1[e] = i1t[e] = 0.0;
+#pragma unroll 1
+        for (int q = 0; q < NQ2; ++q) {
+          const double c = sw[q][0], swq = sw[q][1];
+          const double am = p1[q * NP + mm], an = p1[q * NP + nn];
+          const double pp = am * an, hp = 0.5 * am * an;
+          s1[0] = s1[0] + swq * (pp * d11) * ar;
+          s1[1] = s1[1] + swq * (pp * d22) * ar;
+          s1[2] = s1[2] + swq * (pp * d33) * ar;
+          s1[3] = s1[3] + swq * (hp * n1 * n2) * ar;
+          s1[4] = s1[4] + swq * (hp * n1 * n3) * ar;
+          s1[5] = s1[5] + swq * (hp * n2 * n3) * ar;
+          face_terms(i1, c, g1[q * NP + mm], g1[SG + q * NP + mm], g1[2 * SG + q * NP + mm], an, lam, mu, l2m, n1,
+                     n2, n3);
+          if constexpr (!XCHG)
+            face_terms(i1t, c, g1[q * NP + nn], g1[SG + q * NP + nn], g1[2 * SG + q * NP + nn], am, lam, mu, l2m, n1,
+                       n2, n3);
+        }
+        if constexpr (XCHG) {
+          if (on)
+#pragma unroll
+            for (int e = 0; e < 9; ++e) shX[grp][e][nn * NP + mm] = i1[e];
+          __syncthreads();
+#pragma unroll
+          for (int e = 0; e < 9; ++e) i1t[e] = shX[grp][e][mm * NP + nn];
+        }
+        if (act) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const int e = 3 * i + j;
+              const double v1 = s1[i == j ? i : i + j + 2];
+              sK[e] = sK[e] + v1;
+              if (ADG) sA[e] = sA[e] + v1;
+              sK[e] = sK[e] + theta * i1[e] - i1t[3 * j + i];
+            }
+        }
+        if (interior && on) {
+          double s2[6] = {0, 0, 0, 0, 0, 0}, i2[9], it2[9];
+#pragma unroll
+          for (int e = 0; e < 9; ++e) i2[e] = it2[e] = 0.0;
+#pragma unroll 1
+          for (int q = 0; q < NQ2; ++q) {
+            const double c = sw[q][0], swq = sw[q][1];
+            const double am = p1[q * NP + mm], an = p2[q * NP + nn];
+            const double pp = am * an, hp = 0.5 * am * an;
+            s2[0] = s2[0] - swq * (pp * d11) * ar;
+            s2[1] = s2[1] - swq * (pp * d22) * ar;
+            s2[2] = s2[2] - swq * (pp * d33) * ar;
+            s2[3] = s2[3] - swq * (hp * n1 * n2) * ar;
+            s2[4] = s2[4] - swq * (hp * n1 * n3) * ar;
+            s2[5] = s2[5] - swq * (hp * n2 * n3) * ar;
+            face_terms(i2, -c, g1[q * NP + mm], g1[SG + q * NP + mm], g1[2 * SG + q * NP + mm], an, lam, mu, l2m,
+                       n1, n2, n3);
+            face_terms(it2, c, g2[q * NP + nn], g2[SG + q * NP + nn], g2[2 * SG + q * NP + nn], am, lam, mu, l2m,
+                       n1, n2, n3);
           }
-          if (interior) {
-            const double qn = p2[nn * NQ2 + q];
+          if (poly) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+              for (int j = 0; j < 3; ++j) {
+                const uint32_t o = at(i, j);
+                const double v2 = s2[i == j ? i : i + j + 2];
+                const double kb = fresh ? 0.0 : Kb[o];
+                Kb[o] = kb + theta * i2[3 * i + j] + v2 - it2[3 * i + j];
+                if (ADG) Ab[o] = (fresh ? 0.0 : Ab[o]) + v2;
+              }
+          }
+        }
+      } else {
+        const double kk = interior ? 0.5 : 1.0, sigma = fs.sigma;
+        const double nv[3] = {n1, n2, n3};
+        const double dd[3] = {d11, d22, d33};
+        // T(i,j;X): the traction pattern
+        auto Tij = [&](int i, int j, const double* X) -> double {
+          if (i == j) return l2m * nv[i] * X[i] + mu * nv[(i + 1) % 3] * X[(i + 1) % 3] +
+                             mu * nv[(i + 2) % 3] * X[(i + 2) % 3];
+          return lam * nv[j] * X[i] + mu * nv[i] * X[j];
+        };
+        if (act && on) {
+          double PPs = 0.0, BP[3] = {0, 0, 0}, BPt[3] = {0, 0, 0};
+#pragma unroll 2
+          for (int q = 0; q < NQ2; ++q) {
+            const double w = sw[q][0];
+            const double am = p1[q * NP + mm], an = p1[q * NP + nn];
+            const double wpm = w * am, wpn = w * an;
+            PPs += wpm * an;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+              BP[d] += g1[d * SG + q * NP + mm] * wpn;
+              BPt[d] += g1[d * SG + q * NP + nn] * wpm;
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const double cij = (i == j) ? dd[i] : 0.5 * nv[i] * nv[j];
+              const double s1 = sigma * ar * PPs * cij;
+              const double i1 = kk * ar * Tij(i, j, BP);
+              const double i1t = kk * ar * Tij(j, i, BPt);
+              sK[3 * i + j] = sK[3 * i + j] + s1;
+              if (ADG) sA[3 * i + j] = sA[3 * i + j] + s1;
+              sK[3 * i + j] = sK[3 * i + j] + theta * i1 - i1t;
+            }
+        }
+        if (interior && on) {
+          double PQs = 0.0, CP[3] = {0, 0, 0}, DQ[3] = {0, 0, 0};
+#pragma unroll 2
+          for (int q = 0; q < NQ2; ++q) {
+            const double w = sw[q][0];
+            const double wpm = w * p1[q * NP + mm], qn = p2[q * NP + nn];
             const double wqn = w * qn;
             PQs += wpm * qn;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-              CP[d] += g1[d * SG + mm * NQ2 + q] * wqn;
-              DQ[d] += g2[d * SG + nn * NQ2 + q] * wpm;
+              CP[d] += g1[d * SG + q * NP + mm] * wqn;
+              DQ[d] += g2[d * SG + q * NP + nn] * wpm;
             }
           }
+          if (poly)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+              for (int j = 0; j < 3; ++j) {
+                const double cij = (i == j) ? dd[i] : 0.5 * nv[i] * nv[j];
+                const double i2 = -0.5 * ar * Tij(i, j, CP);
+                const double it2 = 0.5 * ar * Tij(i, j, DQ);
+                const double s2 = -(sigma * ar * PQs * cij);
+                const uint32_t o = at(i, j);
+                const double kb = fresh ? 0.0 : Kb[o];
+                Kb[o] = kb + theta * i2 + s2 - it2;
+                if (ADG) Ab[o] = (fresh ? 0.0 : Ab[o]) + s2;
+              }
         }
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            const double cij = (i == j) ? dd[i] : 0.5 * nv[i] * nv[j];
-            const double s1 = sigma * ar * PPs * cij;
-            const double i1 = kk * ar * Tij(i, j, BP);
-            const double i1t = kk * ar * Tij(j, i, BPt);
-            const size_t o = kpos(N3, i * NP + mm, j * NP + nn);
-            Ks[o] = Ks[o] + s1;
-            if (keepA) As[o] = As[o] + s1;
-            Ks[o] = Ks[o] + theta * i1 - i1t;
-            if (interior) {
-              const double i2 = -0.5 * ar * Tij(i, j, CP);
-              const double it2 = 0.5 * ar * Tij(i, j, DQ);
-              const double s2 = -(sigma * ar * PQs * cij);
-              Kb[o] = Kb[o] + theta * i2 + s2;
-              if (keepA) Ab[o] = Ab[o] + s2;
-              Kb[o] = Kb[o] - it2;
-            }
-          }
       }
+      __syncthreads();  // as after a volume chunk
     }
   }
-
+  if (!poly) return;
+  double* Ks = K + (size_t)r0 * D::BS;
+  double* As = ADG ? A + (size_t)r0 * D::BS : nullptr;
+  if (on) {
+    M[(size_t)Pp * NP * NP + mm * NP + nn] = sMr;
+    Mm[(size_t)Pp * NP * NP + mm * NP + nn] = sM;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {
+      Ks[at(e / 3, e % 3)] = sK[e];
+      if (ADG) As[at(e / 3, e % 3)] = sA[e];
+    }
+  }
+  if constexpr (N3 % 2 == 1) {  // the padding column
+    for (int i = lt; i < (r1 - r0) * N3; i += TG) {
+      const size_t o = (size_t)(r0 + i / N3) * D::BS + kpos(N3, i % N3, N3);
+      K[o] = 0.0;
+      if (ADG) A[o] = 0.0;
+    }
+  }
 }
 
 // Cholesky of both mass blocks of a polyhedron (cholesky,
@@ -625,55 +725,75 @@ __global__ __launch_bounds__(64) void k_cholesky(const double* __restrict__ M,
 
 // ---------------------------------------------------------------------------
 // RHS (MAKE_RHS_FREE, src/matrix_free.f90:467-843) and L2 projection
-// (COMPUTE_MODAL_COEFFICIENTS_FREE, :847-997).  One 128-thread workgroup per
-// polyhedron, entry (i, m) owned by one thread.
+// (COMPUTE_MODAL_COEFFICIENTS_FREE, :847-997).  One workgroup per polyhedron,
+// entry (i, m) owned by one thread; bound by the data's sines and the basis
+// values, both formed once per point (tab1d): p = 3, 13,824 polyhedra, RHS 2.07
+// -> 0.88 ms, projection 0.98 -> 0.53 ms.
 // ---------------------------------------------------------------------------
 template <int P>
-__global__ __launch_bounds__(128) void k_rhs(MeshDev m, int prob, double alpha, double theta,
+constexpr int rhs_threads() { return P == 1 ? 64 : (P == 2 ? 128 : 256); }
+
+template <int P>
+__global__ __launch_bounds__(rhs_threads<P>(), 4) void k_rhs(MeshDev m, int prob, double alpha, double theta,
                                              double* __restrict__ rhs,
                                              const double* __restrict__ tabv = nullptr,
                                              const double* __restrict__ tabf = nullptr) {
   using D = Dims<P>;
-  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2;
-  __shared__ double phi[NP * NQ3];
-  __shared__ double gb[3 * NP * NQ2];
-  __shared__ double spt[NQ3 * 3];
+  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2, TPB = rhs_threads<P>();
+  constexpr int VOLSZ = NP * NQ3, FACESZ = 4 * NP * NQ2;
+  union Tabs {
+    Tab1<P, NQ3> vol;
+    Tab1<P, NQ2> face;
+  };
+  __shared__ double T[VOLSZ > FACESZ ? VOLSZ : FACESZ];
+  __shared__ Tabs t1;
   __shared__ double sval[NQ3 * 3];
   __shared__ int sbl[NP * 3];
   const int tid = threadIdx.x;
   const int Pp = blockIdx.x;
-  for (int i = tid; i < NP * 3; i += blockDim.x) sbl[i] = m.blist[i];
-  double bbP[6];
-  for (int d = 0; d < 6; ++d) bbP[d] = m.bbox[Pp * 6 + d];
+  for (int i = tid; i < NP * 3; i += TPB) sbl[i] = m.blist[i];
+  const double* bbP = m.bbox + (size_t)Pp * 6;
   double* r = rhs + (size_t)Pp * N3;
+  const int ci = tid / NP, mm = tid % NP;  // this thread's entry
   double racc = 0.0;  // running rhs entry of this thread
   for (int a = m.ptet_ptr[Pp]; a < m.ptet_ptr[Pp + 1]; ++a) {
     const int t = m.ptet[a];
+    const double* vt = m.tet_xyz + (size_t)t * 12;
     double v[12], Fk[12], Jdet;
-    for (int i = 0; i < 12; ++i) v[i] = m.tet_xyz[(size_t)t * 12 + i];
+    for (int i = 0; i < 12; ++i) v[i] = vt[i];
     affine_map(v, Fk, Jdet);
     const double aJ = fabs(Jdet);
     const double rho = m.rho[t], lam = m.lam[t], mu = m.mu[t];
     __syncthreads();
-    for (int q = tid; q < NQ3; q += blockDim.x) {
-      map_point(Fk, &m.qtet[q * 4], &spt[q * 3]);
-      if (tabv) {  // values of the caller's forcing at k_rhs_points' volume points
-        for (int c = 0; c < 3; ++c) sval[q * 3 + c] = tabv[((size_t)t * NQ3 + q) * 3 + c];
+    for (int i = tid; i < 4 * NQ3; i += TPB) {
+      if (i < NQ3) {  // the data, times the weight
+        double val[3];
+        if (tabv) {  // values of the caller's forcing at k_rhs_points' volume points
+          for (int c = 0; c < 3; ++c) val[c] = tabv[((size_t)t * NQ3 + i) * 3 + c];
+        } else {
+          double x[3];
+          map_point(Fk, &m.qtet[i * 4], x);
+          forcing(prob, lam, mu, x, rho, val);
+        }
+        const double aw = aJ * m.wtet[i];
+        for (int c = 0; c < 3; ++c) sval[i * 3 + c] = aw * val[c];
       } else {
-        forcing(prob, lam, mu, &spt[q * 3], rho, &sval[q * 3]);
+        const int d = i / NQ3 - 1, q = i % NQ3;
+        double rw[4];
+        affine_row(vt, d, rw);
+        tab1d<P, NQ3>(t1.vol, d, q, map_coord(rw, &m.qtet[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
       }
     }
     __syncthreads();
-    for (int e = tid; e < NP * NQ3; e += blockDim.x) {
-      const int f = e / NQ3, q = e % NQ3;
-      double d0, d1, d2;
-      basis_at(&sbl[f * 3], bbP, &spt[q * 3], phi[e], d0, d1, d2);
+    for (int e = tid; e < NP * NQ3; e += TPB) {
+      const int q = e / NP, f = e % NP;
+      T[e] = t1.vol.v[0][sbl[f * 3]][q] * t1.vol.v[1][sbl[f * 3 + 1]][q] * t1.vol.v[2][sbl[f * 3 + 2]][q];
     }
     __syncthreads();
     if (tid < N3) {
-      const int i = tid / NP, mm = tid % NP;
       double s = 0.0;
-      for (int q = 0; q < NQ3; ++q) s = s + aJ * m.wtet[q] * sval[q * 3 + i] * phi[mm * NQ3 + q];
+#pragma unroll 4
+      for (int q = 0; q < NQ3; ++q) s = s + sval[q * 3 + ci] * T[q * NP + mm];
       racc = racc + s;
     }
     for (int f = 0; f < 4; ++f) {
@@ -682,27 +802,33 @@ __global__ __launch_bounds__(128) void k_rhs(MeshDev m, int prob, double alpha, 
       __syncthreads();
       const double* nrm = &m.normal[(t * 4 + f) * 3];
       const int tag = m.bc_space[t * 4 + f];
-      for (int q = tid; q < NQ2; q += blockDim.x) {
-        double xr[3];
-        face_point(Fk, f, &m.qtri[q * 4], &spt[q * 3]);
-        face_point_rhs(Fk, f, &m.qtri[q * 4], xr);
-        if (tabf) {  // the caller's Dirichlet / Neumann data at k_rhs_points' face points
-          for (int c = 0; c < 3; ++c) sval[q * 3 + c] = tabf[(((size_t)t * 4 + f) * NQ2 + q) * 3 + c];
-        } else if (e2 == -1) {
-          dirichlet(prob, xr, tag, &sval[q * 3]);
+      for (int i = tid; i < 4 * NQ2; i += TPB) {
+        if (i < NQ2) {
+          if (tabf) {  // the caller's Dirichlet / Neumann data at k_rhs_points' face points
+            for (int c = 0; c < 3; ++c) sval[i * 3 + c] = tabf[(((size_t)t * 4 + f) * NQ2 + i) * 3 + c];
+          } else {
+            double xr[3];
+            face_point_rhs(Fk, f, &m.qtri[i * 4], xr);
+            if (e2 == -1) dirichlet(prob, xr, tag, &sval[i * 3]);
+            else neumann(prob, lam, mu, nrm, xr, tag, &sval[i * 3]);
+          }
         } else {
-          neumann(prob, lam, mu, nrm, xr, tag, &sval[q * 3]);
+          const int d = i / NQ2 - 1, q = i % NQ2;
+          double rw[4];
+          affine_row(vt, d, rw);
+          tab1d<P, NQ2>(t1.face, d, q, face_coord(rw, f, &m.qtri[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
         }
       }
       __syncthreads();
-      for (int e = tid; e < NP * NQ2; e += blockDim.x) {
-        const int fb = e / NQ2, q = e % NQ2;
-        basis_at(&sbl[fb * 3], bbP, &spt[q * 3], phi[e], gb[(0 * NP + fb) * NQ2 + q],
-                 gb[(1 * NP + fb) * NQ2 + q], gb[(2 * NP + fb) * NQ2 + q]);
+      constexpr int SG = NP * NQ2;
+      for (int e = tid; e < SG; e += TPB) {
+        const int q = e / NP, fb = e % NP;
+        basis_row<P, NQ2>(t1.face, sbl[fb * 3], sbl[fb * 3 + 1], sbl[fb * 3 + 2], q, T[e], T[SG + e], T[2 * SG + e],
+                          T[3 * SG + e]);
       }
       __syncthreads();
       if (tid < N3) {
-        const int i = tid / NP, mm = tid % NP;
+        const int i = ci;
         const double n1 = nrm[0], n2 = nrm[1], n3 = nrm[2];
         const double ar = m.area[t * 4 + f];
         const double l2m = lam + 2 * mu;
@@ -711,10 +837,9 @@ __global__ __launch_bounds__(128) void k_rhs(MeshDev m, int prob, double alpha, 
         for (int q = 0; q < NQ2; ++q) {
           const double w = m.wtri[q];
           const double* dd = &sval[q * 3];
-          const double ph = phi[mm * NQ2 + q];
+          const double ph = T[q * NP + mm];
           if (e2 == -1) {
-            const double gg1 = gb[(0 * NP + mm) * NQ2 + q], gg2 = gb[(1 * NP + mm) * NQ2 + q],
-                         gg3 = gb[(2 * NP + mm) * NQ2 + q];
+            const double gg1 = T[SG + q * NP + mm], gg2 = T[2 * SG + q * NP + mm], gg3 = T[3 * SG + q * NP + mm];
             double tm, t2;
             if (i == 0) {
               tm = l2m * gg1 * dd[0] * n1 + mu * gg2 * dd[0] * n2 + mu * gg3 * dd[0] * n3 +
@@ -825,55 +950,120 @@ __device__ __forceinline__ void solve_packed(const double* __restrict__ R, doubl
   }
 }
 
+// M^-1 of three right-hand sides across one wave, lane i on row i of all three
+// (NP <= 64): the forward sweep broadcasts y_j = s_j / R_jj from lane j and the
+// rows below subtract R_ji y_j (ascending j, as solve_packed), the backward
+// sweep runs the columns from the last.  NP dependent steps per sweep instead
+// of NP(NP+1)/2 on one lane.
+template <int NP>
+__device__ __forceinline__ void solve_rows(const double* __restrict__ R, double& x0, double& x1, double& x2, int i) {
+  static_assert(NP <= 64, "one lane per row");
+  const int ri = pk_off(NP, i < NP ? i : 0);
+#pragma unroll 5
+  for (int j = 0; j < NP; ++j) {
+    const int rj = pk_off(NP, j);
+    const double rjj = R[rj];
+    const double y0 = __shfl(x0, j, 64) / rjj, y1 = __shfl(x1, j, 64) / rjj, y2 = __shfl(x2, j, 64) / rjj;
+    if (i == j) {
+      x0 = y0;
+      x1 = y1;
+      x2 = y2;
+    } else if (i > j && i < NP) {
+      const double r = R[rj + (i - j)];
+      x0 = x0 - r * y0;
+      x1 = x1 - r * y1;
+      x2 = x2 - r * y2;
+    }
+  }
+#pragma unroll 5
+  for (int j = NP - 1; j >= 0; --j) {
+    const double rjj = R[pk_off(NP, j)];
+    const double y0 = __shfl(x0, j, 64) / rjj, y1 = __shfl(x1, j, 64) / rjj, y2 = __shfl(x2, j, 64) / rjj;
+    if (i == j) {
+      x0 = y0;
+      x1 = y1;
+      x2 = y2;
+    } else if (i < j) {
+      const double r = R[ri + (j - i)];
+      x0 = x0 - r * y0;
+      x1 = x1 - r * y1;
+      x2 = x2 - r * y2;
+    }
+  }
+}
+
 template <int P>
-__global__ __launch_bounds__(128) void k_project(MeshDev m, int fn, const double* __restrict__ RMm,
+__global__ __launch_bounds__(rhs_threads<P>(), 4) void k_project(MeshDev m, int fn, const double* __restrict__ RMm,
                                                  double* __restrict__ out,
                                                  const double* __restrict__ tabv) {
   using D = Dims<P>;
-  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3;
+  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, TPB = rhs_threads<P>();
   __shared__ double phi[NP * NQ3];
-  __shared__ double spt[NQ3 * 3];
+  __shared__ Tab1<P, NQ3> t1;
   __shared__ double sval[NQ3 * 3];
   __shared__ double sb[N3];
+  __shared__ double sR[D::NPK];
   __shared__ int sbl[NP * 3];
   const int tid = threadIdx.x;
   const int Pp = blockIdx.x;
-  for (int i = tid; i < NP * 3; i += blockDim.x) sbl[i] = m.blist[i];
-  double bbP[6];
-  for (int d = 0; d < 6; ++d) bbP[d] = m.bbox[Pp * 6 + d];
+  for (int i = tid; i < NP * 3; i += TPB) sbl[i] = m.blist[i];
+  for (int i = tid; i < D::NPK; i += TPB) sR[i] = RMm[(size_t)Pp * D::NPK + i];
+  const double* bbP = m.bbox + (size_t)Pp * 6;
+  const int ci = tid / NP, mm = tid % NP;
   double acc = 0.0;
   for (int a = m.ptet_ptr[Pp]; a < m.ptet_ptr[Pp + 1]; ++a) {
     const int t = m.ptet[a];
+    const double* vt = m.tet_xyz + (size_t)t * 12;
     double v[12], Fk[12], Jdet;
-    for (int i = 0; i < 12; ++i) v[i] = m.tet_xyz[(size_t)t * 12 + i];
+    for (int i = 0; i < 12; ++i) v[i] = vt[i];
     affine_map(v, Fk, Jdet);
     const double aJ = fabs(Jdet);
     __syncthreads();
-    for (int q = tid; q < NQ3; q += blockDim.x) {
-      map_point(Fk, &m.qtet[q * 4], &spt[q * 3]);
-      if (tabv) {  // the caller's field at k_rhs_points' volume points
-        for (int c = 0; c < 3; ++c) sval[q * 3 + c] = tabv[((size_t)t * NQ3 + q) * 3 + c];
+    for (int i = tid; i < 4 * NQ3; i += TPB) {
+      if (i < NQ3) {  // the field, times the weight
+        double val[3];
+        if (tabv) {  // the caller's field at k_rhs_points' volume points
+          for (int c = 0; c < 3; ++c) val[c] = tabv[((size_t)t * NQ3 + i) * 3 + c];
+        } else {
+          double x[3];
+          map_point(Fk, &m.qtet[i * 4], x);
+          field(fn, x, val);
+        }
+        const double aw = aJ * m.wtet[i];
+        for (int c = 0; c < 3; ++c) sval[i * 3 + c] = aw * val[c];
       } else {
-        field(fn, &spt[q * 3], &sval[q * 3]);
+        const int d = i / NQ3 - 1, q = i % NQ3;
+        double rw[4];
+        affine_row(vt, d, rw);
+        tab1d<P, NQ3>(t1, d, q, map_coord(rw, &m.qtet[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
       }
     }
     __syncthreads();
-    for (int e = tid; e < NP * NQ3; e += blockDim.x) {
-      const int f = e / NQ3, q = e % NQ3;
-      double d0, d1, d2;
-      basis_at(&sbl[f * 3], bbP, &spt[q * 3], phi[e], d0, d1, d2);
+    for (int e = tid; e < NP * NQ3; e += TPB) {
+      const int q = e / NP, f = e % NP;
+      phi[e] = t1.v[0][sbl[f * 3]][q] * t1.v[1][sbl[f * 3 + 1]][q] * t1.v[2][sbl[f * 3 + 2]][q];
     }
     __syncthreads();
-    if (tid < N3) {
-      const int i = tid / NP, mm = tid % NP;
-      for (int q = 0; q < NQ3; ++q) acc = acc + aJ * m.wtet[q] * sval[q * 3 + i] * phi[mm * NQ3 + q];
-    }
+    if (tid < N3)
+#pragma unroll 4
+      for (int q = 0; q < NQ3; ++q) acc = acc + sval[q * 3 + ci] * phi[q * NP + mm];
   }
   if (tid < N3) sb[tid] = acc;
   __syncthreads();
-  if (tid < 3) solve_packed<NP>(RMm + (size_t)Pp * D::NPK, sb + tid * NP);
-  __syncthreads();
-  if (tid < N3) out[(size_t)Pp * N3 + tid] = sb[tid];
+  if (tid >= 64) return;  // one wave solves the three components
+  const bool row = tid < NP;
+  double x0 = row ? sb[tid] : 0.0, x1 = row ? sb[NP + tid] : 0.0, x2 = row ? sb[2 * NP + tid] : 0.0;
+  solve_rows<NP>(sR, x0, x1, x2, tid);
+  if (row) {
+    double* o = out + (size_t)Pp * N3 + tid;
+    o[0] = x0;
+    o[NP] = x1;
+    o[2 * NP] = x2;
+  }
+}
+
+__global__ void k_fill(double* __restrict__ a, double v, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -2828,14 +3018,22 @@ __global__ void k_l2_terms(const double* __restrict__ Mm, const double* __restri
   part[id] = el;
 }
 
-// Sequential sum in index order (the reference accumulates the error terms
-// element by element); one thread: called once per error evaluation.
-__global__ void k_seq_sum(const double* __restrict__ part, int n, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s = s + part[i];
-    out[0] = s;
+// Sum of n error terms by one workgroup in a fixed order: thread t adds terms
+// t, t + 1024, ... eight at a time, then a tree over the threads.  (One thread
+// adding them one after the other, as the reference's element loop does, took
+// 3.3 ms on average for 28,606 and 85,818 terms; this 9.4 us.)
+__global__ __launch_bounds__(1024) void k_sum_terms(const double* __restrict__ part, int n, double* __restrict__ out) {
+  __shared__ double red[1024];
+  double s = 0.0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < n; i += 1024) s = s + part[i];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = 512; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
+    __syncthreads();
   }
+  if (threadIdx.x == 0) out[0] = red[0];
 }
 
 __global__ void k_sub(const double* __restrict__ a, const double* __restrict__ b,

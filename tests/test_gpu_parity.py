@@ -839,3 +839,34 @@ def test_double_couple_sources_match_oracle(name, p):
     assert t_gpu == t
     assert np.abs(un).max() > 0
     assert rel(u, un) < 1e-11, rel(u, un)
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("build", ["reference", "factored"])
+def test_build_of_a_polyhedron_with_a_long_block_row(p, build):
+    """One polyhedron of a 5^3 cube's inner tets with more than 64 single-tet
+    neighbours (the build tracks the first 64 blocks of a row as stored or
+    not, and clears the rest): every block against the oracle's to 1e-13, on
+    memory that held another operator before."""
+    m0 = M.cube_mesh(5)
+    bc = m0.xyz[m0.tet_vert].mean(axis=1)
+    inner = np.abs(bc - 0.5).max(axis=1) < 0.25
+    poly = np.cumsum(~inner)  # 0 = the inner polyhedron
+    poly[inner] = 0
+    _, poly = np.unique(poly, return_inverse=True)
+    m = M.Mesh(m0.xyz, m0.tet_vert, poly, m0.tria_vert, m0.tria_tag, m0.tag_space)
+    o = oracle_for(m, p)
+    o.build_operator()
+    with L.Context(m, p) as ctx:
+        ctx.set_build("factored")
+        ctx.make_matrices_free()
+        ctx.set_build(build)
+        ctx.make_matrices_free()
+        rp, _ = ctx.pattern()
+        assert np.diff(rp).max() > 65, np.diff(rp).max()
+        say(f"[long row] p={p} {build}: {np.diff(rp).max()} blocks")
+        K, A, _, _ = ctx.export_operator()
+        oK, oA = o.K(), o.Adg()
+        for b in range(K.shape[0]):
+            assert rel(K[b], oK[b]) < 1e-13, (b, rel(K[b], oK[b]))
+            assert rel(A[b], oA[b]) < 1e-13
