@@ -179,33 +179,30 @@ int dispatch_p(int p, F&& f) {
   return fail(LYMPH_ERR_ARG, "polynomial degree must be 1..4");
 }
 
-// Step-kernel variants per degree: (column pairs per unrolled load group,
-// neighbour-coefficient broadcast mode); index 0 is the default until
-// lymph_autotune picks one.
 // Step-kernel variants per degree: column pairs per unrolled load group,
 // neighbour-coefficient broadcast mode (0 scalar loads, 1 lane broadcast,
 // 2 packed: 64/3Np polyhedra per wave, coefficients through LDS), waves per
-// polyhedron; index 0 is the default until lymph_autotune picks one.
+// polyhedron; default_variant() names the one a context starts with.
 template <int P> struct StepVar;
 template <> struct StepVar<1> {
-  static constexpr int unr[] = {6, 6, 3, 2, 6, 1, 1, 1, 1};
-  static constexpr int xs[] = {1, 0, 1, 1, 1, 2, 3, 2, 3};
-  static constexpr int wpp[] = {1, 1, 1, 1, 2, 1, 1, 4, 4};
+  static constexpr int unr[] = {6, 6, 3, 2, 6, 1, 1, 1, 1, 6, 6};
+  static constexpr int xs[] = {1, 0, 1, 1, 1, 2, 3, 2, 3, 1, 1};
+  static constexpr int wpp[] = {1, 1, 1, 1, 2, 1, 1, 4, 4, 4, 8};
 };
 template <> struct StepVar<2> {
-  static constexpr int unr[] = {5, 5, 15, 3, 15, 5, 5, 1, 1, 1, 1};
-  static constexpr int xs[] = {1, 0, 1, 1, 0, 1, 1, 2, 3, 2, 3};
-  static constexpr int wpp[] = {1, 1, 1, 1, 1, 2, 4, 1, 1, 4, 4};
+  static constexpr int unr[] = {5, 5, 15, 3, 15, 5, 5, 1, 1, 1, 1, 15, 15};
+  static constexpr int xs[] = {1, 0, 1, 1, 0, 1, 1, 2, 3, 2, 3, 1, 1};
+  static constexpr int wpp[] = {1, 1, 1, 1, 1, 2, 4, 1, 1, 4, 4, 4, 8};
 };
 template <> struct StepVar<3> {
-  static constexpr int unr[] = {10, 10, 5, 6, 15, 30, 30, 3, 30, 10, 30, 15};
-  static constexpr int xs[] = {1, 0, 1, 1, 1, 1, 0, 1, 1, 1, 1, 1};
-  static constexpr int wpp[] = {1, 1, 1, 1, 1, 1, 1, 1, 2, 4, 4, 2};
+  static constexpr int unr[] = {10, 10, 5, 6, 15, 30, 30, 3, 30, 10, 30, 15, 30};
+  static constexpr int xs[] = {1, 0, 1, 1, 1, 1, 0, 1, 1, 1, 1, 1, 1};
+  static constexpr int wpp[] = {1, 1, 1, 1, 1, 1, 1, 1, 2, 4, 4, 2, 8};
 };
 template <> struct StepVar<4> {
-  static constexpr int unr[] = {4, 4, 2, 8, 1, 4, 4, 4, 2, 8, 8};
-  static constexpr int xs[] = {1, 0, 1, 1, 1, 0, 1, 0, 1, 1, 0};
-  static constexpr int wpp[] = {1, 1, 1, 1, 1, 2, 2, 4, 4, 4, 4};
+  static constexpr int unr[] = {4, 4, 2, 8, 1, 4, 4, 4, 2, 8, 8, 8, 14, 14};
+  static constexpr int xs[] = {1, 0, 1, 1, 1, 0, 1, 0, 1, 1, 0, 0, 1, 1};
+  static constexpr int wpp[] = {1, 1, 1, 1, 1, 2, 2, 4, 4, 4, 4, 8, 4, 8};
 };
 template <int P> constexpr int n_var() { return (int)(sizeof(StepVar<P>::unr) / sizeof(int)); }
 
@@ -257,24 +254,24 @@ void launch_leapfrog(int variant, int grid, hipStream_t st, const double* K, con
 
 template <int P> struct StepVar32;
 template <> struct StepVar32<1> {
-  static constexpr int unr[] = {3, 1, 3, 1, 1, 1, 1};
-  static constexpr int wpp[] = {1, 1, 2, 1, 1, 4, 4};
-  static constexpr int pk[] = {0, 0, 0, 1, 2, 1, 2};
+  static constexpr int unr[] = {3, 1, 3, 1, 1, 1, 1, 3, 3};
+  static constexpr int wpp[] = {1, 1, 2, 1, 1, 4, 4, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 1, 2, 1, 2, 0, 0};
 };
 template <> struct StepVar32<2> {
-  static constexpr int unr[] = {4, 2, 8, 4, 4, 1, 1, 1, 1};
-  static constexpr int wpp[] = {1, 1, 1, 2, 4, 1, 1, 4, 4};
-  static constexpr int pk[] = {0, 0, 0, 0, 0, 1, 2, 1, 2};
+  static constexpr int unr[] = {4, 2, 8, 4, 4, 1, 1, 1, 1, 8, 8};
+  static constexpr int wpp[] = {1, 1, 1, 2, 4, 1, 1, 4, 4, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 0, 0, 1, 2, 1, 2, 0, 0};
 };
 template <> struct StepVar32<3> {
-  static constexpr int unr[] = {5, 3, 15, 5, 5, 15, 15, 8};
-  static constexpr int wpp[] = {1, 1, 1, 2, 4, 2, 4, 4};
-  static constexpr int pk[] = {0, 0, 0, 0, 0, 0, 0, 0};
+  static constexpr int unr[] = {5, 3, 15, 5, 5, 15, 15, 8, 15};
+  static constexpr int wpp[] = {1, 1, 1, 2, 4, 2, 4, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 };
 template <> struct StepVar32<4> {
-  static constexpr int unr[] = {3, 1, 9, 3, 3, 9, 9, 13};
-  static constexpr int wpp[] = {1, 1, 1, 2, 4, 2, 4, 4};
-  static constexpr int pk[] = {0, 0, 0, 0, 0, 0, 0, 0};
+  static constexpr int unr[] = {3, 1, 9, 3, 3, 9, 9, 13, 13, 26};
+  static constexpr int wpp[] = {1, 1, 1, 2, 4, 2, 4, 4, 8, 4};
+  static constexpr int pk[] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 };
 template <int P> constexpr int n_var32() { return (int)(sizeof(StepVar32<P>::unr) / sizeof(int)); }
 // 48-bit apply (k_leapfrog48): column quads per load group, waves per
@@ -282,24 +279,24 @@ template <int P> constexpr int n_var32() { return (int)(sizeof(StepVar32<P>::unr
 // workgroup; pk = 2: the same with the joint block walk; p <= 2)
 template <int P> struct StepVar48;
 template <> struct StepVar48<1> {  // quads per load group: even (the corrections come in quad pairs)
-  static constexpr int unr[] = {4, 4, 4, 1, 1, 1, 1};
-  static constexpr int wpp[] = {1, 2, 4, 1, 4, 1, 4};
-  static constexpr int pk[] = {0, 0, 0, 1, 1, 2, 2};
+  static constexpr int unr[] = {4, 4, 4, 1, 1, 1, 1, 4};
+  static constexpr int wpp[] = {1, 2, 4, 1, 4, 1, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 1, 1, 2, 2, 0};
 };
 template <> struct StepVar48<2> {
-  static constexpr int unr[] = {8, 8, 8, 1, 1, 1, 1};
-  static constexpr int wpp[] = {1, 2, 4, 1, 4, 1, 4};
-  static constexpr int pk[] = {0, 0, 0, 1, 1, 2, 2};
+  static constexpr int unr[] = {8, 8, 8, 1, 1, 1, 1, 8};
+  static constexpr int wpp[] = {1, 2, 4, 1, 4, 1, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 1, 1, 2, 2, 0};
 };
 template <> struct StepVar48<3> {
-  static constexpr int unr[] = {6, 16, 6, 16, 6, 16};
-  static constexpr int wpp[] = {1, 1, 2, 2, 4, 4};
-  static constexpr int pk[] = {0, 0, 0, 0, 0, 0};
+  static constexpr int unr[] = {6, 16, 6, 16, 6, 16, 16};
+  static constexpr int wpp[] = {1, 1, 2, 2, 4, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 0, 0, 0, 0};
 };
 template <> struct StepVar48<4> {
-  static constexpr int unr[] = {14, 14, 14};
-  static constexpr int wpp[] = {1, 2, 4};
-  static constexpr int pk[] = {0, 0, 0};
+  static constexpr int unr[] = {14, 14, 14, 14};
+  static constexpr int wpp[] = {1, 2, 4, 8};
+  static constexpr int pk[] = {0, 0, 0, 0};
 };
 template <int P> constexpr int n_var48() { return (int)(sizeof(StepVar48<P>::unr) / sizeof(int)); }
 // lymph_autotune reports into caller arrays of 16 entries
@@ -394,6 +391,49 @@ void launch_leapfrog48(int variant, int grid, hipStream_t st, const float* K, co
     }
     launch_leapfrog48<P, MODE, I + 1>(variant, grid, st, K, Kr, rp, col, rs, rd, u, wa, out, g, c1,
                                       c2, gsel, gtab, ord, dyn);
+  }
+}
+
+// The step variant a context starts with (before lymph_autotune or
+// lymph_set_step_variant), by apply, degree and mesh.  What decides is whether
+// the polyhedra alone fill the chip's 1024 SIMDs:
+//  - few polyhedra (below 256, or below 1024 where uneven polyhedra make long
+//    block rows): the step is one chain of memory trips, so 8 waves share a
+//    polyhedron and each has a whole block in flight.  125 polyhedra, us per
+//    step, one wave per polyhedron / 8 waves: FP64 p = 1..4 5.9 / 3.9, 12.5 /
+//    5.9, 30.7 / 12.0, 96 / 34; 32-bit 5.0 / 3.0, 12.2 / 3.3, 17.3 / 4.7, 53 /
+//    11; 48-bit p = 2, 3 9.9 / 4.1, 30.2 / 6.3;
+//  - up to 3000 polyhedra 4 waves (p <= 2; 1000 polyhedra, FP64 p = 2: 11.9
+//    us against 24.8 with one wave and 13.5 with 8);
+//  - beyond, p <= 2 packs 64 / 3Np polyhedra into a wave (32,768 polyhedra, p
+//    = 1: FP64 83 -> 45 us, 32-bit 58 -> 25; p = 2 32-bit 199 -> 138);
+//  - p >= 3 keeps several waves at every size: a wave's 64 lanes then stream
+//    consecutive blocks (32,768 polyhedra, p = 3: FP64 1004 -> 937 us, 32-bit
+//    513 -> 468 with 8, 48-bit 771 -> 704).  With the 5-block rows of
+//    single-tet polyhedra 8 waves leave three idle: 4 (2 for 48-bit p = 4).
+int default_variant(const LymphCtx* c, int bits) {
+  const int n = c->n_poly;
+  const bool uneven = c->order != nullptr;
+  const bool few = n < 256 || (uneven && n < 1024);
+  const bool mid = n < 3000;
+  const bool long_rows = c->n_blk >= 6 * (size_t)n;
+  switch (c->p) {
+    case 1:
+      if (bits == 64) return n < 2000 ? 10 : (mid ? 9 : (uneven ? 6 : 5));
+      if (bits == 32) return n < 2000 ? 8 : (mid ? 7 : (uneven || n >= 16384 ? 6 : 3));
+      return n < 2000 ? 7 : (mid ? 2 : (uneven || n >= 16384 ? 5 : 3));
+    case 2:
+      if (bits == 64) return few ? 12 : (mid ? 11 : 8);
+      if (bits == 32) return n < 2000 ? 10 : (mid ? 9 : 7);
+      return few ? 7 : (mid ? 2 : 4);
+    case 3:
+      if (bits == 64) return few ? 12 : 10;
+      if (bits == 32) return few || (long_rows && !mid) ? 8 : 6;
+      return few || long_rows || !mid ? 6 : 5;
+    default:
+      if (bits == 64) return 13;
+      if (bits == 32) return few ? 8 : 7;
+      return n < 256 ? 3 : (long_rows ? 2 : 1);
   }
 }
 
@@ -1163,6 +1203,7 @@ int lymph_ctx_create(const LymphMesh* mesh, int p, double alpha, double theta, L
   m.bbox = d_bbox; m.hk = d_hk; m.ptet_ptr = d_ptr; m.ptet = d_ptet; m.row_ptr = d_rowp;
   m.col = d_col; m.face_blk = d_fblk; m.qtet = d_qtet; m.wtet = d_wtet; m.qtri = d_qtri;
   m.wtri = d_wtri; m.blist = d_bl;
+  c->step_variant = default_variant(c, 64);
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     lymph_ctx_destroy(c);
     return fail(LYMPH_ERR_HIP, "hipStreamCreate failed");
@@ -1815,7 +1856,7 @@ int lymph_set_apply_precision(LymphCtx* c, int bits) {
   if (bits != 64)
     if (int rc = sym32_build(c)) return rc;  // pairs stored once: the 32- and 48-bit copies too
   c->apply_bits = bits;
-  c->step_variant = 0;
+  c->step_variant = default_variant(c, bits);
   return 0;
 }
 

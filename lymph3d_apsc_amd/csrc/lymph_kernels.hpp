@@ -895,64 +895,41 @@ __global__ void k_rhs_points(MeshDev m, int n_tet, double* __restrict__ vpts,
   }
 }
 
-// Forward/backward substitution with the packed factor in the reference's
-// order (solve_LU with L = R^T, src/vet_mat_operations.f90:123-153); x in place.
-// M^-1 w = R^-1 R^-T w across one wave, lane = (component cc, row ii) of a
-// 3Np <= 64 vector held one entry per lane (lanes >= 3Np pass through): the
-// forward sweep broadcasts y_j = s_j / R_jj from lane (cc, j) and the rows
-// below subtract R_ji y_j (ascending j, as solve_packed); the backward sweep
-// runs the columns from the last, the rows above subtracting R_ij x_j.  NP
-// dependent steps per sweep instead of Np(Np+1)/2 on one lane.
+// M^-1 w = R^-1 R^-T w (solve_LU with L = R^T, src/vet_mat_operations.f90:
+// 123-153) across a group of 3Np lanes from lane `base`, one entry of the
+// vector per lane: r = component x Np + row (other lanes pass through).  The
+// forward sweep broadcasts y_j = s_j / R_jj and the rows below subtract R_ji
+// y_j, in ascending j as the reference does; the backward sweep runs the
+// columns from the last, the rows above subtracting R_ij x_j.  NP dependent
+// steps per sweep instead of Np(Np+1)/2 on one lane, which the step kernels'
+// tails paid before (125 polyhedra: 6 us of a step at p = 2, 50 at p = 4).
 template <int NP>
-__device__ __forceinline__ double solve_wave(const double* __restrict__ R, double w, int lane) {
-  const bool row = lane < 3 * NP;
-  const int cc = lane / NP, ii = lane % NP;
+__device__ __forceinline__ double solve_group(const double* __restrict__ R, double w, int base, int r, bool on) {
+  const int cc = on ? r / NP : 0, ii = r % NP, from = on ? base + cc * NP : 0;
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const int rj = pk_off(NP, j);
-    const double yj = __shfl(w, row ? cc * NP + j : j, 64) / R[rj];
-    if (row && ii == j)
+    const double yj = __shfl(w, from + j, 64) / R[rj];
+    if (on && ii == j)
       w = yj;
-    else if (row && ii > j)
+    else if (on && ii > j)
       w = w - R[rj + (ii - j)] * yj;
   }
-  const int ri = pk_off(NP, row ? ii : 0);
+  const int ri = pk_off(NP, on ? ii : 0);
 #pragma unroll
   for (int j = NP - 1; j >= 0; --j) {
-    const double xj = __shfl(w, row ? cc * NP + j : j, 64) / R[pk_off(NP, j)];
-    if (row && ii == j)
+    const double xj = __shfl(w, from + j, 64) / R[pk_off(NP, j)];
+    if (on && ii == j)
       w = xj;
-    else if (row && ii < j)
+    else if (on && ii < j)
       w = w - R[ri + (j - ii)] * xj;
   }
   return w;
 }
 
-template <int NP>
-__device__ __forceinline__ void solve_packed(const double* __restrict__ R, double* x) {
-  // loops kept rolled: fully unrolled, the compiler hoists all Np(Np+1)/2
-  // factor entries into registers and the step kernel drops to one wave/SIMD
-  x[0] = x[0] / R[0];
-#pragma unroll 1
-  for (int i = 1; i < NP; ++i) {
-    double s = x[i];
-#pragma unroll 1
-    for (int j = 0; j < i; ++j) s = s - R[pk_off(NP, j) + (i - j)] * x[j];
-    x[i] = s / R[pk_off(NP, i)];
-  }
-  x[NP - 1] = x[NP - 1] / R[pk_off(NP, NP - 1)];
-#pragma unroll 1
-  for (int i = NP - 2; i >= 0; --i) {
-    double s = x[i];
-#pragma unroll 1
-    for (int j = i + 1; j < NP; ++j) s = s - R[pk_off(NP, i) + (j - i)] * x[j];
-    x[i] = s / R[pk_off(NP, i)];
-  }
-}
-
 // M^-1 of three right-hand sides across one wave, lane i on row i of all three
 // (NP <= 64): the forward sweep broadcasts y_j = s_j / R_jj from lane j and the
-// rows below subtract R_ji y_j (ascending j, as solve_packed), the backward
+// rows below subtract R_ji y_j (ascending j), the backward
 // sweep runs the columns from the last.  NP dependent steps per sweep instead
 // of NP(NP+1)/2 on one lane.
 template <int NP>
@@ -1079,6 +1056,15 @@ __global__ void k_fill(double* __restrict__ a, double v, size_t n) {
 //   MODE 1: out = (c1*x + u) + c2*wa           (c1 = dt^2/2, u = u^0, wa = v^0, c2 = dt)
 //   MODE 2: part[P] = sum_r u_r (K u)_r        (DG error: K = A_dg, u = uh - uex)
 // ---------------------------------------------------------------------------
+// LDS ordering within one wave (the rocPRIM wave barrier: fences at
+// wavefront scope around a code-motion barrier); enough for a workgroup of
+// one wave, and it does not wait on the wave's global loads and stores.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Broadcast lane `l`'s double to the whole wave (v_readlane on both halves).
 __device__ __forceinline__ double lane_bcast(double v, int l) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
@@ -1106,6 +1092,28 @@ __device__ inline int step_poly(const int* __restrict__ order) {
   const int i = step_poly();
   return order ? order[i] : i;
 }
+
+// The vectors a row's update reads besides the block products.  With several
+// waves per polyhedron (few polyhedra: latency counts) they are fetched before
+// the blocks, otherwise after them, where other waves cover the wait and the
+// registers are free.
+template <int N3, int RPL>
+struct StepEnds {
+  double s[RPL], d[RPL], u[RPL], a[RPL];
+  __device__ __forceinline__ void load(const double* __restrict__ rs, const double* __restrict__ rd,
+                                       const double* __restrict__ uu, const double* __restrict__ wa, size_t o,
+                                       int lane) {
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) {
+      const int r = lane + 64 * k;
+      const bool row = r < N3;
+      s[k] = row ? rs[o + r] : 0.0;
+      d[k] = row ? rd[o + r] : 0.0;
+      u[k] = row ? uu[o + r] : 0.0;
+      a[k] = row ? wa[o + r] : 0.0;
+    }
+  }
+};
 
 // UNR = column pairs whose loads are issued together (register footprint vs
 // loads in flight).  XS = how the neighbour's coefficients reach the lanes:
@@ -1136,6 +1144,9 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
   if (Pp >= n_poly) return;  // padding workgroups of the last XCD share
   if (MODE != 2)
     for (int k = threadIdx.x; k < D::NPK; k += 64 * WPP) sR[k] = Rp[(size_t)Pp * D::NPK + k];
+  StepEnds<N3, RPL> ends;
+  if constexpr (WPP > 1 && MODE != 2)
+    if (wv == 0) ends.load(rs, rd, u, wa, (size_t)Pp * N3, lane);
   double acc[RPL];
 #pragma unroll
   for (int k = 0; k < RPL; ++k) acc[k] = 0.0;
@@ -1215,6 +1226,7 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
       const int r = lane + 64 * k;
       if (r < N3 && wv == 0) {
         double a = sblk[r];
+#pragma unroll 4
         for (int j = 1; j < b1 - b0; ++j) a = a + sblk[(size_t)j * N3 + r];
         acc[k] = a;
       }
@@ -1235,41 +1247,42 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
     }
     return;
   }
+  if constexpr (WPP == 1) __syncthreads();  // sR
+  if (wv != 0) return;  // no barrier of the workgroup follows
+  if constexpr (WPP == 1) ends.load(rs, rd, u, wa, o, lane);
   // time factor: one scalar, or per source group (ensembles whose instances
   // carry their own wavelet; the table is filled for this step)
   const double gp = gsel ? gtab[gsel[Pp]] : g;
-  if constexpr (P == 3) {
-    // one row per lane: wave 0 solves across its lanes (p = 3 only: at p <= 2
-    // the packed variants keep solve_packed, and every variant of a degree
-    // must give the same bits)
-    __syncthreads();  // sR
-    if (wv != 0) return;  // no barrier follows
-    double w = lane < N3 ? -acc[0] + rs[o + lane] + rd[o + lane] * gp : 0.0;
-    w = solve_wave<NP>(sR, w, lane);
-    if (lane < N3) {
-      if (MODE == 0)
-        out[o + lane] = c1 * w + 2.0 * u[o + lane] - wa[o + lane];
-      else
-        out[o + lane] = c1 * w + u[o + lane] + c2 * wa[o + lane];
+  double w[RPL];
+#pragma unroll
+  for (int k = 0; k < RPL; ++k) w[k] = -acc[k] + ends.s[k] + ends.d[k] * gp;
+  if constexpr (RPL == 1) {  // one row per lane: the wave solves across its lanes
+    w[0] = solve_group<NP>(sR, w[0], 0, lane, lane < N3);
+  } else {  // lane i takes row i of the three components
+#pragma unroll
+    for (int k = 0; k < RPL; ++k)
+      if (lane + 64 * k < N3) sw[lane + 64 * k] = w[k];
+    wave_lds_sync();
+    const bool row = lane < NP;
+    double x0 = row ? sw[lane] : 0.0, x1 = row ? sw[NP + lane] : 0.0, x2 = row ? sw[2 * NP + lane] : 0.0;
+    solve_rows<NP>(sR, x0, x1, x2, lane);
+    if (row) {
+      sw[lane] = x0;
+      sw[NP + lane] = x1;
+      sw[2 * NP + lane] = x2;
     }
-    return;
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) w[k] = lane + 64 * k < N3 ? sw[lane + 64 * k] : 0.0;
   }
 #pragma unroll
   for (int k = 0; k < RPL; ++k) {
     const int r = lane + 64 * k;
-    if (r < N3 && wv == 0) sw[r] = -acc[k] + rs[o + r] + rd[o + r] * gp;
-  }
-  __syncthreads();
-  if (threadIdx.x < 3) solve_packed<NP>(sR, sw + threadIdx.x * NP);
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < RPL; ++k) {
-    const int r = lane + 64 * k;
-    if (r < N3 && wv == 0) {
+    if (r < N3) {
       if (MODE == 0)
-        out[o + r] = c1 * sw[r] + 2.0 * u[o + r] - wa[o + r];
+        out[o + r] = c1 * w[k] + 2.0 * ends.u[k] - ends.a[k];
       else
-        out[o + r] = c1 * sw[r] + u[o + r] + c2 * wa[o + r];
+        out[o + r] = c1 * w[k] + ends.u[k] + c2 * ends.a[k];
     }
   }
 }
@@ -1300,15 +1313,6 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
 // triangular products through LDS, and the update of k_leapfrog.  p <= 3
 // (3Np <= 64 rows, whole column pairs).
 __host__ __device__ constexpr int self_upper_off(int c2i) { return 2 * c2i * (c2i + 1); }
-
-// LDS ordering within one wave (the rocPRIM wave barrier: fences at
-// wavefront scope around a code-motion barrier); enough for a workgroup of
-// one wave, and it does not wait on the wave's global loads and stores.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // One stored block of k_sym_products (self: a self block's packed upper
 // triangle; otherwise a pair block K_PQ with its transposed product).  Kb is
@@ -2110,14 +2114,8 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __rest
     w = -acc + rs[o] + rd[o] * gp;
   }
   if constexpr (TB == 64) {
-    if (act) sw[sub][r] = w;
-    lsync<WPW>();
-    if (lane < 3 * G) {
-      const int sp = lane / 3, comp = lane % 3;
-      if (P0 + sp < n_poly) solve_packed<NP>(sR[sp], sw[sp] + comp * NP);
-    }
-    lsync<WPW>();
-    if (act) w = sw[sub][r];
+    lsync<WPW>();  // sR
+    w = solve_group<NP>(sR[act ? sub : 0], w, sub * N3, r, act);
   }
   if (act) {
     if (MODE == 0)
@@ -2301,14 +2299,8 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restr
     w = -acc + rs[o] + rd[o] * gp;
   }
   if constexpr (TB == 64) {
-    if (act) sw[sub][r] = w;
-    lsync<WPW>();
-    if (lane < 3 * G) {
-      const int sp = lane / 3, comp = lane % 3;
-      if (P0 + sp < n_poly) solve_packed<NP>(sR[sp], sw[sp] + comp * NP);
-    }
-    lsync<WPW>();
-    if (act) w = sw[sub][r];
+    lsync<WPW>();  // sR
+    w = solve_group<NP>(sR[act ? sub : 0], w, sub * N3, r, act);
   }
   if (act) {
     if (MODE == 0)
@@ -2567,6 +2559,9 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict
   double acc[RPL];
 #pragma unroll
   for (int k = 0; k < RPL; ++k) acc[k] = 0.0;
+  StepEnds<N3, RPL> ends;
+  if constexpr (WPP > 1)
+    if (wv == 0) ends.load(rs, rd, u, wa, (size_t)Pp * N3, lane);
   const int b0 = row_ptr[Pp], b1 = row_ptr[Pp + 1];
   for (int b = b0 + wv; b < b1; b += WPP) {
     const int cb = __builtin_amdgcn_readfirstlane(col[b]);
@@ -2658,12 +2653,14 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict
       const int r = lane + 64 * k;
       if (r < N3) {
         double a = sblk[r];
+#pragma unroll 4
         for (int j = 1; j < b1 - b0; ++j) a = a + sblk[(size_t)j * N3 + r];
         acc[k] = a;
       }
     }
   }
   const size_t o = (size_t)Pp * N3;
+  if constexpr (WPP == 1) ends.load(rs, rd, u, wa, o, lane);
   // time factor: one scalar, or per source group (ensembles whose instances
   // carry their own wavelet; the table is filled for this step)
   const double gp = gsel ? gtab[gsel[Pp]] : g;
@@ -2671,11 +2668,11 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict
   for (int k = 0; k < RPL; ++k) {
     const int r = lane + 64 * k;
     if (r < N3) {
-      const double w = -acc[k] + rs[o + r] + rd[o + r] * gp;
+      const double w = -acc[k] + ends.s[k] + ends.d[k] * gp;
       if (MODE == 0)
-        out[o + r] = c1 * w + 2.0 * u[o + r] - wa[o + r];
+        out[o + r] = c1 * w + 2.0 * ends.u[k] - ends.a[k];
       else
-        out[o + r] = c1 * w + u[o + r] + c2 * wa[o + r];
+        out[o + r] = c1 * w + ends.u[k] + c2 * ends.a[k];
     }
   }
 }
@@ -2712,6 +2709,9 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog48(const float* __restrict
   double acc[RPL];
 #pragma unroll
   for (int k = 0; k < RPL; ++k) acc[k] = 0.0;
+  StepEnds<N3, RPL> ends;
+  if constexpr (WPP > 1)
+    if (wv == 0) ends.load(rs, rd, u, wa, (size_t)Pp * N3, lane);
   const int b0 = row_ptr[Pp], b1 = row_ptr[Pp + 1];
   for (int b = b0 + wv; b < b1; b += WPP) {
     const int cb = __builtin_amdgcn_readfirstlane(col[b]);
@@ -2825,22 +2825,24 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog48(const float* __restrict
       const int r = lane + 64 * k;
       if (r < N3) {
         double a = sblk[r];
+#pragma unroll 4
         for (int j = 1; j < b1 - b0; ++j) a = a + sblk[(size_t)j * N3 + r];
         acc[k] = a;
       }
     }
   }
   const size_t o = (size_t)Pp * N3;
+  if constexpr (WPP == 1) ends.load(rs, rd, u, wa, o, lane);
   const double gp = gsel ? gtab[gsel[Pp]] : g;
 #pragma unroll
   for (int k = 0; k < RPL; ++k) {
     const int r = lane + 64 * k;
     if (r < N3) {
-      const double w = -acc[k] + rs[o + r] + rd[o + r] * gp;
+      const double w = -acc[k] + ends.s[k] + ends.d[k] * gp;
       if (MODE == 0)
-        out[o + r] = c1 * w + 2.0 * u[o + r] - wa[o + r];
+        out[o + r] = c1 * w + 2.0 * ends.u[k] - ends.a[k];
       else
-        out[o + r] = c1 * w + u[o + r] + c2 * wa[o + r];
+        out[o + r] = c1 * w + ends.u[k] + c2 * ends.a[k];
     }
   }
 }
