@@ -728,7 +728,7 @@ __global__ __launch_bounds__(64) void k_cholesky(const double* __restrict__ M,
 // (COMPUTE_MODAL_COEFFICIENTS_FREE, :847-997).  One workgroup per polyhedron,
 // entry (i, m) owned by one thread; bound by the data's sines and the basis
 // values, both formed once per point (tab1d): p = 3, 13,824 polyhedra, RHS 2.07
-// -> 0.88 ms, projection 0.98 -> 0.53 ms.
+// -> 0.88 ms, projection 0.98 -> 0.56 ms.
 // ---------------------------------------------------------------------------
 template <int P>
 constexpr int rhs_threads() { return P == 1 ? 64 : (P == 2 ? 128 : 256); }
@@ -895,6 +895,15 @@ __global__ void k_rhs_points(MeshDev m, int n_tet, double* __restrict__ vpts,
   }
 }
 
+// LDS ordering within one wave (the rocPRIM wave barrier: fences at
+// wavefront scope around a code-motion barrier); enough for a workgroup of
+// one wave, and it does not wait on the wave's global loads and stores.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // M^-1 w = R^-1 R^-T w (solve_LU with L = R^T, src/vet_mat_operations.f90:
 // 123-153) across a group of 3Np lanes from lane `base`, one entry of the
 // vector per lane: r = component x Np + row (other lanes pass through).  The
@@ -927,15 +936,12 @@ __device__ __forceinline__ double solve_group(const double* __restrict__ R, doub
   return w;
 }
 
-// M^-1 of three right-hand sides across one wave, lane i on row i of all three
-// (NP <= 64): the forward sweep broadcasts y_j = s_j / R_jj from lane j and the
-// rows below subtract R_ji y_j (ascending j), the backward
-// sweep runs the columns from the last.  NP dependent steps per sweep instead
-// of NP(NP+1)/2 on one lane.
+// R^-T of three right-hand sides across one wave, lane i on row i of all three
+// (NP <= 64): broadcasts y_j = s_j / R_jj from lane j, the rows below subtract
+// R_ji y_j (ascending j, as the reference).
 template <int NP>
-__device__ __forceinline__ void solve_rows(const double* __restrict__ R, double& x0, double& x1, double& x2, int i) {
+__device__ __forceinline__ void forward_rows(const double* __restrict__ R, double& x0, double& x1, double& x2, int i) {
   static_assert(NP <= 64, "one lane per row");
-  const int ri = pk_off(NP, i < NP ? i : 0);
 #pragma unroll 5
   for (int j = 0; j < NP; ++j) {
     const int rj = pk_off(NP, j);
@@ -952,6 +958,15 @@ __device__ __forceinline__ void solve_rows(const double* __restrict__ R, double&
       x2 = x2 - r * y2;
     }
   }
+}
+
+// M^-1 of three right-hand sides across one wave: forward_rows, then the
+// columns from the last.  NP dependent steps per sweep instead of NP(NP+1)/2
+// on one lane.
+template <int NP>
+__device__ __forceinline__ void solve_rows(const double* __restrict__ R, double& x0, double& x1, double& x2, int i) {
+  forward_rows<NP>(R, x0, x1, x2, i);
+  const int ri = pk_off(NP, i < NP ? i : 0);
 #pragma unroll 5
   for (int j = NP - 1; j >= 0; --j) {
     const double rjj = R[pk_off(NP, j)];
@@ -966,6 +981,22 @@ __device__ __forceinline__ void solve_rows(const double* __restrict__ R, double&
       x1 = x1 - r * y1;
       x2 = x2 - r * y2;
     }
+  }
+}
+
+// R^-1 y in place on one lane, every row's terms in ascending columns as the
+// reference adds them.  The projections keep this order: the 32-bit apply
+// turns a last-bit change of the initial data into 1e-6 of the state within
+// 100 steps.  The products of four columns are formed ahead of the chain.
+template <int NP>
+__device__ __forceinline__ void back_ascending(const double* __restrict__ R, double* __restrict__ x) {
+#pragma unroll 1
+  for (int i = NP - 1; i >= 0; --i) {
+    const double* __restrict__ Ri = R + pk_off(NP, i) - i;
+    double s = x[i];
+#pragma unroll 4
+    for (int j = i + 1; j < NP; ++j) s = s - Ri[j] * x[j];
+    x[i] = s / Ri[i];
   }
 }
 
@@ -1027,16 +1058,20 @@ __global__ __launch_bounds__(rhs_threads<P>(), 4) void k_project(MeshDev m, int 
   }
   if (tid < N3) sb[tid] = acc;
   __syncthreads();
-  if (tid >= 64) return;  // one wave solves the three components
-  const bool row = tid < NP;
-  double x0 = row ? sb[tid] : 0.0, x1 = row ? sb[NP + tid] : 0.0, x2 = row ? sb[2 * NP + tid] : 0.0;
-  solve_rows<NP>(sR, x0, x1, x2, tid);
-  if (row) {
-    double* o = out + (size_t)Pp * N3 + tid;
-    o[0] = x0;
-    o[NP] = x1;
-    o[2 * NP] = x2;
+  if (tid < 64) {  // one wave sweeps forward, a lane per component back
+    const bool row = tid < NP;
+    double x0 = row ? sb[tid] : 0.0, x1 = row ? sb[NP + tid] : 0.0, x2 = row ? sb[2 * NP + tid] : 0.0;
+    forward_rows<NP>(sR, x0, x1, x2, tid);
+    if (row) {
+      sb[tid] = x0;
+      sb[NP + tid] = x1;
+      sb[2 * NP + tid] = x2;
+    }
+    wave_lds_sync();
+    if (tid < 3) back_ascending<NP>(sR, sb + tid * NP);
   }
+  __syncthreads();
+  if (tid < N3) out[(size_t)Pp * N3 + tid] = sb[tid];
 }
 
 __global__ void k_fill(double* __restrict__ a, double v, size_t n) {
@@ -1056,15 +1091,6 @@ __global__ void k_fill(double* __restrict__ a, double v, size_t n) {
 //   MODE 1: out = (c1*x + u) + c2*wa           (c1 = dt^2/2, u = u^0, wa = v^0, c2 = dt)
 //   MODE 2: part[P] = sum_r u_r (K u)_r        (DG error: K = A_dg, u = uh - uex)
 // ---------------------------------------------------------------------------
-// LDS ordering within one wave (the rocPRIM wave barrier: fences at
-// wavefront scope around a code-motion barrier); enough for a workgroup of
-// one wave, and it does not wait on the wave's global loads and stores.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Broadcast lane `l`'s double to the whole wave (v_readlane on both halves).
 __device__ __forceinline__ double lane_bcast(double v, int l) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
