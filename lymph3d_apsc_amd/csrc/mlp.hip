@@ -12,8 +12,9 @@
 // the forward pass (X W^T), the input gradient (dZ W) and the weight
 // gradient (dZ^T X) without transposed copies.  Epilogues fuse bias + GELU
 // (forward, keeping the FP32 pre-activation) and the GELU derivative
-// (backward).  Networks up to 512 wide take the fragment-order kernels further
-// down instead (k_slab, k_layer, k_update).
+// (backward).  Networks whose inputs and hidden layers are at most 512 wide take
+// the fragment-order kernels further down instead (k_slab, k_layer, k_wide,
+// k_update).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -337,7 +338,8 @@ __global__ void k_to_bf16(const float* __restrict__ a, bf16_t* __restrict__ b, s
 
 
 // ---------------------------------------------------------------------------
-// Networks whose layers are all at most kSlabW wide (the receiver network).
+// Networks whose inputs and hidden layers are at most kSlabW wide (the receiver
+// network; the all-traces network, whose output layer is wide).
 //
 // Weights are kept in the order the matrix cores read them (pack_pos: W for
 // the forward pass, its columns for the input gradients), and so are the
@@ -367,7 +369,8 @@ struct SlabArgs {
   const bf16_t* Wf[kSlabL]; // W_l packed
   const float* bias[kSlabL];
   const float* X;           // inputs [B][w[0]]
-  float* Y;                 // outputs [B][w[L]]
+  float* Y;                 // outputs [B][w[L]]; null: the last layer's gelu goes to Hp
+  bf16_t* Hp;               // packed [rows][w[L]] (a wide output layer follows)
 };
 
 // fragment f of the packed matrix: a uniform base and the lane's 16 bytes
@@ -491,9 +494,9 @@ __global__ __launch_bounds__(512, 2) void k_slab(SlabArgs g) {
   f32x4 acc[4][MT];
   for (int l = 0; l < g.L; ++l) {
     const int N = g.w[l + 1], tpw = tpw_of(N), nt = tiles_of(N);
-    const bool last = l + 1 == g.L;
+    const bool last = g.Y && l + 1 == g.L;
     slab_product_any<MR, PF>(acc, pf, g.Wf[l], tpw, steps_of(g.w[l]), sH, wave, lane);
-    if (!last) frag_first_any<PF>(pf, g.Wf[l + 1], tpw_of(g.w[l + 2]), steps_of(N), wave, lane);
+    if (l + 1 < g.L) frag_first_any<PF>(pf, g.Wf[l + 1], tpw_of(g.w[l + 2]), steps_of(N), wave, lane);
     __syncthreads();  // every wave has read this layer's input
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -516,7 +519,11 @@ __global__ __launch_bounds__(512, 2) void k_slab(SlabArgs g) {
         if (in)
 #pragma unroll
           for (int r = 0; r < 4; ++r) h[r] = f2bf(gelu(acc[i][m][r] + b[r]));
-        slab_put(sH, m * 16 + mr, n0, h);
+        if (l + 1 < g.L)
+          slab_put(sH, m * 16 + mr, n0, h);
+        else if (in)
+          *reinterpret_cast<uint2*>(g.Hp + pack_pos(row, n0, steps_of(N))) =
+              make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
       }
     }
     if (nt & 1) {  // the last step's second tile
@@ -533,26 +540,76 @@ __global__ __launch_bounds__(512, 2) void k_slab(SlabArgs g) {
 // 16 x 16 tile of a layer is a wave of its own (512 of them at 256 x 512),
 // all its fragments in flight at once: one trip to memory per launch, 3.7 to
 // 4.7 us each.  Receiver network, batch 256: a step of 30 launches took 178
-// us, these 12 take 61 us (k_update 17 us of them).
-enum { LAYER_FWD = 0, LAYER_LOSS = 1, LAYER_BWD = 2 };
+// us, these 12 take 57 us (k_update 11 us of them; 61 and 16 while the
+// transposed copies were rows, of which a load takes 64 bytes at a time).
+enum { LAYER_FWD = 0, LAYER_LOSS = 1, LAYER_BWD = 2, LAYER_OUT = 3 };
 struct LayerArgs {
-  int N, K, B, ldb;    // output width, contraction, rows
+  int N, K, B, ts;     // output width, contraction, rows, steps of a transposed copy's row
   const bf16_t* W;     // packed [N][K]
   const bf16_t* in;    // packed [rows][K]; null: rows idx[b] of X
   const float* X;
   const int* idx;
-  bf16_t* XT;          // X's rows in bf16, transposed [K][ldb]
+  bf16_t* XT;          // X's rows in bf16, transposed and packed [K][rows]
   const float* bias;   // forward
   bf16_t* out;         // packed [rows][N]: gelu(z), dY or dZ
-  bf16_t* outT;        // transposed [N][ldb]
+  bf16_t* outT;        // transposed, packed [N][rows]
   f32x4* dg;           // gelu'(z) as the lanes hold it, one per tile and lane
   const float* T;      // loss: targets, row idx[b]
   float scale;         // loss: 2 / (B N)
-  float* part;         // loss: per tile, sum of (y - t)^2
+  float* part;         // loss: per wave, sum of (y - t)^2
+  float* Y;            // LAYER_OUT: outputs [B][N]
+  int rw;              // k_wide: waves of a workgroup along the rows
 };
 
 // workgroups of 2 waves: column tile wg % tiles, row tiles 2 (wg / tiles) + wave
 __host__ __device__ inline int layer_wgs(int N, int B) { return tiles_of(N) * ((B + 31) >> 5); }
+
+// End of one 16 x 16 tile from its sums; dg, bv, tv: gelu'(z), bias and target
+// of the lane's four columns.  With sT the transposed copy goes there (its
+// column 0, row 0 of the tile).  Returns the lane's part of the loss.
+template <int EPI>
+__device__ __forceinline__ float layer_end(const LayerArgs& g, int mt, int t, int lane, f32x4 acc, f32x4 dg,
+                                           float4 bv, float4 tv, bf16_t* sT = nullptr, int ldT = 0) {
+  const int nt = tiles_of(g.N), row = mt * 16 + (lane & 15), n0 = t * 16 + (lane >> 4) * 4;
+  const bool ok = n0 < g.N && row < g.B;  // widths are multiples of 8: all four columns or none
+  const float b[4] = {bv.x, bv.y, bv.z, bv.w}, tt[4] = {tv.x, tv.y, tv.z, tv.w};
+  if (EPI == LAYER_OUT) {
+    if (ok)
+      *reinterpret_cast<float4*>(g.Y + (size_t)row * g.N + n0) =
+          make_float4(acc[0] + b[0], acc[1] + b[1], acc[2] + b[2], acc[3] + b[3]);
+    return 0.f;
+  }
+  uint32_t h[4] = {0u, 0u, 0u, 0u};
+  float d2 = 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (EPI == LAYER_FWD) {
+      const float z = acc[r] + b[r];
+      const float e1 = 1.0f + erff(z * 0.70710678118654752f);
+      h[r] = f2bf(0.5f * z * e1);
+      dg[r] = 0.5f * e1 + z * 0.39894228040143268f * expf(-0.5f * z * z);
+    } else if (EPI == LAYER_BWD) {
+      h[r] = f2bf(acc[r] * dg[r]);
+    } else {
+      const float d = (acc[r] + b[r]) - tt[r];
+      if (ok) d2 += d * d;
+      h[r] = f2bf(g.scale * d);
+    }
+  }
+  if (EPI == LAYER_FWD) g.dg[((size_t)mt * nt + t) * 64 + lane] = dg;
+  if (ok) {
+    if (g.out)
+      *reinterpret_cast<uint2*>(g.out + pack_pos(row, n0, steps_of(g.N))) =
+          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    if (!sT)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) g.outT[pack_pos(n0 + r, row, g.ts)] = (bf16_t)h[r];
+  }
+  if (sT)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sT[((lane >> 4) * 4 + r) * ldT + (lane & 15)] = (bf16_t)h[r];
+  return d2;
+}
 
 template <int EPI, bool GATHER>
 __device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
@@ -560,7 +617,7 @@ __device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
   const int nt = tiles_of(g.N), t = wg % nt, mt = wg / nt * 2 + wave;
   if (mt * 16 >= g.B) return;
   const int steps = steps_of(g.K);
-  const int mr = lane & 15, row = mt * 16 + mr, n0 = t * 16 + (lane >> 4) * 4;
+  const int row = mt * 16 + (lane & 15), n0 = t * 16 + (lane >> 4) * 4;
   const bool in = n0 < g.N, ok = in && row < g.B;  // widths are multiples of 8: all four columns or none
   f32x4 dg = {0.f, 0.f, 0.f, 0.f};
   if (EPI == LAYER_BWD) dg = g.dg[((size_t)mt * nt + t) * 64 + lane];
@@ -588,7 +645,7 @@ __device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
           v[4] = f2bf(b.x); v[5] = f2bf(b.y); v[6] = f2bf(b.z); v[7] = f2bf(b.w);
           if (t == 0 && s0 + s < steps)
 #pragma unroll
-            for (int r = 0; r < 8; ++r) g.XT[(size_t)(k + r) * g.ldb + row] = (bf16_t)v[r];
+            for (int r = 0; r < 8; ++r) g.XT[pack_pos(k + r, row, g.ts)] = (bf16_t)v[r];
         }
         h[s] = u32x4{v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
       }
@@ -599,37 +656,168 @@ __device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[s]),
                                                       __builtin_bit_cast(bf16x8, h[s]), acc, 0, 0, 0);
   }
-  const float b[4] = {bv.x, bv.y, bv.z, bv.w}, tt[4] = {tv.x, tv.y, tv.z, tv.w};
-  uint32_t h[4] = {0u, 0u, 0u, 0u};
-  float d2 = 0.f;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    if (EPI == LAYER_FWD) {
-      const float z = acc[r] + b[r];
-      const float e1 = 1.0f + erff(z * 0.70710678118654752f);
-      h[r] = f2bf(0.5f * z * e1);
-      dg[r] = 0.5f * e1 + z * 0.39894228040143268f * expf(-0.5f * z * z);
-    } else if (EPI == LAYER_BWD) {
-      h[r] = f2bf(acc[r] * dg[r]);
-    } else {
-      const float d = (acc[r] + b[r]) - tt[r];
-      if (ok) d2 += d * d;
-      h[r] = f2bf(g.scale * d);
-    }
-  }
-  if (EPI == LAYER_FWD) g.dg[((size_t)mt * nt + t) * 64 + lane] = dg;
-  if (ok) {
-    if (g.out)
-      *reinterpret_cast<uint2*>(g.out + pack_pos(row, n0, steps_of(g.N))) =
-          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-#pragma unroll
-    for (int r = 0; r < 4; ++r) g.outT[(size_t)(n0 + r) * g.ldb + row] = (bf16_t)h[r];
-  }
+  float d2 = layer_end<EPI>(g, mt, t, lane, acc, dg, bv, tv);
   if (EPI == LAYER_LOSS) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) d2 += __shfl_down(d2, o, 64);
     if (lane == 0) g.part[(size_t)mt * nt + t] = d2;
   }
+}
+
+// acc[i][j] += W tile (t0 + i) times row tile (m0 + j) over steps s0..s1 - 1,
+// both in fragment order, D steps' fragments in flight.  Tiles past the last are the last one again.
+template <int T, int D>
+__device__ __forceinline__ void block_product(f32x4 (&acc)[T][T], const bf16_t* W, const bf16_t* in, int t0, int nt,
+                                              int m0, int nm, int steps, int s0, int s1, int lane) {
+  size_t wt[T], ht[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    wt[i] = (size_t)min(t0 + i, nt - 1) * steps;
+    ht[i] = (size_t)min(m0 + i, nm - 1) * steps;
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  u32x4 w[D][T], h[D][T];
+  auto get = [&](int d, int s) {
+    s = min(s, s1 - 1);
+#pragma unroll
+    for (int i = 0; i < T; ++i) w[d][i] = frag(W, wt[i] + s, lane);
+#pragma unroll
+    for (int i = 0; i < T; ++i) h[d][i] = frag(in, ht[i] + s, lane);
+  };
+  auto use = [&](int d) {
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int j = 0; j < T; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[d][i]),
+                                                            __builtin_bit_cast(bf16x8, h[d][j]), acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) get(d, s0 + d);
+  int s = s0;
+#pragma unroll 1
+  for (; s + D <= s1; s += D)
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      use(d);
+      get(d, s + D + d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (s + d < s1) use(d);
+}
+
+// LDS ordering within one wave: fences at wavefront scope around a
+// code-motion barrier
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A wide output layer, forward: every wave T x T tiles of 16 x 16, so that
+// W's fragments are read B / 16 T times and the rows' N / 16 T times where k_layer reads them once per tile.  4 waves a workgroup, rw of
+// them along the rows; an XCD takes every eighth group of columns for all
+// rows, so W comes into one L2 only.  Bound by the way of W and the targets
+// (39 MB each at 256 x 38,400) from HBM, of the gradients back (two copies of
+// 20 MB) and of the rows from L2.  EPI LAYER_LOSS fuses the loss: outputs are
+// not stored.
+template <int T, int EPI>
+__global__ __launch_bounds__(256, 2) void k_wide(LayerArgs g) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt = tiles_of(g.N), nm = tiles_of(g.B), steps = steps_of(g.K);
+  const int wr = (nm + T * g.rw - 1) / (T * g.rw), li = blockIdx.x >> 3;
+  const int m0 = (li % wr * g.rw + wave % g.rw) * T;
+  const int t0 = ((li / wr * 8 + (blockIdx.x & 7)) * (4 / g.rw) + wave / g.rw) * T;
+  float d2 = 0.f;
+  // a wave's gradients transposed: they leave as whole fragments
+  constexpr int LDT = 16 * T + 8;
+  __shared__ __attribute__((aligned(16))) bf16_t sT[EPI == LAYER_LOSS ? 4 * 16 * T * LDT : 8];
+  bf16_t* st = sT + (EPI == LAYER_LOSS ? wave * 16 * T * LDT : 0);
+  if (m0 < nm && t0 < nt) {
+    float4 bv[T], tv[T][T];  // biases and targets on their way while the products run
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      const int row = (m0 + j) * 16 + (lane & 15);
+      const int src = EPI == LAYER_LOSS && row < g.B ? g.idx[row] : -1;
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        const int n0 = (t0 + i) * 16 + (lane >> 4) * 4;
+        tv[i][j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (src >= 0 && n0 < g.N) tv[i][j] = *reinterpret_cast<const float4*>(g.T + (size_t)src * g.N + n0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      const int n0 = (t0 + i) * 16 + (lane >> 4) * 4;
+      bv[i] = n0 < g.N ? *reinterpret_cast<const float4*>(g.bias + n0) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    f32x4 acc[T][T];
+    block_product<T, T == 4 ? 2 : 4>(acc, g.W, g.in, t0, nt, m0, nm, steps, 0, steps, lane);
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int j = 0; j < T; ++j)
+        if (t0 + i < nt && m0 + j < nm)
+          d2 += layer_end<EPI>(g, m0 + j, t0 + i, lane, acc[i][j], f32x4{0.f, 0.f, 0.f, 0.f}, bv[i], tv[i][j],
+                               EPI == LAYER_LOSS ? st + i * 16 * LDT + j * 16 : nullptr, LDT);
+    if (EPI == LAYER_LOSS) {
+      wave_lds_sync();
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T / 2; ++j) {  // whole fragments: T is even, and so is m0
+          const int n = (t0 + i) * 16 + (lane & 15), c = j * 32 + (lane >> 4) * 8;
+          if (n < g.N && m0 * 16 + c < g.B)
+            *reinterpret_cast<uint4*>(g.outT + ((size_t)(t0 + i) * g.ts + m0 / 2 + j) * 512 + lane * 8) =
+                *reinterpret_cast<const uint4*>(st + (i * 16 + (lane & 15)) * LDT + c);
+        }
+    }
+  }
+  if (EPI == LAYER_LOSS) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) d2 += __shfl_down(d2, o, 64);
+    if (lane == 0) g.part[(size_t)blockIdx.x * 4 + wave] = d2;
+  }
+}
+
+// Its input gradient: a long contraction (N of the output layer) for few
+// tiles, so the contraction is split as in gemm() and the parts, stored as the
+// lanes hold them, are added in order by k_split_end.  An XCD takes every
+// eighth part, whose operands then fit its L2.  256 x 512 from 38,400: 28 us
+// (2 x 2 tiles a wave 39; more steps in flight change nothing) and 5 for the
+// sums, where the GEMM and its sums took 47.
+template <int T>
+__global__ __launch_bounds__(256, 2) void k_split(LayerArgs g, int S, int chunk, f32x4* ws) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt = tiles_of(g.N), nm = tiles_of(g.B), steps = steps_of(g.K);
+  const int wr = (nm + 2 * T - 1) / (2 * T), wgs = wr * ((nt + 2 * T - 1) / (2 * T)), li = blockIdx.x >> 3;
+  const int z = li / wgs * 8 + (blockIdx.x & 7), o = li % wgs;
+  const int m0 = (o % wr * 2 + (wave & 1)) * T, t0 = (o / wr * 2 + (wave >> 1)) * T;
+  if (z >= S || m0 >= nm || t0 >= nt) return;
+  f32x4 acc[T][T];
+  block_product<T, 4>(acc, g.W, g.in, t0, nt, m0, nm, steps, z * chunk, min(steps, (z + 1) * chunk), lane);
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j)
+      if (t0 + i < nt && m0 + j < nm)
+        ws[(((size_t)z * nm + m0 + j) * nt + t0 + i) * 64 + lane] = acc[i][j];
+}
+
+__global__ __launch_bounds__(64) void k_split_end(LayerArgs g, int S, const f32x4* ws) {
+  const int lane = threadIdx.x, nt = tiles_of(g.N), nm = tiles_of(g.B);
+  const int mt = blockIdx.x / nt, t = blockIdx.x % nt;
+  const f32x4 dg = g.dg[((size_t)mt * nt + t) * 64 + lane];
+  const size_t stride = (size_t)nm * nt * 64;
+  const f32x4* p = ws + ((size_t)mt * nt + t) * 64 + lane;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int z = 0; z < S; ++z) v += p[z * stride];
+  const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+  layer_end<LAYER_BWD>(g, mt, t, lane, v, dg, none, none);
 }
 
 struct AdamArgs {
@@ -658,12 +846,12 @@ __global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __re
 
 struct UpdateLayer {
   int N, K, first;      // W is [N][K]; first workgroup of its weight tiles
-  const bf16_t *DT, *HT;  // dZ^T [N][ldb], H^T [K][ldb]
+  const bf16_t *DT, *HT;  // dZ^T [N][rows], H^T [K][rows], packed
   size_t woff, boff;
   bf16_t *Wf, *Wd, *Wb;  // packed copies and the row-major copy, where kept
 };
 struct UpdateArgs {
-  int L, B, ldb, first_bias, n_part;
+  int L, B, ts, first_bias, n_part;  // ts: steps of DT's and HT's rows
   UpdateLayer y[kSlabL];
   float *P, *M, *V;  // ADAM: updated in place
   float* G;          // !ADAM: gradients
@@ -677,7 +865,7 @@ struct UpdateArgs {
 // Adam update of the master weights, both moments and the bf16 copies in the
 // epilogue (ADAM), or the gradients stored (!ADAM).  64 x 16 (k x n) of W per
 // workgroup of 2 waves, 32 x 16 per wave, fragments straight from the
-// transposed operands (both contiguous along the batch, 16 bytes a lane); D
+// transposed operands (packed along the batch); D
 // fragments hold four neighbouring k of one n, so masters and moments move in
 // 16-byte pieces.  Bound by their 24 bytes per weight and by the trip to
 // memory (a gradient buffer in between would add 8 bytes and a launch).
@@ -692,6 +880,7 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
   if (wg == (int)gridDim.x - 1) {  // the loss
     __shared__ double red[128];
     double s = 0.0;
+#pragma unroll 8
     for (int i = tid; i < u.n_part; i += 128) s += u.part[i];
     red[tid] = s;
     __syncthreads();
@@ -709,7 +898,7 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
     const int gp = lane & 31, half = lane >> 5;
     const int n = o * 4 + wave * 2 + half;  // widths are multiples of 8
     float s = 0.f;
-    for (int b = gp; b < u.B; b += 32) s += bf2f(y.DT[(size_t)n * u.ldb + b]);
+    for (int b = gp; b < u.B; b += 32) s += bf2f(y.DT[pack_pos(n, b, u.ts)]);
     float t = 0.f;
 #pragma unroll
     for (int j = 0; j < 32; ++j) t += __shfl(s, half * 32 + j, 64);
@@ -757,11 +946,13 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
     for (int s = 0; s < CH; ++s) {
       const int bb = s0 + 32 * s + fk, n = n0 + fr;
       b[s] = a[s][0] = a[s][1] = make_uint4(0u, 0u, 0u, 0u);
-      if (bb < u.B && n < y.N) b[s] = *reinterpret_cast<const uint4*>(y.DT + (size_t)n * u.ldb + bb);
+      const size_t st = (size_t)(s0 / 32 + s) * 512 + lane * 8;
+      if (bb < u.B && n < y.N) b[s] = *reinterpret_cast<const uint4*>(y.DT + (size_t)(n0 >> 4) * u.ts * 512 + st);
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int k = k0 + 16 * i + fr;
-        if (bb < u.B && k < y.K) a[s][i] = *reinterpret_cast<const uint4*>(y.HT + (size_t)k * u.ldb + bb);
+        if (bb < u.B && k < y.K)
+          a[s][i] = *reinterpret_cast<const uint4*>(y.HT + (size_t)((k0 >> 4) + i) * u.ts * 512 + st);
       }
     }
 #pragma unroll
@@ -798,6 +989,171 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
       y.Wd[pack_pos(k + 1, n, sn)] = (bf16_t)h1;
       y.Wd[pack_pos(k + 2, n, sn)] = (bf16_t)h2;
       y.Wd[pack_pos(k + 3, n, sn)] = (bf16_t)h3;
+    }
+  }
+}
+
+// k_update of a wide output layer: 32 x 128 (n x k) of W per workgroup of 4
+// waves.  The products go to LDS, from where masters, moments and gradients
+// move as whole rows and both packed copies as whole fragments.  Bound by its
+// 28 bytes per weight: 38,400 x 512 in 117 us (4.9 TB/s; with 256 k 150, with
+// 64 183, as k_update's tiles 231), where the gradient product, the column sums
+// and the update took 130.
+constexpr int kUpN = 32, kUpK = 128, kUpT = kUpK / 64, kUpLd = kUpK + 4, kUpLb = kUpK + 8;
+template <bool ADAM>
+__global__ __launch_bounds__(256, 3) void k_update_wide(UpdateArgs u, int l) {
+  __shared__ __attribute__((aligned(16))) float sG[kUpN * kUpLd];
+  __shared__ __attribute__((aligned(16))) bf16_t sW[kUpN * kUpLb];
+  __shared__ float sB[kUpN][33];
+  const UpdateLayer& y = u.y[l];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tk = (y.K + kUpK - 1) / kUpK;
+  const int k0 = (int)(blockIdx.x % tk) * kUpK, n0 = (int)(blockIdx.x / tk) * kUpN;
+  const int kw = min(kUpK, y.K - k0), rowq = kw / 4;  // k of this workgroup, pieces of 4 per row
+  const bool bias = k0 == 0 && wave == 0;  // its products' rows are the biases' terms
+  constexpr int E = kUpN * kUpK / 4 / 256;
+  float4 pw[E], pm[E], pv[E];
+  const int fr = lane & 15, fk = (lane >> 4) * 8;
+  f32x4 acc[kUpT][2];
+#pragma unroll
+  for (int i = 0; i < kUpT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float sum[2][8] = {};
+  constexpr int CH = 4;
+  uint4 a[CH][kUpT], b[CH][2];
+  auto get = [&](int s0) {
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+      const int bb = s0 + 32 * s + fk;
+      const size_t st = (size_t)(s0 / 32 + s) * 512 + lane * 8;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        b[s][j] = make_uint4(0u, 0u, 0u, 0u);
+        if (bb < u.B && n0 + 16 * j + fr < y.N)
+          b[s][j] = *reinterpret_cast<const uint4*>(y.DT + (size_t)(n0 / 16 + j) * u.ts * 512 + st);
+      }
+#pragma unroll
+      for (int i = 0; i < kUpT; ++i) {
+        const int k = (wave * kUpT + i) * 16 + fr;
+        a[s][i] = make_uint4(0u, 0u, 0u, 0u);
+        if (bb < u.B && k < kw)
+          a[s][i] = *reinterpret_cast<const uint4*>(y.HT + (size_t)(k0 / 16 + wave * kUpT + i) * u.ts * 512 + st);
+      }
+    }
+  };
+  auto use = [&]() {
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+#pragma unroll
+      for (int i = 0; i < kUpT; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s][i]),
+                                                              __builtin_bit_cast(bf16x8, b[s][j]), acc[i][j], 0, 0, 0);
+      if (bias)  // column sums in k_colsum's order: the rows 32 apart first
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t h[4] = {b[s][j].x, b[s][j].y, b[s][j].z, b[s][j].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            sum[j][2 * q] += bf2f((bf16_t)(h[q] & 0xffffu));
+            sum[j][2 * q + 1] += bf2f((bf16_t)(h[q] >> 16));
+          }
+        }
+    }
+  };
+  get(0);
+#pragma unroll 1
+  for (int s0 = 32 * CH; s0 < u.B; s0 += 32 * CH) {
+    use();
+    get(s0);
+  }
+  // masters and moments on their way while the last products run
+  if (ADAM) {
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const int e = tid + 256 * j, n = n0 + e / rowq;
+      if (e < kUpN * rowq && n < y.N) {
+        const size_t at = y.woff + (size_t)n * y.K + k0 + e % rowq * 4;
+        pw[j] = *reinterpret_cast<const float4*>(u.P + at);
+        pm[j] = *reinterpret_cast<const float4*>(u.M + at);
+        pv[j] = *reinterpret_cast<const float4*>(u.V + at);
+      }
+    }
+  }
+  use();
+#pragma unroll
+  for (int i = 0; i < kUpT; ++i)  // lane: four neighbouring k of one n
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      *reinterpret_cast<f32x4*>(sG + (16 * j + fr) * kUpLd + wave * 16 * kUpT + 16 * i + (lane >> 4) * 4) = acc[i][j];
+  if (ADAM && kw < kUpK)  // the copies' last steps and tiles are padded with zeros
+    for (int e = tid; e < kUpN * kUpLb / 8; e += 256) reinterpret_cast<uint4*>(sW)[e] = make_uint4(0u, 0u, 0u, 0u);
+  if (bias)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) sB[16 * j + fr][fk + q] = sum[j][q];
+  __syncthreads();
+  if (bias && tid < kUpN && n0 + tid < y.N) {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < 32; ++q) t += sB[tid][q];
+    const size_t i = y.boff + n0 + tid;
+    if (ADAM) {
+      float w = u.P[i], m = u.M[i], v = u.V[i];
+      adam_one(w, m, v, t, u.a);
+      u.P[i] = w; u.M[i] = m; u.V[i] = v;
+    } else {
+      u.G[i] = t;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < E; ++j) {
+    const int e = tid + 256 * j;
+    if (e >= kUpN * rowq) continue;
+    const int r = e / rowq, k = e % rowq * 4, n = n0 + r;
+    uint2 hw = make_uint2(0u, 0u);
+    if (n < y.N) {
+      const f32x4 g = *reinterpret_cast<const f32x4*>(sG + r * kUpLd + k);
+      const size_t at = y.woff + (size_t)n * y.K + k0 + k;
+      if (!ADAM) {
+        *reinterpret_cast<f32x4*>(u.G + at) = g;
+        continue;
+      }
+      float4 w = pw[j], m = pm[j], v = pv[j];
+      const uint32_t h0 = f2bf(adam_one(w.x, m.x, v.x, g[0], u.a));
+      const uint32_t h1 = f2bf(adam_one(w.y, m.y, v.y, g[1], u.a));
+      const uint32_t h2 = f2bf(adam_one(w.z, m.z, v.z, g[2], u.a));
+      const uint32_t h3 = f2bf(adam_one(w.w, m.w, v.w, g[3], u.a));
+      *reinterpret_cast<float4*>(u.P + at) = w;
+      *reinterpret_cast<float4*>(u.M + at) = m;
+      *reinterpret_cast<float4*>(u.V + at) = v;
+      hw = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
+    }
+    if (ADAM) *reinterpret_cast<uint2*>(sW + r * kUpLb + k) = hw;
+  }
+  if (!ADAM) return;
+  __syncthreads();
+  // fragments of both copies: (n tile, k step) and k tile x this n step
+  const int sk = steps_of(y.K), sn = steps_of(y.N);
+  for (int f = wave; f < kUpK / 8; f += 4) {
+    if (f < kUpK / 16) {
+      const int t = n0 / 16 + (f & 1), st = k0 / 32 + (f >> 1);
+      if (t < tiles_of(y.N) && st < sk)
+        *reinterpret_cast<uint4*>(y.Wf + ((size_t)t * sk + st) * 512 + lane * 8) =
+            *reinterpret_cast<const uint4*>(sW + ((f & 1) * 16 + fr) * kUpLb + (f >> 1) * 32 + fk);
+    } else {
+      const int t = k0 / 16 + f - kUpK / 16;
+      if (t >= tiles_of(y.K)) continue;
+      uint32_t h[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bf16_t* c = sW + (fk + 2 * q) * kUpLb + (f - kUpK / 16) * 16 + fr;
+        h[q] = (uint32_t)c[0] | ((uint32_t)c[kUpLb] << 16);
+      }
+      *reinterpret_cast<uint4*>(y.Wd + ((size_t)t * sn + n0 / 32) * 512 + lane * 8) = make_uint4(h[0], h[1], h[2], h[3]);
     }
   }
 }
@@ -844,9 +1200,12 @@ struct LymphMlp {
   size_t dorder_cap = 0;
   float* dloss = nullptr;
   size_t dloss_cap = 0;
-  // slab networks (all widths <= kSlabW): packed weights, transposed
-  // activations and gradients, gelu' per slab; grown with the batch
-  bool slab = false;
+  // slab networks (inputs and hidden layers <= kSlabW; wide: the output layer
+  // is wider): packed weights, activations and gradients, packed and
+  // transposed, and gelu' per tile
+  bool slab = false, wide = false;
+  bf16_t* hp = nullptr;  // forward of a wide network: the last activations, packed
+  size_t hp_cap = 0;
   std::vector<bf16_t*> Wf, Wd, HT, DT, HP, DP;
   std::vector<f32x4*> dg;
   // inputs and outputs of host-side calls: one batch with the network, grown
@@ -879,28 +1238,35 @@ int dalloc(LymphMlp* m, T** p, size_t n) {
 // output layer: k = 38,400) is split along k over up to kMaxSplit workgroups
 // per tile (32 x 32 = 1024 workgroups there) and reduced in order.
 constexpr int kMaxSplit = 32;
+// parts of a contraction over K for an [M][N] result, of kchunk each
+int split_of(int M, int N, int K, int* kchunk) {
+  const int TM = blocks(N, 128) * blocks(M, 128) >= 256 ? 128 : 64;
+  int S = 1;
+  if (blocks(N, TM) * blocks(M, TM) < 256 && K > 1024) S = std::min<int>(kMaxSplit, (K + 1023) / 1024);
+  *kchunk = (int)(blocks(blocks(K, S), BK) * BK);
+  return (int)blocks(K, *kchunk);
+}
+// split-k workspace: grown on the first call of a larger shape
+int need_ws(LymphMlp* m, size_t floats) {
+  if (floats <= m->ws_floats) return 0;
+  (void)hipStreamSynchronize(m->stream);
+  if (m->ws) (void)hipFree(m->ws);
+  m->ws = nullptr;
+  m->ws_floats = 0;
+  if (hipMalloc(&m->ws, floats * sizeof(float)) != hipSuccess)
+    return fail(LYMPH_MLP_ERR_HIP, "hipMalloc of the split-k workspace failed");
+  m->ws_floats = floats;
+  return 0;
+}
 template <bool A_KC, bool B_KC, int EPI>
 int gemm(LymphMlp* m, GemmArgs a) {
   if (a.M <= 0 || a.N <= 0 || a.K <= 0) return 0;
   const bool big = blocks(a.N, 128) * blocks(a.M, 128) >= 256;
   const int TM = big ? 128 : 64;
-  const unsigned tiles = blocks(a.N, TM) * blocks(a.M, TM);
-  int S = 1;
-  if (tiles < 256 && a.K > 1024) S = std::min<int>(kMaxSplit, (a.K + 1023) / 1024);
-  a.kchunk = (int)(blocks(blocks(a.K, S), BK) * BK);
-  S = (int)blocks(a.K, a.kchunk);
+  const int S = split_of(a.M, a.N, a.K, &a.kchunk);
   a.part = nullptr;
   if (S > 1) {
-    const size_t need = (size_t)S * a.M * a.N;
-    if (need > m->ws_floats) {  // grown once, on the first call of a larger shape
-      (void)hipStreamSynchronize(m->stream);
-      if (m->ws) (void)hipFree(m->ws);
-      m->ws = nullptr;
-      m->ws_floats = 0;
-      if (hipMalloc(&m->ws, need * sizeof(float)) != hipSuccess)
-        return fail(LYMPH_MLP_ERR_HIP, "hipMalloc of the split-k workspace failed");
-      m->ws_floats = need;
-    }
+    if (int rc = need_ws(m, (size_t)S * a.M * a.N)) return rc;
     a.part = m->ws;
   }
   dim3 grid(blocks(a.N, TM), blocks(a.M, TM), S);
@@ -978,39 +1344,92 @@ int grow(LymphMlp* m, LymphMlp::Buf& b, size_t n) {
   return 0;
 }
 
-// Outputs of n rows (device).  16 rows a slab until every CU has one (4096
-// rows), then 32: the weights are read once per slab, and two slabs of 32 fit
-// a CU's registers.
+// Tiles of 16 per wave and direction of a wide layer's k_wide, 1: k_layer.
+// The larger a wave's block, the less of the rows' activations every group of
+// columns reads again (256 rows x 38,400: 47 us with 4 x 4 tiles, 57 with 2 x
+// 2, 70 with 4 x 1), as long as about two waves a SIMD are left: 1024 blocks
+// of 4 x 4, 512 of 2 x 2.
+int wide_tile(int N, int B) {
+  const size_t t = (size_t)tiles_of(N) * tiles_of(B);
+  return t >= 16 * 1024 ? 4 : t >= 4 * 512 ? 2 : 1;
+}
+// its launch; returns the waves (entries of the loss sum)
+template <int EPI>
+int launch_wide(LymphMlp* m, LayerArgs& a) {
+  const int T = wide_tile(a.N, a.B), nt = tiles_of(a.N), nm = tiles_of(a.B);
+  if (T == 1) {
+    k_layer<EPI, false><<<(unsigned)layer_wgs(a.N, a.B), 128, 0, m->stream>>>(a);
+    return nt * nm;
+  }
+  a.rw = nm > 2 * T ? 4 : nm > T ? 2 : 1;
+  const unsigned wr = blocks(nm, T * a.rw), cg = blocks(nt, T * (4 / a.rw));
+  const unsigned wgs = 8 * blocks(cg, 8) * wr;
+  if (T == 4) k_wide<4, EPI><<<wgs, 256, 0, m->stream>>>(a);
+  else k_wide<2, EPI><<<wgs, 256, 0, m->stream>>>(a);
+  return (int)wgs * 4;
+}
+
+// Rows of a forward pass at a time: at most 64 MB of outputs, a batch at least
+int chunk_rows(const LymphMlp* m) {
+  return std::max(m->max_batch, (int)((16u << 20) / (unsigned)m->w[m->L]) / 32 * 32);
+}
+
+// Outputs of n <= chunk_rows() rows (device).  16 rows a slab until every CU
+// has one (4096 rows), then 32: the weights are read once per slab, and two
+// slabs of 32 fit a CU's registers.  A wide output layer takes the slabs'
+// activations from memory in a launch of its own, which spreads it over the chip.
 int slab_forward(LymphMlp* m, int n, const float* X, float* Y) {
   if (n <= 0) return 0;
   SlabArgs a{};
-  a.L = m->L;
+  a.L = m->wide ? m->L - 1 : m->L;
   a.B = n;
-  for (int l = 0; l <= m->L; ++l) a.w[l] = m->w[l];
-  for (int l = 0; l < m->L; ++l) {
+  for (int l = 0; l <= a.L; ++l) a.w[l] = m->w[l];
+  for (int l = 0; l < a.L; ++l) {
     a.Wf[l] = m->Wf[l];
     a.bias[l] = m->P + m->boff[l];
   }
   a.X = X;
-  a.Y = Y;
+  if (m->wide) {
+    const size_t need = pack_size((n + 31) / 32 * 32, a.w[a.L]);
+    if (need > m->hp_cap) {  // zeros: the padding of the last step is never written
+      HIP_TRY(hipStreamSynchronize(m->stream));
+      if (m->hp) (void)hipFree(m->hp);
+      m->hp = nullptr;
+      m->hp_cap = 0;
+      HIP_TRY(hipMalloc(&m->hp, need * sizeof(bf16_t)));
+      HIP_TRY(hipMemsetAsync(m->hp, 0, need * sizeof(bf16_t), m->stream));
+      m->hp_cap = need;
+    }
+    a.Hp = m->hp;
+  } else {
+    a.Y = Y;
+  }
   if (n <= 4096)
     k_slab<16, 16><<<blocks(n, 16), 512, 0, m->stream>>>(a);
   else
     k_slab<32, 16><<<blocks(n, 32), 512, 0, m->stream>>>(a);
+  if (m->wide) {
+    const int l = m->L - 1;
+    LayerArgs o{};
+    o.N = m->w[m->L]; o.K = m->w[l]; o.B = n;
+    o.W = m->Wf[l]; o.in = m->hp; o.bias = m->P + m->boff[l]; o.Y = Y;
+    launch_wide<LAYER_OUT>(m, o);
+  }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("k_slab: ") + hipGetErrorString(e));
 }
 
 // One step on rows idx of X, T: gradients into G (adam == null) or applied.
-// L forward launches, L - 1 backward, one update.
+// L forward launches, L - 1 backward (a wide layer's in two), one update.
 int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx, float* loss,
               const AdamArgs* adam) {
   const size_t ny = (size_t)B * m->w[m->L];
   const int L = m->L;
   hipStream_t st = m->stream;
+  int n_part = tiles_of(B) * tiles_of(m->w[L]);
   for (int l = 0; l < L; ++l) {
     LayerArgs a{};
-    a.N = m->w[l + 1]; a.K = m->w[l]; a.B = B; a.ldb = m->max_batch;
+    a.N = m->w[l + 1]; a.K = m->w[l]; a.B = B; a.ts = steps_of(m->max_batch);
     a.W = m->Wf[l];
     a.in = m->HP[l];
     a.X = X; a.idx = idx; a.XT = m->HT[0];
@@ -1023,32 +1442,49 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
     } else {
       a.out = m->DP[l]; a.outT = m->DT[l];
       a.T = T; a.scale = 2.0f / (float)ny; a.part = m->part;
-      if (l == 0) k_layer<LAYER_LOSS, true><<<wgs, 128, 0, st>>>(a);
+      if (m->wide) n_part = launch_wide<LAYER_LOSS>(m, a);
+      else if (l == 0) k_layer<LAYER_LOSS, true><<<wgs, 128, 0, st>>>(a);
       else k_layer<LAYER_LOSS, false><<<wgs, 128, 0, st>>>(a);
     }
   }
   for (int l = L - 1; l >= 1; --l) {  // dZ_{l-1} = (dZ_l W_l) gelu'(z_{l-1})
     LayerArgs a{};
-    a.N = m->w[l]; a.K = m->w[l + 1]; a.B = B; a.ldb = m->max_batch;
+    a.N = m->w[l]; a.K = m->w[l + 1]; a.B = B; a.ts = steps_of(m->max_batch);
     a.W = m->Wd[l];
     a.in = m->DP[l];
     a.out = l > 1 ? m->DP[l - 1] : nullptr; a.outT = m->DT[l - 1]; a.dg = m->dg[l - 1];
-    k_layer<LAYER_BWD, false><<<(unsigned)layer_wgs(a.N, B), 128, 0, st>>>(a);
+    int kchunk = 0;
+    const int S = l == L - 1 && m->wide ? split_of(B, a.N, a.K, &kchunk) : 1;
+    if (S == 1) {
+      k_layer<LAYER_BWD, false><<<(unsigned)layer_wgs(a.N, B), 128, 0, st>>>(a);
+      continue;
+    }
+    const int nt = tiles_of(a.N), nm = tiles_of(B);
+    if (int rc = need_ws(m, (size_t)S * nt * nm * 256)) return rc;
+    f32x4* ws = reinterpret_cast<f32x4*>(m->ws);
+    if (nm >= 8)
+      k_split<4><<<8 * blocks(S, 8) * blocks(nm, 8) * blocks(nt, 8), 256, 0, st>>>(a, S, kchunk / 32, ws);
+    else
+      k_split<2><<<8 * blocks(S, 8) * blocks(nm, 4) * blocks(nt, 4), 256, 0, st>>>(a, S, kchunk / 32, ws);
+    k_split_end<<<(unsigned)(nt * nm), 64, 0, st>>>(a, S, ws);
   }
   UpdateArgs u{};
   u.L = L;
   u.B = B;
-  u.ldb = m->max_batch;
+  u.ts = steps_of(m->max_batch);
   u.P = m->P; u.M = m->Mo; u.V = m->Vo; u.G = m->G;
   if (adam) u.a = *adam;
+  // a wide layer's weights in a launch of their own where it fills the chip
+  const int big = (int)(blocks(m->w[L], kUpN) * blocks(m->w[L - 1], kUpK));
+  const int apart = m->wide && big >= 256 ? L - 1 : -1;
   int wgs = 0, bias = 0;
   for (int l = 0; l < L; ++l) {
     UpdateLayer& y = u.y[l];
     y.N = m->w[l + 1];
     y.K = m->w[l];
     y.first = wgs;
-    wgs += (int)(blocks(y.N, 16) * blocks(y.K, 64));
-    bias += y.N / 4;
+    if (l != apart) wgs += (int)(blocks(y.N, 16) * blocks(y.K, 64));
+    if (l != apart) bias += y.N / 4;
     y.DT = m->DT[l];
     y.HT = m->HT[l];
     y.woff = m->woff[l];
@@ -1058,9 +1494,13 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
   }
   u.first_bias = wgs;
   u.part = m->part;
-  u.n_part = tiles_of(B) * tiles_of(m->w[L]);
+  u.n_part = n_part;
   u.part_scale = 1.0f / (float)ny;
   u.loss = loss;
+  if (apart >= 0) {
+    if (adam) k_update_wide<true><<<big, 256, 0, st>>>(u, apart);
+    else k_update_wide<false><<<big, 256, 0, st>>>(u, apart);
+  }
   if (adam) k_update<true><<<wgs + bias + 1, 128, 0, st>>>(u);
   else k_update<false><<<wgs + bias + 1, 128, 0, st>>>(u);
   hipError_t e = hipGetLastError();
@@ -1080,6 +1520,7 @@ int lymph_mlp_destroy(LymphMlp* m) {
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   for (void* p : m->owned) (void)hipFree(p);
   if (m->ws) (void)hipFree(m->ws);
+  if (m->hp) (void)hipFree(m->hp);
   if (m->dorder) (void)hipFree(m->dorder);
   if (m->dloss) (void)hipFree(m->dloss);
   if (m->in.own) (void)hipFree(m->in.p);
@@ -1127,16 +1568,18 @@ int lymph_mlp_create(int n_layers, const int32_t* widths, int max_batch, LymphMl
   zero(&m->Vo, off);
   al(&m->G, off);
   const int NL = m->w[n_layers];
-  m->slab = n_layers <= kSlabL && *std::max_element(m->w.begin(), m->w.end()) <= kSlabW;
-  const size_t ldb = (size_t)max_batch;
+  m->wide = n_layers > 1 && NL > kSlabW;
+  m->slab = n_layers <= kSlabL && *std::max_element(m->w.begin(), m->w.end() - 1) <= kSlabW &&
+            (NL <= kSlabW || m->wide);
+  m->wide = m->wide && m->slab;
   if (m->slab) {
     for (auto* v : {&m->Wf, &m->Wd, &m->HT, &m->DT, &m->HP, &m->DP}) v->assign(n_layers, nullptr);
     m->dg.assign(n_layers, nullptr);
     for (int l = 0; l < n_layers; ++l) {
       const int N = m->w[l + 1], K = m->w[l];
       zero(&m->Wf[l], pack_size(N, K));
-      al(&m->HT[l], ldb * K);
-      al(&m->DT[l], ldb * N);
+      al(&m->HT[l], pack_size(K, max_batch));
+      al(&m->DT[l], pack_size(N, max_batch));
       if (l > 0) {  // operands of the next layer's launch, either way
         zero(&m->Wd[l], pack_size(K, N));
         zero(&m->HP[l], pack_size(max_batch, K));
@@ -1155,7 +1598,10 @@ int lymph_mlp_create(int n_layers, const int32_t* widths, int max_batch, LymphMl
     al(&m->dZa, (size_t)max_batch * maxh);
     al(&m->dZb, (size_t)max_batch * maxh);
   }
-  al(&m->part, std::max((size_t)blocks((size_t)max_batch * NL, 256), (size_t)tiles_of(max_batch) * tiles_of(NL)));
+  // k_loss: a sum per workgroup; the layer kernels: one per wave, of whole
+  // groups of 8 workgroups (launch_wide: 2 x 2 tiles a wave or more)
+  const size_t mt = tiles_of(max_batch), nt = tiles_of(NL);
+  al(&m->part, std::max((size_t)blocks((size_t)max_batch * NL, 256), mt * nt + 16 * mt + 2 * nt + 128));
   al(&m->loss, 1);
   al(&m->idx, (size_t)max_batch);
   m->in.cap = (size_t)max_batch * m->w[0];
@@ -1340,11 +1786,15 @@ int lymph_mlp_predict(LymphMlp* m, int n, const float* x, float* y) {
       hipMemcpyAsync(dx, x, (size_t)n * w0 * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
     rc = fail(LYMPH_MLP_ERR_HIP, "upload failed");
   if (m->slab) {
-    if (!rc) rc = grow(m, m->out, (size_t)std::max(1, n) * NL);
-    if (!rc) rc = slab_forward(m, n, dx, m->out.p);
-    if (!rc && n > 0 &&
-        hipMemcpyAsync(y, m->out.p, (size_t)n * NL * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
-      rc = fail(LYMPH_MLP_ERR_HIP, "download failed");
+    const int chunk = chunk_rows(m);
+    if (!rc) rc = grow(m, m->out, (size_t)std::max(1, std::min(n, chunk)) * NL);
+    for (int b0 = 0; b0 < n && !rc; b0 += chunk) {
+      const int B = std::min(chunk, n - b0);
+      rc = slab_forward(m, B, dx + (size_t)b0 * w0, m->out.p);
+      if (!rc && hipMemcpyAsync(y + (size_t)b0 * NL, m->out.p, (size_t)B * NL * 4, hipMemcpyDeviceToHost,
+                                m->stream) != hipSuccess)
+        rc = fail(LYMPH_MLP_ERR_HIP, "download failed");
+    }
     if (hipStreamSynchronize(m->stream) != hipSuccess && !rc) rc = fail(LYMPH_MLP_ERR_HIP, "prediction failed");
     return rc;
   }
@@ -1371,8 +1821,9 @@ int lymph_mlp_time_predict(LymphMlp* m, int n, int reps, double* ms) {
   std::vector<int> id(m->max_batch);
   for (int i = 0; i < m->max_batch; ++i) id[i] = i;
   HIP_TRY(hipMemcpyAsync(m->idx, id.data(), 4 * m->max_batch, hipMemcpyHostToDevice, m->stream));
+  const int chunk = chunk_rows(m);
   if (m->slab)
-    if (int rc = grow(m, m->out, (size_t)n * m->w[m->L])) return rc;
+    if (int rc = grow(m, m->out, (size_t)std::min(n, chunk) * m->w[m->L])) return rc;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
@@ -1380,7 +1831,8 @@ int lymph_mlp_time_predict(LymphMlp* m, int n, int reps, double* ms) {
   HIP_TRY(hipEventRecord(e0, m->stream));
   for (int r = 0; r < reps && !rc; ++r) {
     if (m->slab) {
-      rc = slab_forward(m, n, m->X, m->out.p);
+      for (int b0 = 0; b0 < n && !rc; b0 += chunk)
+        rc = slab_forward(m, std::min(chunk, n - b0), m->X + (size_t)b0 * m->w[0], m->out.p);
       continue;
     }
     for (int b0 = 0; b0 < n && !rc; b0 += m->max_batch) {

@@ -128,3 +128,15 @@ def test_narrow_networks_at_tile_edges_match_oracle(widths, batch):
         with Mlp(widths, max_batch=batch, seed=0) as other:
             other.set_params(net.params())
             assert np.array_equal(other.predict(x[:33]), net.predict(x[:33]))
+
+
+# a wide output layer behind hidden layers of at most 512: one tile a wave (520),
+# 2 x 2 (8000 x 72) and 4 x 4 (16,408 x 264) with remainders both ways, the
+# contraction of its input gradient in one, 2, 8 and 17 parts
+WIDE = [([8, 16, 520], 8), ([24, 72, 40, 1032], 24), ([8, 512, 8000], 72), ([16, 40, 16408], 264)]
+
+
+@pytest.mark.parametrize("widths,batch", WIDE)
+def test_wide_outputs_at_tile_edges_match_oracle(widths, batch):
+    """The checks above; 4200 rows of 16,408 outputs come in several chunks."""
+    test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
