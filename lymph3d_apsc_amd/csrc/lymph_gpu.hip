@@ -400,8 +400,8 @@ void launch_leapfrog48(int variant, int grid, hipStream_t st, const float* K, co
 //  - few polyhedra (below 256, or below 1024 where uneven polyhedra make long
 //    block rows): the step is one chain of memory trips, so 8 waves share a
 //    polyhedron and each has a whole block in flight.  125 polyhedra, us per
-//    step, one wave per polyhedron / 8 waves: FP64 p = 1..4 5.9 / 3.9, 12.5 /
-//    5.9, 30.7 / 12.0, 96 / 34; 32-bit 5.0 / 3.0, 12.2 / 3.3, 17.3 / 4.7, 53 /
+//    step, one wave per polyhedron / 8 waves: FP64 p = 1..4 6.3 / 3.9, 11.9 /
+//    5.3, 28.4 / 9.7, 88 / 26; 32-bit 5.0 / 3.0, 12.2 / 3.3, 17.3 / 4.7, 53 /
 //    11; 48-bit p = 2, 3 9.9 / 4.1, 30.2 / 6.3;
 //  - up to 3000 polyhedra 4 waves (p <= 2; 1000 polyhedra, FP64 p = 2: 11.9
 //    us against 24.8 with one wave and 13.5 with 8);

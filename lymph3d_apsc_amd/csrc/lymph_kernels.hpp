@@ -904,36 +904,70 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Broadcast lane `l`'s double to the whole wave (v_readlane on both halves).
+__device__ __forceinline__ double lane_bcast(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+
+// A divisor b of many quotients: y = 1 / b rounded, then quot() gives a / b to
+// the bits of the division in five dependent operations instead of a dozen
+// (Markstein, IBM J. Res. Dev. 34, 1990: the remainder a - b q is exact in one
+// fused multiply-add, the first correction makes q faithful, the second rounds
+// it correctly).  Quotients that are not finite come from the division's own
+// rule: q = a y is then the infinity or NaN it gives.
+struct Divisor {
+  double b, y;
+  __device__ __forceinline__ explicit Divisor(double v) : b(v), y(1.0 / v) {}
+  // within this range no quotient of a normal number leaves the exponents
+  // where the remainder is exact; outside it the solves divide
+  __device__ __forceinline__ bool plain() const { return fabs(b) > 0x1p-400 && fabs(b) < 0x1p400; }
+};
+__device__ __forceinline__ double quot(double a, const Divisor& d) {
+  const double q0 = a * d.y;
+  const double q1 = fma(fma(-d.b, q0, a), d.y, q0);
+  const double q2 = fma(fma(-d.b, q1, a), d.y, q1);
+  return fabs(q0) < __builtin_inf() ? q2 : q0;
+}
+
 // M^-1 w = R^-1 R^-T w (solve_LU with L = R^T, src/vet_mat_operations.f90:
 // 123-153) across a group of 3Np lanes from lane `base`, one entry of the
-// vector per lane: r = component x Np + row (other lanes pass through).  The
-// forward sweep broadcasts y_j = s_j / R_jj and the rows below subtract R_ji
-// y_j, in ascending j as the reference does; the backward sweep runs the
-// columns from the last, the rows above subtracting R_ij x_j.  NP dependent
-// steps per sweep instead of Np(Np+1)/2 on one lane, which the step kernels'
-// tails paid before (125 polyhedra: 6 us of a step at p = 2, 50 at p = 4).
-template <int NP>
-__device__ __forceinline__ double solve_group(const double* __restrict__ R, double w, int base, int r, bool on) {
-  const int cc = on ? r / NP : 0, ii = r % NP, from = on ? base + cc * NP : 0;
+// vector per lane: r = component x Np + row (other lanes' results are not
+// used).  The forward sweep broadcasts y_j = s_j / R_jj and the rows below
+// subtract R_ji y_j, in ascending j as the reference does; the backward sweep
+// runs the columns from the last, the rows above subtracting R_ij x_j.  NP
+// dependent steps per sweep instead of Np(Np+1)/2 on one lane.  A lane past its
+// own step goes on with values that nothing reads, which keeps the selects off
+// the chain.  The solves are the tail of a step on few polyhedra: with divisions
+// and selects on the chain 162 single-tet polyhedra took 6.2, 10.4 and 30.9 us
+// a step at p = 2, 3, 4, now 5.2, 8.6 and 22.7.
+template <int NP, bool PLAIN>
+__device__ __forceinline__ double solve_group_as(const double* __restrict__ R, const Divisor& d, double w, int ii,
+                                                 int from) {
+  double y = 0.0;
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
-    const int rj = pk_off(NP, j);
-    const double yj = __shfl(w, from + j, 64) / R[rj];
-    if (on && ii == j)
-      w = yj;
-    else if (on && ii > j)
-      w = w - R[rj + (ii - j)] * yj;
+    const double t = PLAIN ? quot(w, d) : w / d.b;
+    if (ii == j) y = t;
+    w = w - R[pk_off(NP, j) + (ii > j ? ii - j : 0)] * __shfl(t, from + j, 64);
   }
-  const int ri = pk_off(NP, on ? ii : 0);
+  const int ri = pk_off(NP, ii);
+  w = y;
 #pragma unroll
   for (int j = NP - 1; j >= 0; --j) {
-    const double xj = __shfl(w, from + j, 64) / R[pk_off(NP, j)];
-    if (on && ii == j)
-      w = xj;
-    else if (on && ii < j)
-      w = w - R[ri + (j - ii)] * xj;
+    const double t = PLAIN ? quot(w, d) : w / d.b;
+    if (ii == j) y = t;
+    w = w - R[ri + (ii < j ? j - ii : 0)] * __shfl(t, from + j, 64);
   }
-  return w;
+  return y;
+}
+template <int NP>
+__device__ __forceinline__ double solve_group(const double* __restrict__ R, const Divisor& d, double w, int base,
+                                              int r, bool on) {
+  const int cc = on ? r / NP : 0, ii = on ? r % NP : 0, from = on ? base + cc * NP : 0;
+  return __all(!on || d.plain()) ? solve_group_as<NP, true>(R, d, w, ii, from)
+                                 : solve_group_as<NP, false>(R, d, w, ii, from);
 }
 
 // R^-T of three right-hand sides across one wave, lane i on row i of all three
@@ -960,28 +994,44 @@ __device__ __forceinline__ void forward_rows(const double* __restrict__ R, doubl
   }
 }
 
-// M^-1 of three right-hand sides across one wave: forward_rows, then the
-// columns from the last.  NP dependent steps per sweep instead of NP(NP+1)/2
-// on one lane.
-template <int NP>
-__device__ __forceinline__ void solve_rows(const double* __restrict__ R, double& x0, double& x1, double& x2, int i) {
-  forward_rows<NP>(R, x0, x1, x2, i);
-  const int ri = pk_off(NP, i < NP ? i : 0);
+// M^-1 of three right-hand sides across one wave, lane i on row i of all three
+// (NP <= 64), the sweeps as in solve_group; d: the divisor R_ii of lane i.
+// Broadcasts by v_readlane (24.2 us above with __shfl).
+template <int NP, bool PLAIN>
+__device__ __forceinline__ void solve_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
+  double y[3] = {0.0, 0.0, 0.0};
 #pragma unroll 5
-  for (int j = NP - 1; j >= 0; --j) {
-    const double rjj = R[pk_off(NP, j)];
-    const double y0 = __shfl(x0, j, 64) / rjj, y1 = __shfl(x1, j, 64) / rjj, y2 = __shfl(x2, j, 64) / rjj;
-    if (i == j) {
-      x0 = y0;
-      x1 = y1;
-      x2 = y2;
-    } else if (i < j) {
-      const double r = R[ri + (j - i)];
-      x0 = x0 - r * y0;
-      x1 = x1 - r * y1;
-      x2 = x2 - r * y2;
+  for (int j = 0; j < NP; ++j) {
+    const double r = R[pk_off(NP, j) + (i < NP && i > j ? i - j : 0)];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
+      if (i == j) y[c] = t;
+      x[c] = x[c] - r * lane_bcast(t, j);
     }
   }
+  const int ri = pk_off(NP, i < NP ? i : 0);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) x[c] = y[c];
+#pragma unroll 5
+  for (int j = NP - 1; j >= 0; --j) {
+    const double r = R[ri + (i < NP && i < j ? j - i : 0)];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
+      if (i == j) y[c] = t;
+      x[c] = x[c] - r * lane_bcast(t, j);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) x[c] = y[c];
+}
+template <int NP>
+__device__ __forceinline__ void solve_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
+  if (__all(i >= NP || d.plain()))
+    solve_rows_as<NP, true>(R, d, x, i);
+  else
+    solve_rows_as<NP, false>(R, d, x, i);
 }
 
 // R^-1 y in place on one lane, every row's terms in ascending columns as the
@@ -1091,13 +1141,6 @@ __global__ void k_fill(double* __restrict__ a, double v, size_t n) {
 //   MODE 1: out = (c1*x + u) + c2*wa           (c1 = dt^2/2, u = u^0, wa = v^0, c2 = dt)
 //   MODE 2: part[P] = sum_r u_r (K u)_r        (DG error: K = A_dg, u = uh - uex)
 // ---------------------------------------------------------------------------
-// Broadcast lane `l`'s double to the whole wave (v_readlane on both halves).
-__device__ __forceinline__ double lane_bcast(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-  return __hiloint2double(hi, lo);
-}
-
 // Polyhedron of this workgroup.  Workgroups are dealt to the 8 XCDs round
 // robin (workgroup b runs on XCD b % 8), each XCD with its own L2; the grid is
 // padded to a multiple of 8 and XCD x is given the x-th eighth of the
@@ -1171,8 +1214,13 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
   if (MODE != 2)
     for (int k = threadIdx.x; k < D::NPK; k += 64 * WPP) sR[k] = Rp[(size_t)Pp * D::NPK + k];
   StepEnds<N3, RPL> ends;
+  const int drow = RPL == 1 ? (lane < N3 ? lane % NP : 0) : (lane < NP ? lane : 0);  // the lane's row in the solve
+  Divisor diag(1.0);
   if constexpr (WPP > 1 && MODE != 2)
-    if (wv == 0) ends.load(rs, rd, u, wa, (size_t)Pp * N3, lane);
+    if (wv == 0) {
+      ends.load(rs, rd, u, wa, (size_t)Pp * N3, lane);
+      diag = Divisor(Rp[(size_t)Pp * D::NPK + pk_off(NP, drow)]);
+    }
   double acc[RPL];
 #pragma unroll
   for (int k = 0; k < RPL; ++k) acc[k] = 0.0;
@@ -1282,21 +1330,22 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
   double w[RPL];
 #pragma unroll
   for (int k = 0; k < RPL; ++k) w[k] = -acc[k] + ends.s[k] + ends.d[k] * gp;
+  if constexpr (WPP == 1) diag = Divisor(sR[pk_off(NP, drow)]);
   if constexpr (RPL == 1) {  // one row per lane: the wave solves across its lanes
-    w[0] = solve_group<NP>(sR, w[0], 0, lane, lane < N3);
+    w[0] = solve_group<NP>(sR, diag, w[0], 0, lane, lane < N3);
   } else {  // lane i takes row i of the three components
 #pragma unroll
     for (int k = 0; k < RPL; ++k)
       if (lane + 64 * k < N3) sw[lane + 64 * k] = w[k];
     wave_lds_sync();
     const bool row = lane < NP;
-    double x0 = row ? sw[lane] : 0.0, x1 = row ? sw[NP + lane] : 0.0, x2 = row ? sw[2 * NP + lane] : 0.0;
-    solve_rows<NP>(sR, x0, x1, x2, lane);
-    if (row) {
-      sw[lane] = x0;
-      sw[NP + lane] = x1;
-      sw[2 * NP + lane] = x2;
-    }
+    double x[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) x[c] = row ? sw[c * NP + lane] : 0.0;
+    solve_rows<NP>(sR, diag, x, lane);
+    if (row)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) sw[c * NP + lane] = x[c];
     wave_lds_sync();
 #pragma unroll
     for (int k = 0; k < RPL; ++k) w[k] = lane + 64 * k < N3 ? sw[lane + 64 * k] : 0.0;
@@ -2141,7 +2190,8 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __rest
   }
   if constexpr (TB == 64) {
     lsync<WPW>();  // sR
-    w = solve_group<NP>(sR[act ? sub : 0], w, sub * N3, r, act);
+    const double* R = sR[act ? sub : 0];
+    w = solve_group<NP>(R, Divisor(act ? R[pk_off(NP, r % NP)] : 1.0), w, sub * N3, r, act);
   }
   if (act) {
     if (MODE == 0)
@@ -2326,7 +2376,8 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restr
   }
   if constexpr (TB == 64) {
     lsync<WPW>();  // sR
-    w = solve_group<NP>(sR[act ? sub : 0], w, sub * N3, r, act);
+    const double* R = sR[act ? sub : 0];
+    w = solve_group<NP>(R, Divisor(act ? R[pk_off(NP, r % NP)] : 1.0), w, sub * N3, r, act);
   }
   if (act) {
     if (MODE == 0)

@@ -899,3 +899,34 @@ def test_build_of_a_polyhedron_with_a_long_block_row(p, build):
         for b in range(K.shape[0]):
             assert rel(K[b], oK[b]) < 1e-13, (b, rel(K[b], oK[b]))
             assert rel(A[b], oA[b]) < 1e-13
+
+
+@pytest.mark.parametrize("p", [1, 2, 3, 4])
+def test_mass_solves_by_reciprocals_give_the_divisions_bits(p):
+    """Densities times 2^900 take the mass factor out of the range in which the
+    step kernels correct products with reciprocals (they divide there): from
+    zero displacement the accelerations must be the plain ones' bits times
+    2^-900, for every variant, zeros and infinities in the load among them."""
+    say(f"[mass solve] p={p}")
+    m = M.cube_mesh(3, agglomerate=True)
+    out = []
+    for scale in (1.0, 2.0 ** 900):
+        m.rho = np.full(m.n_tet, 1.3) * scale
+        with L.Context(m, p) as ctx:
+            ctx.make_matrices_free()
+            z = ctx.vec()
+            f = np.random.default_rng(p).standard_normal(z.size).reshape(m.n_poly, -1)
+            f[1] = 0.0
+            f[2, ::3] = 0.0
+            f[3, 1] = np.inf
+            ctx.set_slot(_lib.SLOT_RHS_STAT, z)
+            ctx.set_slot(_lib.SLOT_RHS_DYN, f.ravel() * np.sqrt(scale))
+            got = []
+            for v in range(ctx.n_step_variants()):
+                ctx.set_step_variant(v)
+                got.append(ctx.time_step_matrix_free(1.0, 1.0, z, z) * np.sqrt(scale))
+            out.append(got)
+    assert np.isfinite(out[0][0].reshape(m.n_poly, -1)[[0, 1, 2]]).all() and np.abs(out[0][0][:10]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, out[0][0], equal_nan=True)
+        assert np.array_equal(a, b, equal_nan=True)
