@@ -210,45 +210,65 @@ template <int P> constexpr int n_var() { return (int)(sizeof(StepVar<P>::unr) / 
 // block row) must stay within this; otherwise variant 0 runs instead
 constexpr size_t kMaxDynLds = 64 * 1024;
 
+// Step kernels read the operator with streaming loads, or (keep) with cached
+// ones where it stays on the chip from one step to the next
+template <int MODE, class F>
+void with_nt(bool keep, F&& launch) {
+  if constexpr (MODE == 2) {
+    launch(std::true_type{});
+  } else {
+    if (keep) launch(std::false_type{});
+    else launch(std::true_type{});
+  }
+}
+
 template <int P, int MODE, int I = 0>
 void launch_leapfrog(int variant, int grid, hipStream_t st, const double* K, const int* rp,
                      const int* col, const double* Rp, const double* rs, const double* rd,
                      const double* u, const double* wa, double* out, double g, double c1,
-                     double c2, const int* gsel, const double* gtab, const int* ord, size_t dyn) {
+                     double c2, const int* gsel, const double* gtab, const int* ord, size_t dyn, bool keep) {
   if constexpr (I < n_var<P>()) {
     if (variant == I) {
       constexpr int W = StepVar<P>::wpp[I];
       if constexpr (StepVar<P>::xs[I] == 2) {
         constexpr int G = 64 / (3 * np_of(P));
         const int groups = (grid + G - 1) / G;
-        k_leapfrog_packed<P, MODE, 64, W><<<step_grid((groups + W - 1) / W), 64 * W, 0, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog_packed<P, MODE, 64, W, decltype(nt)::value>
+              <<<step_grid((groups + W - 1) / W), 64 * W, 0, st>>>(
             K, nullptr, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid);
+        });
         return;
       } else if constexpr (StepVar<P>::xs[I] == 3) {
         constexpr int G = 64 / (3 * np_of(P));
         if ((size_t)W * G * dyn > kMaxDynLds) {
           launch_leapfrog<P, MODE, 0>(0, grid, st, K, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2,
-                                      gsel, gtab, ord, dyn);
+                                      gsel, gtab, ord, dyn, keep);
           return;
         }
         const int groups = (grid + G - 1) / G;
-        k_leapfrog_joint<P, MODE, 64, W><<<step_grid((groups + W - 1) / W), 64 * W, W * G * dyn, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog_joint<P, MODE, 64, W, decltype(nt)::value>
+              <<<step_grid((groups + W - 1) / W), 64 * W, W * G * dyn, st>>>(
             K, nullptr, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid, (int)(G * dyn / 8));
+        });
         return;
       } else {
       if (W > 1 && dyn > kMaxDynLds) {
         launch_leapfrog<P, MODE, 0>(0, grid, st, K, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2,
-                                    gsel, gtab, ord, dyn);
+                                    gsel, gtab, ord, dyn, keep);
         return;
       }
-      k_leapfrog<P, MODE, StepVar<P>::unr[I], StepVar<P>::xs[I], W>
-          <<<step_grid(grid), 64 * W, W > 1 ? dyn : 0, st>>>(K, rp, col, Rp, rs, rd, u, wa, out, g,
+      with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog<P, MODE, StepVar<P>::unr[I], StepVar<P>::xs[I], W, decltype(nt)::value>
+              <<<step_grid(grid), 64 * W, W > 1 ? dyn : 0, st>>>(K, rp, col, Rp, rs, rd, u, wa, out, g,
                                                              c1, c2, gsel, gtab, grid, ord);
+        });
       return;
       }
     }
     launch_leapfrog<P, MODE, I + 1>(variant, grid, st, K, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2,
-                                    gsel, gtab, ord, dyn);
+                                    gsel, gtab, ord, dyn, keep);
   }
 }
 
@@ -313,41 +333,49 @@ template <int P, int MODE, int I = 0>
 void launch_leapfrog32(int variant, int grid, hipStream_t st, const float* K, const int* rp,
                        const int* col, const double* Rp, const double* rs, const double* rd,
                        const double* u, const double* wa, double* out, double g, double c1,
-                       double c2, const int* gsel, const double* gtab, const int* ord, size_t dyn) {
+                       double c2, const int* gsel, const double* gtab, const int* ord, size_t dyn, bool keep) {
   if constexpr (I < n_var32<P>()) {
     if (variant == I) {
       constexpr int W = StepVar32<P>::wpp[I];
       if constexpr (StepVar32<P>::pk[I] == 1) {
         constexpr int G = 64 / (3 * np_of(P));
         const int groups = (grid + G - 1) / G;
-        k_leapfrog_packed<P, MODE, 32, W><<<step_grid((groups + W - 1) / W), 64 * W, 0, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog_packed<P, MODE, 32, W, decltype(nt)::value>
+              <<<step_grid((groups + W - 1) / W), 64 * W, 0, st>>>(
             K, nullptr, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid);
+        });
         return;
       } else if constexpr (StepVar32<P>::pk[I] == 2) {
         constexpr int G = 64 / (3 * np_of(P));
         if ((size_t)W * G * dyn > kMaxDynLds) {
           launch_leapfrog32<P, MODE, 0>(0, grid, st, K, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2,
-                                        gsel, gtab, ord, dyn);
+                                        gsel, gtab, ord, dyn, keep);
           return;
         }
         const int groups = (grid + G - 1) / G;
-        k_leapfrog_joint<P, MODE, 32, W><<<step_grid((groups + W - 1) / W), 64 * W, W * G * dyn, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog_joint<P, MODE, 32, W, decltype(nt)::value>
+              <<<step_grid((groups + W - 1) / W), 64 * W, W * G * dyn, st>>>(
             K, nullptr, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid, (int)(G * dyn / 8));
+        });
         return;
       } else {
       if (W > 1 && dyn > kMaxDynLds) {
         launch_leapfrog32<P, MODE, 0>(0, grid, st, K, rp, col, Rp, rs, rd, u, wa, out, g, c1, c2,
-                                      gsel, gtab, ord, dyn);
+                                      gsel, gtab, ord, dyn, keep);
         return;
       }
-      k_leapfrog32<P, MODE, StepVar32<P>::unr[I], W>
-          <<<step_grid(grid), 64 * W, W > 1 ? dyn : 0, st>>>(K, rp, col, Rp, rs, rd, u, wa, out, g,
+      with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog32<P, MODE, StepVar32<P>::unr[I], W, decltype(nt)::value>
+              <<<step_grid(grid), 64 * W, W > 1 ? dyn : 0, st>>>(K, rp, col, Rp, rs, rd, u, wa, out, g,
                                                              c1, c2, gsel, gtab, grid, ord);
+        });
       return;
       }
     }
     launch_leapfrog32<P, MODE, I + 1>(variant, grid, st, K, rp, col, Rp, rs, rd, u, wa, out, g, c1,
-                                      c2, gsel, gtab, ord, dyn);
+                                      c2, gsel, gtab, ord, dyn, keep);
   }
 }
 
@@ -355,7 +383,7 @@ template <int P, int MODE, int I = 0>
 void launch_leapfrog48(int variant, int grid, hipStream_t st, const float* K, const _Float16* Kr,
                        const int* rp, const int* col, const double* rs, const double* rd,
                        const double* u, const double* wa, double* out, double g, double c1,
-                       double c2, const int* gsel, const double* gtab, const int* ord, size_t dyn) {
+                       double c2, const int* gsel, const double* gtab, const int* ord, size_t dyn, bool keep) {
   if constexpr (I < n_var48<P>()) {
     if (variant == I) {
       constexpr int W = StepVar48<P>::wpp[I];
@@ -363,34 +391,43 @@ void launch_leapfrog48(int variant, int grid, hipStream_t st, const float* K, co
         static_assert(3 * np_of(P) <= 32, "packed step needs 3Np <= 32");
         constexpr int G = 64 / (3 * np_of(P));
         const int groups = (grid + G - 1) / G;
-        k_leapfrog_packed<P, MODE, 48, W><<<step_grid((groups + W - 1) / W), 64 * W, 0, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog_packed<P, MODE, 48, W, decltype(nt)::value>
+              <<<step_grid((groups + W - 1) / W), 64 * W, 0, st>>>(
             K, Kr, rp, col, nullptr, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid);
+        });
         return;
       } else if constexpr (StepVar48<P>::pk[I] == 2) {
         static_assert(3 * np_of(P) <= 32, "joint packed step needs 3Np <= 32");
         constexpr int G = 64 / (3 * np_of(P));
         if ((size_t)W * G * dyn > kMaxDynLds) {
           launch_leapfrog48<P, MODE, 0>(0, grid, st, K, Kr, rp, col, rs, rd, u, wa, out, g, c1, c2,
-                                        gsel, gtab, ord, dyn);
+                                        gsel, gtab, ord, dyn, keep);
           return;
         }
         const int groups = (grid + G - 1) / G;
-        k_leapfrog_joint<P, MODE, 48, W><<<step_grid((groups + W - 1) / W), 64 * W, W * G * dyn, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog_joint<P, MODE, 48, W, decltype(nt)::value>
+              <<<step_grid((groups + W - 1) / W), 64 * W, W * G * dyn, st>>>(
             K, Kr, rp, col, nullptr, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid, (int)(G * dyn / 8));
+        });
         return;
       } else {
         if (W > 1 && dyn > kMaxDynLds) {
           launch_leapfrog48<P, MODE, 0>(0, grid, st, K, Kr, rp, col, rs, rd, u, wa, out, g, c1, c2,
-                                        gsel, gtab, ord, dyn);
+                                        gsel, gtab, ord, dyn, keep);
           return;
         }
-        k_leapfrog48<P, MODE, StepVar48<P>::unr[I], W><<<step_grid(grid), 64 * W, W > 1 ? dyn : 0, st>>>(
+        with_nt<MODE>(keep, [&](auto nt) {
+          k_leapfrog48<P, MODE, StepVar48<P>::unr[I], W, decltype(nt)::value>
+              <<<step_grid(grid), 64 * W, W > 1 ? dyn : 0, st>>>(
             K, Kr, rp, col, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, grid, ord);
+        });
         return;
       }
     }
     launch_leapfrog48<P, MODE, I + 1>(variant, grid, st, K, Kr, rp, col, rs, rd, u, wa, out, g, c1,
-                                      c2, gsel, gtab, ord, dyn);
+                                      c2, gsel, gtab, ord, dyn, keep);
   }
 }
 
@@ -488,11 +525,27 @@ int d2h_vec(LymphCtx* c, const double* d, double* h) {
   return 0;
 }
 
+// Whether the step's operator reads should stay in the caches: the eight L2s
+// hold 32 MB, the Infinity Cache 256 MB; beyond, a cached read only displaces
+// the vectors.  us per step, streaming / cached: 2,197 polyhedra p = 1 (17 MB)
+// 11.1 / 8.2; 125 p = 3 (21 MB) 9.7 / 7.5; 512 p = 2 (23 MB) 8.8 / 6.8; 32-bit 1,000 p =
+// 2 (23 MB) 6.9 / 5.1; p = 2 98 MB 18.7 / 16.9, 193 MB 33.7 / 31.4; deck of 28,606
+// tets p = 1 (161 MB) 31.7 / 30.4.  At p = 3 the two are even or streaming wins
+// between (46 MB 9.6 / 9.7, 92 MB 18.2 / 19.3), then 184 MB 34.4 / 31.8, 207 MB
+// 33.6 / 32.6.  Past the Infinity Cache streaming wins everywhere: 320 MB 60.6 /
+// 68.8, 354 MB 66 / 76.
+bool keep_operator(const LymphCtx* c) {
+  const size_t bytes = (size_t)c->n_blk * c->n3 * c->n3 * c->apply_bits / 8;
+  constexpr size_t kL2 = (size_t)32 << 20, kMall = (size_t)208 << 20;
+  return bytes <= kL2 || (bytes <= kMall && (c->p <= 2 || bytes >= 4 * kL2));
+}
+
 int launch_step(LymphCtx* c, int mode, double g, double c1, double c2, const double* u,
                 const double* wa, double* out, bool grouped = false) {
   const int* gsel = grouped ? c->gsel : nullptr;
   const double* gtab = grouped ? c->gtab : nullptr;
   const size_t dyn = (size_t)c->max_row * c->n3 * sizeof(double);
+  const bool keep = keep_operator(c);
   return dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
     // the 32-bit apply works on mass-orthonormal vectors: ~F from tilde_rhs
@@ -535,17 +588,17 @@ int launch_step(LymphCtx* c, int mode, double g, double c1, double c2, const dou
     } else if (c->apply_bits == 48) {
       if (mode == 0)
         launch_leapfrog48<P, 0>(c->step_variant, c->n_poly, c->stream, c->K32, c->K16, c->md.row_ptr,
-                                c->md.col, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn);
+                                c->md.col, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn, keep);
       else
         launch_leapfrog48<P, 1>(c->step_variant, c->n_poly, c->stream, c->K32, c->K16, c->md.row_ptr,
-                                c->md.col, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn);
+                                c->md.col, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn, keep);
     } else if (c->apply_bits == 32) {
       if (mode == 0)
         launch_leapfrog32<P, 0>(c->step_variant, c->n_poly, c->stream, c->K32, c->md.row_ptr,
-                                c->md.col, c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn);
+                                c->md.col, c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn, keep);
       else
         launch_leapfrog32<P, 1>(c->step_variant, c->n_poly, c->stream, c->K32, c->md.row_ptr,
-                                c->md.col, c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn);
+                                c->md.col, c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn, keep);
     } else if (c->Ks) {
       if constexpr (3 * np_of(P) <= 64 && (3 * np_of(P)) % 2 == 0) {
         const int n_pair = (c->n_blk - c->n_poly) / 2;
@@ -582,10 +635,10 @@ int launch_step(LymphCtx* c, int mode, double g, double c1, double c2, const dou
       }
     } else if (mode == 0) {
       launch_leapfrog<P, 0>(c->step_variant, c->n_poly, c->stream, c->K, c->md.row_ptr, c->md.col,
-                            c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn);
+                            c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn, keep);
     } else {
       launch_leapfrog<P, 1>(c->step_variant, c->n_poly, c->stream, c->K, c->md.row_ptr, c->md.col,
-                            c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn);
+                            c->RM, rs, rd, u, wa, out, g, c1, c2, gsel, gtab, c->order, dyn, keep);
     }
     return check_launch("k_leapfrog");
   });
@@ -937,7 +990,7 @@ int errors_dev(LymphCtx* c, const double* uh, const double* ue, double* l2sq, do
       k_sub<<<grid1(n, 256), 256, 0, c->stream>>>(uh, ue, c->stage[2], n);
       launch_leapfrog<P, 2>(0, c->n_poly, c->stream, c->A, c->md.row_ptr, c->md.col, nullptr,
                             nullptr, nullptr, c->stage[2], nullptr, c->part, 0.0, 0.0, 0.0,
-                            nullptr, nullptr, c->order, 0);
+                            nullptr, nullptr, c->order, 0, false);
       k_sum_terms<<<1, 1024, 0, c->stream>>>(c->part, c->n_poly, c->dsum + 1);
     }
     return check_launch("error kernels");

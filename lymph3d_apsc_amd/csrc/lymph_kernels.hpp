@@ -28,18 +28,22 @@ struct Dims {
   static constexpr size_t BS = (size_t)N3 * N3C;
 };
 
-// Operator blocks are read exactly once per step and never again before the
-// next step has streamed ~all of HBM past the caches: non-temporal loads keep
-// them from displacing the coefficient vectors (which neighbours re-read).
+// Operator blocks are read exactly once per step.  Where the operator does not
+// stay in the caches until the next step, non-temporal loads (NT) keep them
+// from displacing the coefficient vectors (which neighbours re-read).
 typedef double lymph_dv2 __attribute__((ext_vector_type(2)));
 typedef float lymph_fv4 __attribute__((ext_vector_type(4)));
 typedef float lymph_fv2 __attribute__((ext_vector_type(2)));
+template <bool NT = true>
 __device__ inline double2 load_stream(const double* p) {
-  const lymph_dv2 t = __builtin_nontemporal_load(reinterpret_cast<const lymph_dv2*>(p));
+  const auto* q = reinterpret_cast<const lymph_dv2*>(p);
+  const lymph_dv2 t = NT ? __builtin_nontemporal_load(q) : *q;
   return make_double2(t.x, t.y);
 }
+template <bool NT = true>
 __device__ inline float4 load_stream(const float* p) {
-  const lymph_fv4 t = __builtin_nontemporal_load(reinterpret_cast<const lymph_fv4*>(p));
+  const auto* q = reinterpret_cast<const lymph_fv4*>(p);
+  const lymph_fv4 t = NT ? __builtin_nontemporal_load(q) : *q;
   return make_float4(t.x, t.y, t.z, t.w);
 }
 // the tail columns of a 32-bit block row (N3 % 4 of them; 1 or 2 for p <= 4)
@@ -97,11 +101,15 @@ LYMPH_HD size_t kpos16(int N3, int r, int c) {
 // halves, non-temporal like the operator's own.
 typedef _Float16 lymph_hv4 __attribute__((ext_vector_type(4)));
 typedef _Float16 lymph_hv8 __attribute__((ext_vector_type(8)));
+template <bool NT = true>
 __device__ inline lymph_hv8 load_stream_h8(const _Float16* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const lymph_hv8*>(p));
+  const auto* q = reinterpret_cast<const lymph_hv8*>(p);
+  return NT ? __builtin_nontemporal_load(q) : *q;
 }
+template <bool NT = true>
 __device__ inline lymph_hv4 load_stream_h4(const _Float16* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const lymph_hv4*>(p));
+  const auto* q = reinterpret_cast<const lymph_hv4*>(p);
+  return NT ? __builtin_nontemporal_load(q) : *q;
 }
 LYMPH_HD size_t kpos32(int N3, int r, int c) {
   const int c0 = N3 / 4 * 4;
@@ -1189,7 +1197,7 @@ struct StepEnds {
 // 0 = wave-uniform scalar loads per pair, 1 = one coalesced vector load per
 // block (lane c holds x[c]) broadcast with v_readlane, so the inner loop waits
 // only on the block's own HBM loads.  Chosen per degree by lymph_autotune.
-template <int P, int MODE, int UNR, int XS, int WPP = 1>
+template <int P, int MODE, int UNR, int XS, int WPP, bool NT>
 __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict__ K,
                                                  const int* __restrict__ row_ptr,
                                                  const int* __restrict__ col,
@@ -1252,7 +1260,7 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
         for (int k = 0; k < RPL; ++k) {
           const int r = lane + 64 * k;
           if ((NPAIR % UNR == 0 || c2i < NPAIR) && r < N3)
-            kv[uu][k] = load_stream(Kb + ((size_t)c2i * N3 + r) * 2);
+            kv[uu][k] = load_stream<NT>(Kb + ((size_t)c2i * N3 + r) * 2);
         }
       }
 #pragma unroll
@@ -2030,7 +2038,7 @@ __device__ inline void lsync() {
 // operator in column pairs), 32 (mass-orthonormal FP32 operator in column
 // quads, no solves) or 48 (the FP32 operator plus its 16-bit corrections Kr,
 // with k_leapfrog48's arithmetic in its order: bit-identical to it).
-template <int P, int MODE, int TB, int WPW = 1>
+template <int P, int MODE, int TB, int WPW, bool NT>
 __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __restrict__ Kv,
                                                         const _Float16* __restrict__ Kr,
                                                         const int* __restrict__ row_ptr,
@@ -2086,20 +2094,20 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __rest
       if constexpr (TB == 64) {
         const double* Kb = static_cast<const double*>(Kv) + (size_t)b * D::BS;
 #pragma unroll
-        for (int c2i = 0; c2i < NPAIR; ++c2i) kd[c2i] = load_stream(Kb + ((size_t)c2i * N3 + r) * 2);
+        for (int c2i = 0; c2i < NPAIR; ++c2i) kd[c2i] = load_stream<NT>(Kb + ((size_t)c2i * N3 + r) * 2);
       } else {
         const float* Kb = static_cast<const float*>(Kv) + (size_t)b * Dims32<P>::BS;
 #pragma unroll
-        for (int q = 0; q < NQUAD; ++q) kf[q] = load_stream(Kb + ((size_t)q * N3 + r) * 4);
+        for (int q = 0; q < NQUAD; ++q) kf[q] = load_stream<NT>(Kb + ((size_t)q * N3 + r) * 4);
         if constexpr (TAIL > 0) load_tail<TAIL>(Kb + (size_t)4 * NQUAD * N3 + (size_t)r * TAIL, kt);
         if constexpr (TB == 48) {
           const _Float16* Rb = Kr + (size_t)b * Dims16<P>::BS;
 #pragma unroll
           for (int k = 0; k < (NQUAD + 1) / 2; ++k) {
             if (2 * k + 1 < NQUAD) {
-              kr[k] = load_stream_h8(Rb + ((size_t)k * N3 + r) * 8);
+              kr[k] = load_stream_h8<NT>(Rb + ((size_t)k * N3 + r) * 8);
             } else {  // the last quad of an odd count: 4 values per row
-              const lymph_hv4 h = load_stream_h4(Rb + Dims16<P>::HALF0 + (size_t)r * 4);
+              const lymph_hv4 h = load_stream_h4<NT>(Rb + Dims16<P>::HALF0 + (size_t)r * 4);
               kr[k] = lymph_hv8{h.x, h.y, h.z, h.w, 0, 0, 0, 0};
             }
           }
@@ -2210,7 +2218,7 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __rest
 // order, so results are bit-identical to k_leapfrog (TB = 48: to
 // k_leapfrog48, with Kr its 16-bit corrections).  Dynamic LDS: the products
 // of the wave's longest block range (G x longest row x 3Np doubles).
-template <int P, int MODE, int TB, int WPW = 1>
+template <int P, int MODE, int TB, int WPW, bool NT>
 __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restrict__ Kv,
                                                        const _Float16* __restrict__ Kr,
                                                        const int* __restrict__ row_ptr,
@@ -2266,20 +2274,20 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restr
       if constexpr (TB == 64) {
         const double* Kb = static_cast<const double*>(Kv) + (size_t)bj * D::BS;
 #pragma unroll
-        for (int c2i = 0; c2i < NPAIR; ++c2i) kd[c2i] = load_stream(Kb + ((size_t)c2i * N3 + r) * 2);
+        for (int c2i = 0; c2i < NPAIR; ++c2i) kd[c2i] = load_stream<NT>(Kb + ((size_t)c2i * N3 + r) * 2);
       } else {
         const float* Kb = static_cast<const float*>(Kv) + (size_t)bj * Dims32<P>::BS;
 #pragma unroll
-        for (int q = 0; q < NQUAD; ++q) kf[q] = load_stream(Kb + ((size_t)q * N3 + r) * 4);
+        for (int q = 0; q < NQUAD; ++q) kf[q] = load_stream<NT>(Kb + ((size_t)q * N3 + r) * 4);
         if constexpr (TAIL > 0) load_tail<TAIL>(Kb + (size_t)4 * NQUAD * N3 + (size_t)r * TAIL, kt);
         if constexpr (TB == 48) {
           const _Float16* Rb = Kr + (size_t)bj * Dims16<P>::BS;
 #pragma unroll
           for (int kk = 0; kk < (NQUAD + 1) / 2; ++kk) {
             if (2 * kk + 1 < NQUAD) {
-              kr[kk] = load_stream_h8(Rb + ((size_t)kk * N3 + r) * 8);
+              kr[kk] = load_stream_h8<NT>(Rb + ((size_t)kk * N3 + r) * 8);
             } else {  // the last quad of an odd count: 4 values per row
-              const lymph_hv4 h = load_stream_h4(Rb + Dims16<P>::HALF0 + (size_t)r * 4);
+              const lymph_hv4 h = load_stream_h4<NT>(Rb + Dims16<P>::HALF0 + (size_t)r * 4);
               kr[kk] = lymph_hv8{h.x, h.y, h.z, h.w, 0, 0, 0, 0};
             }
           }
@@ -2612,7 +2620,7 @@ __global__ __launch_bounds__(64) void k_tilde_back(const double* __restrict__ RM
   }
 }
 
-template <int P, int MODE, int UNR, int WPP = 1>
+template <int P, int MODE, int UNR, int WPP, bool NT>
 __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict__ K,
                                                    const int* __restrict__ row_ptr,
                                                    const int* __restrict__ col,
@@ -2663,7 +2671,7 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict
         for (int k = 0; k < RPL; ++k) {
           const int r = lane + 64 * k;
           if ((NQUAD % UNR == 0 || q < NQUAD) && r < N3)
-            kv[uu][k] = load_stream(Kb + ((size_t)q * N3 + r) * 4);
+            kv[uu][k] = load_stream<NT>(Kb + ((size_t)q * N3 + r) * 4);
         }
       }
 #pragma unroll
@@ -2762,7 +2770,7 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict
 // per operator entry; the state stays within about 1e-9 of the FP64 step's
 // over 1000 steps where the 32-bit apply drifts to 1e-5.
 
-template <int P, int MODE, int UNR, int WPP>
+template <int P, int MODE, int UNR, int WPP, bool NT>
 __global__ __launch_bounds__(64 * WPP) void k_leapfrog48(const float* __restrict__ K,
                                                    const _Float16* __restrict__ Kr,
                                                    const int* __restrict__ row_ptr,
@@ -2819,12 +2827,12 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog48(const float* __restrict
         for (int k = 0; k < RPL; ++k) {
           const int r = lane + 64 * k;
           if (q < NQUAD && r < N3) {
-            kv[uu][k] = load_stream(Kb + ((size_t)q * N3 + r) * 4);
+            kv[uu][k] = load_stream<NT>(Kb + ((size_t)q * N3 + r) * 4);
             if ((uu & 1) == 0) {
               if (q + 1 < NQUAD) {
-                tv[uu / 2][k] = load_stream_h8(Rb + ((size_t)(q >> 1) * N3 + r) * 8);
+                tv[uu / 2][k] = load_stream_h8<NT>(Rb + ((size_t)(q >> 1) * N3 + r) * 8);
               } else {  // the last quad of an odd count: 4 values per row
-                const lymph_hv4 h = load_stream_h4(Rb + Dims16<P>::HALF0 + (size_t)r * 4);
+                const lymph_hv4 h = load_stream_h4<NT>(Rb + Dims16<P>::HALF0 + (size_t)r * 4);
                 tv[uu / 2][k] = lymph_hv8{h.x, h.y, h.z, h.w, 0, 0, 0, 0};
               }
             }
