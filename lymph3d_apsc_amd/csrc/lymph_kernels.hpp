@@ -1002,9 +1002,35 @@ __device__ __forceinline__ void forward_rows(const double* __restrict__ R, doubl
   }
 }
 
-// M^-1 of three right-hand sides across one wave, lane i on row i of all three
-// (NP <= 64), the sweeps as in solve_group; d: the divisor R_ii of lane i.
+// R^-1 of three right-hand sides across one wave, lane i on row i of all three
+// (NP <= 64), the columns from the last; d: the divisor R_ii of lane i.
 // Broadcasts by v_readlane (24.2 us above with __shfl).
+template <int NP, bool PLAIN>
+__device__ __forceinline__ void back_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
+  double y[3] = {0.0, 0.0, 0.0};
+  const int ri = pk_off(NP, i < NP ? i : 0);
+#pragma unroll 5
+  for (int j = NP - 1; j >= 0; --j) {
+    const double r = R[ri + (i < NP && i < j ? j - i : 0)];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
+      if (i == j) y[c] = t;
+      x[c] = x[c] - r * lane_bcast(t, j);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) x[c] = y[c];
+}
+template <int NP>
+__device__ __forceinline__ void back_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
+  if (__all(i >= NP || d.plain()))
+    back_rows_as<NP, true>(R, d, x, i);
+  else
+    back_rows_as<NP, false>(R, d, x, i);
+}
+
+// M^-1: both sweeps
 template <int NP, bool PLAIN>
 __device__ __forceinline__ void solve_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
   double y[3] = {0.0, 0.0, 0.0};
@@ -1018,21 +1044,9 @@ __device__ __forceinline__ void solve_rows_as(const double* __restrict__ R, cons
       x[c] = x[c] - r * lane_bcast(t, j);
     }
   }
-  const int ri = pk_off(NP, i < NP ? i : 0);
 #pragma unroll
   for (int c = 0; c < 3; ++c) x[c] = y[c];
-#pragma unroll 5
-  for (int j = NP - 1; j >= 0; --j) {
-    const double r = R[ri + (i < NP && i < j ? j - i : 0)];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
-      if (i == j) y[c] = t;
-      x[c] = x[c] - r * lane_bcast(t, j);
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) x[c] = y[c];
+  back_rows_as<NP, PLAIN>(R, d, x, i);
 }
 template <int NP>
 __device__ __forceinline__ void solve_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
@@ -2573,11 +2587,9 @@ __global__ __launch_bounds__(64) void k_tilde(const double* __restrict__ RM,
   }
 }
 
-// u = R^-1 ~u (mode 1 of the transforms above) with one wave per polyhedron: lane i keeps
-// row i's partial sums of the three components, and the columns are swept
-// from the last: y_j = s_j / R_jj is broadcast from lane j, then every row
-// above subtracts R_ij y_j.  NP steps instead of NP(NP+1)/2 dependent ones
-// per thread; row i subtracts its terms in descending column order.
+// u = R^-1 ~u (mode 1 of the transforms above) with one wave per polyhedron:
+// back_rows, the factor staged in LDS in one trip (read from memory column by
+// column, with divisions on the chain, 64 polyhedra took 16 us at p = 4, now 8).
 template <int P>
 __global__ __launch_bounds__(64) void k_tilde_back(const double* __restrict__ RM,
                                                    const double* __restrict__ in,
@@ -2585,39 +2597,23 @@ __global__ __launch_bounds__(64) void k_tilde_back(const double* __restrict__ RM
                                                    const int* __restrict__ list, int n) {
   using D = Dims<P>;
   constexpr int NP = D::NP;
-  static_assert(NP <= 64, "one lane per row");
+  __shared__ double sR[D::NPK];
   const int w = blockIdx.x;
   if (w >= n) return;
   const int Pp = list ? list[w] : w;
   const int i = threadIdx.x;
   const bool row = i < NP;
   const double* R = RM + (size_t)Pp * D::NPK;
-  const double* x = in + (size_t)Pp * D::N3;
-  double* y = out + (size_t)Pp * D::N3;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  if (row) {
-    s0 = x[i];
-    s1 = x[NP + i];
-    s2 = x[2 * NP + i];
-  }
-  const int ri = row ? pk_off(NP, i) : 0;
+  const Divisor d(R[pk_off(NP, row ? i : 0)]);
+  for (int k = i; k < D::NPK; k += 64) sR[k] = R[k];
+  double x[3];
 #pragma unroll
-  for (int j = NP - 1; j >= 0; --j) {
-    const double rjj = R[pk_off(NP, j)];
-    const double y0 = __shfl(s0, j, 64) / rjj;
-    const double y1 = __shfl(s1, j, 64) / rjj;
-    const double y2 = __shfl(s2, j, 64) / rjj;
-    if (i == j) {
-      y[i] = y0;
-      y[NP + i] = y1;
-      y[2 * NP + i] = y2;
-    } else if (i < j) {
-      const double r = R[ri + (j - i)];
-      s0 = s0 - r * y0;
-      s1 = s1 - r * y1;
-      s2 = s2 - r * y2;
-    }
-  }
+  for (int c = 0; c < 3; ++c) x[c] = row ? in[(size_t)Pp * D::N3 + c * NP + i] : 0.0;
+  wave_lds_sync();
+  back_rows<NP>(sR, d, x, i);
+  if (row)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) out[(size_t)Pp * D::N3 + c * NP + i] = x[c];
 }
 
 template <int P, int MODE, int UNR, int WPP, bool NT>
@@ -3163,34 +3159,35 @@ __global__ void k_to_fortran(const double* __restrict__ p, double* __restrict__ 
 
 // Receivers: value of the modal field at a point, sum_i u_i Lx Ly Lz on the
 // polyhedron's bounding box, as EXPORT_SOLUTION evaluates it
-// (src/solution_processing.f90:150-170).  One thread per (receiver, comp);
-// out[r*3 + comp] of record row `row`.
+// (src/solution_processing.f90:150-170).  One wave per receiver, a basis
+// function per lane, the terms added in the functions' order: 64 receivers at
+// p = 4 took 21 us with a thread per component, now 5; out[r*3 + comp] of
+// record row `row`.
 template <int P>
-__global__ void k_sample(const double* __restrict__ u, const int* __restrict__ rpoly,
+__global__ __launch_bounds__(64) void k_sample(const double* __restrict__ u, const int* __restrict__ rpoly,
                          const double* __restrict__ rxyz, const double* __restrict__ bbox,
                          const int* __restrict__ blist, int n, double* __restrict__ out) {
   using D = Dims<P>;
   constexpr int NP = D::NP;
-  const int id = blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= 3 * n) return;
-  const int r = id / 3, comp = id % 3;
+  const int r = blockIdx.x, i = threadIdx.x;
+  if (r >= n) return;
   const int Pp = rpoly[r];
   const double* bb = bbox + (size_t)Pp * 6;
-  double xp[3], sq[3];
+  const int f = i < NP ? i : 0;
+  double v[3];
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
     const double hb = (bb[2 * d + 1] - bb[2 * d]) / 2.0, mb = (bb[2 * d + 1] + bb[2 * d]) / 2.0;
-    xp[d] = (rxyz[r * 3 + d] - mb) / hb;
-    sq[d] = sqrt(hb);
+    v[d] = leg(blist[f * 3 + d], (rxyz[r * 3 + d] - mb) / hb) / sqrt(hb);
   }
-  const double* uu = u + (size_t)Pp * D::N3 + comp * NP;
-  double s = 0.0;
-  for (int i = 0; i < NP; ++i) {
-    const double vx = leg(blist[i * 3 + 0], xp[0]) / sq[0];
-    const double vy = leg(blist[i * 3 + 1], xp[1]) / sq[1];
-    const double vz = leg(blist[i * 3 + 2], xp[2]) / sq[2];
-    s = s + uu[i] * vx * vy * vz;
-  }
-  out[id] = s;
+  double t[3], s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) t[c] = u[(size_t)Pp * D::N3 + c * NP + f] * v[0] * v[1] * v[2];
+#pragma unroll
+  for (int j = 0; j < NP; ++j)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) s[c] = s[c] + lane_bcast(t[c], j);
+  if (i < 3) out[r * 3 + i] = i == 0 ? s[0] : (i == 1 ? s[1] : s[2]);
 }
 
 // Point forces: rhs[P_k][i*Np+m] += f_k,i phi_m(x_k), sources applied in order
