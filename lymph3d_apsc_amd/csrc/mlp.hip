@@ -786,8 +786,8 @@ __global__ __launch_bounds__(256, 2) void k_wide(LayerArgs g) {
 // Its input gradient: a long contraction (N of the output layer) for few
 // tiles, so the contraction is split as in gemm() and the parts, stored as the
 // lanes hold them, are added in order by k_split_end.  An XCD takes every
-// eighth part, whose operands then fit its L2.  256 x 512 from 38,400: 28 us
-// (2 x 2 tiles a wave 39; more steps in flight change nothing) and 5 for the
+// eighth part, whose operands then fit its L2.  256 x 512 from 38,400: 28 us,
+// 19 where dZ and W are still in the Infinity Cache (2 x 2 tiles a wave 39; more steps in flight change nothing) and 5 for the
 // sums, where the GEMM and its sums took 47.
 template <int T>
 __global__ __launch_bounds__(256, 2) void k_split(LayerArgs g, int S, int chunk, f32x4* ws) {
@@ -993,14 +993,28 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
   }
 }
 
+// four floats, streaming (NT) or cached
+template <bool NT>
+__device__ __forceinline__ float4 load4(const float* p) {
+  const auto* q = reinterpret_cast<const f32x4*>(p);
+  const f32x4 t = NT ? __builtin_nontemporal_load(q) : *q;
+  return make_float4(t[0], t[1], t[2], t[3]);
+}
+template <bool NT>
+__device__ __forceinline__ void store4(float* p, float4 v) {
+  const f32x4 t = {v.x, v.y, v.z, v.w};
+  if (NT) __builtin_nontemporal_store(t, reinterpret_cast<f32x4*>(p));
+  else *reinterpret_cast<f32x4*>(p) = t;
+}
+
 // k_update of a wide output layer: 32 x 128 (n x k) of W per workgroup of 4
 // waves.  The products go to LDS, from where masters, moments and gradients
 // move as whole rows and both packed copies as whole fragments.  Bound by its
-// 28 bytes per weight: 38,400 x 512 in 117 us (4.9 TB/s; with 256 k 150, with
-// 64 183, as k_update's tiles 231), where the gradient product, the column sums
+// 28 bytes per weight: 38,400 x 512 in 110 us (5.2 TB/s; with 256 k 150, with
+// 64 183, as k_update's tiles 231; NT: see wide_nt), where the gradient product, the column sums
 // and the update took 130.
 constexpr int kUpN = 32, kUpK = 128, kUpT = kUpK / 64, kUpLd = kUpK + 4, kUpLb = kUpK + 8;
-template <bool ADAM>
+template <bool ADAM, bool NT>
 __global__ __launch_bounds__(256, 3) void k_update_wide(UpdateArgs u, int l) {
   __shared__ __attribute__((aligned(16))) float sG[kUpN * kUpLd];
   __shared__ __attribute__((aligned(16))) bf16_t sW[kUpN * kUpLb];
@@ -1076,9 +1090,9 @@ __global__ __launch_bounds__(256, 3) void k_update_wide(UpdateArgs u, int l) {
       const int e = tid + 256 * j, n = n0 + e / rowq;
       if (e < kUpN * rowq && n < y.N) {
         const size_t at = y.woff + (size_t)n * y.K + k0 + e % rowq * 4;
-        pw[j] = *reinterpret_cast<const float4*>(u.P + at);
-        pm[j] = *reinterpret_cast<const float4*>(u.M + at);
-        pv[j] = *reinterpret_cast<const float4*>(u.V + at);
+        pw[j] = load4<NT>(u.P + at);
+        pm[j] = load4<NT>(u.M + at);
+        pv[j] = load4<NT>(u.V + at);
       }
     }
   }
@@ -1127,9 +1141,9 @@ __global__ __launch_bounds__(256, 3) void k_update_wide(UpdateArgs u, int l) {
       const uint32_t h1 = f2bf(adam_one(w.y, m.y, v.y, g[1], u.a));
       const uint32_t h2 = f2bf(adam_one(w.z, m.z, v.z, g[2], u.a));
       const uint32_t h3 = f2bf(adam_one(w.w, m.w, v.w, g[3], u.a));
-      *reinterpret_cast<float4*>(u.P + at) = w;
-      *reinterpret_cast<float4*>(u.M + at) = m;
-      *reinterpret_cast<float4*>(u.V + at) = v;
+      store4<NT>(u.P + at, w);
+      store4<NT>(u.M + at, m);
+      store4<NT>(u.V + at, v);
       hw = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
     }
     if (ADAM) *reinterpret_cast<uint2*>(sW + r * kUpLb + k) = hw;
@@ -1347,7 +1361,7 @@ int grow(LymphMlp* m, LymphMlp::Buf& b, size_t n) {
 // Tiles of 16 per wave and direction of a wide layer's k_wide, 1: k_layer.
 // The larger a wave's block, the less of the rows' activations every group of
 // columns reads again (256 rows x 38,400: 47 us with 4 x 4 tiles, 57 with 2 x
-// 2, 70 with 4 x 1), as long as about two waves a SIMD are left: 1024 blocks
+// 2, 70 with 4 x 1; 40 since wide_nt), as long as about two waves a SIMD are left: 1024 blocks
 // of 4 x 4, 512 of 2 x 2.
 int wide_tile(int N, int B) {
   const size_t t = (size_t)tiles_of(N) * tiles_of(B);
@@ -1417,6 +1431,16 @@ int slab_forward(LymphMlp* m, int n, const float* X, float* Y) {
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("k_slab: ") + hipGetErrorString(e));
+}
+
+// Whether a wide layer's masters and moments are streamed past the caches: from
+// half of the Infinity Cache on they push out the packed weights, the gradients
+// and the targets that the step's other launches read.  us per step of an
+// 8-512x3-N network at batch 256, cached / streamed: 49 MB of them 80.9 / 84.8,
+// 98 MB 107 / 112, 123 MB 128 / 129, 147 MB 144 / 139, 184 MB 187 / 159, 236 MB
+// (N = 38,400) 235 / 198.
+bool wide_nt(const LymphMlp* m) {
+  return (size_t)m->w[m->L] * m->w[m->L - 1] * 12 > ((size_t)128 << 20);
 }
 
 // One step on rows idx of X, T: gradients into G (adam == null) or applied.
@@ -1498,8 +1522,9 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
   u.part_scale = 1.0f / (float)ny;
   u.loss = loss;
   if (apart >= 0) {
-    if (adam) k_update_wide<true><<<big, 256, 0, st>>>(u, apart);
-    else k_update_wide<false><<<big, 256, 0, st>>>(u, apart);
+    if (!adam) k_update_wide<false, false><<<big, 256, 0, st>>>(u, apart);
+    else if (wide_nt(m)) k_update_wide<true, true><<<big, 256, 0, st>>>(u, apart);
+    else k_update_wide<true, false><<<big, 256, 0, st>>>(u, apart);
   }
   if (adam) k_update<true><<<wgs + bias + 1, 128, 0, st>>>(u);
   else k_update<false><<<wgs + bias + 1, 128, 0, st>>>(u);

@@ -140,3 +140,9 @@ WIDE = [([8, 16, 520], 8), ([24, 72, 40, 1032], 24), ([8, 512, 8000], 72), ([16,
 def test_wide_outputs_at_tile_edges_match_oracle(widths, batch):
     """The checks above; 4200 rows of 16,408 outputs come in several chunks."""
     test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
+
+
+def test_wide_update_with_streamed_masters_matches_oracle():
+    """The checks above with masters and moments of the output layer above 128
+    MB (512 x 21,896: remainders in n), where the update streams them."""
+    test_narrow_networks_at_tile_edges_match_oracle([8, 512, 21896], 24)
