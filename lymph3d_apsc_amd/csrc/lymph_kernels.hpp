@@ -923,20 +923,29 @@ __device__ __forceinline__ double lane_bcast(double v, int l) {
 // the bits of the division in five dependent operations instead of a dozen
 // (Markstein, IBM J. Res. Dev. 34, 1990: the remainder a - b q is exact in one
 // fused multiply-add, the first correction makes q faithful, the second rounds
-// it correctly).  Quotients that are not finite come from the division's own
-// rule: q = a y is then the infinity or NaN it gives.
+// it correctly), for divisors that are plain() and numerators that are
+// quotable().  Quotients that are zero, infinite or NaN are q = a y, which has
+// the division's sign.
 struct Divisor {
   double b, y;
   __device__ __forceinline__ explicit Divisor(double v) : b(v), y(1.0 / v) {}
-  // within this range no quotient of a normal number leaves the exponents
-  // where the remainder is exact; outside it the solves divide
-  __device__ __forceinline__ bool plain() const { return fabs(b) > 0x1p-400 && fabs(b) < 0x1p400; }
+  __device__ __forceinline__ bool plain() const { return fabs(b) > 0x1p-100 && fabs(b) < 0x1p100; }
 };
 __device__ __forceinline__ double quot(double a, const Divisor& d) {
   const double q0 = a * d.y;
   const double q1 = fma(fma(-d.b, q0, a), d.y, q0);
   const double q2 = fma(fma(-d.b, q1, a), d.y, q1);
-  return fabs(q0) < __builtin_inf() ? q2 : q0;
+  constexpr int kNonzeroFinite = 0x008 | 0x010 | 0x080 | 0x100;  // -normal, -subnormal, +subnormal, +normal
+  return __builtin_amdgcn_class(q0, kNonzeroFinite) ? q2 : q0;
+}
+// Numerators whose quotients by a plain divisor are exact above: the quotient
+// stays within 2^-960 and 2^1000, the last bit of the remainder (2^-106 of the
+// numerator) above the smallest subnormal; zeros, infinities and NaN pass.  The
+// solves test the numerators that they used once at their end and divide if one
+// fails: in a wave front's first trace, or next to overflow.
+__device__ __forceinline__ bool quotable(double a) {
+  const double m = fabs(a);
+  return (m >= 0x1p-860 && m <= 0x1p900) || m == 0.0 || !(m < __builtin_inf());
 }
 
 // M^-1 w = R^-1 R^-T w (solve_LU with L = R^T, src/vet_mat_operations.f90:
@@ -952,12 +961,15 @@ __device__ __forceinline__ double quot(double a, const Divisor& d) {
 // a step at p = 2, 3, 4, now 5.2, 8.6 and 22.7.
 template <int NP, bool PLAIN>
 __device__ __forceinline__ double solve_group_as(const double* __restrict__ R, const Divisor& d, double w, int ii,
-                                                 int from) {
-  double y = 0.0;
+                                                 int from, bool& ok) {
+  double y = 0.0, af = 0.0, ab = 0.0;  // the lane's results and numerators
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const double t = PLAIN ? quot(w, d) : w / d.b;
-    if (ii == j) y = t;
+    if (ii == j) {
+      y = t;
+      af = w;
+    }
     w = w - R[pk_off(NP, j) + (ii > j ? ii - j : 0)] * __shfl(t, from + j, 64);
   }
   const int ri = pk_off(NP, ii);
@@ -965,17 +977,25 @@ __device__ __forceinline__ double solve_group_as(const double* __restrict__ R, c
 #pragma unroll
   for (int j = NP - 1; j >= 0; --j) {
     const double t = PLAIN ? quot(w, d) : w / d.b;
-    if (ii == j) y = t;
+    if (ii == j) {
+      y = t;
+      ab = w;
+    }
     w = w - R[ri + (ii < j ? j - ii : 0)] * __shfl(t, from + j, 64);
   }
+  ok = !PLAIN || (quotable(af) && quotable(ab));
   return y;
 }
 template <int NP>
 __device__ __forceinline__ double solve_group(const double* __restrict__ R, const Divisor& d, double w, int base,
                                               int r, bool on) {
   const int cc = on ? r / NP : 0, ii = on ? r % NP : 0, from = on ? base + cc * NP : 0;
-  return __all(!on || d.plain()) ? solve_group_as<NP, true>(R, d, w, ii, from)
-                                 : solve_group_as<NP, false>(R, d, w, ii, from);
+  bool ok;
+  if (__all(!on || d.plain())) {
+    const double y = solve_group_as<NP, true>(R, d, w, ii, from, ok);
+    if (__all(!on || ok)) return y;
+  }
+  return solve_group_as<NP, false>(R, d, w, ii, from, ok);
 }
 
 // R^-T of three right-hand sides across one wave, lane i on row i of all three
@@ -1006,8 +1026,8 @@ __device__ __forceinline__ void forward_rows(const double* __restrict__ R, doubl
 // (NP <= 64), the columns from the last; d: the divisor R_ii of lane i.
 // Broadcasts by v_readlane (24.2 us above with __shfl).
 template <int NP, bool PLAIN>
-__device__ __forceinline__ void back_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
-  double y[3] = {0.0, 0.0, 0.0};
+__device__ __forceinline__ bool back_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
+  double y[3] = {0.0, 0.0, 0.0}, a[3] = {0.0, 0.0, 0.0};  // the lane's results and numerators
   const int ri = pk_off(NP, i < NP ? i : 0);
 #pragma unroll 5
   for (int j = NP - 1; j >= 0; --j) {
@@ -1015,45 +1035,65 @@ __device__ __forceinline__ void back_rows_as(const double* __restrict__ R, const
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
-      if (i == j) y[c] = t;
+      if (i == j) {
+        y[c] = t;
+        a[c] = x[c];
+      }
       x[c] = x[c] - r * lane_bcast(t, j);
     }
   }
 #pragma unroll
   for (int c = 0; c < 3; ++c) x[c] = y[c];
+  return !PLAIN || (quotable(a[0]) && quotable(a[1]) && quotable(a[2]));
 }
 template <int NP>
 __device__ __forceinline__ void back_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
-  if (__all(i >= NP || d.plain()))
-    back_rows_as<NP, true>(R, d, x, i);
-  else
-    back_rows_as<NP, false>(R, d, x, i);
+  if (__all(i >= NP || d.plain())) {
+    double y[3] = {x[0], x[1], x[2]};
+    const bool ok = back_rows_as<NP, true>(R, d, y, i);
+    if (__all(ok)) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) x[c] = y[c];
+      return;
+    }
+  }
+  back_rows_as<NP, false>(R, d, x, i);
 }
 
 // M^-1: both sweeps
 template <int NP, bool PLAIN>
-__device__ __forceinline__ void solve_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
-  double y[3] = {0.0, 0.0, 0.0};
+__device__ __forceinline__ bool solve_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
+  double y[3] = {0.0, 0.0, 0.0}, a[3] = {0.0, 0.0, 0.0};
 #pragma unroll 5
   for (int j = 0; j < NP; ++j) {
     const double r = R[pk_off(NP, j) + (i < NP && i > j ? i - j : 0)];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
-      if (i == j) y[c] = t;
+      if (i == j) {
+        y[c] = t;
+        a[c] = x[c];
+      }
       x[c] = x[c] - r * lane_bcast(t, j);
     }
   }
 #pragma unroll
   for (int c = 0; c < 3; ++c) x[c] = y[c];
-  back_rows_as<NP, PLAIN>(R, d, x, i);
+  const bool ok = back_rows_as<NP, PLAIN>(R, d, x, i);
+  return ok && (!PLAIN || (quotable(a[0]) && quotable(a[1]) && quotable(a[2])));
 }
 template <int NP>
 __device__ __forceinline__ void solve_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
-  if (__all(i >= NP || d.plain()))
-    solve_rows_as<NP, true>(R, d, x, i);
-  else
-    solve_rows_as<NP, false>(R, d, x, i);
+  if (__all(i >= NP || d.plain())) {
+    double y[3] = {x[0], x[1], x[2]};
+    const bool ok = solve_rows_as<NP, true>(R, d, y, i);
+    if (__all(ok)) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) x[c] = y[c];
+      return;
+    }
+  }
+  solve_rows_as<NP, false>(R, d, x, i);
 }
 
 // R^-1 y in place on one lane, every row's terms in ascending columns as the

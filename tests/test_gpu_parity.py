@@ -930,3 +930,72 @@ def test_mass_solves_by_reciprocals_give_the_divisions_bits(p):
     for a, b in zip(*out):
         assert np.array_equal(a, out[0][0], equal_nan=True)
         assert np.array_equal(a, b, equal_nan=True)
+
+
+def mass_factor(M):
+    """R of M = R^T R for every block (n, Np, Np), as k_cholesky orders its sums."""
+    R = np.zeros_like(M)
+    for j in range(M.shape[1]):
+        s = M[:, j, j].copy()
+        for k in range(j):
+            s = s - R[:, k, j] * R[:, k, j]
+        R[:, j, j] = np.sqrt(s)
+        for i in range(j + 1, M.shape[1]):
+            t = M[:, j, i].copy()
+            for k in range(j):
+                t = t - R[:, k, j] * R[:, k, i]
+            R[:, j, i] = t / R[:, j, j]
+    return R
+
+
+def mass_solve(R, x):
+    """R^-1 R^-T x by divisions, x (n, 3, Np): both sweeps column by column, as
+    the step kernels run them."""
+    x = x.copy()
+    n = R.shape[1]
+    for sweep in (range(n), range(n - 1, -1, -1)):
+        forward = sweep.step > 0
+        for j in sweep:
+            x[:, :, j] = x[:, :, j] / R[:, None, j, j]
+            for i in range(j + 1, n) if forward else range(j):
+                x[:, :, i] = x[:, :, i] - (R[:, None, j, i] if forward else R[:, None, i, j]) * x[:, :, j]
+    return x
+
+
+@pytest.mark.parametrize("p", [1, 2, 3, 4])
+def test_mass_solves_of_tiny_and_signed_zero_loads_give_the_divisions_bits(p):
+    """Loads whose quotients by the mass factor end near or below the smallest
+    normal number, load entries next to the largest one, and negative zeros: a
+    step from (signed) zero displacement gives the bits of a solve by divisions,
+    for every variant, and the 32-bit apply's back transform too."""
+    say(f"[mass solve, tiny loads] p={p}")
+    m = M.cube_mesh(4, agglomerate=True)
+    rng = np.random.default_rng(p)
+    with L.Context(m, p) as ctx:
+        ctx.make_matrices_free()
+        R = mass_factor(ctx.export_operator()[2])
+        f = rng.standard_normal((m.n_poly, 3, ctx.Np))
+        for k in range(1, m.n_poly):
+            f[k] *= 2.0 ** rng.integers(-60, 60)
+        f[1:40] *= 2.0 ** rng.integers(-1060, -960, (39, 1, 1))  # whole polyhedra
+        f[40:44] *= 2.0 ** rng.integers(-1000, 0, (4, 3, ctx.Np))  # neighbouring entries far apart
+        f[44] = -0.0
+        f[45, 0] = -0.0
+        f[46, :, 0] = 1.7e308
+        f[47] = 1e-310
+        zero = np.zeros(f.size)
+        ctx.set_slot(_lib.SLOT_RHS_STAT, -zero)
+        ctx.set_slot(_lib.SLOT_RHS_DYN, f.ravel())
+        with np.errstate(all="ignore"):
+            ref = mass_solve(R, f).ravel()
+        assert (np.abs(ref[(ref != 0) & np.isfinite(ref)]) < 2.0 ** -1022).any() and (np.signbit(ref) & (ref == 0)).any()
+        finite = np.isfinite(ref)
+        for v in range(ctx.n_step_variants()):
+            ctx.set_step_variant(v)
+            # c1 w + 2 u - a: -0 only where w is
+            got = ctx.time_step_matrix_free(1.0, 1.0, zero, -zero)
+            assert np.array_equal(np.isfinite(got), finite), v
+            assert np.array_equal(got[finite].view(np.int64), ref[finite].view(np.int64)), v
+        ctx.set_apply_precision(32)
+        got = ctx.time_step_matrix_free(1.0, 1.0, zero, zero)
+        assert np.array_equal(got[finite], ref[finite])
