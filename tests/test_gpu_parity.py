@@ -988,7 +988,9 @@ def test_mass_solves_of_tiny_and_signed_zero_loads_give_the_divisions_bits(p):
         ctx.set_slot(_lib.SLOT_RHS_DYN, f.ravel())
         with np.errstate(all="ignore"):
             ref = mass_solve(R, f).ravel()
-        assert (np.abs(ref[(ref != 0) & np.isfinite(ref)]) < 2.0 ** -1022).any() and (np.signbit(ref) & (ref == 0)).any()
+        assert (np.abs(ref[(ref != 0) & np.isfinite(ref)]) < 2.0 ** -1022).any()
+        # (beyond p = 1 the sweeps' differences turn every negative zero positive)
+        assert p > 1 or (np.signbit(ref) & (ref == 0)).any()
         finite = np.isfinite(ref)
         for v in range(ctx.n_step_variants()):
             ctx.set_step_variant(v)
