@@ -224,6 +224,10 @@ int lymph_autotune(LymphCtx* ctx, int reps, int* n_variants, int* unr, int* xmod
  * current apply precision) without timing; *n_variants (may be NULL) = count.
  * No reference counterpart. */
 int lymph_set_step_variant(LymphCtx* ctx, int index, int* n_variants);
+/* The step-kernel variant in use (chosen by mesh, degree and apply until one
+ * is selected or autotuned) and the count for the current apply precision;
+ * either may be NULL.  No reference counterpart. */
+int lymph_get_step_variant(const LymphCtx* ctx, int* index, int* n_variants);
 
 /* Operator precision of the step's block apply: 64 (default), 32 or 48.
  * With 32 the steps run in the mass-orthonormal basis u~ = R u (M = R^T R per

@@ -1850,6 +1850,15 @@ int lymph_set_step_variant(LymphCtx* c, int index, int* n_variants) {
   });
 }
 
+int lymph_get_step_variant(const LymphCtx* c, int* index, int* n_variants) {
+  if (int rc = need_ctx(c)) return rc;
+  if (index) *index = c->step_variant;
+  return dispatch_p(c->p, [&](auto pc) -> int {
+    if (n_variants) *n_variants = n_var_of<decltype(pc)::value>(c->apply_bits);
+    return 0;
+  });
+}
+
 int lymph_set_apply_precision(LymphCtx* c, int bits) {
   if (int rc = need_built(c)) return rc;
   if (bits != 32 && bits != 48 && bits != 64)

@@ -216,6 +216,12 @@ module lymph_gpu
       integer(c_int), intent(out) :: n_variants
       integer(c_int) :: rc
     end function
+    function lymph_get_step_variant(ctx, idx, n_variants) bind(C, name='lymph_get_step_variant') result(rc)
+      import :: c_int, c_ptr
+      type(c_ptr), value :: ctx
+      integer(c_int), intent(out) :: idx, n_variants
+      integer(c_int) :: rc
+    end function
     function lymph_set_apply_precision(ctx, bits) bind(C, name='lymph_set_apply_precision') result(rc)
       import :: c_int, c_ptr
       type(c_ptr), value :: ctx

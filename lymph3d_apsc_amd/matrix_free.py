@@ -214,9 +214,15 @@ class Context:
         check(lib().lymph_set_step_variant(self.h, int(index), C.byref(nv)), "lymph_set_step_variant")
         return nv.value
 
+    def step_variant(self):
+        """Index of the step-kernel variant in use."""
+        v = C.c_int()
+        check(lib().lymph_get_step_variant(self.h, C.byref(v), None), "lymph_get_step_variant")
+        return v.value
+
     def n_step_variants(self):
         nv = C.c_int()
-        check(lib().lymph_set_step_variant(self.h, 0, C.byref(nv)), "lymph_set_step_variant")
+        check(lib().lymph_get_step_variant(self.h, None, C.byref(nv)), "lymph_get_step_variant")
         return nv.value
 
     def set_apply_precision(self, bits):

@@ -1001,3 +1001,21 @@ def test_mass_solves_of_tiny_and_signed_zero_loads_give_the_divisions_bits(p):
         ctx.set_apply_precision(32)
         got = ctx.time_step_matrix_free(1.0, 1.0, zero, zero)
         assert np.array_equal(got[finite], ref[finite])
+
+
+def test_asking_for_the_variants_keeps_the_one_in_use():
+    """n_step_variants() neither selects a variant nor changes a step: a context
+    keeps the variant chosen for its mesh (not number 0 here), one that was
+    selected, and one that autotune kept."""
+    say("[variant count]")
+    m = M.cube_mesh(5, agglomerate=True)
+    with L.Context(m, 3) as ctx:
+        ctx.make_matrices_free()
+        for bits in (64, 32, 48):
+            ctx.set_apply_precision(bits)
+            v, n = ctx.step_variant(), ctx.n_step_variants()
+            assert 0 < v < n and ctx.step_variant() == v
+            assert ctx.set_step_variant(2) == n == ctx.n_step_variants()
+            assert ctx.step_variant() == 2
+            ctx.autotune(reps=2)
+            assert ctx.n_step_variants() == n and ctx.step_variant() == ctx.chosen_variant
