@@ -47,15 +47,16 @@ __device__ inline float4 load_stream(const float* p) {
   return make_float4(t.x, t.y, t.z, t.w);
 }
 // the tail columns of a 32-bit block row (N3 % 4 of them; 1 or 2 for p <= 4)
-template <int T>
+template <bool NT, int T>
 __device__ inline void load_tail(const float* p, float (&v)[T]) {
   static_assert(T == 1 || T == 2, "tail of 1 or 2 columns");
   if constexpr (T == 2) {
-    const lymph_fv2 t = __builtin_nontemporal_load(reinterpret_cast<const lymph_fv2*>(p));
+    const auto* q = reinterpret_cast<const lymph_fv2*>(p);
+    const lymph_fv2 t = NT ? __builtin_nontemporal_load(q) : *q;
     v[0] = t.x;
     v[1] = t.y;
   } else {
-    v[0] = __builtin_nontemporal_load(p);
+    v[0] = NT ? __builtin_nontemporal_load(p) : *p;
   }
 }
 
@@ -2153,7 +2154,7 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __rest
         const float* Kb = static_cast<const float*>(Kv) + (size_t)b * Dims32<P>::BS;
 #pragma unroll
         for (int q = 0; q < NQUAD; ++q) kf[q] = load_stream<NT>(Kb + ((size_t)q * N3 + r) * 4);
-        if constexpr (TAIL > 0) load_tail<TAIL>(Kb + (size_t)4 * NQUAD * N3 + (size_t)r * TAIL, kt);
+        if constexpr (TAIL > 0) load_tail<NT>(Kb + (size_t)4 * NQUAD * N3 + (size_t)r * TAIL, kt);
         if constexpr (TB == 48) {
           const _Float16* Rb = Kr + (size_t)b * Dims16<P>::BS;
 #pragma unroll
@@ -2333,7 +2334,7 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restr
         const float* Kb = static_cast<const float*>(Kv) + (size_t)bj * Dims32<P>::BS;
 #pragma unroll
         for (int q = 0; q < NQUAD; ++q) kf[q] = load_stream<NT>(Kb + ((size_t)q * N3 + r) * 4);
-        if constexpr (TAIL > 0) load_tail<TAIL>(Kb + (size_t)4 * NQUAD * N3 + (size_t)r * TAIL, kt);
+        if constexpr (TAIL > 0) load_tail<NT>(Kb + (size_t)4 * NQUAD * N3 + (size_t)r * TAIL, kt);
         if constexpr (TB == 48) {
           const _Float16* Rb = Kr + (size_t)bj * Dims16<P>::BS;
 #pragma unroll
@@ -2749,7 +2750,7 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog32(const float* __restrict
         const int r = lane + 64 * k;
         if (r < N3) {
           float kt[TAIL];
-          load_tail<TAIL>(Kb + (size_t)C0 * N3 + (size_t)r * TAIL, kt);
+          load_tail<NT>(Kb + (size_t)C0 * N3 + (size_t)r * TAIL, kt);
 #pragma unroll
           for (int j = 0; j < TAIL; ++j) s[k] = s[k] + kt[j] * xt[j];
         }
