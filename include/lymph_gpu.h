@@ -229,6 +229,14 @@ int lymph_set_step_variant(LymphCtx* ctx, int index, int* n_variants);
  * either may be NULL.  No reference counterpart. */
 int lymph_get_step_variant(const LymphCtx* ctx, int* index, int* n_variants);
 
+/* For contexts that step at the same time (captured solves replayed on several
+ * streams): `others` = bytes of their operators kept in the caches between
+ * steps (0 by default, negative: leave as it is), so that this context streams
+ * its own where both do not fit; *own (may be NULL) = the bytes this context
+ * keeps under the current apply, 0 if it streams.  Holds for launches and
+ * captures from here on; no result depends on it.  No reference counterpart. */
+int lymph_ctx_share_cache(LymphCtx* ctx, int64_t others, int64_t* own);
+
 /* Operator precision of the step's block apply: 64 (default), 32 or 48.
  * With 32 the steps run in the mass-orthonormal basis u~ = R u (M = R^T R per
  * polyhedron): the blocks R_P^-T K_PQ R_Q^-1 are formed in FP64 and rounded

@@ -39,7 +39,7 @@ EXPORTS = [
     "lymph_error_l2", "lymph_error_dg", "lymph_error_slots", "lymph_run", "lymph_check_finite",
     "lymph_build_rhs_fn", "lymph_project_fn",
     "lymph_time_function", "lymph_autotune", "lymph_set_step_variant",
-    "lymph_get_step_variant", "lymph_set_receivers",
+    "lymph_get_step_variant", "lymph_ctx_share_cache", "lymph_set_receivers",
     "lymph_sample_receivers", "lymph_step_n_record", "lymph_get_traces",
     "lymph_set_apply_precision", "lymph_set_source_groups", "lymph_ctx_set_keep_adg", "lymph_ctx_set_build", "lymph_release_fp64_operator", "lymph_set_symmetric_storage",
     "lymph_add_point_sources", "lymph_add_point_sources_noalloc", "lymph_add_double_couples", "lymph_set_ricker", "lymph_ricker",
@@ -112,6 +112,7 @@ def lib():
         "lymph_autotune": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
         "lymph_set_step_variant": (_i, [_vp, _i, _vp]),
         "lymph_get_step_variant": (_i, [_vp, _vp, _vp]),
+        "lymph_ctx_share_cache": (_i, [_vp, C.c_int64, _vp]),
         "lymph_set_receivers": (_i, [_vp, _i, _vp, _vp, _i]),
         "lymph_sample_receivers": (_i, [_vp, _i, _vp]),
         "lymph_step_n_record": (_i, [_vp, _i, _i, _d, _d, _i, _vp]),

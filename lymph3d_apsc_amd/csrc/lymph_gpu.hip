@@ -106,6 +106,7 @@ struct LymphCtx {
   int n_tet = 0, n_poly = 0, n_blk = 0;
   int layout = LYMPH_LAYOUT_POLY;
   int step_variant = 0;
+  size_t held_beside = 0;  // bytes that contexts stepping at the same time keep in the caches
   int apply_bits = 64;
   bool keep_adg = true;
   int build_mode = LYMPH_BUILD_REFERENCE;
@@ -534,9 +535,17 @@ int d2h_vec(LymphCtx* c, const double* d, double* h) {
 // between (46 MB 9.6 / 9.7, 92 MB 18.2 / 19.3), then 184 MB 34.4 / 31.8, 207 MB
 // 33.6 / 32.6.  Past the Infinity Cache streaming wins everywhere: 320 MB 60.6 /
 // 68.8, 354 MB 66 / 76.
+//
+// Solves of two contexts on two streams share the Infinity Cache: one that
+// would come to more than 288 MB with what the others keep there streams.  us
+// per step of both together, 32-bit, p = 2 and 3, both streamed / both cached:
+// 140 + 162 MB 49.7 / 47.6, 193 + 193 67.2 / 69.3 (one cached, one streamed
+// 58.1), 193 + 260 75.8 / 81.7 (70.2).
+size_t operator_bytes(const LymphCtx* c) { return (size_t)c->n_blk * c->n3 * c->n3 * c->apply_bits / 8; }
 bool keep_operator(const LymphCtx* c) {
-  const size_t bytes = (size_t)c->n_blk * c->n3 * c->n3 * c->apply_bits / 8;
-  constexpr size_t kL2 = (size_t)32 << 20, kMall = (size_t)208 << 20;
+  const size_t bytes = operator_bytes(c);
+  constexpr size_t kL2 = (size_t)32 << 20, kMall = (size_t)208 << 20, kShared = (size_t)288 << 20;
+  if (c->held_beside && bytes + c->held_beside > kShared) return false;
   return bytes <= kL2 || (bytes <= kMall && (c->p <= 2 || bytes >= 4 * kL2));
 }
 
@@ -1848,6 +1857,13 @@ int lymph_set_step_variant(LymphCtx* c, int index, int* n_variants) {
     c->step_variant = index;
     return 0;
   });
+}
+
+int lymph_ctx_share_cache(LymphCtx* c, int64_t others, int64_t* own) {
+  if (int rc = need_ctx(c)) return rc;
+  if (others >= 0) c->held_beside = (size_t)others;
+  if (own) *own = keep_operator(c) ? (int64_t)operator_bytes(c) : 0;
+  return 0;
 }
 
 int lymph_get_step_variant(const LymphCtx* c, int* index, int* n_variants) {

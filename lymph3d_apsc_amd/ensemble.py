@@ -133,6 +133,7 @@ class Ensemble:
         self.instances = list(instances)
         self.dt, self.nsteps, self.every, self.f0 = dt, nsteps, every, f0
         self.groups = []
+        held = 0  # operator bytes that the groups so far keep in the caches: all groups step at once
         # seconds per set-up phase, summed over the groups (device work is
         # synchronised at each phase's end)
         self.setup_seconds = dict(union=0.0, context=0.0, operator=0.0, precision=0.0,
@@ -160,6 +161,7 @@ class Ensemble:
             if apply_bits != 64:  # 32- or 48-bit apply: the FP64 blocks are not needed after it
                 ctx.set_apply_precision(apply_bits)
                 ctx.release_fp64_operator()
+            held += ctx.share_cache(held)
             lap("precision", ctx)
             # sources and receivers located in each instance, ids offset into the union
             tet_off = np.cumsum([0] + [m.n_tet for m in meshes])

@@ -222,6 +222,13 @@ module lymph_gpu
       integer(c_int), intent(out) :: idx, n_variants
       integer(c_int) :: rc
     end function
+    function lymph_ctx_share_cache(ctx, others, own) bind(C, name='lymph_ctx_share_cache') result(rc)
+      import :: c_int, c_int64_t, c_ptr
+      type(c_ptr), value :: ctx
+      integer(c_int64_t), value :: others
+      integer(c_int64_t), intent(out) :: own
+      integer(c_int) :: rc
+    end function
     function lymph_set_apply_precision(ctx, bits) bind(C, name='lymph_set_apply_precision') result(rc)
       import :: c_int, c_ptr
       type(c_ptr), value :: ctx

@@ -225,6 +225,15 @@ class Context:
         check(lib().lymph_get_step_variant(self.h, None, C.byref(nv)), "lymph_get_step_variant")
         return nv.value
 
+    def share_cache(self, others=None):
+        """Bytes of this context's operator that its steps keep in the caches (0:
+        streamed); `others` = what contexts stepping at the same time keep there,
+        which decides from here on whether this one's fits beside it."""
+        own = C.c_int64()
+        check(lib().lymph_ctx_share_cache(self.h, -1 if others is None else int(others), C.byref(own)),
+              "lymph_ctx_share_cache")
+        return own.value
+
     def set_apply_precision(self, bits):
         """Precision of the step's operator apply: 64 (default), 32 (FP32
         blocks in the mass-orthonormal basis, FP32 sums) or 48 (those FP32

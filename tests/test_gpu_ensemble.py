@@ -130,3 +130,29 @@ def test_48bit_ensemble_matches_fp64_ensemble():
         say(f"  instance {k}: 48-bit {e48:.2e}, 32-bit {e32:.2e}")
         assert e48 < 1e-7, (k, e48)
         assert e48 < 1e-2 * e32, (k, e48, e32)
+
+
+def test_groups_that_do_not_fit_the_caches_together_are_not_both_kept_there():
+    """A p = 2 group of 193 MB and a p = 3 group of 162 MB (32-bit): each alone
+    is kept in the caches between steps, in one ensemble, whose groups step on
+    two streams at once, only the first; two that fit together both are.  The
+    traces are the same bits either way."""
+    say("[ensemble cache share]")
+    big = E.make_instance(1, (20, 20), (2,)), E.make_instance(2, (12, 12), (3,))
+    small = E.make_instance(1, (10, 10), (2,)), E.make_instance(2, (7, 7), (3,))
+    dt, steps = 1e-4, 20
+
+    def solve(instances):
+        e = E.Ensemble(instances, dt, steps, every=5, autotune=False)
+        out = [g["ctx"].share_cache() for g in e.groups], e.run()
+        e.close()
+        return out
+
+    (a,), ta = solve(big[:1])
+    (b,), tb = solve(big[1:])
+    assert 150e6 < a <= 208 * 2 ** 20 and 150e6 < b <= 208 * 2 ** 20, (a, b)
+    held, t = solve(big)
+    assert held == [a, 0]
+    assert np.array_equal(t[0], ta[0]) and np.array_equal(t[1], tb[0])
+    held, _ = solve(small)
+    assert all(held) and sum(held) <= 288 * 2 ** 20
