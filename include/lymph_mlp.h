@@ -64,7 +64,9 @@ int lymph_mlp_train(LymphMlp* net, int n_steps, int batch, const int32_t* order,
  * parameter gradients in the parameter layout. */
 int lymph_mlp_gradients(LymphMlp* net, int batch, const float* x, const float* y, float* grads,
                         float* loss);
-/* Forward pass of n inputs (any n). */
+/* Forward pass of n inputs (any n).  Inputs and outputs pass through device
+ * buffers of the network of up to 64 MB each (more only for max_batch rows),
+ * which stay with it. */
 int lymph_mlp_predict(LymphMlp* net, int n, const float* x, float* y);
 /* Device time of forward passes over the first n samples of the training
  * set (device-resident inputs), mean over reps, in ms. */

@@ -1223,7 +1223,7 @@ struct LymphMlp {
   std::vector<bf16_t*> Wf, Wd, HT, DT, HP, DP;
   std::vector<f32x4*> dg;
   // inputs and outputs of host-side calls: one batch with the network, grown
-  // (own) to the largest call
+  // (own) up to upload_rows() and chunk_rows()
   struct Buf {
     float* p = nullptr;
     size_t cap = 0;
@@ -1383,9 +1383,16 @@ int launch_wide(LymphMlp* m, LayerArgs& a) {
   return (int)wgs * 4;
 }
 
-// Rows of a forward pass at a time: at most 64 MB of outputs, a batch at least
+// Rows of a forward pass at a time: at most 64 MB of inputs or outputs, a batch
+// at least
 int chunk_rows(const LymphMlp* m) {
-  return std::max(m->max_batch, (int)((16u << 20) / (unsigned)m->w[m->L]) / 32 * 32);
+  return std::max(m->max_batch, (int)((16u << 20) / (unsigned)std::max(m->w[0], m->w[m->L])) / 32 * 32);
+}
+// Rows of host inputs at a time, whole passes of `pass` rows: at most 64 MB, a
+// pass at least.  The buffer stays with the network, so it does not grow with
+// the rows of a call.
+int upload_rows(const LymphMlp* m, int pass) {
+  return std::max(pass, (int)((16u << 20) / (unsigned)m->w[0]) / pass * pass);
 }
 
 // Outputs of n <= chunk_rows() rows (device).  16 rows a slab until every CU
@@ -1804,36 +1811,33 @@ int lymph_mlp_predict(LymphMlp* m, int n, const float* x, float* y) {
   if (int rc = need(m)) return rc;
   if (n < 0 || (n > 0 && (!x || !y))) return fail(LYMPH_MLP_ERR_ARG, "bad inputs");
   const int w0 = m->w[0], NL = m->w[m->L];
-  if (int rc = grow(m, m->in, (size_t)std::max(1, n) * w0)) return rc;
-  float* dx = m->in.p;
+  const int pass = m->slab ? chunk_rows(m) : m->max_batch, up = upload_rows(m, pass);
+  if (int rc = grow(m, m->in, (size_t)std::min(n, up) * w0)) return rc;
+  if (m->slab)
+    if (int rc = grow(m, m->out, (size_t)std::min(n, pass) * NL)) return rc;
+  const float* dx = m->in.p;
   int rc = 0;
-  if (n > 0 &&
-      hipMemcpyAsync(dx, x, (size_t)n * w0 * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
+  std::vector<int> id(m->slab ? 0 : m->max_batch);
+  for (int i = 0; i < (int)id.size(); ++i) id[i] = i;
+  if (!m->slab &&
+      hipMemcpyAsync(m->idx, id.data(), 4 * id.size(), hipMemcpyHostToDevice, m->stream) != hipSuccess)
     rc = fail(LYMPH_MLP_ERR_HIP, "upload failed");
-  if (m->slab) {
-    const int chunk = chunk_rows(m);
-    if (!rc) rc = grow(m, m->out, (size_t)std::max(1, std::min(n, chunk)) * NL);
-    for (int b0 = 0; b0 < n && !rc; b0 += chunk) {
-      const int B = std::min(chunk, n - b0);
-      rc = slab_forward(m, B, dx + (size_t)b0 * w0, m->out.p);
-      if (!rc && hipMemcpyAsync(y + (size_t)b0 * NL, m->out.p, (size_t)B * NL * 4, hipMemcpyDeviceToHost,
-                                m->stream) != hipSuccess)
-        rc = fail(LYMPH_MLP_ERR_HIP, "download failed");
+  for (int b0 = 0; b0 < n && !rc; b0 += pass) {
+    const int B = std::min(pass, n - b0), at = b0 % up;  // up is a multiple of pass
+    if (at == 0 && hipMemcpyAsync(m->in.p, x + (size_t)b0 * w0, (size_t)std::min(up, n - b0) * w0 * 4,
+                                  hipMemcpyHostToDevice, m->stream) != hipSuccess) {
+      rc = fail(LYMPH_MLP_ERR_HIP, "upload failed");
+      break;
     }
-    if (hipStreamSynchronize(m->stream) != hipSuccess && !rc) rc = fail(LYMPH_MLP_ERR_HIP, "prediction failed");
-    return rc;
-  }
-  std::vector<int> id(m->max_batch);
-  for (int i = 0; i < m->max_batch; ++i) id[i] = i;
-  if (!rc &&
-      hipMemcpyAsync(m->idx, id.data(), 4 * m->max_batch, hipMemcpyHostToDevice, m->stream) != hipSuccess)
-    rc = fail(LYMPH_MLP_ERR_HIP, "upload failed");
-  for (int b0 = 0; b0 < n && !rc; b0 += m->max_batch) {
-    const int B = std::min(m->max_batch, n - b0);
-    k_gather<<<blocks((size_t)B * w0, 256), 256, 0, m->stream>>>(dx + (size_t)b0 * w0, w0, m->idx, B, m->H[0]);
-    rc = forward(m, B);
-    if (!rc && hipMemcpyAsync(y + (size_t)b0 * NL, m->Y, (size_t)B * NL * 4, hipMemcpyDeviceToHost,
-                              m->stream) != hipSuccess)
+    const float* xb = dx + (size_t)at * w0;
+    if (m->slab) {
+      rc = slab_forward(m, B, xb, m->out.p);
+    } else {
+      k_gather<<<blocks((size_t)B * w0, 256), 256, 0, m->stream>>>(xb, w0, m->idx, B, m->H[0]);
+      rc = forward(m, B);
+    }
+    if (!rc && hipMemcpyAsync(y + (size_t)b0 * NL, m->slab ? m->out.p : m->Y, (size_t)B * NL * 4,
+                              hipMemcpyDeviceToHost, m->stream) != hipSuccess)
       rc = fail(LYMPH_MLP_ERR_HIP, "download failed");
   }
   if (hipStreamSynchronize(m->stream) != hipSuccess && !rc) rc = fail(LYMPH_MLP_ERR_HIP, "prediction failed");

@@ -146,3 +146,31 @@ def test_wide_update_with_streamed_masters_matches_oracle():
     """The checks above with masters and moments of the output layer above 128
     MB (512 x 21,896: remainders in n), where the update streams them."""
     test_narrow_networks_at_tile_edges_match_oracle([8, 512, 21896], 24)
+
+
+def free_bytes():
+    """Free device memory, from the HIP runtime that the libraries loaded."""
+    import ctypes as C
+    with open("/proc/self/maps") as f:
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("widths,n", [([512, 8], 150000), ([1024, 8], 80000), ([8, 16, 1032], 50000)])
+def test_predict_keeps_no_device_memory_of_a_large_call(widths, n):
+    """300 MB of inputs (both kinds of network) or 200 MB of outputs: at most the
+    two buffers of 64 MB and the hidden activations stay with the network, and
+    every row's output is the same bits as in calls of part of the rows, on
+    either side of the places where the call is split."""
+    from lymph3d_apsc_amd.mlp import Mlp
+    say(f"[mlp predict memory] {widths} {n} rows")
+    x = np.random.default_rng(n).standard_normal((n, widths[0])).astype(np.float32)
+    with Mlp(widths, max_batch=64, seed=2) as net:
+        net.predict(x[:64])
+        before = free_bytes()
+        y = net.predict(x)
+        assert before - free_bytes() < 150 << 20
+        for i in (0, 16000, 32000, 32700, n - 333):
+            assert np.array_equal(net.predict(x[i:i + 333]), y[i:i + 333]), i
