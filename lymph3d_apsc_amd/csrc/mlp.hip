@@ -1177,6 +1177,34 @@ __global__ __launch_bounds__(128) void k_layer(LayerArgs g) {
   layer_tile<EPI, GATHER>(g, blockIdx.x);
 }
 
+// Rows idx of X in bf16 in both fragment orders (a wave per 16 rows x 32
+// columns, transposed through LDS): see rows_apart().
+__global__ __launch_bounds__(256) void k_rows(const float* __restrict__ X, const int* __restrict__ idx, int B, int K,
+                                              int ts, bf16_t* __restrict__ HP, bf16_t* __restrict__ XT) {
+  constexpr int LDR = 24;  // 16 rows, padded to keep 16-byte pieces aligned
+  __shared__ __attribute__((aligned(16))) bf16_t sX[4][32 * LDR];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, steps = steps_of(K);
+  const int w = blockIdx.x * 4 + wave, mt = w / steps, k0 = w % steps * 32;
+  if (mt * 16 >= B) return;
+  const int row = mt * 16 + (lane & 15), q = (lane >> 4) * 8;
+  uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+  if (row < B && k0 + q < K) {
+    const float* x = X + (size_t)idx[row] * K + k0 + q;
+    const float4 a = *reinterpret_cast<const float4*>(x), b = *reinterpret_cast<const float4*>(x + 4);
+    v[0] = f2bf(a.x); v[1] = f2bf(a.y); v[2] = f2bf(a.z); v[3] = f2bf(a.w);
+    v[4] = f2bf(b.x); v[5] = f2bf(b.y); v[6] = f2bf(b.z); v[7] = f2bf(b.w);
+  }
+  *reinterpret_cast<uint4*>(HP + ((size_t)mt * steps + k0 / 32) * 512 + lane * 8) =
+      make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+  bf16_t* s = sX[wave];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) s[(q + r) * LDR + (lane & 15)] = (bf16_t)v[r];
+  wave_lds_sync();
+  const int k = lane >> 1, r0 = (lane & 1) * 8;  // widths and batches are multiples of 8
+  if (k0 + k < K && mt * 16 + r0 < B)
+    *reinterpret_cast<uint4*>(XT + pack_pos(k0 + k, mt * 16 + r0, ts)) = *reinterpret_cast<const uint4*>(s + k * LDR + r0);
+}
+
 // bf16 copies of W [N][K] in both fragment orders
 __global__ void k_pack(const float* __restrict__ W, int N, int K, bf16_t* __restrict__ Wf, bf16_t* __restrict__ Wd) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1450,14 +1478,28 @@ bool wide_nt(const LymphMlp* m) {
   return (size_t)m->w[m->L] * m->w[m->L - 1] * 12 > ((size_t)128 << 20);
 }
 
+// Whether a step's input rows are packed by a launch of their own (k_rows).
+// Every column tile of the first layer otherwise gathers and converts them
+// again, which wide inputs do not hide: us per step, in the layer / apart, one
+// layer of 512 x 512 at batch 256 22 / 12, 4,096 100 / 55, 65,536 1610 / 700
+// (with the GEMMs 28, 75 and 1040); 256 x 256 at 256 15.2 / 12.2.  Inputs of at
+// most 128 cost less than the launch: 128-256x2 at batch 512 21.6 / 23.3,
+// 64-512 at 1,024 18.5 / 20.8, 32-512x5-64 at 256 56.4 / 57.4.
+bool rows_apart(const LymphMlp* m) { return m->w[0] > 128; }
+
 // One step on rows idx of X, T: gradients into G (adam == null) or applied.
-// L forward launches, L - 1 backward (a wide layer's in two), one update.
+// L forward launches (wide inputs packed by one more), L - 1 backward (a wide
+// layer's in two), one update.
 int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx, float* loss,
               const AdamArgs* adam) {
   const size_t ny = (size_t)B * m->w[m->L];
   const int L = m->L;
   hipStream_t st = m->stream;
   int n_part = tiles_of(B) * tiles_of(m->w[L]);
+  const bool packed = rows_apart(m);
+  if (packed)
+    k_rows<<<blocks((size_t)tiles_of(B) * steps_of(m->w[0]), 4), 256, 0, st>>>(X, idx, B, m->w[0], steps_of(m->max_batch),
+                                                                             m->HP[0], m->HT[0]);
   for (int l = 0; l < L; ++l) {
     LayerArgs a{};
     a.N = m->w[l + 1]; a.K = m->w[l]; a.B = B; a.ts = steps_of(m->max_batch);
@@ -1468,13 +1510,13 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
     const unsigned wgs = (unsigned)layer_wgs(a.N, B);
     if (l + 1 < L) {
       a.out = m->HP[l + 1]; a.outT = m->HT[l + 1]; a.dg = m->dg[l];
-      if (l == 0) k_layer<LAYER_FWD, true><<<wgs, 128, 0, st>>>(a);
+      if (l == 0 && !packed) k_layer<LAYER_FWD, true><<<wgs, 128, 0, st>>>(a);
       else k_layer<LAYER_FWD, false><<<wgs, 128, 0, st>>>(a);
     } else {
       a.out = m->DP[l]; a.outT = m->DT[l];
       a.T = T; a.scale = 2.0f / (float)ny; a.part = m->part;
       if (m->wide) n_part = launch_wide<LAYER_LOSS>(m, a);
-      else if (l == 0) k_layer<LAYER_LOSS, true><<<wgs, 128, 0, st>>>(a);
+      else if (l == 0 && !packed) k_layer<LAYER_LOSS, true><<<wgs, 128, 0, st>>>(a);
       else k_layer<LAYER_LOSS, false><<<wgs, 128, 0, st>>>(a);
     }
   }
@@ -1617,6 +1659,7 @@ int lymph_mlp_create(int n_layers, const int32_t* widths, int max_batch, LymphMl
         zero(&m->HP[l], pack_size(max_batch, K));
         zero(&m->DP[l], pack_size(max_batch, N));
       }
+      if (l == 0 && rows_apart(m)) al(&m->HP[0], pack_size(max_batch, K));
       if (l + 1 < n_layers) al(&m->dg[l], (size_t)tiles_of(max_batch) * tiles_of(N) * 64);
     }
   } else {

@@ -174,3 +174,12 @@ def test_predict_keeps_no_device_memory_of_a_large_call(widths, n):
         assert before - free_bytes() < 150 << 20
         for i in (0, 16000, 32000, 32700, n - 333):
             assert np.array_equal(net.predict(x[i:i + 333]), y[i:i + 333]), i
+
+
+# inputs on either side of the width from which they are packed ahead of the
+# first layer (128), whole and ragged steps of 32 and tiles of 16 rows, one
+# layer and several, batches of several thousand rows
+@pytest.mark.parametrize("widths,batch", [([128, 24], 8), ([136, 24], 8), ([136, 520, 8], 24), ([264, 16, 8], 40),
+                                          ([504, 512], 2056), ([512, 40, 1032], 264)])
+def test_wide_inputs_packed_ahead_match_oracle(widths, batch):
+    test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
