@@ -872,17 +872,22 @@ struct UpdateArgs {
 // Joined to the launch of a lower layer's input gradient instead, each layer's
 // update made those launches 8.3 us long where they take 4.2: 75 us a step
 // against 63.  The workgroups from first_bias on sum the biases' columns (in
-// k_colsum's order), the last one the loss.
-template <bool ADAM>
-__global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// k_colsum's order), the last one the loss.  PARTS > 1: that many pairs of
+// waves share the batch and add their sums in order (see update_parts).
+template <bool ADAM, int PARTS>
+__global__ __launch_bounds__(128 * PARTS) void k_update(UpdateArgs u) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6 & 1), part = __builtin_amdgcn_readfirstlane(tid >> 7);
   const int wg = blockIdx.x;
+  __shared__ f32x4 sP[PARTS > 1 ? PARTS - 1 : 1][PARTS > 1 ? 2 : 1][64][2];
   if (wg == (int)gridDim.x - 1) {  // the loss
     __shared__ double red[128];
-    double s = 0.0;
+    if (part == 0) {
+      double s = 0.0;
 #pragma unroll 8
-    for (int i = tid; i < u.n_part; i += 128) s += u.part[i];
-    red[tid] = s;
+      for (int i = tid; i < u.n_part; i += 128) s += u.part[i];
+      red[tid] = s;
+    }
     __syncthreads();
     for (int w = 64; w > 0; w >>= 1) {
       if (tid < w) red[tid] += red[tid + w];
@@ -898,7 +903,17 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
     const int gp = lane & 31, half = lane >> 5;
     const int n = o * 4 + wave * 2 + half;  // widths are multiples of 8
     float s = 0.f;
-    for (int b = gp; b < u.B; b += 32) s += bf2f(y.DT[pack_pos(n, b, u.ts)]);
+    if constexpr (PARTS == 1) {
+      for (int b = gp; b < u.B; b += 32) s += bf2f(y.DT[pack_pos(n, b, u.ts)]);
+    } else {
+#pragma unroll 8
+      for (int b = 32 * part + gp; b < u.B; b += 32 * PARTS) s += bf2f(y.DT[pack_pos(n, b, u.ts)]);
+      if (part > 0) sP[part - 1][wave][lane][0][0] = s;
+      __syncthreads();
+      if (part > 0) return;
+#pragma unroll
+      for (int j = 0; j < PARTS - 1; ++j) s += sP[j][wave][lane][0][0];
+    }
     float t = 0.f;
 #pragma unroll
     for (int j = 0; j < 32; ++j) t += __shfl(s, half * 32 + j, 64);
@@ -919,14 +934,15 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
   const UpdateLayer& y = u.y[l];
   const int tk = (y.K + 63) / 64, o = wg - y.first;
   const int k0 = (o % tk) * 64 + wave * 32, n0 = (o / tk) * 16;
-  if (k0 >= y.K || n0 >= y.N) return;
+  const bool on = k0 < y.K && n0 < y.N;
+  if (PARTS == 1 && !on) return;
   const int fr = lane & 15, fk = (lane >> 4) * 8;
   f32x4 acc[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   // masters and moments on their way while the products run
   float4 pw[2], pm[2], pv[2];
-  if (ADAM) {
+  if (ADAM && part == 0) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int k = k0 + 16 * i + (lane >> 4) * 4, n = n0 + fr;
@@ -940,7 +956,7 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
   }
   constexpr int CH = 4;
 #pragma unroll 1
-  for (int s0 = 0; s0 < u.B; s0 += 32 * CH) {
+  for (int s0 = 32 * CH * part; s0 < u.B && on; s0 += 32 * CH * PARTS) {
     uint4 a[CH][2], b[CH];
 #pragma unroll
     for (int s = 0; s < CH; ++s) {
@@ -962,6 +978,17 @@ __global__ __launch_bounds__(128) void k_update(UpdateArgs u) {
         for (int i = 0; i < 2; ++i)
           acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s][i]),
                                                            __builtin_bit_cast(bf16x8, b[s]), acc[i], 0, 0, 0);
+  }
+  if constexpr (PARTS > 1) {
+    if (part > 0)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sP[part - 1][wave][lane][i] = acc[i];
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int j = 0; j < PARTS - 1; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] += sP[j][wave][lane][i];
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -1487,6 +1514,17 @@ bool wide_nt(const LymphMlp* m) {
 // 64-512 at 1,024 18.5 / 20.8, 32-512x5-64 at 256 56.4 / 57.4.
 bool rows_apart(const LymphMlp* m) { return m->w[0] > 128; }
 
+// Pairs of waves per tile of k_update.  With one, a wave walks the whole batch,
+// and few tiles (wgs workgroups) leave the chip idle meanwhile; four in a
+// workgroup keep four times the loads in flight.  us per step, 1 / 4, at batch
+// 2,048 and 16,384: 64-512 32.1 / 21.8 and 191 / 126 (the GEMMs: 44 and 169),
+// 8-512 27.2 / 18.4 and 169 / 72 (46 and 135), 512-512 (256 workgroups) 33.2 /
+// 24.8 and 190 / 111.  Where the tiles fill the chip both are even: 32-512x5-64
+// (1,088) 121 / 126 and 725 / 707.  Smaller batches keep one sum in the rows'
+// order (64-512 at 1,024: 18.1 / 13.9; at 256 even).
+constexpr int kUpParts = 4;
+int update_parts(int wgs, int B) { return B >= 2048 && wgs <= 256 ? kUpParts : 1; }
+
 // One step on rows idx of X, T: gradients into G (adam == null) or applied.
 // L forward launches (wide inputs packed by one more), L - 1 backward (a wide
 // layer's in two), one update.
@@ -1575,8 +1613,13 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
     else if (wide_nt(m)) k_update_wide<true, true><<<big, 256, 0, st>>>(u, apart);
     else k_update_wide<true, false><<<big, 256, 0, st>>>(u, apart);
   }
-  if (adam) k_update<true><<<wgs + bias + 1, 128, 0, st>>>(u);
-  else k_update<false><<<wgs + bias + 1, 128, 0, st>>>(u);
+  if (update_parts(wgs, B) > 1) {
+    if (adam) k_update<true, kUpParts><<<wgs + bias + 1, 128 * kUpParts, 0, st>>>(u);
+    else k_update<false, kUpParts><<<wgs + bias + 1, 128 * kUpParts, 0, st>>>(u);
+  } else {
+    if (adam) k_update<true, 1><<<wgs + bias + 1, 128, 0, st>>>(u);
+    else k_update<false, 1><<<wgs + bias + 1, 128, 0, st>>>(u);
+  }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("training step: ") + hipGetErrorString(e));
 }

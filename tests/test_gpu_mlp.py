@@ -183,3 +183,12 @@ def test_predict_keeps_no_device_memory_of_a_large_call(widths, n):
                                           ([504, 512], 2056), ([512, 40, 1032], 264)])
 def test_wide_inputs_packed_ahead_match_oracle(widths, batch):
     test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
+
+
+# few weight tiles and a batch of 2048 and more: four pairs of waves share the
+# batch, in lots of 128 rows (remainders of 8 rows up to three lots), tiles past
+# the widths' ends, up to 256 workgroups of tiles; 2040 rows are one sum
+@pytest.mark.parametrize("widths,batch", [([8, 8], 2048), ([72, 40], 2056), ([24, 136, 88, 8], 2424), ([264, 72], 4096),
+                                          ([8, 520], 2176), ([512, 512], 2048), ([504, 8, 520, 16], 2056), ([72, 40], 2040)])
+def test_updates_over_large_batches_match_oracle(widths, batch):
+    test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
