@@ -1315,6 +1315,18 @@ int split_of(int M, int N, int K, int* kchunk) {
   *kchunk = (int)(blocks(blocks(K, S), BK) * BK);
   return (int)blocks(K, *kchunk);
 }
+// The same for a wide layer's input gradient.  Where the GEMM would not split,
+// k_split still does from 4,096 outputs on, into 8 parts (one per XCD): k_layer
+// reads W again for every 16 rows.  us per step, k_layer / split: 8-512x3-38,400
+// at batch 2,048 1047 / 762, 4,096 2050 / 1478 (the GEMM 1934), 8,192 4032 / 3011
+// (3452); 8-512-8,192 at 8,192 901 / 760 (888); 512x2-4,096 at 4,096 239 / 221;
+// 8-512-2,048 at 2,048 even, at 16,384 644 / 690.
+int wide_parts(int M, int N, int K, int* kchunk) {
+  const int S = split_of(M, N, K, kchunk);
+  if (S > 1 || K < 4096) return S;
+  *kchunk = (int)(blocks(blocks(K, 8), BK) * BK);
+  return (int)blocks(K, *kchunk);
+}
 // split-k workspace: grown on the first call of a larger shape
 int need_ws(LymphMlp* m, size_t floats) {
   if (floats <= m->ws_floats) return 0;
@@ -1565,7 +1577,7 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
     a.in = m->DP[l];
     a.out = l > 1 ? m->DP[l - 1] : nullptr; a.outT = m->DT[l - 1]; a.dg = m->dg[l - 1];
     int kchunk = 0;
-    const int S = l == L - 1 && m->wide ? split_of(B, a.N, a.K, &kchunk) : 1;
+    const int S = l == L - 1 && m->wide ? wide_parts(B, a.N, a.K, &kchunk) : 1;
     if (S == 1) {
       k_layer<LAYER_BWD, false><<<(unsigned)layer_wgs(a.N, B), 128, 0, st>>>(a);
       continue;

@@ -192,3 +192,11 @@ def test_wide_inputs_packed_ahead_match_oracle(widths, batch):
                                           ([8, 520], 2176), ([512, 512], 2048), ([504, 8, 520, 16], 2056), ([72, 40], 2040)])
 def test_updates_over_large_batches_match_oracle(widths, batch):
     test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
+
+
+# input gradients of a wide layer over so many rows that a GEMM would not split
+# them: 4096 outputs and more in 8 parts (the last one a remainder, the last row
+# tiles a half block), 4088 in one
+@pytest.mark.parametrize("widths,batch", [([8, 512, 4096], 2048), ([8, 504, 4104], 2056), ([8, 512, 4088], 2048)])
+def test_wide_input_gradients_over_large_batches_match_oracle(widths, batch):
+    test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
