@@ -200,3 +200,20 @@ def test_updates_over_large_batches_match_oracle(widths, batch):
 @pytest.mark.parametrize("widths,batch", [([8, 512, 4096], 2048), ([8, 504, 4104], 2056), ([8, 512, 4088], 2048)])
 def test_wide_input_gradients_over_large_batches_match_oracle(widths, batch):
     test_narrow_networks_at_tile_edges_match_oracle(widths, batch)
+
+
+def test_predict_in_pieces_of_a_large_batch_gives_the_bits_of_small_calls():
+    """4200 rows of 16,408 outputs on a network of that batch: pieces of 2304
+    rows (150 MB of outputs in whole groups of 256); the same rows on a network
+    of batch 64, in pieces of 1,000 and less."""
+    from lymph3d_apsc_amd.mlp import Mlp
+    say("[mlp predict pieces]")
+    widths = [8, 40, 16408]
+    x = np.random.default_rng(9).standard_normal((4200, 8)).astype(np.float32)
+    with Mlp(widths, max_batch=4200, seed=6) as net, Mlp(widths, max_batch=64, seed=6) as small:
+        y = net.predict(x)
+        assert np.isfinite(y).all() and np.abs(y).min(axis=1).max() > 0
+        for a in range(0, 4200, 1000):
+            assert np.array_equal(small.predict(x[a:a + 1000]), y[a:a + 1000]), a
+        y_ref, _ = R.forward(net.params().astype(np.float64), widths, x[2290:2320], emulate=True)
+        assert rel(y[2290:2320], y_ref) < 5e-3
