@@ -848,7 +848,7 @@ struct UpdateLayer {
   int N, K, first;      // W is [N][K]; first workgroup of its weight tiles
   const bf16_t *DT, *HT;  // dZ^T [N][rows], H^T [K][rows], packed
   size_t woff, boff;
-  bf16_t *Wf, *Wd, *Wb;  // packed copies and the row-major copy, where kept
+  bf16_t *Wf, *Wd;      // packed copies
 };
 struct UpdateArgs {
   int L, B, ts, first_bias, n_part;  // ts: steps of DT's and HT's rows
@@ -1008,7 +1008,6 @@ __global__ __launch_bounds__(128 * PARTS) void k_update(UpdateArgs u) {
     *reinterpret_cast<float4*>(u.M + at) = m;
     *reinterpret_cast<float4*>(u.V + at) = v;
     const uint2 hw = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
-    if (y.Wb) *reinterpret_cast<uint2*>(y.Wb + (size_t)n * y.K + k) = hw;
     if (y.Wf) *reinterpret_cast<uint2*>(y.Wf + pack_pos(n, k, steps_of(y.K))) = hw;
     if (y.Wd) {
       const int sn = steps_of(y.N);
