@@ -1019,3 +1019,34 @@ def test_asking_for_the_variants_keeps_the_one_in_use():
             assert ctx.step_variant() == 2
             ctx.autotune(reps=2)
             assert ctx.n_step_variants() == n and ctx.step_variant() == ctx.chosen_variant
+
+
+@pytest.mark.parametrize("near,far,p,bits", [((13, "agg"), (15, "agg"), 3, 32), ((8, "tets"), (15, "agg"), 3, 32),
+                                             ((20, "agg"), (26, "agg"), 1, 32), ((20, "agg"), (26, "agg"), 1, 48),
+                                             ((12, "agg"), (13, "agg"), 2, 32), ((15, "grown"), (16, "grown"), 3, 64),
+                                             ((15, "grown"), (16, "grown"), 4, 32), ((5, "agg"), (7, "agg"), 4, 48)])
+def test_default_variant_changes_across_its_lines_and_keeps_the_bits(near, far, p, bits):
+    """Meshes on either side of a line of the choice (2,000, 3,000 and 16,384
+    polyhedra, 1,024 uneven ones, 256 at p = 4; 5- and 7-block rows) start on
+    different variants, and on each the step has the bits of variant 0."""
+    say(f"[variant lines] {near} {far} p={p} {bits}-bit")
+    chosen = []
+    for n, kind in (near, far):
+        if kind == "grown":
+            m = M.cube_mesh(n, dirichlet_faces={"x0", "x1", "y0", "y1", "z0"}, poly_size=(4, 40), seed=3)
+        else:
+            m = M.cube_mesh(n, agglomerate=kind == "agg")
+        rng = np.random.default_rng(n + p)
+        with L.Context(m, p) as ctx:
+            ctx.set_keep_adg(False)
+            ctx.set_build("factored")
+            ctx.make_matrices_free()
+            ctx.set_apply_precision(bits)
+            u0, u1 = rng.standard_normal(m.n_poly * ctx.n3), rng.standard_normal(m.n_poly * ctx.n3)
+            chosen.append(ctx.step_variant())
+            a = ctx.time_step_matrix_free(0.37, 1e-4, u0, u1)
+            f = ctx.first_time_step_matrix_free(0.37, 1e-4, u0, u1)
+            ctx.set_step_variant(0)
+            assert np.array_equal(a, ctx.time_step_matrix_free(0.37, 1e-4, u0, u1), equal_nan=True)
+            assert np.array_equal(f, ctx.first_time_step_matrix_free(0.37, 1e-4, u0, u1), equal_nan=True)
+    assert chosen[0] != chosen[1], chosen
