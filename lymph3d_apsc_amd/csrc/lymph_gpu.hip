@@ -434,39 +434,65 @@ void launch_leapfrog48(int variant, int grid, hipStream_t st, const float* K, co
 
 // The step variant a context starts with (before lymph_autotune or
 // lymph_set_step_variant), by apply, degree and mesh.  What decides is whether
-// the polyhedra alone fill the chip's 1024 SIMDs:
-//  - few polyhedra (below 256, or below 1024 where uneven polyhedra make long
-//    block rows): the step is one chain of memory trips, so 8 waves share a
-//    polyhedron and each has a whole block in flight.  125 polyhedra, us per
-//    step, one wave per polyhedron / 8 waves: FP64 p = 1..4 6.3 / 3.9, 11.9 /
-//    5.3, 28.4 / 9.7, 88 / 26; 32-bit 5.0 / 3.0, 12.2 / 3.3, 17.3 / 4.7, 53 /
-//    11; 48-bit p = 2, 3 9.9 / 4.1, 30.2 / 6.3;
-//  - up to 3000 polyhedra 4 waves (p <= 2; 1000 polyhedra, FP64 p = 2: 11.9
-//    us against 24.8 with one wave and 13.5 with 8);
-//  - beyond, p <= 2 packs 64 / 3Np polyhedra into a wave (32,768 polyhedra, p
-//    = 1: FP64 83 -> 45 us, 32-bit 58 -> 25; p = 2 32-bit 199 -> 138);
-//  - p >= 3 keeps several waves at every size: a wave's 64 lanes then stream
-//    consecutive blocks (32,768 polyhedra, p = 3: FP64 1004 -> 937 us, 32-bit
-//    513 -> 468 with 8, 48-bit 771 -> 704).  With the 5-block rows of
-//    single-tet polyhedra 8 waves leave three idle: 4 (2 for 48-bit p = 4).
+// the polyhedra alone fill the chip's 1024 SIMDs: below, a step is one chain of
+// memory trips and several waves share a polyhedron; above, p <= 2 packs 64 /
+// 3Np polyhedra into a wave, and p >= 3 keeps several waves, whose lanes stream
+// consecutive blocks.  us per step on agglomerated cubes (6 to 7 blocks a row)
+// unless single tets (5) or uneven polyhedra (11) are named:
+//  - p = 1: 8 waves below 2,000 polyhedra, 4 below 3,000, then packed.  FP64, 1 /
+//    4 / 8 waves / packed: 125 polyhedra 6.6 / 5.0 / 4.5 / 6.1, 1,000 7.4 / 6.0 /
+//    5.7 / 6.0, 2,197 8.7 / 8.2 / 9.4 / 6.4, 3,375 10.5 / 10.4 / 12.6 / 6.9,
+//    32,768 82 / 104 / 148 / 45: packing wins from about 1,500 on already, which
+//    lymph_autotune finds.  Uneven polyhedra walk their blocks jointly: 2,338
+//    polyhedra 4 / 8 waves / joint 12.9 / 14.2 / 15.3, 4,076 17.7 / 23.1 / 17.0 (packed 19.8).
+//    So do 16,384 polyhedra and more at 32 and 48 bits, where packed and joint
+//    are even but for the largest (32,768 at 48 bits 35.5 / 33.6).
+//  - p = 2: 8 waves below 256 polyhedra, or 1,024 uneven ones (32-bit: 2,000 of
+//    either), 4 below 3,000, then packed (FP64: joint).  FP64, 1 / 4 / 8 waves /
+//    joint: 216 polyhedra 12.0 / 6.2 / 5.9 / 8.1, 1,000 18.5 / 10.9 / 12.4 / 12.6,
+//    2,744 25.1 / 24.1 / 28.8 / 24.0, 32,768 269 / 267 / 368 / 257; uneven 999 46.7 /
+//    17.5 / 17.4 / 21.8.  32-bit, 4 / 8 waves / packed: 1,728 9.7 / 10.2 / 11.3, 2,197
+//    13.1 / 12.6 / 13.5, 3,375 16.3 / 17.1 / 16.0.
+//  - p = 3: FP64 and 32-bit 8 waves below 256 polyhedra or 1,024 uneven ones, then
+//    4, and 8 again for 32 bits from 3,000 polyhedra with 6 blocks a row and more;
+//    48 bits 8 waves but for 256 to 3,000 with shorter rows (4).  4 / 8 waves: FP64
+//    216 polyhedra 11.9 / 10.5, 343 15.6 / 16.1, 8,000 232 / 238, uneven 999 55.8 /
+//    54.0; 32-bit 216 6.1 / 5.0, 1,000 15.5 / 15.9, 8,000 124 / 121, 16,464 tets 186 /
+//    188; 48-bit 1,000 23.5 / 23.1, 16,464 tets 273 / 266, 1,296 tets 24.4 / 23.6.
+//  - p = 4: FP64 8 waves at every size, 4 / 8: 125 polyhedra 28.7 / 26.5, 343 41.5 /
+//    43.4, 8,000 713 / 703, 3,072 tets 208 / 205.  32-bit as p = 3 up to there, then
+//    4: 216 15.4 / 12.7, 343 21.5 / 22.0, 8,000 365 / 382.  48-bit 8 waves below
+//    256, then 4, 2 with shorter rows, 2 / 4 / 8: 216 28.5 / 20.1 / 18.2, 343 34.0 /
+//    29.1 / 31.1, 3,072 tets 157 / 160 / 181.
+// One long row sizes the LDS of every workgroup of a joint or shared step.
+// Among few polyhedra its own time decides, which these steps shorten; among
+// many (past 32,768) the occupancy: p <= 2 packs without LDS where a wave would
+// take more than 16 KB, p = 3 takes one wave a polyhedron past 48 KB (32-bit: 8
+// waves at any size).  Single tets but for one row of 136 (68 at p = 2), that /
+// the other: p = 1 105,268 polyhedra 180 / 303 (48-bit 181 / 260), 16,306 85 / 43;
+// p = 2 47,922 275 / 338, 16,386 132 / 120; p = 3 105,268 2282 / 2558 (32-bit 1208
+// / 1425), 10,180 32-bit 117 / 138.
 int default_variant(const LymphCtx* c, int bits) {
   const int n = c->n_poly;
   const bool uneven = c->order != nullptr;
   const bool few = n < 256 || (uneven && n < 1024);
   const bool mid = n < 3000;
   const bool long_rows = c->n_blk >= 6 * (size_t)n;
+  const bool many = n > 32768;
+  const size_t dyn = (size_t)c->max_row * c->n3 * sizeof(double);
+  const bool joint = !(many && (64 / c->n3) * dyn > ((size_t)16 << 10));
   switch (c->p) {
     case 1:
-      if (bits == 64) return n < 2000 ? 10 : (mid ? 9 : (uneven ? 6 : 5));
-      if (bits == 32) return n < 2000 ? 8 : (mid ? 7 : (uneven || n >= 16384 ? 6 : 3));
-      return n < 2000 ? 7 : (mid ? 2 : (uneven || n >= 16384 ? 5 : 3));
+      if (bits == 64) return n < 2000 ? 10 : (mid ? 9 : (uneven && joint ? 6 : 5));
+      if (bits == 32) return n < 2000 ? 8 : (mid ? 7 : ((uneven || n >= 16384) && joint ? 6 : 3));
+      return n < 2000 ? 7 : (mid ? 2 : ((uneven || n >= 16384) && joint ? 5 : 3));
     case 2:
-      if (bits == 64) return few ? 12 : (mid ? 11 : 8);
+      if (bits == 64) return few ? 12 : (mid ? 11 : (joint ? 8 : 7));
       if (bits == 32) return n < 2000 ? 10 : (mid ? 9 : 7);
       return few ? 7 : (mid ? 2 : 4);
     case 3:
-      if (bits == 64) return few ? 12 : 10;
-      if (bits == 32) return few || (long_rows && !mid) ? 8 : 6;
+      if (bits == 64) return few ? 12 : (many && dyn > ((size_t)48 << 10) ? 5 : 10);
+      if (bits == 32) return few || dyn > ((size_t)48 << 10) || (long_rows && !mid) ? 8 : 6;
       return few || long_rows || !mid ? 6 : 5;
     default:
       if (bits == 64) return 13;
@@ -528,13 +554,20 @@ int d2h_vec(LymphCtx* c, const double* d, double* h) {
 
 // Whether the step's operator reads should stay in the caches: the eight L2s
 // hold 32 MB, the Infinity Cache 256 MB; beyond, a cached read only displaces
-// the vectors.  us per step, streaming / cached: 2,197 polyhedra p = 1 (17 MB)
-// 11.1 / 8.2; 125 p = 3 (21 MB) 9.7 / 7.5; 512 p = 2 (23 MB) 8.8 / 6.8; 32-bit 1,000 p =
-// 2 (23 MB) 6.9 / 5.1; p = 2 98 MB 18.7 / 16.9, 193 MB 33.7 / 31.4; deck of 28,606
-// tets p = 1 (161 MB) 31.7 / 30.4.  At p = 3 the two are even or streaming wins
-// between (46 MB 9.6 / 9.7, 92 MB 18.2 / 19.3), then 184 MB 34.4 / 31.8, 207 MB
-// 33.6 / 32.6.  Past the Infinity Cache streaming wins everywhere: 320 MB 60.6 /
-// 68.8, 354 MB 66 / 76.
+// the vectors.  us per step, streaming / cached, at operators of
+//  - up to 32 MiB: p = 1 31 MB 10.5 / 8.4, p = 3 21 MB 7.8 / 7.5, 32-bit 30 MB 8.7 /
+//    6.4, p = 4 32-bit 32 MB 11.5 / 9.1: cached;
+//  - up to 208 MiB at p <= 2: 3 to 15% for cached reads throughout (p = 1 32-bit
+//    154 MB 32.3 / 28.2; p = 2 195 MB 33.9 / 33.2, 48-bit 210 MB 37.2 / 35.3);
+//  - 32 to 128 MiB at p >= 3: streamed, as p = 3 is even or loses up to 5% by
+//    caching (46 MB 9.5 / 9.7, 92 MB 18.2 / 19.1, uneven 79 MB 16.0 / 15.5); p = 4
+//    would win 3 to 25% (64 MB 26.2 / 22.3, 114 MB 29.5 / 28.5);
+//  - 128 to 208 MiB at p >= 3: p = 3 184 MB 34.3 / 31.9, 32-bit 187 MB uneven 33.8 /
+//    31.0, p = 4 186 MB 45.6 / 43.8: cached;
+//  - beyond: up to about 300 MB caching is even or wins up to 5% (p = 3 260 MB 43.4 /
+//    43.3, 247 MB 43.8 / 42.3; p = 1 32-bit 253 MB 54.5 / 46.6), and streaming
+//    leaves the cache to the vectors and to other contexts; from there on it
+//    wins: p = 3 324 MB 54.6 / 58.7, p = 2 386 MB 63.3 / 73.2, p = 4 400 MB 74.0 / 83.4.
 //
 // Solves of two contexts on two streams share the Infinity Cache: one that
 // would come to more than 288 MB with what the others keep there streams.  us

@@ -1050,3 +1050,36 @@ def test_default_variant_changes_across_its_lines_and_keeps_the_bits(near, far, 
             assert np.array_equal(a, ctx.time_step_matrix_free(0.37, 1e-4, u0, u1), equal_nan=True)
             assert np.array_equal(f, ctx.first_time_step_matrix_free(0.37, 1e-4, u0, u1), equal_nan=True)
     assert chosen[0] != chosen[1], chosen
+
+
+def mesh_with_a_long_row(n):
+    """Single tets of an n^3 cube but for one polyhedron of 4 x 3 x 3 cubes: 132
+    neighbours."""
+    m0 = M.cube_mesh(n)
+    cell = np.floor(m0.xyz[m0.tet_vert].mean(axis=1) * n).astype(int) - n // 3
+    inner = ((cell >= 0) & (cell < (4, 3, 3))).all(axis=1)
+    poly = np.zeros(m0.n_tet, np.int64)
+    poly[~inner] = 1 + np.arange((~inner).sum())
+    return M.Mesh(m0.xyz, m0.tet_vert, poly, m0.tria_vert, m0.tria_tag, m0.tag_space)
+
+
+@pytest.mark.parametrize("p,bits,far", [(1, 64, 5), (1, 32, 3), (1, 48, 3), (2, 64, 7), (3, 64, 5), (3, 32, 8)])
+def test_default_variant_with_a_long_row_among_many_polyhedra(p, bits, far):
+    """A block row of 133 makes the LDS of every workgroup of a joint or shared
+    step large: past 32,768 polyhedra a context starts on a variant without it
+    (8 waves at 32 bits, p = 3), with the bits of variant 0."""
+    say(f"[variant, long row] p={p} {bits}-bit")
+    for n, chosen in ((12, None), (18, far)):
+        m = mesh_with_a_long_row(n)
+        rng = np.random.default_rng(n)
+        with L.Context(m, p) as ctx:
+            ctx.set_keep_adg(False)
+            ctx.set_build("factored")
+            ctx.make_matrices_free()
+            assert np.diff(ctx.pattern()[0]).max() == 133
+            ctx.set_apply_precision(bits)
+            assert chosen is None or ctx.step_variant() == chosen
+            u0, u1 = rng.standard_normal(m.n_poly * ctx.n3), rng.standard_normal(m.n_poly * ctx.n3)
+            a = ctx.time_step_matrix_free(0.37, 1e-4, u0, u1)
+            ctx.set_step_variant(0)
+            assert np.array_equal(a, ctx.time_step_matrix_free(0.37, 1e-4, u0, u1), equal_nan=True), n
