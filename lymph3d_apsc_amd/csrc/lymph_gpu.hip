@@ -2147,8 +2147,12 @@ namespace {
 int sample_into(LymphCtx* c, const double* u, double* d_out) {
   return dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    k_sample<P><<<(unsigned)c->n_recv, 64, 0, c->stream>>>(
-        u, c->rpoly, c->rxyz, c->md.bbox, c->md.blist, c->n_recv, d_out);
+    if (c->n_recv <= kSampleWaves)
+      k_sample<P><<<(unsigned)c->n_recv, 64, 0, c->stream>>>(u, c->rpoly, c->rxyz, c->md.bbox, c->md.blist,
+                                                             c->n_recv, d_out);
+    else
+      k_sample_many<P><<<grid1(3 * (size_t)c->n_recv, 128), 128, 0, c->stream>>>(
+          u, c->rpoly, c->rxyz, c->md.bbox, c->md.blist, c->n_recv, d_out);
     return check_launch("k_sample");
   });
 }

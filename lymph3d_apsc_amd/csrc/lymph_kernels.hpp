@@ -300,10 +300,9 @@ struct BuildTet {
 };
 
 template <int P, bool REF, bool ADG>
-__global__ __launch_bounds__(Build<P>::TPB, !REF && (P == 2 || P == 3) ? 4 : 2) void k_build(MeshDev m, double alpha, double theta,
-                                                         double* __restrict__ K, double* __restrict__ A,
-                                                         double* __restrict__ M, double* __restrict__ Mm,
-                                                         int n_poly) {
+__global__ __launch_bounds__(Build<P>::TPB, !REF && (P == 2 || P == 3) ? 4 : 2) void k_build(
+    MeshDev m, double alpha, double theta, double* __restrict__ K, double* __restrict__ A, double* __restrict__ M,
+    double* __restrict__ Mm, int n_poly) {
   using D = Dims<P>;
   using B = Build<P>;
   constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2, QC = B::QC, GP = B::GP, TG = B::TG,
@@ -3200,10 +3199,14 @@ __global__ void k_to_fortran(const double* __restrict__ p, double* __restrict__ 
 
 // Receivers: value of the modal field at a point, sum_i u_i Lx Ly Lz on the
 // polyhedron's bounding box, as EXPORT_SOLUTION evaluates it
-// (src/solution_processing.f90:150-170).  One wave per receiver, a basis
-// function per lane, the terms added in the functions' order: 64 receivers at
-// p = 4 took 21 us with a thread per component, now 5; out[r*3 + comp] of
-// record row `row`.
+// (src/solution_processing.f90:150-170); out[r*3 + comp] of record row `row`.
+// One wave per receiver, a basis function per lane, the terms added in the
+// functions' order: 64 receivers at p = 4 take 5 us, with a thread per
+// component 14.  Beyond kSampleWaves receivers the threads fill the chip
+// (k_sample_many, the same bits): wave / thread us, p = 1 and 4, 2,000 receivers
+// 5.3 / 5.6 and 8.6 / 16.8, 8,000 10.1 / 7.1 and 17.1 / 17.2, 100,000 52 / 10 and
+// 141 / 54.
+constexpr int kSampleWaves = 4096;
 template <int P>
 __global__ __launch_bounds__(64) void k_sample(const double* __restrict__ u, const int* __restrict__ rpoly,
                          const double* __restrict__ rxyz, const double* __restrict__ bbox,
@@ -3229,6 +3232,34 @@ __global__ __launch_bounds__(64) void k_sample(const double* __restrict__ u, con
 #pragma unroll
     for (int c = 0; c < 3; ++c) s[c] = s[c] + lane_bcast(t[c], j);
   if (i < 3) out[r * 3 + i] = i == 0 ? s[0] : (i == 1 ? s[1] : s[2]);
+}
+
+template <int P>
+__global__ void k_sample_many(const double* __restrict__ u, const int* __restrict__ rpoly,
+                              const double* __restrict__ rxyz, const double* __restrict__ bbox,
+                              const int* __restrict__ blist, int n, double* __restrict__ out) {
+  using D = Dims<P>;
+  constexpr int NP = D::NP;
+  const int id = blockIdx.x * blockDim.x + threadIdx.x;
+  if (id >= 3 * n) return;
+  const int r = id / 3, comp = id % 3;
+  const int Pp = rpoly[r];
+  const double* bb = bbox + (size_t)Pp * 6;
+  double xp[3], sq[3];
+  for (int d = 0; d < 3; ++d) {
+    const double hb = (bb[2 * d + 1] - bb[2 * d]) / 2.0, mb = (bb[2 * d + 1] + bb[2 * d]) / 2.0;
+    xp[d] = (rxyz[(size_t)r * 3 + d] - mb) / hb;
+    sq[d] = sqrt(hb);
+  }
+  const double* uu = u + (size_t)Pp * D::N3 + comp * NP;
+  double s = 0.0;
+  for (int i = 0; i < NP; ++i) {
+    const double vx = leg(blist[i * 3 + 0], xp[0]) / sq[0];
+    const double vy = leg(blist[i * 3 + 1], xp[1]) / sq[1];
+    const double vz = leg(blist[i * 3 + 2], xp[2]) / sq[2];
+    s = s + uu[i] * vx * vy * vz;
+  }
+  out[id] = s;
 }
 
 // Point forces: rhs[P_k][i*Np+m] += f_k,i phi_m(x_k), sources applied in order

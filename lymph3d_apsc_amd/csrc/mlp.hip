@@ -665,7 +665,8 @@ __device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
 }
 
 // acc[i][j] += W tile (t0 + i) times row tile (m0 + j) over steps s0..s1 - 1,
-// both in fragment order, D steps' fragments in flight.  Tiles past the last are the last one again.
+// both in fragment order, D steps' fragments in flight.  Tiles past the last are
+// the last one again.
 template <int T, int D>
 __device__ __forceinline__ void block_product(f32x4 (&acc)[T][T], const bf16_t* W, const bf16_t* in, int t0, int nt,
                                               int m0, int nm, int steps, int s0, int s1, int lane) {
@@ -717,10 +718,11 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// A wide output layer, forward: every wave T x T tiles of 16 x 16, so that
-// W's fragments are read B / 16 T times and the rows' N / 16 T times where k_layer reads them once per tile.  4 waves a workgroup, rw of
-// them along the rows; an XCD takes every eighth group of columns for all
-// rows, so W comes into one L2 only.  Bound by the way of W and the targets
+// A wide output layer, forward: every wave T x T tiles of 16 x 16, so that W's
+// fragments are read B / 16 T times and the rows' N / 16 T times where k_layer
+// reads them once per tile.  4 waves a workgroup, rw of them along the rows; an
+// XCD takes every eighth group of columns for all rows, so W comes into one L2
+// only.  Bound by the way of W and the targets
 // (39 MB each at 256 x 38,400) from HBM, of the gradients back (two copies of
 // 20 MB) and of the rows from L2.  EPI LAYER_LOSS fuses the loss: outputs are
 // not stored.
@@ -787,8 +789,9 @@ __global__ __launch_bounds__(256, 2) void k_wide(LayerArgs g) {
 // tiles, so the contraction is split as in gemm() and the parts, stored as the
 // lanes hold them, are added in order by k_split_end.  An XCD takes every
 // eighth part, whose operands then fit its L2.  256 x 512 from 38,400: 28 us,
-// 19 where dZ and W are still in the Infinity Cache (2 x 2 tiles a wave 39; more steps in flight change nothing) and 5 for the
-// sums, where the GEMM and its sums took 47.
+// 19 where dZ and W are still in the Infinity Cache (2 x 2 tiles a wave 39; more
+// steps in flight change nothing) and 5 for the sums, where the GEMM and its
+// sums took 47.
 template <int T>
 __global__ __launch_bounds__(256, 2) void k_split(LayerArgs g, int S, int chunk, f32x4* ws) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1228,7 +1231,8 @@ __global__ __launch_bounds__(256) void k_rows(const float* __restrict__ X, const
   wave_lds_sync();
   const int k = lane >> 1, r0 = (lane & 1) * 8;  // widths and batches are multiples of 8
   if (k0 + k < K && mt * 16 + r0 < B)
-    *reinterpret_cast<uint4*>(XT + pack_pos(k0 + k, mt * 16 + r0, ts)) = *reinterpret_cast<const uint4*>(s + k * LDR + r0);
+    *reinterpret_cast<uint4*>(XT + pack_pos(k0 + k, mt * 16 + r0, ts)) =
+        *reinterpret_cast<const uint4*>(s + k * LDR + r0);
 }
 
 // bf16 copies of W [N][K] in both fragment orders
@@ -1553,8 +1557,8 @@ int slab_step(LymphMlp* m, int B, const float* X, const float* T, const int* idx
   int n_part = tiles_of(B) * tiles_of(m->w[L]);
   const bool packed = rows_apart(m);
   if (packed)
-    k_rows<<<blocks((size_t)tiles_of(B) * steps_of(m->w[0]), 4), 256, 0, st>>>(X, idx, B, m->w[0], steps_of(m->max_batch),
-                                                                             m->HP[0], m->HT[0]);
+    k_rows<<<blocks((size_t)tiles_of(B) * steps_of(m->w[0]), 4), 256, 0, st>>>(
+        X, idx, B, m->w[0], steps_of(m->max_batch), m->HP[0], m->HT[0]);
   for (int l = 0; l < L; ++l) {
     LayerArgs a{};
     a.N = m->w[l + 1]; a.K = m->w[l]; a.B = B; a.ts = steps_of(m->max_batch);

@@ -1083,3 +1083,24 @@ def test_default_variant_with_a_long_row_among_many_polyhedra(p, bits, far):
             a = ctx.time_step_matrix_free(0.37, 1e-4, u0, u1)
             ctx.set_step_variant(0)
             assert np.array_equal(a, ctx.time_step_matrix_free(0.37, 1e-4, u0, u1), equal_nan=True), n
+
+
+@pytest.mark.parametrize("p", [1, 2, 3, 4])
+def test_receivers_on_both_sides_of_the_wave_limit(p):
+    """4,096 receivers are sampled by a wave each, 4,097 by a thread per
+    component: the same bits where they share points, and the oracle's values."""
+    say(f"[many receivers] p={p}")
+    m = hetero_mesh()
+    o = oracle_for(m, p)
+    rng = np.random.default_rng(p)
+    pts = rng.uniform(0.05, 0.95, (4097, 3))
+    with L.Context(m, p) as ctx:
+        u = rng.standard_normal(m.n_poly * ctx.n3)
+        ctx.set_slot(_lib.SLOT_U_CUR, u)
+        tets = ctx.set_receivers(pts)
+        many = ctx.sample_receivers()
+        ctx.set_receivers(pts[:4096], tets=tets[:4096])
+        few = ctx.sample_receivers()
+        assert np.array_equal(many[:4096], few)
+        ref = o.eval_points(pts[::97], tets[::97], u)
+        assert rel(many[::97], ref) < 1e-13
