@@ -1065,6 +1065,16 @@ int project_field(LymphCtx* c, int fn, double* v) {
   });
 }
 
+// p = 1 operator build with one polyhedron a wave instead of four, which walk
+// their tets in step and every face that one of them has: where few polyhedra
+// leave the chip idle anyway, above all large ones.  us, reference order, four a
+// wave / one (with 256 threads a polyhedron): 22 polyhedra of 300 to 600 tets
+// 7839 / 3490 (5383), 2,338 of 4 to 40 1000 / 703, 512 of 6 116 / 110; 1,728 of 6
+// 128 / 149, 9,535 of 4 to 40 1604 / 1844, 27,000 of 6 580 / 1582.
+bool build_one(const LymphCtx* c) {
+  return c->n_poly < 1024 || (c->n_poly < 4096 && c->n_tet >= 16 * c->n_poly);
+}
+
 int need_ctx(const LymphCtx* c) {
   if (!c) return fail(LYMPH_ERR_ARG, "null context");
   return 0;
@@ -1391,10 +1401,16 @@ int lymph_build_operator(LymphCtx* c) {
   int rc = dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
     // every entry of K, A_dg and the mass blocks is stored, none needs clearing
-    const unsigned wgs = grid1(c->n_poly, Build<P>::GP) * Build<P>::SPLIT;
+    auto go_as = [&](auto ref, auto adg, auto one) {
+      using B = Build<P, decltype(one)::value>;
+      k_build<P, decltype(ref)::value, decltype(adg)::value, decltype(one)::value>
+          <<<grid1(c->n_poly, B::GP) * B::SPLIT, B::TPB, 0, c->stream>>>(c->md, c->alpha, c->theta, c->K, c->A, c->M,
+                                                                         c->Mm, c->n_poly);
+    };
     auto go = [&](auto ref, auto adg) {
-      k_build<P, decltype(ref)::value, decltype(adg)::value><<<wgs, Build<P>::TPB, 0, c->stream>>>(
-          c->md, c->alpha, c->theta, c->K, c->A, c->M, c->Mm, c->n_poly);
+      if constexpr (P == 1)
+        if (build_one(c)) return go_as(ref, adg, std::true_type{});
+      go_as(ref, adg, std::false_type{});
     };
     const bool ref = c->build_mode != LYMPH_BUILD_FACTORED;
     if (ref && c->A) go(std::true_type{}, std::true_type{});

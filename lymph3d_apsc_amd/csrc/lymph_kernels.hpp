@@ -250,19 +250,19 @@ __device__ __forceinline__ void basis_row(const Tab1<P, NQ>& t, int a, int b, in
 // -> 11.  At p = 3 the reference order keeps the FP64 units 62% busy; the
 // factored one waits on LDS and barriers.
 // ---------------------------------------------------------------------------
-template <int P>
+template <int P, bool ONE = false>
 struct Build {
   static constexpr int PAIRS = np_of(P) * np_of(P);
-  // p = 1: 16 pairs, four polyhedra a wave; p = 2: 100 pairs in two waves; p =
-  // 3: 400 in seven; p = 4: 1225 in two workgroups of ten (two pairs a thread
-  // in one spilled 210 registers)
-  static constexpr int GP = P == 1 ? 4 : 1;
-  static constexpr int TG = P == 1 ? 16 : (P == 2 ? 128 : (P == 3 ? 448 : 640));
+  // p = 1: 16 pairs, four polyhedra a wave (ONE: one); p = 2: 100 pairs in two
+  // waves; p = 3: 400 in seven; p = 4: 1225 in two workgroups of ten (two pairs
+  // a thread in one spilled 210 registers)
+  static constexpr int GP = P == 1 && !ONE ? 4 : 1;
+  static constexpr int TG = P == 1 ? (ONE ? 64 : 16) : (P == 2 ? 128 : (P == 3 ? 448 : 640));
   static constexpr int SPLIT = (PAIRS + TG - 1) / TG;
   static constexpr int SHARE = (PAIRS + SPLIT - 1) / SPLIT;  // pairs per workgroup
   static constexpr int TPB = GP * TG;
   static constexpr int NQ2 = (P + 1) * (P + 1), NQ3 = NQ2 * (P + 1);
-  static constexpr int NB = P == 1 ? 2 : 8;  // tets fetched at a time
+  static constexpr int NB = GP > 1 ? 2 : 8;  // tets fetched at a time
   static constexpr int QC = P <= 2 ? NQ3 : 2 * NQ2 <= 32 ? 32 : NQ2;  // volume points per table
   static_assert(NQ3 % QC == 0, "whole chunks of the volume rule");
 };
@@ -299,12 +299,12 @@ struct BuildTet {
   BuildFace f[4];
 };
 
-template <int P, bool REF, bool ADG>
-__global__ __launch_bounds__(Build<P>::TPB, !REF && (P == 2 || P == 3) ? 4 : 2) void k_build(
+template <int P, bool REF, bool ADG, bool ONE = false>
+__global__ __launch_bounds__((Build<P, ONE>::TPB), !REF && (P == 2 || P == 3) ? 4 : 2) void k_build(
     MeshDev m, double alpha, double theta, double* __restrict__ K, double* __restrict__ A, double* __restrict__ M,
     double* __restrict__ Mm, int n_poly) {
   using D = Dims<P>;
-  using B = Build<P>;
+  using B = Build<P, ONE>;
   constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2, QC = B::QC, GP = B::GP, TG = B::TG,
                 PAIRS = B::PAIRS;
   constexpr bool XCHG = REF && B::SPLIT == 1;  // the transposed pair's term is in this workgroup

@@ -1104,3 +1104,23 @@ def test_receivers_on_both_sides_of_the_wave_limit(p):
         assert np.array_equal(many[:4096], few)
         ref = o.eval_points(pts[::97], tets[::97], u)
         assert rel(many[::97], ref) < 1e-13
+
+
+@pytest.mark.parametrize("n,size", [(3, (150, 200)), (6, (300, 600)), (11, None), (10, None)])
+def test_p1_build_of_few_large_and_of_many_small_polyhedra(n, size):
+    """One polyhedron a wave (fewer than 1,024) and four (1,331 of 6 tets): every
+    block against the oracle's to 1e-13, both orders of the build."""
+    say(f"[p=1 build] {n}^3 {size}")
+    m = M.cube_mesh(n, poly_size=size, seed=1) if size else M.cube_mesh(n, agglomerate=True)
+    o = oracle_for(m, 1)
+    o.build_operator()
+    oK, oA, oM = o.K(), o.Adg(), o.mass()[0]
+    for build in ("reference", "factored"):
+        with L.Context(m, 1) as ctx:
+            ctx.set_build(build)
+            ctx.make_matrices_free()
+            K, A, Mb, _ = ctx.export_operator()
+            s = np.abs(oK).max(axis=(1, 2))
+            assert (np.abs(K - oK).max(axis=(1, 2)) < 1e-13 * s).all()
+            assert (np.abs(A - oA).max(axis=(1, 2)) < 1e-13 * np.maximum(np.abs(oA).max(axis=(1, 2)), 1e-300)).all()
+            assert rel(Mb, oM) < 1e-13
