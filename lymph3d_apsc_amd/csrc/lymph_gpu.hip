@@ -1045,6 +1045,20 @@ int errors_dev(LymphCtx* c, const double* uh, const double* ue, double* l2sq, do
   return 0;
 }
 
+// launches of k_rhs and k_project
+template <int P, class... A>
+void run_rhs(LymphCtx* c, A... a) {
+  if constexpr (P == 1)
+    if (c->n_poly >= kRhsWave) return (void)k_rhs<1, 64><<<c->n_poly, 64, 0, c->stream>>>(c->md, a...);
+  k_rhs<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, a...);
+}
+template <int P, class... A>
+void run_project(LymphCtx* c, A... a) {
+  if constexpr (P == 1)
+    if (c->n_poly >= kRhsWave) return (void)k_project<1, 64><<<c->n_poly, 64, 0, c->stream>>>(c->md, a...);
+  k_project<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, a...);
+}
+
 // zeros into a vector by a kernel (a fill of hipMemsetAsync recorded into a
 // captured solve is not replayed reliably)
 int fill_zero(LymphCtx* c, double* v) {
@@ -1060,7 +1074,7 @@ int project_field(LymphCtx* c, int fn, double* v) {
   if (fn == LYMPH_FN_ZERO) return fill_zero(c, v);
   return dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    k_project<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, fn, c->RMm, v, nullptr);
+    run_project<P>(c, fn, c->RMm, v, nullptr);
     return check_launch("k_project");
   });
 }
@@ -1523,8 +1537,7 @@ int lymph_build_rhs(LymphCtx* c, int problem, int slot, double* rhs_out) {
   else
     rc = dispatch_p(c->p, [&](auto pc) -> int {
       constexpr int P = decltype(pc)::value;
-      k_rhs<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, problem, c->alpha, c->theta, c->slot[slot],
-                                                              nullptr, nullptr);
+      run_rhs<P>(c, problem, c->alpha, c->theta, c->slot[slot], nullptr, nullptr);
       return check_launch("k_rhs");
     });
   if (rc) return rc;
@@ -1567,7 +1580,7 @@ int lymph_project_fn(LymphCtx* c, lymph_field_fn fld, void* user, int slot, doub
   HIP_TRY_OR(hipMemcpy(dv, tv.data(), 3 * nv * sizeof(double), hipMemcpyHostToDevice), done);
   rc = dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    k_project<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, LYMPH_FN_ZERO, c->RMm, c->slot[slot], dv);
+    run_project<P>(c, LYMPH_FN_ZERO, c->RMm, c->slot[slot], dv);
     return check_launch("k_project");
   });
   if (rc) return done(rc);
@@ -1653,8 +1666,7 @@ int lymph_build_rhs_fn(LymphCtx* c, lymph_forcing_fn f, lymph_dirichlet_fn gd, l
   HIP_TRY_OR(hipMemcpy(df, tf.data(), 3 * nf * sizeof(double), hipMemcpyHostToDevice), done);
   rc = dispatch_p(c->p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
-    k_rhs<P><<<c->n_poly, rhs_threads<P>(), 0, c->stream>>>(c->md, LYMPH_PROB_NULL, c->alpha, c->theta,
-                                                c->slot[slot], dv, df);
+    run_rhs<P>(c, LYMPH_PROB_NULL, c->alpha, c->theta, c->slot[slot], dv, df);
     return check_launch("k_rhs");
   });
   if (rc) return done(rc);

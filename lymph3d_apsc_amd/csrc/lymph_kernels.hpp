@@ -739,15 +739,40 @@ __global__ __launch_bounds__(64) void k_cholesky(const double* __restrict__ M,
 // -> 0.88 ms, projection 0.98 -> 0.56 ms.
 // ---------------------------------------------------------------------------
 template <int P>
-constexpr int rhs_threads() { return P == 1 ? 64 : (P == 2 ? 128 : 256); }
+constexpr int rhs_threads() { return P <= 2 ? 128 : 256; }
+// p = 1: from so many polyhedra on the chip is full and one wave a polyhedron
+// does; below, a second one shortens the walk over a polyhedron's tets.  us of a
+// right-hand side with 64 / 128 threads: 22 polyhedra of 300 to 600 tets 3019 /
+// 2641, 2,338 of 4 to 40 341 / 303, 1,728 of 6 80 / 77; 3,524 of 50 to 100 1015 /
+// 1182, 4,096 of 6 128 / 149.
+constexpr int kRhsWave = 2560;
+// NQ points' data(q) and 3 NQ one-dimensional values tab(i) over a workgroup: the
+// data on the first wave, the values on the others where there are (one wave
+// would run the two one after the other) and the data fit one, or else all in a
+// row
+template <int NQ, int TPB, class Data, class Tab>
+__device__ __forceinline__ void data_and_tabs(int tid, Data&& data, Tab&& tab) {
+  if constexpr (NQ < 64 && TPB > 64) {
+    if (tid < 64) {
+      if (tid < NQ) data(tid);
+    } else {
+      for (int i = tid - 64; i < 3 * NQ; i += TPB - 64) tab(i);
+    }
+  } else {
+    for (int i = tid; i < 4 * NQ; i += TPB) {
+      if (i < NQ) data(i);
+      else tab(i - NQ);
+    }
+  }
+}
 
-template <int P>
-__global__ __launch_bounds__(rhs_threads<P>(), 4) void k_rhs(MeshDev m, int prob, double alpha, double theta,
+template <int P, int TPB = rhs_threads<P>()>
+__global__ __launch_bounds__(TPB, 4) void k_rhs(MeshDev m, int prob, double alpha, double theta,
                                              double* __restrict__ rhs,
                                              const double* __restrict__ tabv = nullptr,
                                              const double* __restrict__ tabf = nullptr) {
   using D = Dims<P>;
-  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2, TPB = rhs_threads<P>();
+  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, NQ2 = D::NQ2;
   constexpr int VOLSZ = NP * NQ3, FACESZ = 4 * NP * NQ2;
   union Tabs {
     Tab1<P, NQ3> vol;
@@ -773,25 +798,26 @@ __global__ __launch_bounds__(rhs_threads<P>(), 4) void k_rhs(MeshDev m, int prob
     const double aJ = fabs(Jdet);
     const double rho = m.rho[t], lam = m.lam[t], mu = m.mu[t];
     __syncthreads();
-    for (int i = tid; i < 4 * NQ3; i += TPB) {
-      if (i < NQ3) {  // the data, times the weight
-        double val[3];
-        if (tabv) {  // values of the caller's forcing at k_rhs_points' volume points
-          for (int c = 0; c < 3; ++c) val[c] = tabv[((size_t)t * NQ3 + i) * 3 + c];
-        } else {
-          double x[3];
-          map_point(Fk, &m.qtet[i * 4], x);
-          forcing(prob, lam, mu, x, rho, val);
-        }
-        const double aw = aJ * m.wtet[i];
-        for (int c = 0; c < 3; ++c) sval[i * 3 + c] = aw * val[c];
-      } else {
-        const int d = i / NQ3 - 1, q = i % NQ3;
-        double rw[4];
-        affine_row(vt, d, rw);
-        tab1d<P, NQ3>(t1.vol, d, q, map_coord(rw, &m.qtet[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
-      }
-    }
+    data_and_tabs<NQ3, TPB>(
+        tid,
+        [&](int i) {  // the data, times the weight
+          double val[3];
+          if (tabv) {  // values of the caller's forcing at k_rhs_points' volume points
+            for (int c = 0; c < 3; ++c) val[c] = tabv[((size_t)t * NQ3 + i) * 3 + c];
+          } else {
+            double x[3];
+            map_point(Fk, &m.qtet[i * 4], x);
+            forcing(prob, lam, mu, x, rho, val);
+          }
+          const double aw = aJ * m.wtet[i];
+          for (int c = 0; c < 3; ++c) sval[i * 3 + c] = aw * val[c];
+        },
+        [&](int i) {
+          const int d = i / NQ3, q = i % NQ3;
+          double rw[4];
+          affine_row(vt, d, rw);
+          tab1d<P, NQ3>(t1.vol, d, q, map_coord(rw, &m.qtet[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
+        });
     __syncthreads();
     for (int e = tid; e < NP * NQ3; e += TPB) {
       const int q = e / NP, f = e % NP;
@@ -810,23 +836,24 @@ __global__ __launch_bounds__(rhs_threads<P>(), 4) void k_rhs(MeshDev m, int prob
       __syncthreads();
       const double* nrm = &m.normal[(t * 4 + f) * 3];
       const int tag = m.bc_space[t * 4 + f];
-      for (int i = tid; i < 4 * NQ2; i += TPB) {
-        if (i < NQ2) {
-          if (tabf) {  // the caller's Dirichlet / Neumann data at k_rhs_points' face points
-            for (int c = 0; c < 3; ++c) sval[i * 3 + c] = tabf[(((size_t)t * 4 + f) * NQ2 + i) * 3 + c];
-          } else {
-            double xr[3];
-            face_point_rhs(Fk, f, &m.qtri[i * 4], xr);
-            if (e2 == -1) dirichlet(prob, xr, tag, &sval[i * 3]);
-            else neumann(prob, lam, mu, nrm, xr, tag, &sval[i * 3]);
-          }
-        } else {
-          const int d = i / NQ2 - 1, q = i % NQ2;
-          double rw[4];
-          affine_row(vt, d, rw);
-          tab1d<P, NQ2>(t1.face, d, q, face_coord(rw, f, &m.qtri[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
-        }
-      }
+      data_and_tabs<NQ2, TPB>(
+          tid,
+          [&](int i) {
+            if (tabf) {  // the caller's Dirichlet / Neumann data at k_rhs_points' face points
+              for (int c = 0; c < 3; ++c) sval[i * 3 + c] = tabf[(((size_t)t * 4 + f) * NQ2 + i) * 3 + c];
+            } else {
+              double xr[3];
+              face_point_rhs(Fk, f, &m.qtri[i * 4], xr);
+              if (e2 == -1) dirichlet(prob, xr, tag, &sval[i * 3]);
+              else neumann(prob, lam, mu, nrm, xr, tag, &sval[i * 3]);
+            }
+          },
+          [&](int i) {
+            const int d = i / NQ2, q = i % NQ2;
+            double rw[4];
+            affine_row(vt, d, rw);
+            tab1d<P, NQ2>(t1.face, d, q, face_coord(rw, f, &m.qtri[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
+          });
       __syncthreads();
       constexpr int SG = NP * NQ2;
       for (int e = tid; e < SG; e += TPB) {
@@ -1112,12 +1139,12 @@ __device__ __forceinline__ void back_ascending(const double* __restrict__ R, dou
   }
 }
 
-template <int P>
-__global__ __launch_bounds__(rhs_threads<P>(), 4) void k_project(MeshDev m, int fn, const double* __restrict__ RMm,
+template <int P, int TPB = rhs_threads<P>()>
+__global__ __launch_bounds__(TPB, 4) void k_project(MeshDev m, int fn, const double* __restrict__ RMm,
                                                  double* __restrict__ out,
                                                  const double* __restrict__ tabv) {
   using D = Dims<P>;
-  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3, TPB = rhs_threads<P>();
+  constexpr int NP = D::NP, N3 = D::N3, NQ3 = D::NQ3;
   __shared__ double phi[NP * NQ3];
   __shared__ Tab1<P, NQ3> t1;
   __shared__ double sval[NQ3 * 3];
@@ -1139,25 +1166,26 @@ __global__ __launch_bounds__(rhs_threads<P>(), 4) void k_project(MeshDev m, int 
     affine_map(v, Fk, Jdet);
     const double aJ = fabs(Jdet);
     __syncthreads();
-    for (int i = tid; i < 4 * NQ3; i += TPB) {
-      if (i < NQ3) {  // the field, times the weight
-        double val[3];
-        if (tabv) {  // the caller's field at k_rhs_points' volume points
-          for (int c = 0; c < 3; ++c) val[c] = tabv[((size_t)t * NQ3 + i) * 3 + c];
-        } else {
-          double x[3];
-          map_point(Fk, &m.qtet[i * 4], x);
-          field(fn, x, val);
-        }
-        const double aw = aJ * m.wtet[i];
-        for (int c = 0; c < 3; ++c) sval[i * 3 + c] = aw * val[c];
-      } else {
-        const int d = i / NQ3 - 1, q = i % NQ3;
-        double rw[4];
-        affine_row(vt, d, rw);
-        tab1d<P, NQ3>(t1, d, q, map_coord(rw, &m.qtet[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
-      }
-    }
+    data_and_tabs<NQ3, TPB>(
+        tid,
+        [&](int i) {  // the field, times the weight
+          double val[3];
+          if (tabv) {  // the caller's field at k_rhs_points' volume points
+            for (int c = 0; c < 3; ++c) val[c] = tabv[((size_t)t * NQ3 + i) * 3 + c];
+          } else {
+            double x[3];
+            map_point(Fk, &m.qtet[i * 4], x);
+            field(fn, x, val);
+          }
+          const double aw = aJ * m.wtet[i];
+          for (int c = 0; c < 3; ++c) sval[i * 3 + c] = aw * val[c];
+        },
+        [&](int i) {
+          const int d = i / NQ3, q = i % NQ3;
+          double rw[4];
+          affine_row(vt, d, rw);
+          tab1d<P, NQ3>(t1, d, q, map_coord(rw, &m.qtet[q * 4]), bbP[2 * d], bbP[2 * d + 1]);
+        });
     __syncthreads();
     for (int e = tid; e < NP * NQ3; e += TPB) {
       const int q = e / NP, f = e % NP;

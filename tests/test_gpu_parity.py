@@ -1124,3 +1124,19 @@ def test_p1_build_of_few_large_and_of_many_small_polyhedra(n, size):
             assert (np.abs(K - oK).max(axis=(1, 2)) < 1e-13 * s).all()
             assert (np.abs(A - oA).max(axis=(1, 2)) < 1e-13 * np.maximum(np.abs(oA).max(axis=(1, 2)), 1e-300)).all()
             assert rel(Mb, oM) < 1e-13
+
+
+@pytest.mark.parametrize("n,size", [(13, None), (14, None), (6, (300, 600))])
+def test_p1_data_of_few_and_of_many_polyhedra(n, size):
+    """p = 1 right-hand sides and projections with two waves a polyhedron (fewer
+    than 2,560) and one (2,744), against the oracle."""
+    say(f"[p=1 data] {n}^3 {size}")
+    m = M.cube_mesh(n, poly_size=size, seed=1) if size else M.cube_mesh(n, agglomerate=True)
+    o = oracle_for(m, 1)
+    o.build_operator()
+    with L.Context(m, 1) as ctx:
+        ctx.make_matrices_free()
+        for prob in (L.PROB_REF_MMS, L.PROB_CUBE_WAVE):
+            assert rel(ctx.make_rhs_free(prob), o.rhs(prob)) < 1e-13, prob
+        for fn in (_lib.FN_REF_VEL, _lib.FN_CUBE_U):
+            assert rel(ctx.compute_modal_coefficients_free(fn, _lib.SLOT_U_CUR), o.project(fn)) < 1e-13, fn
