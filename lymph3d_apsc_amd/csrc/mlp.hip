@@ -548,7 +548,7 @@ struct LayerArgs {
   const bf16_t* W;     // packed [N][K]
   const bf16_t* in;    // packed [rows][K]; null: rows idx[b] of X
   const float* X;
-  const int* idx;
+  const int* idx;      // null: rows 0, 1, ...
   bf16_t* XT;          // X's rows in bf16, transposed and packed [K][rows]
   const float* bias;   // forward
   bf16_t* out;         // packed [rows][N]: gelu(z), dY or dZ
@@ -639,7 +639,7 @@ __device__ __forceinline__ void layer_tile(const LayerArgs& g, int wg) {
         const int k = st * 32 + (lane >> 4) * 8;
         uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
         if (row < g.B && k < g.K) {
-          const float* x = g.X + (size_t)g.idx[row] * g.K + k;
+          const float* x = g.X + (size_t)(g.idx ? g.idx[row] : row) * g.K + k;
           const float4 a = *reinterpret_cast<const float4*>(x), b = *reinterpret_cast<const float4*>(x + 4);
           v[0] = f2bf(a.x); v[1] = f2bf(a.y); v[2] = f2bf(a.z); v[3] = f2bf(a.w);
           v[4] = f2bf(b.x); v[5] = f2bf(b.y); v[6] = f2bf(b.z); v[7] = f2bf(b.w);
@@ -1471,6 +1471,19 @@ int upload_rows(const LymphMlp* m, int pass) {
   return std::max(pass, (int)((16u << 20) / (unsigned)m->w[0]) / pass * pass);
 }
 
+// Whether a forward pass of up to 32 rows takes a launch per layer, through the
+// training's buffers (which hold whole tiles of max_batch rows): in a slab a
+// single CU pulls every layer's weights in turn, which past about 300 KB a layer
+// takes longer than the launches.  us of a pass, slab / launches (the GEMMs), 1
+// row: nine layers of 512 77 / 39 (57), sixteen 136 / 64 (100), six of 512 42 / 28
+// (39), 32-512x5-64 36 / 22 (35); eight of 384 (288 KB each) 39 by the slab (42).
+bool few_rows_by_layer(const LymphMlp* m, int n, int layers) {
+  if (n > 32 || tiles_of(n) > tiles_of(m->max_batch) || layers < 2) return false;
+  size_t bytes = 0;
+  for (int l = 0; l < layers; ++l) bytes += pack_size(m->w[l + 1], m->w[l]) * sizeof(bf16_t);
+  return bytes > (size_t)layers * 300 * 1024;
+}
+
 // Outputs of n <= chunk_rows() rows (device).  16 rows a slab until every CU
 // has one (4096 rows), then 32: the weights are read once per slab, and two
 // slabs of 32 fit a CU's registers.  A wide output layer takes the slabs'
@@ -1486,6 +1499,26 @@ int slab_forward(LymphMlp* m, int n, const float* X, float* Y) {
     a.bias[l] = m->P + m->boff[l];
   }
   a.X = X;
+  if (few_rows_by_layer(m, n, a.L)) {
+    for (int l = 0; l < m->L; ++l) {
+      LayerArgs o{};
+      o.N = m->w[l + 1]; o.K = m->w[l]; o.B = n; o.ts = steps_of(m->max_batch);
+      o.W = m->Wf[l]; o.in = m->HP[l]; o.bias = m->P + m->boff[l];
+      o.X = X; o.XT = m->HT[0]; o.Y = Y;
+      const unsigned wgs = (unsigned)layer_wgs(o.N, n);
+      if (l + 1 < m->L) {
+        o.out = m->HP[l + 1]; o.outT = m->HT[l + 1]; o.dg = m->dg[l];
+        if (l == 0) k_layer<LAYER_FWD, true><<<wgs, 128, 0, m->stream>>>(o);
+        else k_layer<LAYER_FWD, false><<<wgs, 128, 0, m->stream>>>(o);
+      } else if (m->wide) {
+        launch_wide<LAYER_OUT>(m, o);
+      } else {
+        k_layer<LAYER_OUT, false><<<wgs, 128, 0, m->stream>>>(o);
+      }
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : fail(LYMPH_MLP_ERR_HIP, std::string("k_layer: ") + hipGetErrorString(e));
+  }
   if (m->wide) {
     const size_t need = pack_size((n + 31) / 32 * 32, a.w[a.L]);
     if (need > m->hp_cap) {  // zeros: the padding of the last step is never written

@@ -217,3 +217,28 @@ def test_predict_in_pieces_of_a_large_batch_gives_the_bits_of_small_calls():
             assert np.array_equal(small.predict(x[a:a + 1000]), y[a:a + 1000]), a
         y_ref, _ = R.forward(net.params().astype(np.float64), widths, x[2290:2320], emulate=True)
         assert rel(y[2290:2320], y_ref) < 5e-3
+
+
+@pytest.mark.parametrize("widths,max_batch", [([512, 512, 512], 8), ([24, 512, 488, 512, 40], 24), ([8, 512, 512, 512, 1032], 64),
+                                              ([136, 504, 512, 8], 32)])
+def test_predictions_of_few_rows_by_layers_give_the_bits_of_the_slab(widths, max_batch):
+    """Up to 32 rows (of the batch's whole tiles) of a network with large layers
+    go a launch per layer, more rows in slabs: the same bits, also between
+    training steps, whose buffers they pass through."""
+    from lymph3d_apsc_amd.mlp import Mlp
+    say(f"[mlp few rows] {widths} {max_batch}")
+    rng = np.random.default_rng(max_batch)
+    x = rng.standard_normal((100, widths[0])).astype(np.float32)
+    t = rng.standard_normal((100, widths[-1])).astype(np.float32)
+    with Mlp(widths, max_batch=max_batch, seed=8) as net, Mlp(widths, max_batch=max_batch, seed=8) as other:
+        for m in (net, other):
+            m.set_data(x, t)
+        for step in range(3):
+            y = net.predict(x)
+            for n in (1, 7, 8, 16, 17, 31, 32, 33):
+                assert np.array_equal(net.predict(x[:n]), y[:n]), n
+            y_ref, _ = R.forward(net.params().astype(np.float64), widths, x[:16], emulate=True)
+            assert rel(y[:16], y_ref) < 5e-3
+            order = rng.integers(0, 100, 8).astype(np.int32)
+            assert np.array_equal(net.train(order, 8, 1e-3), other.train(order, 8, 1e-3))
+            assert np.array_equal(net.params(), other.params())
