@@ -1235,14 +1235,37 @@ __global__ __launch_bounds__(256) void k_rows(const float* __restrict__ X, const
         *reinterpret_cast<const uint4*>(s + k * LDR + r0);
 }
 
-// bf16 copies of W [N][K] in both fragment orders
-__global__ void k_pack(const float* __restrict__ W, int N, int K, bf16_t* __restrict__ Wf, bf16_t* __restrict__ Wd) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * K) return;
-  const int n = (int)(i / K), k = (int)(i % K);
-  const bf16_t h = f2bf(W[i]);
-  if (Wf) Wf[pack_pos(n, k, steps_of(K))] = h;
-  if (Wd) Wd[pack_pos(k, n, steps_of(N))] = h;
+// bf16 copies of every layer's W [N][K] in both fragment orders, a lane's 16
+// bytes of a fragment per thread, Wf's fragments first; all layers in one launch
+// (with one each and 2-byte stores 32-512x5-64's parameters took 20 us longer)
+struct PackLayer {
+  const float* W;
+  int N, K;
+  bf16_t *Wf, *Wd;    // Wd: null for the first layer
+  unsigned first;     // workgroup
+};
+struct PackArgs {
+  int L;
+  PackLayer y[kSlabL];
+};
+__global__ __launch_bounds__(256) void k_pack(PackArgs p) {
+  int l = p.L - 1;
+  while (blockIdx.x < p.y[l].first) --l;
+  const PackLayer& y = p.y[l];
+  const size_t nf = (size_t)tiles_of(y.N) * steps_of(y.K) * 64, nd = (size_t)tiles_of(y.K) * steps_of(y.N) * 64;
+  size_t i = (size_t)(blockIdx.x - y.first) * 256 + threadIdx.x;
+  if (i >= nf + (y.Wd ? nd : 0)) return;
+  const bool f = i < nf;
+  if (!f) i -= nf;
+  // row r of the packed matrix, columns c..c + 7: W's row r, or its column r
+  const int steps = steps_of(f ? y.K : y.N), lane = (int)(i & 63);
+  const int r = (int)(i / 64 / steps) * 16 + (lane & 15), c = (int)(i / 64 % steps) * 32 + (lane >> 4) * 8;
+  uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+  if (r < (f ? y.N : y.K) && c < (f ? y.K : y.N))  // widths are multiples of 8
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = f2bf(f ? y.W[(size_t)r * y.K + c + q] : y.W[(size_t)(c + q) * y.K + r]);
+  *reinterpret_cast<uint4*>((f ? y.Wf : y.Wd) + i * 8) =
+      make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
 }
 
 unsigned blocks(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
@@ -1815,9 +1838,16 @@ int lymph_mlp_set_params(LymphMlp* m, const float* p) {
   if (!p) return fail(LYMPH_MLP_ERR_ARG, "null params");
   HIP_TRY(hipMemcpyAsync(m->P, p, m->n_params * 4, hipMemcpyHostToDevice, m->stream));
   if (m->slab) {
-    for (int l = 0; l < m->L; ++l)
-      k_pack<<<blocks((size_t)m->w[l + 1] * m->w[l], 256), 256, 0, m->stream>>>(m->P + m->woff[l], m->w[l + 1],
-                                                                                m->w[l], m->Wf[l], m->Wd[l]);
+    PackArgs p{};
+    p.L = m->L;
+    unsigned wgs = 0;
+    for (int l = 0; l < m->L; ++l) {
+      const int N = m->w[l + 1], K = m->w[l];
+      p.y[l] = {m->P + m->woff[l], N, K, m->Wf[l], m->Wd[l], wgs};
+      const size_t nf = (size_t)tiles_of(N) * steps_of(K), nd = (size_t)tiles_of(K) * steps_of(N);
+      wgs += blocks((nf + (m->Wd[l] ? nd : 0)) * 64, 256);
+    }
+    k_pack<<<wgs, 256, 0, m->stream>>>(p);
   } else {
     k_to_bf16<<<blocks(m->n_params, 256), 256, 0, m->stream>>>(m->P, m->Wb, m->n_params);
   }
