@@ -149,10 +149,11 @@ def test_wide_update_with_streamed_masters_matches_oracle():
 
 
 def free_bytes():
-    """Free device memory, from the HIP runtime that the libraries loaded."""
+    """Free device memory, from the HIP runtime that liblymph_mlp.so is linked to
+    (found through its handle; the process may hold another one)."""
     import ctypes as C
-    with open("/proc/self/maps") as f:
-        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    from lymph3d_apsc_amd import mlp
+    hip = mlp.lib()
     free, total = C.c_size_t(), C.c_size_t()
     assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
     return free.value
