@@ -967,12 +967,12 @@ __device__ __forceinline__ double quot(double a, const Divisor& d) {
 }
 // Numerators whose quotients by a plain divisor are exact above: the quotient
 // stays within 2^-960 and 2^1000, the last bit of the remainder (2^-106 of the
-// numerator) above the smallest subnormal; zeros, infinities and NaN pass.  The
-// solves test the numerators that they used once at their end and divide if one
-// fails: in a wave front's first trace, or next to overflow.
+// numerator) above the smallest subnormal.  The solves test the numerators that
+// they used once at their end and divide if one fails: in a wave front's first
+// trace, next to overflow, or with infinities and NaN.
 __device__ __forceinline__ bool quotable(double a) {
   const double m = fabs(a);
-  return (m >= 0x1p-860 && m <= 0x1p900) || m == 0.0 || !(m < __builtin_inf());
+  return (m >= 0x1p-860 && m <= 0x1p900) || m == 0.0;
 }
 
 // M^-1 w = R^-1 R^-T w (solve_LU with L = R^T, src/vet_mat_operations.f90:
@@ -982,35 +982,31 @@ __device__ __forceinline__ bool quotable(double a) {
 // subtract R_ji y_j, in ascending j as the reference does; the backward sweep
 // runs the columns from the last, the rows above subtracting R_ij x_j.  NP
 // dependent steps per sweep instead of Np(Np+1)/2 on one lane.  A lane past its
-// own step goes on with values that nothing reads, which keeps the selects off
-// the chain.  The solves are the tail of a step on few polyhedra: with divisions
+// own step goes on, subtracting zeros (R[NPK] is one), so that it keeps its
+// numerator and the selects stay off the chain.  The solves are the tail of a step on few polyhedra: with divisions
 // and selects on the chain 162 single-tet polyhedra took 6.2, 10.4 and 30.9 us
-// a step at p = 2, 3, 4, now 5.2, 8.6 and 22.7.
+// a step at p = 2, 3, 4, now 5.2, 7.3 and 23.5.
 template <int NP, bool PLAIN>
 __device__ __forceinline__ double solve_group_as(const double* __restrict__ R, const Divisor& d, double w, int ii,
                                                  int from, bool& ok) {
-  double y = 0.0, af = 0.0, ab = 0.0;  // the lane's results and numerators
+  constexpr int ZERO = NP * (NP + 1) / 2;
+  double y = 0.0;
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const double t = PLAIN ? quot(w, d) : w / d.b;
-    if (ii == j) {
-      y = t;
-      af = w;
-    }
-    w = w - R[pk_off(NP, j) + (ii > j ? ii - j : 0)] * __shfl(t, from + j, 64);
+    if (ii == j) y = t;
+    w = w - R[ii > j ? pk_off(NP, j) + ii - j : ZERO] * __shfl(t, from + j, 64);
   }
+  ok = !PLAIN || quotable(w);
   const int ri = pk_off(NP, ii);
   w = y;
 #pragma unroll
   for (int j = NP - 1; j >= 0; --j) {
     const double t = PLAIN ? quot(w, d) : w / d.b;
-    if (ii == j) {
-      y = t;
-      ab = w;
-    }
-    w = w - R[ri + (ii < j ? j - ii : 0)] * __shfl(t, from + j, 64);
+    if (ii == j) y = t;
+    w = w - R[ii < j ? ri + j - ii : ZERO] * __shfl(t, from + j, 64);
   }
-  ok = !PLAIN || (quotable(af) && quotable(ab));
+  ok = ok && (!PLAIN || quotable(w));
   return y;
 }
 template <int NP>
@@ -1054,24 +1050,23 @@ __device__ __forceinline__ void forward_rows(const double* __restrict__ R, doubl
 // Broadcasts by v_readlane (24.2 us above with __shfl).
 template <int NP, bool PLAIN>
 __device__ __forceinline__ bool back_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
-  double y[3] = {0.0, 0.0, 0.0}, a[3] = {0.0, 0.0, 0.0};  // the lane's results and numerators
+  constexpr int ZERO = NP * (NP + 1) / 2;
+  double y[3] = {0.0, 0.0, 0.0};
   const int ri = pk_off(NP, i < NP ? i : 0);
 #pragma unroll 5
   for (int j = NP - 1; j >= 0; --j) {
-    const double r = R[ri + (i < NP && i < j ? j - i : 0)];
+    const double r = R[i < j ? ri + j - i : ZERO];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
-      if (i == j) {
-        y[c] = t;
-        a[c] = x[c];
-      }
+      if (i == j) y[c] = t;
       x[c] = x[c] - r * lane_bcast(t, j);
     }
   }
+  const bool ok = !PLAIN || i >= NP || (quotable(x[0]) && quotable(x[1]) && quotable(x[2]));
 #pragma unroll
   for (int c = 0; c < 3; ++c) x[c] = y[c];
-  return !PLAIN || (quotable(a[0]) && quotable(a[1]) && quotable(a[2]));
+  return ok;
 }
 template <int NP>
 __device__ __forceinline__ void back_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
@@ -1090,24 +1085,22 @@ __device__ __forceinline__ void back_rows(const double* __restrict__ R, const Di
 // M^-1: both sweeps
 template <int NP, bool PLAIN>
 __device__ __forceinline__ bool solve_rows_as(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
-  double y[3] = {0.0, 0.0, 0.0}, a[3] = {0.0, 0.0, 0.0};
+  constexpr int ZERO = NP * (NP + 1) / 2;
+  double y[3] = {0.0, 0.0, 0.0};
 #pragma unroll 5
   for (int j = 0; j < NP; ++j) {
-    const double r = R[pk_off(NP, j) + (i < NP && i > j ? i - j : 0)];
+    const double r = R[i < NP && i > j ? pk_off(NP, j) + i - j : ZERO];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double t = PLAIN ? quot(x[c], d) : x[c] / d.b;
-      if (i == j) {
-        y[c] = t;
-        a[c] = x[c];
-      }
+      if (i == j) y[c] = t;
       x[c] = x[c] - r * lane_bcast(t, j);
     }
   }
+  const bool ok = !PLAIN || i >= NP || (quotable(x[0]) && quotable(x[1]) && quotable(x[2]));
 #pragma unroll
   for (int c = 0; c < 3; ++c) x[c] = y[c];
-  const bool ok = back_rows_as<NP, PLAIN>(R, d, x, i);
-  return ok && (!PLAIN || (quotable(a[0]) && quotable(a[1]) && quotable(a[2])));
+  return back_rows_as<NP, PLAIN>(R, d, x, i) && ok;
 }
 template <int NP>
 __device__ __forceinline__ void solve_rows(const double* __restrict__ R, const Divisor& d, double (&x)[3], int i) {
@@ -1291,18 +1284,18 @@ __global__ __launch_bounds__(64 * WPP) void k_leapfrog(const double* __restrict_
                                                  double* __restrict__ out, double g, double c1,
                                                  double c2, const int* __restrict__ gsel,
                                                  const double* __restrict__ gtab, int n_poly,
-    const int* __restrict__ order) {
+                                                 const int* __restrict__ order) {
   using D = Dims<P>;
   constexpr int NP = D::NP, N3 = D::N3, NPAIR = D::NPAIR;
   constexpr int RPL = (N3 + 63) / 64;
   __shared__ double sw[N3];
-  __shared__ double sR[D::NPK];
+  __shared__ double sR[D::NPK + 1];  // the factor and a zero
   extern __shared__ double sblk[];  // WPP > 1: per-block products [block][row]
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int Pp = step_poly(order);
   if (Pp >= n_poly) return;  // padding workgroups of the last XCD share
   if (MODE != 2)
-    for (int k = threadIdx.x; k < D::NPK; k += 64 * WPP) sR[k] = Rp[(size_t)Pp * D::NPK + k];
+    for (int k = threadIdx.x; k <= D::NPK; k += 64 * WPP) sR[k] = k < D::NPK ? Rp[(size_t)Pp * D::NPK + k] : 0.0;
   StepEnds<N3, RPL> ends;
   const int drow = RPL == 1 ? (lane < N3 ? lane % NP : 0) : (lane < NP ? lane : 0);  // the lane's row in the solve
   Divisor diag(1.0);
@@ -2143,20 +2136,20 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_packed(const void* __rest
   // neighbour coefficients, double-buffered by block parity: one barrier per block
   __shared__ double sxa[WPW][2][G][N3 + 1];
   __shared__ double swa[WPW][G][N3];
-  __shared__ double sRa[WPW][G][D::NPK];
+  __shared__ double sRa[WPW][G][D::NPK + 1];  // the factors, each and a zero
   const int wv = threadIdx.x >> 6;
   double(&sx)[2][G][N3 + 1] = sxa[wv];
   double(&sw)[G][N3] = swa[wv];
-  double(&sR)[G][D::NPK] = sRa[wv];
+  double(&sR)[G][D::NPK + 1] = sRa[wv];
   const int lane = threadIdx.x & 63;
   const int sub = lane / N3, r = lane % N3;
   const int P0 = (step_poly() * WPW + wv) * G;
   const int Pp = P0 + sub;
   const bool act = sub < G && Pp < n_poly;
   if (MODE != 2 && TB == 64)
-    for (int k = lane; k < G * D::NPK; k += 64) {
-      const int sp = k / D::NPK, e = k % D::NPK, Q = P0 + sp;
-      if (Q < n_poly) sR[sp][e] = Rp[(size_t)Q * D::NPK + e];
+    for (int k = lane; k < G * (D::NPK + 1); k += 64) {
+      const int sp = k / (D::NPK + 1), e = k % (D::NPK + 1), Q = P0 + sp;
+      if (Q < n_poly) sR[sp][e] = e < D::NPK ? Rp[(size_t)Q * D::NPK + e] : 0.0;
     }
   const int b0 = act ? row_ptr[Pp] : 0, cnt = act ? row_ptr[Pp + 1] - b0 : 0;
   double xn = cnt > 0 ? u[(size_t)col[b0] * N3 + r] : 0.0;  // neighbour value of the next block
@@ -2322,11 +2315,11 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restr
   constexpr int NQUAD = Dims32<P>::NQ, TAIL = Dims32<P>::T;
   __shared__ double sxa[WPW][2][G][N3 + 1];
   __shared__ double swa[WPW][G][N3];
-  __shared__ double sRa[WPW][G][D::NPK];
+  __shared__ double sRa[WPW][G][D::NPK + 1];  // the factors, each and a zero
   const int wv = threadIdx.x >> 6;
   double(&sx)[2][G][N3 + 1] = sxa[wv];
   double(&sw)[G][N3] = swa[wv];
-  double(&sR)[G][D::NPK] = sRa[wv];
+  double(&sR)[G][D::NPK + 1] = sRa[wv];
   extern __shared__ double prod_all[];  // per wave: [block - B0][row]
   const int lane = threadIdx.x & 63;
   const int sub = lane / N3, r = lane % N3;
@@ -2334,9 +2327,9 @@ __global__ __launch_bounds__(64 * WPW) void k_leapfrog_joint(const void* __restr
   const int Pp = P0 + sub;
   const bool act = sub < G && Pp < n_poly;
   if (MODE != 2 && TB == 64)
-    for (int k = lane; k < G * D::NPK; k += 64) {
-      const int sp = k / D::NPK, e = k % D::NPK, Q = P0 + sp;
-      if (Q < n_poly) sR[sp][e] = Rp[(size_t)Q * D::NPK + e];
+    for (int k = lane; k < G * (D::NPK + 1); k += 64) {
+      const int sp = k / (D::NPK + 1), e = k % (D::NPK + 1), Q = P0 + sp;
+      if (Q < n_poly) sR[sp][e] = e < D::NPK ? Rp[(size_t)Q * D::NPK + e] : 0.0;
     }
   if (P0 >= n_poly) return;  // padding group: the wave exits before any barrier
   double* prod = prod_all + (size_t)wv * prod_stride;
@@ -2665,7 +2658,7 @@ __global__ __launch_bounds__(64) void k_tilde_back(const double* __restrict__ RM
                                                    const int* __restrict__ list, int n) {
   using D = Dims<P>;
   constexpr int NP = D::NP;
-  __shared__ double sR[D::NPK];
+  __shared__ double sR[D::NPK + 1];  // the factor and a zero
   const int w = blockIdx.x;
   if (w >= n) return;
   const int Pp = list ? list[w] : w;
@@ -2673,7 +2666,7 @@ __global__ __launch_bounds__(64) void k_tilde_back(const double* __restrict__ RM
   const bool row = i < NP;
   const double* R = RM + (size_t)Pp * D::NPK;
   const Divisor d(R[pk_off(NP, row ? i : 0)]);
-  for (int k = i; k < D::NPK; k += 64) sR[k] = R[k];
+  for (int k = i; k <= D::NPK; k += 64) sR[k] = k < D::NPK ? R[k] : 0.0;
   double x[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) x[c] = row ? in[(size_t)Pp * D::N3 + c * NP + i] : 0.0;
