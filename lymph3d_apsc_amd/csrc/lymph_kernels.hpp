@@ -247,8 +247,9 @@ __device__ __forceinline__ void basis_row(const Tab1<P, NQ>& t, int a, int b, in
 // now, reference / factored order, both operators, agglomerated cubes: p = 1
 // (64,000 polyhedra) 17.6 -> 1.3 / 7.1 -> 1.1; p = 2 (32,768) 35.9 -> 6.5 / 11.7
 // -> 4.0; p = 3 (13,824) 123 -> 20 / 29.6 -> 10.5; p = 4 (4,096) 233 -> 32 / 31
-// -> 11.  At p = 3 the reference order keeps the FP64 units 62% busy; the
-// factored one waits on LDS and barriers.
+// -> 11.  At p = 3 the reference order keeps the vector units 62% busy, 58% of
+// the time with FP64; the factored one 40%, with as many LDS instructions for a
+// quarter of the FP64 ones.
 // ---------------------------------------------------------------------------
 template <int P, bool ONE = false>
 struct Build {

@@ -1584,9 +1584,9 @@ bool wide_nt(const LymphMlp* m) {
 
 // Whether a step's input rows are packed by a launch of their own (k_rows).
 // Every column tile of the first layer otherwise gathers and converts them
-// again, which wide inputs do not hide: us per step, in the layer / apart, one
-// layer of 512 x 512 at batch 256 22 / 12, 4,096 100 / 55, 65,536 1610 / 700
-// (with the GEMMs 28, 75 and 1040); 256 x 256 at 256 15.2 / 12.2.  Inputs of at
+// again, which wide inputs do not hide: us per step, in the layer / apart (both
+// with one sum per tile of k_update), one layer of 512 x 512 at batch 256 22 /
+// 12, 4,096 100 / 55, 65,536 1610 / 700 (with the GEMMs 28, 75 and 1040); 256 x 256 at 256 15.2 / 12.2.  Inputs of at
 // most 128 cost less than the launch: 128-256x2 at batch 512 21.6 / 23.3,
 // 64-512 at 1,024 18.5 / 20.8, 32-512x5-64 at 256 56.4 / 57.4.
 bool rows_apart(const LymphMlp* m) { return m->w[0] > 128; }
