@@ -482,7 +482,6 @@ __global__ __launch_bounds__((Build<P, ONE>::TPB), !REF && (P == 2 || P == 3) ? 
       const double d11 = fabs(n1) * fabs(n1) + 0.5 * (fabs(n2) * fabs(n2)) + 0.5 * (fabs(n3) * fabs(n3));
       const double d22 = fabs(n2) * fabs(n2) + 0.5 * (fabs(n1) * fabs(n1)) + 0.5 * (fabs(n3) * fabs(n3));
       const double d33 = fabs(n3) * fabs(n3) + 0.5 * (fabs(n1) * fabs(n1)) + 0.5 * (fabs(n2) * fabs(n2));
-      const double dd[3] = {d11, d22, d33};
       for (int i = lt; i < 3 * NQ2 * (interior ? 2 : 1); i += TG) {
         const int side = i / (3 * NQ2), d = i / NQ2 % 3, q = i % NQ2;
         double r[4];
